@@ -9,13 +9,12 @@
 
 namespace sfx {
 
-constexpr int kB3Ranks = 4;     // ranks per launch at most
-constexpr int kB3TanRanks = 2;  // ranks per tangent or FP64 launch at most (that region fits two workgroups per CU)
-// ranks per launch at most of a variant
-template <typename T>
-constexpr int b3_max_ranks(bool tangent) {
-  return (tangent || sizeof(T) == 8) ? kB3TanRanks : kB3Ranks;
-}
+// ranks per launch at most. Four rather than two: a launch of the 64^3 melt
+// costs 4-6 us before and after its ranks (dispatch, the region's loads, the
+// maximum), which two ranks pay twice. FP32 tangents, two chains: 14.4 / 16.2 us
+// (forward / composing) for four ranks, 8.7 / 11.0 us for two; FP64 at 128^3:
+// 65 / 113 us against 32 / 64 us, the region read half as often.
+constexpr int kB3Ranks = 4;
 
 // Ranks s0+1 .. s0+nr of one chain, all of one segment state.
 template <typename T>
@@ -52,8 +51,7 @@ struct B3Launch {
 };
 
 // Splits chain steps a..b (ascending) into launches: a launch ends at a grid
-// line ((step - g0 + 1) % grid == 0; grid is b3_max_ranks of the variant), before a step of another segment
-// state, or before a step that split() marks. f(first, last) per launch. The
+// line ((step - g0 + 1) % grid == 0), before a step of another segment state, or before a step that split() marks. f(first, last) per launch. The
 // grid makes the partition of any stretch that starts on a grid line equal
 // to that of the whole chain, so a recomputed stretch reproduces it bit for bit.
 template <class State, class Split, class F>

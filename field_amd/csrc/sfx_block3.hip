@@ -6,18 +6,26 @@
 // direction (a lattice with bounds extends by periodic wrap or by reflection,
 // mirror1 about the face and mirror2 about the first layer, which is what the
 // per-rank halo copies of Lat3D.cpp:892-1562 amount to), then computes rank k
-// on the tile widened by nr - k, ping-ponging between two LDS buffers:
+// on the tile widened by nr - k:
 //   G_k(r) = g(r) (1/6) sum_6 G_{k-1}(r + e)            (Lat3D1stO.cpp:53-260)
 //   dG_k(r) = g(r) ((1/6) sum_6 dG_{k-1} - v(r) (1/6) sum_6 G_{k-1})
-// Every thread owns one tile site: it stores that site's value of every rank,
-// composes acc += G_k G_pair c_k (ConnectG, Lat3D1stO.cpp:299-312; tangent
-// dacc += (dG_k G_pair + G_k dG_pair) c_k) in a register with the partner
-// values prefetched at launch start, and adds it to HBM once. In FP32 the
-// widened ranks are computed four z sites per work item with float4 LDS
-// accesses (consecutive items take consecutive 16-byte words of whole rows);
-// in FP64 by (y, z) columns, several threads per column along x, consecutive
-// threads on consecutive LDS words. LDS reads are conflict-free either way,
-// and HBM accesses coalesce along z.
+// Two threads hold one (y, z) column of the widened tile, half of its x planes
+// each, in registers, with g (and v) beside them: the x neighbours are
+// registers, the y and z neighbours come from LDS, where every rank is
+// exchanged, at addresses that differ from the thread's own by constants. The
+// owned sites of every rank are stored and composed from those registers,
+// acc += G_k G_pair c_k (ConnectG, Lat3D1stO.cpp:299-312; tangent
+// dacc += (dG_k G_pair + G_k dG_pair) c_k), and acc goes to HBM once.
+//
+// What bounds it: at 64^3 the instructions a wave issues one after the other
+// (the arrays stay in the caches), at 128^3 the LDS exchange and HBM. The form
+// before gave each thread of a 1024-thread workgroup one site at a time and
+// spent most of its instructions on the divisions that found it; its reads
+// from LDS were seven a site, now five. Four ranks of two chains at 64^3,
+// FP32: 17.5 / 21.5 us then, 9.4 / 11.2 us now (forward / composing), tangents
+// 25 / 29 us then, 14.4 / 16.2 us now; FP64 at 128^3, four ranks: 122 / 160 us
+// then, 65 / 113 us now. One thread per column (twice the planes each) took
+// 11.7 / 14.7 us in FP32: half the waves, each twice as long.
 //
 // FP32 scaling: the input is divided by max(rank s0) and every rank by the
 // lattice maximum of g, so no rank exceeds 1 and at most nr ranks decay
@@ -33,17 +41,28 @@ namespace sfx {
 
 constexpr int kTX = 8, kTY = 8, kTZ = 16;
 constexpr int kH = kB3Ranks;  // largest widening: the lattice-side bound of block3_ok
-// the tile widened by h (the most ranks a launch of the variant advances)
-template <typename T, bool TANGENT>
+// the tile widened by H layers; one (y, z) column of it is two threads, each
+// with px of its x planes in registers
+template <int H>
 struct B3Region {
-  static constexpr int h = b3_max_ranks<T>(TANGENT);
-  static constexpr int rx = kTX + 2 * h, ry = kTY + 2 * h, rz = kTZ + 2 * h;
-  static constexpr int ryz = ry * rz;
-  static constexpr int r = rx * ryz;  // region sites
+  static constexpr int rx = kTX + 2 * H, ry = kTY + 2 * H, rz = kTZ + 2 * H;
+  static constexpr int px = rx / 2;
+  static constexpr int half = (ry * rz + 63) / 64 * 64;  // threads of one half
+  static constexpr int threads = 2 * half;
+  // LDS words of one rank: planes 1..px-1 of each half (the outermost plane is
+  // nobody's y or z neighbour), a row of padding below and above
+  static constexpr int words = 2 * (px - 1) * half + 2 * rz;
 };
-constexpr int kT = kTX * kTY * kTZ;
-constexpr int kB3 = 1024;  // threads per workgroup, one per tile site
-static_assert(kB3 == kT, "a thread owns one tile site");
+// two LDS buffers (one barrier per rank) where they leave room for three
+// workgroups per CU, else one buffer and two barriers
+template <typename T, bool TANGENT, int H>
+constexpr bool b3_double() {
+  return 2 * (TANGENT ? 2 : 1) * B3Region<H>::words * (int)sizeof(T) <= 53 * 1024;
+}
+template <typename T, bool TANGENT, int H>
+constexpr int b3_lds() {
+  return (b3_double<T, TANGENT, H>() ? 2 : 1) * (TANGENT ? 2 : 1) * B3Region<H>::words * (int)sizeof(T);
+}
 
 bool block3_ok(const DevLattice& L) {
   return L.grad == 3 && L.kind == ST_3D_SC && L.order == 1 && L.nx > kH && L.ny > kH && L.nz > kH;
@@ -59,39 +78,55 @@ __device__ __forceinline__ int extend(int c, int n, int periodic, int m2lo, int 
   return c < 1 ? 1 : (c > n ? n : c);
 }
 
-template <typename T>
-__device__ __forceinline__ T block_max_T(T m, float* red) {
-  float v = (float)m;
+// float maximum over the workgroup; valid in thread 0
+template <int NT>
+__device__ __forceinline__ float block_max_f(float v, float* red) {
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
   float r = red[0];
-  for (int i = 1; i < kB3 / 64; i++) r = fmaxf(r, red[i]);
-  return (T)r;
+  for (int i = 1; i < NT / 64; i++) r = fmaxf(r, red[i]);
+  return r;
 }
 
-template <typename T, bool TANGENT, bool SCALED, bool CONNECT>
-// FP32 tangent variants fit two workgroups per CU in LDS; the bound asks the
-// compiler for the register budget (64 VGPRs) that lets them (the FP64 base
-// variants, also two per CU, stay below it unasked)
-__global__ void __launch_bounds__(kB3) __attribute__((amdgpu_waves_per_eu((TANGENT && sizeof(T) == 4) ? 8 : 1)))
-k_block3(DevLattice L, B3Launch<T> la, int nb) {
-  constexpr int kH = B3Region<T, TANGENT>::h;
-  constexpr int kRZ = B3Region<T, TANGENT>::rz, kRYZ = B3Region<T, TANGENT>::ryz, kR = B3Region<T, TANGENT>::r;
+template <typename T, bool TANGENT, bool SCALED, bool CONNECT, int H>
+__global__ void __launch_bounds__(B3Region<H>::threads) k_block3(DevLattice L, B3Launch<T> la, int nb) {
+  using R = B3Region<H>;
+  constexpr int PX = R::px, RX = R::rx, RZ = R::rz, NT = R::half;
+  constexpr int OX = PX - H;  // owned planes of a half: its planes H..PX-1
+  constexpr bool DB = b3_double<T, TANGENT, H>();
   // chain of this workgroup and its tile number within that chain's grid
   const int chain = (int)blockIdx.x >= nb ? 1 : 0;
   const int bl = (int)blockIdx.x - chain * nb;
   const B3Args<T>& a = la.a[chain];
-  extern __shared__ __align__(16) unsigned char smem[];
-  T* G0 = (T*)smem;
-  T* G1 = G0 + kR;
-  T* gl = G1 + kR;
-  T* D0 = TANGENT ? gl + kR : nullptr;
-  T* D1 = TANGENT ? D0 + kR : nullptr;
-  T* vl = TANGENT ? D1 + kR : nullptr;
-  __shared__ float red[kB3 / 64];
+  __shared__ __align__(16) T lds[b3_lds<T, TANGENT, H>() / sizeof(T)];
+  __shared__ float red[R::threads / 64], scl[2];
+  __shared__ T cfac[kB3Ranks];
 
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, lane = t & 63;
+  const int nr = a.nr;
+
+  // the maxima and logs the scale factors build on were written by earlier
+  // launches: the first wave asks for them before anything else, so that they
+  // arrive before the region and are worked on while it is in flight
+  float ma = 0.f, mb = 0.f;
+  double lnv0 = 0.0, lnp = 0.0, lref = 0.0;
+  if constexpr (SCALED) {
+    if (t < 64) {
+      ma = __uint_as_float(a.maxv[(long long)a.s0 * kStepWords + lane * kSlotStride]);
+      mb = __uint_as_float(a.gmax[lane * kSlotStride]);
+      lnv0 = a.lnv[a.s0];
+      if constexpr (CONNECT) {
+        int pi = a.pidx[0];
+#pragma unroll
+        for (int k = 1; k < kB3Ranks; k++)
+          if (lane == k) pi = a.pidx[k];
+        if (lane < nr) lnp = a.lnpair[pi];
+        lref = *a.ref;
+      }
+    }
+  }
+
   const int nbz = (L.nz + kTZ - 1) / kTZ, nby = (L.ny + kTY - 1) / kTY;
   // XCD-aware: each XCD takes a contiguous run of tiles (x-slabs), so the y / z
   // halos its tiles share stay in that XCD's L2
@@ -101,243 +136,193 @@ k_block3(DevLattice L, B3Launch<T> la, int nb) {
   const int by = b % nby;
   const int bx = b / nby;
   const int x0 = 1 + bx * kTX, y0 = 1 + by * kTY, z0 = 1 + bz * kTZ;  // tile origin (interior coords)
-  const int nr = a.nr;
 
-  // the tile site this thread owns (kB3 == kT): z fastest, so HBM accesses coalesce
-  const int oZ = t % kTZ, oY = (t / kTZ) % kTY, oX = t / (kTZ * kTY);
-  const bool owner = x0 + oX <= L.nx && y0 + oY <= L.ny && z0 + oZ <= L.nz;
-  const long long ogi = owner ? sidx(L, x0 + oX, y0 + oY, z0 + oZ) : 0;
-  const int oidx = (kH + oX) * kRYZ + (kH + oY) * kRZ + (kH + oZ);
-
-  // the logs the scale factors build on were written by earlier launches: load
-  // them now, so their latency overlaps the region loads below
-  const int lane = t & 63;
-  double lnv0 = 0.0, lnp = 0.0, lref = 0.0;
-  if constexpr (SCALED) {
-    lnv0 = a.lnv[a.s0];
-    if constexpr (CONNECT) {
-      int pi = 0;
+  // this thread's (y, z) column and its half of it: plane j of the lower half
+  // is region plane j, of the upper half region plane RX-1-j, so that in both
+  // plane j-1 lies outwards, j+1 inwards, rank k needs the planes j >= k, and
+  // the planes H.. are owned where (y, z) lies in the tile and in the lattice
+  const int half = __builtin_amdgcn_readfirstlane(t >= NT ? 1 : 0);
+  const int c = t - half * NT;
+  const int Y = c / RZ, Z = c - Y * RZ;
+  const bool owner = Y >= H && Y < H + kTY && Z >= H && Z < H + kTZ && y0 + Y - H <= L.ny && z0 + Z - H <= L.nz;
+  const int yy = extend(y0 + Y - H, L.ny, L.periodic[1], L.mirror2_1[1], L.mirror2_2[1]);
+  const int zz = extend(z0 + Z - H, L.nz, L.periodic[2], L.mirror2_1[2], L.mirror2_2[2]);
+  const unsigned yz = (unsigned)(yy * L.MZ + zz);
+  // plane offsets: one lane each, then into scalar registers
+  const int xl = x0 - H + (half ? RX - 1 - lane : lane);
+  const unsigned xoff =
+      (unsigned)extend(xl, L.nx, L.periodic[0], L.mirror2_1[0], L.mirror2_2[0]) * (unsigned)L.jx;
+  unsigned px[PX];
 #pragma unroll
-      for (int k = 0; k < kB3Ranks; k++)
-        if (lane == k) pi = a.pidx[k];
-      if (lane < nr) lnp = a.lnpair[pi];
-      lref = *a.ref;
-    }
+  for (int j = 0; j < PX; j++) px[j] = (unsigned)__builtin_amdgcn_readlane((int)xoff, j);
+  // owned plane j lies in the lattice
+  auto inside = [&](int j) { return x0 + (half ? kTX - 1 - (j - H) : j - H) <= L.nx; };
+
+  // rank s0 (and its tangent), g (and v) of the column: the plane's offset is
+  // uniform, the lane's is one 32-bit word
+  T G[PX], g[PX], D[TANGENT ? PX : 1], v[TANGENT ? PX : 1];
+#pragma unroll
+  for (int j = 0; j < PX; j++) {
+    G[j] = (a.in + px[j])[yz];
+    if constexpr (TANGENT) D[j] = (a.din + px[j])[yz];
+  }
+#pragma unroll
+  for (int j = 1; j < PX; j++) {
+    g[j] = (a.g + px[j])[yz];
+    if constexpr (TANGENT) v[j] = (a.v + px[j])[yz];
   }
 
-  // issue the loads of rank s0 (and its tangent), g (and v) on the tile widened
-  // by nr first: the scale factors below are computed while they are in flight,
-  // and no LDS store waits on them before that
-  constexpr int kIt = (kR + kB3 - 1) / kB3;
-  const int wlo = kH - nr, wy = kTY + 2 * nr, wz = kTZ + 2 * nr;
-  const int nreg = (kTX + 2 * nr) * wy * wz;
-  T vg[kIt], vgg[kIt], vd[kIt], vv[kIt];
-  int li[kIt];
-#pragma unroll
-  for (int j = 0; j < kIt; j++) {
-    const int i = t + j * kB3;
-    li[j] = -1;
-    if (i < nreg) {
-      const int Z = i % wz, r = i / wz, Y = r % wy, X = r / wy;
-      const int x = extend(x0 + wlo + X - kH, L.nx, L.periodic[0], L.mirror2_1[0], L.mirror2_2[0]);
-      const int y = extend(y0 + wlo + Y - kH, L.ny, L.periodic[1], L.mirror2_1[1], L.mirror2_2[1]);
-      const int z = extend(z0 + wlo + Z - kH, L.nz, L.periodic[2], L.mirror2_1[2], L.mirror2_2[2]);
-      const long long gi = sidx(L, x, y, z);
-      li[j] = (wlo + X) * kRYZ + (wlo + Y) * kRZ + (wlo + Z);
-      vg[j] = a.in[gi];
-      vgg[j] = a.g[gi];
-      if constexpr (TANGENT) {
-        vd[j] = a.din[gi];
-        vv[j] = a.v[gi];
-      }
-    }
-  }
-
-  // the partner ranks are needed only from the first composition on
-  T pr[kB3Ranks], dpr[kB3Ranks];
-  if constexpr (CONNECT) {
-#pragma unroll
-    for (int k = 0; k < kB3Ranks; k++) {
-      pr[k] = (owner && k < nr) ? a.pair[k][ogi] : T(0);
-      if constexpr (TANGENT) dpr[k] = (owner && k < nr) ? a.dpair[k][ogi] : T(0);
-    }
-  }
-
-  // scale factors of this launch. They are uniform, so every wave evaluates
-  // each FP64 log / exp once in one lane and broadcasts it: lanes 0 and 1 the
-  // logs of the two divisors, lane k the composition factor of rank k + 1.
-  // The FP64 logs and exponentials are evaluated by the first wave alone,
-  // which shares the composition factors through LDS (read after the first
-  // rank's barrier); the other waves go on to the LDS stores meanwhile.
-  T in_scale = T(1), ginv = T(1);
+  // scale factors of this launch: the FP64 logs and exponentials are evaluated
+  // by the first wave alone (lanes 0 and 1 the logs of the two divisors, lane k
+  // the composition factor of rank k + 1) while the region is in flight
   double ln_base = 0.0, lng = 0.0;
-  __shared__ T cfac[kB3Ranks];
   if constexpr (SCALED) {
-    float m0, gm;
-    block_step_max2(a.maxv, a.s0, a.gmax, 0, m0, gm);
-    if (!(m0 > 0.f)) m0 = 1.f;
-    if (!(gm > 0.f)) gm = 1.f;
-    in_scale = (T)(1.f / m0);
-    ginv = (T)(1.f / gm);
     if (t < 64) {
-      const double lv = lane == 0 ? log((double)m0) : (lane == 1 ? log((double)gm) : 0.0);
-      ln_base = lnv0 + __shfl(lv, 0, 64);
-      lng = __shfl(lv, 1, 64);
-      if constexpr (CONNECT) {
-        const double c = lane < nr ? exp(ln_base + (lane + 1) * lng + lnp - lref) : 1.0;
-        if (lane < kB3Ranks) cfac[lane] = (T)c;
+      for (int o = 32; o > 0; o >>= 1) {
+        ma = fmaxf(ma, __shfl_xor(ma, o, 64));
+        mb = fmaxf(mb, __shfl_xor(mb, o, 64));
       }
-    }
-  } else if constexpr (CONNECT) {
-    if (t < kB3Ranks) cfac[t] = T(1);
-  }
-
-#pragma unroll
-  for (int j = 0; j < kIt; j++) {
-    if (li[j] >= 0) {
-      G0[li[j]] = vg[j] * in_scale;
-      gl[li[j]] = vgg[j];
-      if constexpr (TANGENT) {
-        D0[li[j]] = vd[j] * in_scale;
-        vl[li[j]] = vv[j];
+      if (!(ma > 0.f)) ma = 1.f;
+      if (!(mb > 0.f)) mb = 1.f;
+      if (lane == 0) {
+        scl[0] = 1.f / ma;
+        scl[1] = 1.f / mb;
       }
-    }
-  }
-  __syncthreads();
-
-  T* src = G0;
-  T* dst = G1;
-  T* dsrc = D0;
-  T* ddst = D1;
-  T acc = T(0), mloc = T(0);
-  const T sixth = T(1.0 / 6.0);
-  for (int k = 1; k <= nr; k++) {
-    // rank k on the tile widened by e = nr - k: threads take (y, z) columns,
-    // several threads per column split it along x. Consecutive threads cover
-    // whole LDS rows of kRZ (threads on the ring outside the widened tile
-    // idle), so a wave reads consecutive LDS words, free of bank conflicts.
-    const int e = nr - k;
-    const int lo = kH - e;
-    const int bxn = kTX + 2 * e, byn = kTY + 2 * e, bzn = kTZ + 2 * e;
-    if constexpr (sizeof(T) == 4) {
-      // FP32: a work item is four consecutive z sites of one (x, y) row, read
-      // and written as float4 (rows start on 16-byte boundaries: kRZ and kRYZ
-      // are multiples of 4). Items cover the widened z range rounded out to
-      // whole quads; the extra sites at the row ends read in-buffer
-      // neighbours, and no later rank reads them. Same additions in the same
-      // order as one site at a time, so the same bits.
-      static_assert(kRZ % 4 == 0 && kRYZ % 4 == 0, "float4 rows");
-      const int c0 = lo >> 2, nch = ((lo + bzn + 3) >> 2) - c0;
-      const int items = bxn * byn * nch;
-      for (int it = t; it < items; it += kB3) {
-        const int ch = c0 + it % nch, r = it / nch;
-        const int idx = (lo + r / byn) * kRYZ + (lo + r % byn) * kRZ + ch * 4;
-        const float4 c = *(const float4*)&src[idx];
-        const float4 xm = *(const float4*)&src[idx - kRYZ], xp = *(const float4*)&src[idx + kRYZ];
-        const float4 ym = *(const float4*)&src[idx - kRZ], yp = *(const float4*)&src[idx + kRZ];
-        const float zm = src[idx - 1], zp = src[idx + 4];
-        const float4 gq = *(const float4*)&gl[idx];
-        const float4 sv = make_float4((xm.x + xp.x + ym.x + yp.x + zm + c.y) * sixth,
-                                      (xm.y + xp.y + ym.y + yp.y + c.x + c.z) * sixth,
-                                      (xm.z + xp.z + ym.z + yp.z + c.y + c.w) * sixth,
-                                      (xm.w + xp.w + ym.w + yp.w + c.z + zp) * sixth);
-        const float4 gv = make_float4(gq.x * ginv, gq.y * ginv, gq.z * ginv, gq.w * ginv);
-        *(float4*)&dst[idx] = make_float4(gv.x * sv.x, gv.y * sv.y, gv.z * sv.z, gv.w * sv.w);
-        if constexpr (TANGENT) {
-          const float4 dc = *(const float4*)&dsrc[idx];
-          const float4 dxm = *(const float4*)&dsrc[idx - kRYZ], dxp = *(const float4*)&dsrc[idx + kRYZ];
-          const float4 dym = *(const float4*)&dsrc[idx - kRZ], dyp = *(const float4*)&dsrc[idx + kRZ];
-          const float dzm = dsrc[idx - 1], dzp = dsrc[idx + 4];
-          const float4 vq = *(const float4*)&vl[idx];
-          const float4 ds = make_float4((dxm.x + dxp.x + dym.x + dyp.x + dzm + dc.y) * sixth,
-                                        (dxm.y + dxp.y + dym.y + dyp.y + dc.x + dc.z) * sixth,
-                                        (dxm.z + dxp.z + dym.z + dyp.z + dc.y + dc.w) * sixth,
-                                        (dxm.w + dxp.w + dym.w + dyp.w + dc.z + dzp) * sixth);
-          *(float4*)&ddst[idx] = make_float4(gv.x * (ds.x - vq.x * sv.x), gv.y * (ds.y - vq.y * sv.y),
-                                             gv.z * (ds.z - vq.z * sv.z), gv.w * (ds.w - vq.w * sv.w));
-        }
-      }
-    } else {
-      const int ncol = byn * kRZ;
-      const int per = kB3 / ncol > 0 ? kB3 / ncol : 1;
-      const int c = t % ncol, xs = t / ncol, RZ = c % kRZ;
-      if (t < per * ncol && RZ >= lo && RZ < lo + bzn) {
-        const int base = (lo + c / kRZ) * kRZ + RZ;
-        for (int X = lo + xs; X < lo + bxn; X += per) {
-          const int idx = X * kRYZ + base;
-          const T s = (src[idx - kRYZ] + src[idx + kRYZ] + src[idx - kRZ] + src[idx + kRZ] + src[idx - 1] +
-                       src[idx + 1]) * sixth;
-          const T gv = gl[idx] * ginv;
-          dst[idx] = gv * s;
-          if constexpr (TANGENT) {
-            const T ds = (dsrc[idx - kRYZ] + dsrc[idx + kRYZ] + dsrc[idx - kRZ] + dsrc[idx + kRZ] + dsrc[idx - 1] +
-                          dsrc[idx + 1]) * sixth;
-            ddst[idx] = gv * (ds - vl[idx] * s);
-          }
+      if (CONNECT || bl == 0) {
+        const double lv = log((double)(lane == 1 ? mb : ma));
+        ln_base = lnv0 + __shfl(lv, 0, 64);
+        lng = __shfl(lv, 1, 64);
+        if constexpr (CONNECT) {
+          const double cf = lane < nr ? exp(ln_base + (lane + 1) * lng + lnp - lref) : 1.0;
+          if (lane < kB3Ranks) cfac[lane] = (T)cf;
         }
       }
     }
     __syncthreads();
-    // the owned tile site of rank k: store, compose, track the last rank's max
-    if (owner) {
-      const T val = dst[oidx];
-      T dval = T(0);
-      if constexpr (TANGENT) dval = ddst[oidx];
-      T* outk = a.out[k - 1];
-      if (outk) outk[ogi] = val;
-      if constexpr (TANGENT) {
-        T* doutk = a.dout[k - 1];
-        if (doutk) doutk[ogi] = dval;
-      }
-      if constexpr (CONNECT) {
-        if constexpr (TANGENT)
-          acc += (dval * pr[k - 1] + val * dpr[k - 1]) * cfac[k - 1];
-        else
-          acc += val * pr[k - 1] * cfac[k - 1];
-      }
-      if (k == nr) mloc = val;
+    const T in_scale = (T)scl[0], ginv = (T)scl[1];
+#pragma unroll
+    for (int j = 0; j < PX; j++) {
+      G[j] *= in_scale;
+      if (j) g[j] *= ginv;
+      if constexpr (TANGENT) D[j] *= in_scale;
     }
-    T* tmp = src;
-    src = dst;
-    dst = tmp;
-    if constexpr (TANGENT) {
-      tmp = dsrc;
-      dsrc = ddst;
-      ddst = tmp;
+  }
+
+  T acc[CONNECT ? OX : 1];
+  if constexpr (CONNECT) {
+#pragma unroll
+    for (int i = 0; i < OX; i++) acc[i] = T(0);
+  }
+  const T sixth = T(1.0 / 6.0);
+  const unsigned own = (unsigned)(RZ + c + half * (PX - 1) * NT), other = (unsigned)(RZ + c + (1 - half) * (PX - 1) * NT);
+#pragma unroll
+  for (int k = 1; k <= H; k++) {
+    if (k <= nr) {
+      // the partner values of this rank, in flight through the exchange
+      T pr[CONNECT ? OX : 1], dpr[CONNECT && TANGENT ? OX : 1];
+      if constexpr (CONNECT) {
+        if (owner) {
+#pragma unroll
+          for (int i = 0; i < OX; i++) {
+            pr[i] = (a.pair[k - 1] + px[H + i])[yz];
+            if constexpr (TANGENT) dpr[i] = (a.dpair[k - 1] + px[H + i])[yz];
+          }
+        }
+      }
+      T* const buf = lds + (DB && (k & 1) ? (TANGENT ? 2 : 1) * R::words : 0);
+      T* const dbuf = buf + R::words;
+      if (!DB && k > 1) __syncthreads();  // the previous rank's reads are done
+#pragma unroll
+      for (int j = k; j < PX; j++) {
+        buf[own + (j - 1) * NT] = G[j];
+        if constexpr (TANGENT) dbuf[own + (j - 1) * NT] = D[j];
+      }
+      __syncthreads();
+      T co = G[k - 1], dco = TANGENT ? D[k - 1] : T(0);  // the next plane outwards, old rank
+#pragma unroll
+      for (int j = k; j < PX; j++) {
+        const unsigned o = own + (j - 1) * NT;
+        const T cc = G[j];
+        const T ci = j + 1 < PX ? G[j + 1 < PX ? j + 1 : j] : buf[other + (PX - 2) * NT];
+        const T s = (co + ci + buf[o - RZ] + buf[o + RZ] + buf[o - 1] + buf[o + 1]) * sixth;
+        G[j] = g[j] * s;
+        co = cc;
+        if constexpr (TANGENT) {
+          const T dc = D[j];
+          const T dci = j + 1 < PX ? D[j + 1 < PX ? j + 1 : j] : dbuf[other + (PX - 2) * NT];
+          const T ds = (dco + dci + dbuf[o - RZ] + dbuf[o + RZ] + dbuf[o - 1] + dbuf[o + 1]) * sixth;
+          D[j] = g[j] * (ds - v[j] * s);
+          dco = dc;
+        }
+      }
+      // the owned tile sites of rank k: store and compose
+      if (owner) {
+        T* const outk = a.out[k - 1];
+        T* const doutk = TANGENT ? a.dout[k - 1] : nullptr;
+        if (outk) {
+#pragma unroll
+          for (int j = H; j < PX; j++)
+            if (inside(j)) {
+              (outk + px[j])[yz] = G[j];
+              if constexpr (TANGENT) (doutk + px[j])[yz] = D[j];
+            }
+        }
+        if constexpr (CONNECT) {
+          const T cf = SCALED ? cfac[k - 1] : T(1);
+#pragma unroll
+          for (int i = 0; i < OX; i++) {
+            if constexpr (TANGENT)
+              acc[i] += (D[H + i] * pr[i] + G[H + i] * dpr[i]) * cf;
+            else
+              acc[i] += G[H + i] * pr[i] * cf;
+          }
+        }
+      }
     }
   }
 
   if constexpr (CONNECT) {
-    if (owner) a.acc[ogi] += acc;
+    if (owner) {
+#pragma unroll
+      for (int i = 0; i < OX; i++)
+        if (inside(H + i)) (a.acc + px[H + i])[yz] += acc[i];
+    }
   }
   if constexpr (SCALED) {
-    const T m = block_max_T<T>(mloc, red);
+    T mloc = T(0);
+    if (owner) {
+#pragma unroll
+      for (int j = H; j < PX; j++)
+        if (inside(j)) mloc = mloc > G[j] ? mloc : G[j];
+    }
+    const float m = block_max_f<R::threads>((float)mloc, red);
     if (t == 0) {
-      put_step_max(a.maxv, a.s0 + nr, (float)m);
+      put_step_max(a.maxv, a.s0 + nr, m);
       if (bl == 0)
         for (int k = 1; k <= nr; k++) a.lnv[a.s0 + k] = ln_base + k * lng;
     }
   }
 }
 
-template <typename T, bool TANGENT>
-static size_t b3_lds() {
-  return (TANGENT ? 6 : 3) * (size_t)B3Region<T, TANGENT>::r * sizeof(T);
-}
-
-template <typename T, bool TG, bool SC, bool CN>
+template <typename T, bool TG, bool SC, bool CN, int H>
 static void b3_launch(const DevLattice& L, const B3Launch<T>& a, unsigned nb, hipStream_t st, hipEvent_t ev0,
                       hipEvent_t ev1) {
-  static bool attr = false;  // dynamic LDS above the default limit needs the attribute once
-  const size_t lds = b3_lds<T, TG>();
-  if (!attr) {
-    SFX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_block3<T, TG, SC, CN>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr = true;
-  }
+  static_assert(b3_lds<T, TG, H>() <= 64 * 1024, "static LDS");
   // with events: recorded by the dispatch itself at kernel start and end
-  hipExtLaunchKernelGGL(k_block3<T, TG, SC, CN>, dim3(nb * (unsigned)a.nchains), dim3(kB3), (uint32_t)lds, st, ev0,
-                        ev1, 0u, L, a, (int)nb);
+  hipExtLaunchKernelGGL((k_block3<T, TG, SC, CN, H>), dim3(nb * (unsigned)a.nchains), dim3(B3Region<H>::threads), 0,
+                        st, ev0, ev1, 0u, L, a, (int)nb);
+}
+template <typename T, bool TG, bool SC, bool CN>
+static void b3_launch_h(int nr, const DevLattice& L, const B3Launch<T>& a, unsigned nb, hipStream_t st,
+                        hipEvent_t ev0, hipEvent_t ev1) {
+  // launches of one or two ranks (a chain's ends, a change of the segment
+  // state) load and compute a smaller region: 7.2 / 9.1 us instead of 14 / 16
+  // at 75 x 61 x 90 in FP32
+  if (nr <= 2) {
+    b3_launch<T, TG, SC, CN, 2>(L, a, nb, st, ev0, ev1);
+    return;
+  }
+  b3_launch<T, TG, SC, CN, kB3Ranks>(L, a, nb, st, ev0, ev1);
 }
 
 template <typename T>
@@ -353,20 +338,21 @@ template <typename T>
 void launch_block3(const DevLattice& L, const B3Launch<T>& a, bool tangent, bool scaled, bool connect,
                    hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
   SFX_REQUIRE(a.nchains == 1 || a.nchains == 2, SFX_E_INVALID, "a blocked launch advances one or two chains");
-  for (int c = 0; c < a.nchains; c++)
-    SFX_REQUIRE(a.a[c].nr >= 1 && a.a[c].nr <= b3_max_ranks<T>(tangent), SFX_E_INVALID,
-                "blocked launch of 1..4 ranks (1..2 for tangents and FP64)");
+  int nr = 0;
+  for (int c = 0; c < a.nchains; c++) {
+    SFX_REQUIRE(a.a[c].nr >= 1 && a.a[c].nr <= kB3Ranks, SFX_E_INVALID, "blocked launch of 1..4 ranks");
+    nr = std::max(nr, a.a[c].nr);
+  }
   SFX_REQUIRE(!(tangent && sizeof(T) == 8), SFX_E_UNSUPPORTED, "FP64 tangent sweeps run rank by rank");
-  const size_t lds_base = b3_lds<T, false>(), lds_tan = b3_lds<T, true>();
-  SFX_REQUIRE((lds_base <= 160 * 1024 && (sizeof(T) == 8 || lds_tan <= 160 * 1024)), SFX_E_UNSUPPORTED,
-              "blocked tile exceeds LDS");
   const unsigned nb = (unsigned)(((L.nx + kTX - 1) / kTX) * ((L.ny + kTY - 1) / kTY) * ((L.nz + kTZ - 1) / kTZ));
-#define B3(TG, SC, CN) b3_launch<T, TG, SC, CN>(L, a, nb, st, ev0, ev1)
+#define B3(TG, SC, CN) b3_launch_h<T, TG, SC, CN>(nr, L, a, nb, st, ev0, ev1)
   if (tangent) {
-    if (scaled) {
-      if (connect) B3(true, true, true); else B3(true, true, false);
-    } else {
-      if (connect) B3(true, false, true); else B3(true, false, false);
+    if constexpr (sizeof(T) == 4) {
+      if (scaled) {
+        if (connect) B3(true, true, true); else B3(true, true, false);
+      } else {
+        if (connect) B3(true, false, true); else B3(true, false, false);
+      }
     }
   } else {
     if (scaled) {
