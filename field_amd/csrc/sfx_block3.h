@@ -28,6 +28,7 @@ struct B3Args {
   const T* pair[kB3Ranks];     // composition partner of rank s0+k
   const T* dpair[kB3Ranks];
   T* acc;                      // accumulator of the state (phi, or dphi for tangents)
+  T* bacc;                     // tangent sweeps: phi's accumulator too, unless the base has been swept (nullptr)
   int nr;
   // FP32 log-scaling: the input is divided by max(rank s0) (maxv[s0]) and
   // every rank by the lattice maximum of g (gmax); lnv[s] is the log of the

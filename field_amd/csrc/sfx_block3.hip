@@ -208,10 +208,13 @@ __global__ void __launch_bounds__(B3Region<H>::threads) k_block3(DevLattice L, B
     }
   }
 
-  T acc[CONNECT ? OX : 1];
+  T acc[CONNECT ? OX : 1], bacc[CONNECT && TANGENT ? OX : 1];
   if constexpr (CONNECT) {
 #pragma unroll
-    for (int i = 0; i < OX; i++) acc[i] = T(0);
+    for (int i = 0; i < OX; i++) {
+      acc[i] = T(0);
+      if constexpr (TANGENT) bacc[i] = T(0);
+    }
   }
   const T sixth = T(1.0 / 6.0);
   const unsigned own = (unsigned)(RZ + c + half * (PX - 1) * NT), other = (unsigned)(RZ + c + (1 - half) * (PX - 1) * NT);
@@ -271,10 +274,12 @@ __global__ void __launch_bounds__(B3Region<H>::threads) k_block3(DevLattice L, B
           const T cf = SCALED ? cfac[k - 1] : T(1);
 #pragma unroll
           for (int i = 0; i < OX; i++) {
-            if constexpr (TANGENT)
+            if constexpr (TANGENT) {
               acc[i] += (D[H + i] * pr[i] + G[H + i] * dpr[i]) * cf;
-            else
+              bacc[i] += G[H + i] * pr[i] * cf;
+            } else {
               acc[i] += G[H + i] * pr[i] * cf;
+            }
           }
         }
       }
@@ -285,7 +290,11 @@ __global__ void __launch_bounds__(B3Region<H>::threads) k_block3(DevLattice L, B
     if (owner) {
 #pragma unroll
       for (int i = 0; i < OX; i++)
-        if (inside(H + i)) (a.acc + px[H + i])[yz] += acc[i];
+        if (inside(H + i)) {
+          (a.acc + px[H + i])[yz] += acc[i];
+          if constexpr (TANGENT)
+            if (a.bacc) (a.bacc + px[H + i])[yz] += bacc[i];
+        }
     }
   }
   if constexpr (SCALED) {

@@ -16,7 +16,8 @@ void launch_prop2f(const DevLattice& L, bool tangent, const T* Win, const T* dWi
 // from Wp = W_f(s-1) (null for s = 1, where G_f = g); sc.pmaxv: the forward maxima
 template <typename T>
 void launch_prop2b(const DevLattice& L, bool tangent, const T* Gin, const T* dGin, const T* g, const T* v, T* Gout,
-                   T* dGout, const T* Wp, const T* dWp, T* acc, double S, const RankScale& sc, hipStream_t st);
+                   T* dGout, const T* Wp, const T* dWp, T* acc, double S, const RankScale& sc, hipStream_t st,
+                   T* bacc = nullptr);
 // forward rank 1 in W form (G = g, tangent -v g)
 template <typename T>
 void launch_init2f(const DevLattice& L, bool tangent, const T* g, const T* v, T* W, T* dW, double S,
@@ -24,7 +25,7 @@ void launch_init2f(const DevLattice& L, bool tangent, const T* g, const T* v, T*
 // backward rank N (G = g, tangent -v g) composed with G_f(N) recovered from Wp = W_f(N-1)
 template <typename T>
 void launch_init2b(const DevLattice& L, bool tangent, const T* g, const T* v, T* G, T* dG, const T* Wp,
-                   const T* dWp, T* acc, const RankScale& sc, hipStream_t st);
+                   const T* dWp, T* acc, const RankScale& sc, hipStream_t st, T* bacc = nullptr);
 // per-block weighted sums over the six components of G (and dG)
 template <typename T>
 int launch_wsum6(const DevLattice& L, const T* G, const T* dG, double* p1, double* p2, hipStream_t st);

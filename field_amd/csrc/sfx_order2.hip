@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(kB2) k_prop2b(DevLattice L, const T* __restric
                                                 const T* __restrict__ g, const T* __restrict__ v,
                                                 T* __restrict__ Gout, T* __restrict__ dGout,
                                                 const T* __restrict__ Wp, const T* __restrict__ dWp,
-                                                T* __restrict__ acc, T S, RankScale sc) {
+                                                T* __restrict__ acc, T* __restrict__ bacc, T S, RankScale sc) {
   long long q = site_ordinal();
   const long long M = L.M;
   const bool in = q < L.V;
@@ -291,7 +291,7 @@ __global__ void __launch_bounds__(kB2) k_prop2b(DevLattice L, const T* __restric
   const T Lw = (T(1) - S) / T(4);
   long long r = 0;
   T o[6], d[6], pa[6], dpa[6], zz[6], dz[6];
-  T graw = T(0), vv = T(0), acc0 = T(0);
+  T graw = T(0), vv = T(0), acc0 = T(0), bacc0 = T(0);
 #pragma unroll
   for (int k = 0; k < 6; k++) o[k] = d[k] = zz[k] = dz[k] = T(0);
   if (in) {
@@ -324,6 +324,8 @@ __global__ void __launch_bounds__(kB2) k_prop2b(DevLattice L, const T* __restric
     if constexpr (TANGENT) vv = v[r];
     pair_rows<T, TANGENT, CURVED>(L, Wp, dWp, M, x, nbr, fl, r, pa, dpa);
     acc0 = acc[r];
+    if constexpr (TANGENT)
+      if (bacc) bacc0 = bacc[r];
   }
   // outside the per-site branch: lanes without a site transfer zeros (the
   // matrix-core form needs the whole wave)
@@ -360,10 +362,12 @@ __global__ void __launch_bounds__(kB2) k_prop2b(DevLattice L, const T* __restric
         da += dk * gp[k] + ok * dgp[k];
       }
     }
-    if constexpr (TANGENT)
+    if constexpr (TANGENT) {
       acc[r] = acc0 + da * cfac;
-    else
+      if (bacc) bacc[r] = bacc0 + a * cfac;
+    } else {
       acc[r] = acc0 + a * cfac;
+    }
   }
   if constexpr (SCALED) {
     __shared__ float sm[kB2 / 64];
@@ -426,7 +430,7 @@ __global__ void k_init2f(DevLattice L, const T* __restrict__ g, const T* __restr
 template <typename T, bool SCALED, bool TANGENT, bool CURVED>
 __global__ void k_init2b(DevLattice L, const T* __restrict__ g, const T* __restrict__ v, T* __restrict__ G,
                          T* __restrict__ dG, const T* __restrict__ Wp, const T* __restrict__ dWp,
-                         T* __restrict__ acc, RankScale sc) {
+                         T* __restrict__ acc, T* __restrict__ bacc, RankScale sc) {
   long long q = site_ordinal();
   const long long M = L.M;
   T pscale = T(1);
@@ -448,12 +452,13 @@ __global__ void k_init2b(DevLattice L, const T* __restrict__ g, const T* __restr
     neighbours(L, x, y, z, nbr, fl);
     T gp[6], dgp[6];
     pair_rank<T, TANGENT, CURVED>(L, Wp, dWp, gv, vv, M, x, nbr, fl, r, pscale, gp, dgp);
-    T a = T(0);
+    T a = T(0), ba = T(0);
     for (int k = 0; k < 6; k++) {
       G[(long long)k * M + r] = gv;
       if constexpr (TANGENT) {
         dG[(long long)k * M + r] = -vv * gv;
         a += -vv * gv * gp[k] + gv * dgp[k];
+        ba += gv * gp[k];
       } else {
         a += gv * gp[k];
       }
@@ -461,6 +466,8 @@ __global__ void k_init2b(DevLattice L, const T* __restrict__ g, const T* __restr
     T c = T(1);
     if constexpr (SCALED) c = (T)exp(sc.lnpair[sc.pair] - *sc.ref);
     acc[r] += a * c;
+    if constexpr (TANGENT)
+      if (bacc) bacc[r] += ba * c;
     m = (float)gv;
   }
   if constexpr (SCALED) {
@@ -565,18 +572,19 @@ void launch_prop2f(const DevLattice& L, bool tangent, const T* Win, const T* dWi
 
 template <typename T>
 void launch_prop2b(const DevLattice& L, bool tangent, const T* Gin, const T* dGin, const T* g, const T* v, T* Gout,
-                   T* dGout, const T* Wp, const T* dWp, T* acc, double S, const RankScale& sc, hipStream_t st) {
+                   T* dGout, const T* Wp, const T* dWp, T* acc, double S, const RankScale& sc, hipStream_t st,
+                   T* bacc) {
   const unsigned nb = grid1(L.V, kB2);
   const bool sc_on = sc.maxv != nullptr;
   const T s = (T)S;
   if (use_mfma(L, tangent, sizeof(T))) {
 #define K(SC, TG, CV) \
-  k_prop2b<T, SC, TG, CV, true><<<nb, kB2, 0, st>>>(L, Gin, dGin, g, v, Gout, dGout, Wp, dWp, acc, s, sc)
+  k_prop2b<T, SC, TG, CV, true><<<nb, kB2, 0, st>>>(L, Gin, dGin, g, v, Gout, dGout, Wp, dWp, acc, bacc, s, sc)
     SFX_O2_DISPATCH(K);
 #undef K
   } else {
 #define K(SC, TG, CV) \
-  k_prop2b<T, SC, TG, CV, false><<<nb, kB2, 0, st>>>(L, Gin, dGin, g, v, Gout, dGout, Wp, dWp, acc, s, sc)
+  k_prop2b<T, SC, TG, CV, false><<<nb, kB2, 0, st>>>(L, Gin, dGin, g, v, Gout, dGout, Wp, dWp, acc, bacc, s, sc)
     SFX_O2_DISPATCH(K);
 #undef K
   }
@@ -594,10 +602,10 @@ void launch_init2f(const DevLattice& L, bool tangent, const T* g, const T* v, T*
 
 template <typename T>
 void launch_init2b(const DevLattice& L, bool tangent, const T* g, const T* v, T* G, T* dG, const T* Wp,
-                   const T* dWp, T* acc, const RankScale& sc, hipStream_t st) {
+                   const T* dWp, T* acc, const RankScale& sc, hipStream_t st, T* bacc) {
   const unsigned nb = grid1(L.V, kB2);
   const bool sc_on = sc.maxv != nullptr;
-#define K(SC, TG, CV) k_init2b<T, SC, TG, CV><<<nb, kB2, 0, st>>>(L, g, v, G, dG, Wp, dWp, acc, sc)
+#define K(SC, TG, CV) k_init2b<T, SC, TG, CV><<<nb, kB2, 0, st>>>(L, g, v, G, dG, Wp, dWp, acc, bacc, sc)
   SFX_O2_DISPATCH(K);
 #undef K
 }
@@ -616,18 +624,18 @@ template void launch_prop2f<float>(const DevLattice&, bool, const float*, const 
                                    float*, float*, double, const RankScale&, hipStream_t);
 template void launch_prop2b<double>(const DevLattice&, bool, const double*, const double*, const double*,
                                     const double*, double*, double*, const double*, const double*, double*, double,
-                                    const RankScale&, hipStream_t);
+                                    const RankScale&, hipStream_t, double*);
 template void launch_prop2b<float>(const DevLattice&, bool, const float*, const float*, const float*, const float*,
                                    float*, float*, const float*, const float*, float*, double, const RankScale&,
-                                   hipStream_t);
+                                   hipStream_t, float*);
 template void launch_init2f<double>(const DevLattice&, bool, const double*, const double*, double*, double*, double,
                                     const RankScale&, hipStream_t);
 template void launch_init2f<float>(const DevLattice&, bool, const float*, const float*, float*, float*, double,
                                    const RankScale&, hipStream_t);
 template void launch_init2b<double>(const DevLattice&, bool, const double*, const double*, double*, double*,
-                                    const double*, const double*, double*, const RankScale&, hipStream_t);
+                                    const double*, const double*, double*, const RankScale&, hipStream_t, double*);
 template void launch_init2b<float>(const DevLattice&, bool, const float*, const float*, float*, float*, const float*,
-                                   const float*, float*, const RankScale&, hipStream_t);
+                                   const float*, float*, const RankScale&, hipStream_t, float*);
 template int launch_wsum6<double>(const DevLattice&, const double*, const double*, double*, double*, hipStream_t);
 template int launch_wsum6<float>(const DevLattice&, const float*, const float*, double*, double*, hipStream_t);
 

@@ -214,6 +214,10 @@ struct System {
   // call allocates nothing after the first)
   void abi_vectors(double*& in, double*& out);
   void compute_phi(int precision);  // from d_u
+  // compute_phi before and after the molecules' sweeps: a caller that sweeps
+  // base and tangent propagators together puts its own sweeps in between
+  void start_phi(int precision);
+  void finish_phi(int precision);
   void residual_internal(int precision);  // d_u -> d_f
   void finish_range(int m);  // range_restricted: the range condition fixes molecule m's constant
   bool has_range() const;

@@ -873,7 +873,7 @@ void System::sweep_blocked(int m, bool scaled) {
                            st);
 }
 
-void System::compute_phi(int prec) {
+void System::start_phi(int prec) {
   const DevLattice& L = lat.d;
   const bool gmax = prec == SFX_FP32 && use_block3;
   launch_swf(L, d_u, d_itmask, ns, d_st_itvar, d_swf, d_swf32, stream, gmax ? d_gmax : nullptr, ns * kStepWords);
@@ -882,6 +882,10 @@ void System::compute_phi(int prec) {
     launch_gmax(L, d_swf32, ns, d_gmax, stream, true);
     gmax_valid = true;
   }
+}
+
+void System::compute_phi(int prec) {
+  start_phi(prec);
   // non-solvent molecules first, the solvent closes phi_b (SF_MolList1stO.cpp:280-292)
   for (int pass = 0; pass < 2; pass++)
     for (int m = 0; m < nm; m++) {
@@ -893,6 +897,11 @@ void System::compute_phi(int prec) {
         sweep<double, double>(m, false);
       if (mols[m].freedom == SFX_RANGE_RESTRICTED) finish_range(m);
     }
+  finish_phi(prec);
+}
+
+void System::finish_phi(int prec) {
+  const DevLattice& L = lat.d;
   launch_phi_total(L, ns, nm, d_phi_m, d_mol_uses, d_fprof, d_frozen, d_phi, d_phitot, stream, &sp, d_molscal,
                    d_phib_state, d_cbulk);
   launch_sides(L, ns, d_phi, d_rho, stream);
