@@ -16,7 +16,7 @@
 #include <cmath>
 #include <type_traits>
 
-#include "sfx_device.h"
+#include "sfx_scf.h"
 #include "sfx_order2.h"
 #include "sfx_block3.h"
 #include "sfx_solve.h"
@@ -191,11 +191,11 @@ __global__ void __launch_bounds__(kTB) k_tprop(DevLattice L, const T* __restrict
   float m = 0.f;
   if (in) {
     T Go = gv * a * scale;
-    T dGo = gv * (da - vr * a) * scale;
+    T dGo = gv * tan_step(da, vr, a) * scale;
     Gout[r] = Go;
     dGout[r] = dGo;
     if constexpr (CONNECT) {
-      dacc[r] = dac + (dGo * gpr + Go * dgpr) * cfac;
+      dacc[r] = dac + tan_compose(dGo, gpr, Go, dgpr) * cfac;
       if (acc) acc[r] = ac + Go * gpr * cfac;
     }
     m = (float)Go;
@@ -224,7 +224,7 @@ __global__ void k_tconnect(DevLattice L, const T* __restrict__ A, const T* __res
   int x, y, z;
   interior_coords(L, q, x, y, z);
   long long r = sidx(L, x, y, z);
-  dacc[r] += (dA[r] * B[r] + A[r] * dB[r]) * c;
+  dacc[r] += tan_compose(dA[r], B[r], A[r], dB[r]) * c;
   if (acc) acc[r] += A[r] * B[r] * c;
 }
 
@@ -322,30 +322,8 @@ __global__ void k_tmol_finalize(MolParams mp, const double* p1, const double* p2
     s1 += r1[i];
     s2 += r2[i];
   }
-  double* d = dmol + mp.index * 4;
-  double dln = (p1 && n > 0) ? s2 / s1 : 0.0;
-  const double* ms = molscal + mp.index * MS_COUNT;
-  double phib = ms[MS_PHIB];
-  // the prefactor of the tangent sweep's scaling (its own reference log-scale)
-  const double f = mp.kind == 2 ? 2.0 : mp.kind == 3 ? 1.0 / 6.0 : 1.0;
-  if (mp.freedom == SFX_RESTRICTED)
-    d[3] = f * exp(log(mp.theta) - ms[MS_LNGN] - (mp.kind == 0 ? 0.0 : log((double)mp.N)) + ms[MS_REF]);
-  else
-    d[3] = f * (mp.kind == 0 ? phib : phib / mp.N) * exp(ms[MS_REF]);
-  d[0] = dln;
-  if (mp.freedom == SFX_RESTRICTED) {
-    d[1] = -dln;
-    d[2] = -phib * dln;
-  } else if (mp.freedom == SFX_SOLVENT) {
-    double dpb = 0;
-    for (int m = 0; m < nmol; m++)
-      if (m != mp.index) dpb -= dmol[m * 4 + 2];
-    d[2] = dpb;
-    d[1] = phib != 0 ? dpb / phib : 0.0;
-  } else {
-    d[1] = 0;
-    d[2] = 0;
-  }
+  tmol_scalars(mp, p1 && n > 0, s1, s2, molscal + mp.index * MS_COUNT, nmol, [&](int m) { return dmol[m * 4 + 2]; },
+               dmol + mp.index * 4);
 }
 
 // dphi_{m,t} at interior sites
@@ -359,18 +337,11 @@ __global__ void k_tmol_phi(DevLattice L, unsigned uses, int ns, const double* __
   int x, y, z;
   interior_coords(L, q, x, y, z);
   const long long r0 = sidx(L, x, y, z);
-  const double rel = dm[1];
   for (int t = 0; t < ns; t++) {  // every state of the molecule (bit t of uses), arrays [state][M]
     if (!((uses >> t) & 1u)) continue;
     const long long r = (long long)t * L.M + r0;
-    const double ph = phi_m[r];
-    const double gv = g[r];
-    double out;
-    if (monomer)
-      out = ph * (rel - v[r]);
-    else
-      out = gv > 0 ? ph * (rel + v[r]) + dm[3] * ((double)dacc[r] + (dacc2 ? (double)dacc2[r] : 0.0)) / gv : 0.0;
-    dphi_m[r] = out;
+    const double da = monomer ? 0.0 : (double)dacc[r] + (dacc2 ? (double)dacc2[r] : 0.0);
+    dphi_m[r] = tphi_site(monomer != 0, phi_m[r], g[r], v[r], da, dm);
   }
 }
 
@@ -421,29 +392,9 @@ __global__ void k_jres(DevLattice L, SysParams sp, const unsigned char* __restri
     for (int k = 0; k < nv; k++) jv[(long long)k * L.M + i] = 0.0;
     return;
   }
-  double pt = phitot[i], dpt = dphitot[i];
-  double du[SFX_MAXS];
-  double av = 0;
-  for (int k = 0; k < nv; k++) {
-    int t = sp.itvar_rep[k];
-    double ci = 0, dci = 0, dcb = 0;
-    for (int j = 0; j < sp.ns; j++) {
-      double c = sp.chi[t * SFX_MAXS + j];
-      if (c == 0) continue;
-      ci += c * rho[(long long)j * L.M + i];
-      dci += c * drho[(long long)j * L.M + i];
-      if (!sp.melt && !sp.frozen[j]) {
-        double dpb = 0;
-        for (int m = 0; m < sp.nm; m++) dpb += dmol[m * 4 + 2] * sp.mol_frac[m * SFX_MAXS + j];
-        dcb += c * dpb;
-      }
-    }
-    double d = v[(long long)k * L.M + i] - dci / pt + ci * dpt / (pt * pt) + dcb;
-    du[k] = d;
-    av += d;
-  }
-  av /= nv;
-  for (int k = 0; k < nv; k++) jv[(long long)k * L.M + i] = -dpt / (pt * pt) + du[k] - av;
+  jres_site(sp, phitot[i], dphitot[i], dmol, [&](int k) { return v[(long long)k * L.M + i]; },
+            [&](int t) { return rho[(long long)t * L.M + i]; }, [&](int t) { return drho[(long long)t * L.M + i]; },
+            [&](int k, double d) { jv[(long long)k * L.M + i] = d; });
 }
 
 // per-state direction v_t = v_{itvar(t)} (zero for frozen states), in T
@@ -1053,10 +1004,29 @@ static void require_products(const System& S) {
               "Jacobian products of range_restricted molecules are not built; solve with DIIS or Newton");
 }
 
+// the product of a 1-D system in one launch, where that applies
+static bool one_launch_product(System& S, Tangent& W, const double* v, double* jv, int precision, bool base) {
+  if (!S.one_launch(precision, true)) return false;
+  Scf1Args a = S.scf1_args();
+  a.base = base;
+  a.v = v;
+  a.dstore = W.dstore.p;
+  a.dphi_m = W.dphi_m.p;
+  a.jv = jv;
+  launch_scf1d(S.lat.d, a, true, S.stream);
+  if (base) {
+    S.gmax_valid = false;
+    S.phi_valid = true;
+    S.last_precision = precision;
+  }
+  return true;
+}
+
 // J v at the base state of the last compute_phi / residual at S.d_u.
 void jvp_at_base(System& S, const double* v, double* jv, int precision) {
   require_products(S);
   Tangent& W = tangent(S);
+  if (one_launch_product(S, W, v, jv, precision, false)) return;
   tangent_sweeps(S, W, v, precision, false);
   tangent_residual(S, W, v, jv);
 }
@@ -1069,6 +1039,7 @@ void jvp_internal(System& S, const double* v, double* jv, int precision) {
   if (S.has_range()) S.compute_phi(precision);  // phi stays defined after the refusal
   require_products(S);
   Tangent& W = tangent(S);
+  if (one_launch_product(S, W, v, jv, precision, true)) return;
   S.start_phi(precision);
   tangent_sweeps(S, W, v, precision, true);
   S.finish_phi(precision);

@@ -23,4 +23,40 @@ bool chain1d_ok(const DevLattice& L);
 void launch_chain1d(const DevLattice& L, const double* in0, const Chain1Step* steps, int n, double* last,
                     hipStream_t st);
 
+// a run of consecutive ranks of one state, and a molecule as k_scf1d sees it
+struct Chain1Run {
+  int state, count;
+};
+struct Chain1Mol {
+  int index, N, freedom, kind;
+  int run0, nruns;  // its runs, in rank order
+  unsigned uses;
+  int lo, hi;       // range_restricted: the box
+  double phib, theta, phi_range;
+};
+
+// arrays of a 1-D system as System holds them
+struct Scf1Args {
+  SysParams sp;
+  unsigned shared;        // states of more than one molecule
+  Chain1Mol mols[SFX_MAXM];  // in the order of evaluation
+  const Chain1Run* runs;
+  int nruns;
+  const double* u;
+  const unsigned char* itmask;
+  const double* fprof;
+  double* swf;
+  float* swf32;
+  double *store, *phi_m, *phi, *rho, *phitot, *molscal, *phib_state, *cbulk;
+  double* f;              // may be null: phi only
+  // tangent
+  int base;               // with the base evaluation
+  const double* v;
+  double *dstore, *dphi_m, *jv;
+};
+
+// one workgroup evaluates the whole system (up to 1024 layers whose arrays fit LDS)
+bool scf1d_ok(const DevLattice& L, int ns, bool tangent);
+void launch_scf1d(const DevLattice& L, const Scf1Args& a, bool tangent, hipStream_t st);
+
 }  // namespace sfx

@@ -66,6 +66,22 @@ __device__ __forceinline__ int nb(int c, int d, int n, int b1, int b2) {
   return v == 0 ? b1 : (v == n + 1 ? b2 : v);
 }
 
+// The 1-D step from a site's value b and its neighbours a below and c above
+// (Lat1DFlat1stO.cpp:44-46, Lat1DCyl1stO.cpp:22-23), rounded as written: every
+// kernel gives the same bits, and so does a layer's mirror image (a and c
+// exchanged), which lets a kernel compute the layers behind a bound as images
+template <typename T>
+__device__ __forceinline__ T step1_flat(T l1, T a, T b, T c) {
+#pragma clang fp contract(off)
+  return fma(l1, (a - b) + (c - b), b);
+}
+template <typename T>
+__device__ __forceinline__ T step1_curved(T lm, T lp, T a, T b, T c) {
+#pragma clang fp contract(off)
+  const T below = lm * (a - b), above = lp * (c - b);
+  return b + (below + above);
+}
+
 // Propagator stencil sum without the segment weight: sum_k lambda_k G(r+e_k).
 // Surface neighbours contribute zero. 1-D: Lat1DFlat1stO.cpp:44-46 and
 // Lat1DCyl1stO.cpp:22-23; 2-D: Lat2DFlat1stO.cpp:44, Lat2DCyl1stO.cpp:27-30;
@@ -76,8 +92,8 @@ __device__ __forceinline__ T stencil(const DevLattice& L, const T* __restrict__ 
     T b = G[x];
     T a = (x == 1) ? (L.surf1[0] ? T(0) : G[L.b1[0]]) : G[x - 1];
     T c = (x == L.nx) ? (L.surf2[0] ? T(0) : G[L.b2[0]]) : G[x + 1];
-    if (L.curved) return b + T(L.lm[x]) * (a - b) + T(L.lp[x]) * (c - b);
-    return b + T(L.l1) * (a - b - b + c);
+    if (L.curved) return step1_curved(T(L.lm[x]), T(L.lp[x]), a, b, c);
+    return step1_flat(T(L.l1), a, b, c);
   } else if constexpr (KIND == ST_2D) {
     const long long jx = L.jx;
     long long r = (long long)x * jx + y;
@@ -114,23 +130,25 @@ __device__ __forceinline__ T stencil(const DevLattice& L, const T* __restrict__ 
 // Weight of an interior site in ComputeLnGN (Lat1DFlat1stO.cpp:301-316,
 // Lat1DCyl1stO.cpp:258-270, Lat2DFlat1stO.cpp:293-330, Lat2DCyl1stO.cpp:388-438,
 // Lat3D1stO.cpp:345-370 via SubtractBoundaries).
-__device__ __forceinline__ double lngn_weight(const DevLattice& L, int x, int y, int z) {
+__device__ __forceinline__ double lngn_weight1(const DevLattice& L, int x) {  // 1-D
   double w = 1.0;
-  if (L.grad == 1) {
-    if (L.curved) {
-      w = L.Lw[x];
-      if (x == 1 && L.mirror2_1[0]) w *= 0.5;
-      if (x == L.nx && L.mirror2_2[0]) w *= 0.5;
-    } else {
-      if (x == 1) {
-        w = L.ladj;
-        if (L.mirror2_1[0]) w *= 0.5;
-      } else if (x == L.nx) {
-        w = L.mirror2_2[0] ? 0.5 : 2 - L.ladj;
-      }
+  if (L.curved) {
+    w = L.Lw[x];
+    if (x == 1 && L.mirror2_1[0]) w *= 0.5;
+    if (x == L.nx && L.mirror2_2[0]) w *= 0.5;
+  } else {
+    if (x == 1) {
+      w = L.ladj;
+      if (L.mirror2_1[0]) w *= 0.5;
+    } else if (x == L.nx) {
+      w = L.mirror2_2[0] ? 0.5 : 2 - L.ladj;
     }
-    return w;
   }
+  return w;
+}
+__device__ __forceinline__ double lngn_weight(const DevLattice& L, int x, int y, int z) {
+  if (L.grad == 1) return lngn_weight1(L, x);
+  double w = 1.0;
   int c[3] = {x, y, z};
   int n[3] = {L.nx, L.ny, L.nz};
   for (int k = 0; k < L.grad; k++) {
@@ -171,6 +189,25 @@ __device__ __forceinline__ double fe_weight(const DevLattice& L, int x, int y, i
   return w;
 }
 
+// contact average of a 1-D lattice, x not a halo layer unless of a surface
+// (Lat1DFlat.cpp:510-524, Lat1DCylinder.cpp:160-171)
+__device__ __forceinline__ double side_at1(const DevLattice& L, const double* __restrict__ P, int x) {
+  const long long M = L.MX;
+  if (x == 0) {
+    double lp = L.curved ? L.lpc[0] : L.l1chi;
+    return P[0] + lp * (-P[0] - P[0] + P[1]);
+  }
+  if (x == L.nx + 1) {
+    double lm = L.curved ? L.lmc[M - 1] : L.l1chi;
+    return P[M - 1] + lm * (-P[M - 1] - P[M - 1] + P[M - 2]);
+  }
+  const double b = P[x];
+  const double a = P[remap(x - 1, L.nx, L.surf1[0] ? 0 : L.b1[0], L.surf2[0] ? L.nx + 1 : L.b2[0])];
+  const double c = P[remap(x + 1, L.nx, L.surf1[0] ? 0 : L.b1[0], L.surf2[0] ? L.nx + 1 : L.b2[0])];
+  if (L.curved) return b + L.lpc[x] * (c - b) + L.lmc[x] * (a - b);
+  return b + L.l1chi * (a - b - b + c);
+}
+
 // contact averages <phi_t> (SideFraction / Sides) on every site
 __device__ inline double side_at(const DevLattice& L, const double* __restrict__ P, int x, int y, int z) {
   // remap halo coordinates that are not surfaces
@@ -190,21 +227,7 @@ __device__ inline double side_at(const DevLattice& L, const double* __restrict__
     if (L.grad >= 3) Z = remap(Z, L.nz, L.b1[2], L.b2[2]);
     return P[sidx(L, X, Y, Z)];
   };
-  if (L.grad == 1) {
-    // Lat1DFlat.cpp:510-524, Lat1DCylinder.cpp:160-171
-    const long long M = L.MX;
-    if (x == 0) {
-      double lp = L.curved ? L.lpc[0] : L.l1chi;
-      return P[0] + lp * (-P[0] - P[0] + P[1]);
-    }
-    if (x == L.nx + 1) {
-      double lm = L.curved ? L.lmc[M - 1] : L.l1chi;
-      return P[M - 1] + lm * (-P[M - 1] - P[M - 1] + P[M - 2]);
-    }
-    double b = P[x], a = at(x - 1, 0, 0), c = at(x + 1, 0, 0);
-    if (L.curved) return b + L.lpc[x] * (c - b) + L.lmc[x] * (a - b);
-    return b + L.l1chi * (a - b - b + c);
-  }
+  if (L.grad == 1) return side_at1(L, P, x);
   if (L.grad == 2) {
     // Lat2DFlat.cpp:996-1053, Lat2DCylinder.cpp:205-320 (standard lattice, l2 = 0)
     double b = P[sidx(L, x, y, 0)];

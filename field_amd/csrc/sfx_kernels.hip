@@ -6,7 +6,7 @@
 #include "sfx_device.h"
 #include <algorithm>
 
-#include "sfx_kernels.h"
+#include "sfx_scf.h"
 
 namespace sfx {
 
@@ -200,8 +200,7 @@ __global__ void k_wsum(DevLattice L, const T* __restrict__ G, double* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// Molecule scalars after a sweep (one thread). Normalisation per freedom:
-// SF_Monomer1stO.cpp:110-130, SF_Homopol1stO.cpp:599-619, SF_Copol1stO.cpp:1242-1275.
+// Molecule scalars after a sweep (mol_scalars), one workgroup
 __global__ void k_mol_finalize(MolParams mp, const double* __restrict__ partial, int nparts,
                                double* __restrict__ scal, const double* __restrict__ lnfN,
                                const double* __restrict__ allscal, int nmol) {
@@ -215,41 +214,9 @@ __global__ void k_mol_finalize(MolParams mp, const double* __restrict__ partial,
   if (threadIdx.x != 0) return;
   s = 0;
   for (int i = 0; i < (int)(blockDim.x >> 6); i++) s += red[i];
-  double lnsum = mp.kind == 3 ? log(s / 6.0) : log(s);  // second order: Lat3D2ndO.cpp:1024
-  double lnscale = lnfN ? *lnfN : 0.0;  // FP32: log-scale of the final rank
-  double lnGN = lnsum + lnscale;
-  double ref = scal[MS_REF];
-  double N = mp.N;
-  double phib = mp.phib, lnC, lnpref;
-  if (mp.freedom == SFX_SOLVENT) {
-    phib = 1.0;
-    for (int m = 0; m < nmol; m++)
-      if (m != mp.index) phib -= allscal[m * MS_COUNT + MS_PHIB];
-  }
-  // half-stored chains (SymMatrix1 factor 2); second order divides by 6 (Lat3D2ndO.cpp:1037)
-  double f = mp.kind == 2 ? 2.0 : mp.kind == 3 ? 1.0 / 6.0 : 1.0;
-  double pref;
-  if (mp.freedom == SFX_RANGE_RESTRICTED) {
-    // the profile before the range condition fixes its constant (k_range_finalize)
-    lnC = 0.0;
-    phib = 0.0;
-    pref = f * exp(ref);
-  } else if (mp.freedom == SFX_RESTRICTED) {
-    lnC = log(mp.theta) - lnGN - (mp.kind == 0 ? 0.0 : log(N));
-    phib = mp.theta / exp(lnGN);
-    lnpref = lnC;
-    pref = f * exp(lnpref + ref);
-  } else {
-    // phi = (phi_b / N) G G_inv / g: phi_b multiplies directly, since the
-    // solvent closure can make it negative (NormPhiFree, Lat1DFlat1stO.cpp:317-331)
-    const double C = mp.kind == 0 ? phib : phib / N;
-    lnC = log(C);  // NaN for phi_b <= 0, as ln of the reference's lnCb; used by the free energy only
-    pref = f * C * exp(ref);
-  }
-  scal[MS_LNGN] = lnGN;
-  scal[MS_LNC] = lnC;
-  scal[MS_PHIB] = phib;
-  scal[MS_PREF] = pref;
+  // FP32: log-scale of the final rank
+  mol_scalars(mp, s, lnfN ? *lnfN : 0.0, scal[MS_REF], nmol, [&](int m) { return allscal[m * MS_COUNT + MS_PHIB]; },
+              scal);
 }
 
 // phi_{m,t} = pref_m * acc_{m,t} / g_t (g>0, else 0); monomers phi = pref * g.
@@ -268,7 +235,7 @@ __global__ void k_mol_phi(DevLattice L, const A* __restrict__ acc, const A* __re
   if (monomer)
     v = pref * gv;
   else
-    v = gv > 0 ? (((double)acc[r] + (acc2 ? (double)acc2[r] : 0.0)) / gv) * pref : 0.0;
+    v = phi_site((double)acc[r] + (acc2 ? (double)acc2[r] : 0.0), gv, pref);
   phi_m[r] = v;
 }
 
@@ -282,9 +249,6 @@ void launch_set_ref_pair(double* scal, const double* lna, int ia, const double* 
 
 // state totals over molecules + frozen profiles, halos from their sources;
 // phitot on interior sites.
-__device__ void bulk_fractions(const SysParams& sp, const double* __restrict__ molscal, double* __restrict__ phib_state,
-                               double* __restrict__ cbulk);
-
 // state totals; the first thread also derives the bulk fractions and ChemIntBulk
 // from the molecules' phi_b (no dependence on the sites)
 __global__ void k_phi_total(DevLattice L, int nstates, int nmol, const double* __restrict__ phi_m,
@@ -323,40 +287,10 @@ __global__ void k_sides(DevLattice L, int nstates, const double* __restrict__ ph
   if (i >= L.M) return;
   int x, y, z;
   site_coords(L, i, x, y, z);
-  bool inside = is_interior(L, x, y, z);
-  bool surf = false;
-  if (!inside) {
-    int c[3] = {x, y, z}, n[3] = {L.nx, L.ny, L.nz};
-    for (int k = 0; k < L.grad; k++)
-      if ((c[k] == 0 && L.surf1[k]) || (c[k] == n[k] + 1 && L.surf2[k])) surf = true;
-  }
+  const bool side = has_side(L, x, y, z);
   for (int t = 0; t < nstates; t++) {
     const double* P = phi + (long long)t * L.M;
-    rho[(long long)t * L.M + i] = (inside || surf) ? side_at(L, P, x, y, z) : 0.0;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// segment bulk fractions and ChemIntBulk (SF_MolStructure.cpp:605-612,
-// SF_SegmentList.cpp:610-623); one thread
-__device__ void bulk_fractions(const SysParams& sp, const double* __restrict__ molscal, double* __restrict__ phib_state,
-                               double* __restrict__ cbulk) {
-  for (int t = 0; t < sp.ns; t++) {
-    double pb = 0;
-    if (sp.melt)
-      pb = sp.melt_phib[t];
-    else if (!sp.frozen[t])
-      for (int m = 0; m < sp.nm; m++) pb += molscal[m * MS_COUNT + MS_PHIB] * sp.mol_frac[m * SFX_MAXS + t];
-    phib_state[t] = pb;
-  }
-  for (int t = 0; t < sp.ns; t++) {
-    double c = 0;
-    if (!sp.frozen[t])
-      for (int j = 0; j < sp.ns; j++) {
-        double x = sp.chi[t * SFX_MAXS + j];
-        if (x != 0) c += x * phib_state[j];
-      }
-    cbulk[t] = c;
+    rho[(long long)t * L.M + i] = side ? side_at(L, P, x, y, z) : 0.0;
   }
 }
 
@@ -373,24 +307,9 @@ __global__ void k_residual(DevLattice L, SysParams sp, const unsigned char* __re
     for (int k = 0; k < nv; k++) f[(long long)k * L.M + i] = 0.0;
     return;
   }
-  double up[SFX_MAXS];
-  double pt = phitot[i];
-  double av = 0;
-  for (int k = 0; k < nv; k++) {
-    int t = sp.itvar_rep[k];
-    double ci = 0;
-    for (int j = 0; j < sp.ns; j++) {
-      double x = sp.chi[t * SFX_MAXS + j];
-      if (x != 0) ci += x * rho[(long long)j * L.M + i];
-    }
-    double v = -log(swf[(long long)t * L.M + i]);
-    v -= ci / pt;
-    v += cbulk[t];
-    up[k] = v;
-    av += v;
-  }
-  av /= nv;
-  for (int k = 0; k < nv; k++) f[(long long)k * L.M + i] = -1.0 + 1.0 / pt + up[k] - av;
+  residual_site(sp, phitot[i], cbulk, [&](int t) { return swf[(long long)t * L.M + i]; },
+                [&](int t) { return rho[(long long)t * L.M + i]; },
+                [&](int k, double v) { f[(long long)k * L.M + i] = v; });
 }
 
 // per-site free-energy density, block partials (SF_MolList1stO.cpp:815-940)
@@ -614,7 +533,7 @@ __global__ void k_mol_phi_states(DevLattice L, unsigned uses, int ns, const A* _
     if (!((uses >> t) & 1u)) continue;
     const long long i = (long long)t * L.M + r;
     const double gv = g[i];
-    phi_m[i] = gv > 0 ? (((double)acc[i] + (acc2 ? (double)acc2[i] : 0.0)) / gv) * pref : 0.0;
+    phi_m[i] = phi_site((double)acc[i] + (acc2 ? (double)acc2[i] : 0.0), gv, pref);
   }
 }
 
@@ -750,12 +669,7 @@ __global__ void k_range_finalize(const double* __restrict__ partial, int nparts,
   if (threadIdx.x != 0) return;
   s = 0;
   for (int i = 0; i < (int)(blockDim.x >> 6); i++) s += red[i];
-  const double C = phi_range / s;
-  scal[MS_RANGE_C] = C;
-  scal[MS_PREF] *= C;
-  scal[MS_LNC] = log(C);
-  // theta = sum_z L phi = C N G_N (every rank composes to G_N), so phi_b = theta / G_N = N C
-  scal[MS_PHIB] = (double)N * C;
+  range_scalars(s, phi_range, N, scal);
 }
 
 __global__ void k_range_scale(DevLattice L, unsigned uses, int ns, const double* __restrict__ scal,

@@ -155,6 +155,13 @@ struct System {
   // one launch of the stretch `which` of molecule m (building its list on
   // first use from the host steps)
   void chain1_run(int m, int which, const std::vector<Chain1Step>& host, const double* in0, double* last);
+  // a 1-D system evaluated by one workgroup in one launch (sfx_chain1d.hip):
+  // FP64, full store, no kernel timing (which reports per-rank launches)
+  bool one_launch(int precision, bool tangent) const;
+  Scf1Args scf1_args();  // the system's arrays; builds the list of runs on first use
+  std::vector<Chain1Mol> scf1_mols;
+  int scf1_nruns = 0;
+  Chain1Run* scf1_runs = nullptr;
   SysParams sp{};
   hipStream_t stream = nullptr;      // where every call of this system runs
   hipStream_t own_stream = nullptr;  // created with the system, used unless a caller sets one

@@ -69,7 +69,7 @@ System::~System() {
   void* ptrs[] = {d_u, d_f, d_swf, d_swf32, d_phi_m, d_acc, d_acc2, d_phi, d_rho, d_phitot, d_fprof, d_frozen,
                   d_st_itvar, d_mol_uses, d_itmask, d_sites, d_store, d_pp, d_pp2, d_molscal, d_lnf, d_lnb,
                   d_maxf, d_maxb, d_partial, d_phib_state, d_cbulk, d_scalar, d_xabi, d_gmax,
-                  d_abi_in, d_abi_out};
+                  d_abi_in, d_abi_out, scf1_runs};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   tangent_free(tan);
@@ -884,7 +884,70 @@ void System::start_phi(int prec) {
   }
 }
 
+bool System::one_launch(int prec, bool tangent) const {
+  return prec == SFX_FP64 && use_chain1 && !checkpointed && !prof.on && scf1d_ok(lat.d, ns, tangent);
+}
+
+Scf1Args System::scf1_args() {
+  if (!scf1_runs) {
+    std::vector<Chain1Mol> hm;
+    std::vector<Chain1Run> hr;
+    for (int pass = 0; pass < 2; pass++)  // non-solvent molecules first, as compute_phi
+      for (int m = 0; m < nm; m++) {
+        const Molecule& mo = mols[m];
+        if ((pass == 0) == (mo.freedom == SFX_SOLVENT)) continue;
+        Chain1Mol c{m, mo.N, mo.freedom, mo.kind, (int)hr.size(), 0, mo.uses_mask(), mo.range.lo[0], mo.range.hi[0],
+                    mo.phib, mo.theta, mo.phi_range};
+        for (int s = 0; s < mo.N; s++) {
+          if (s == 0 || mo.seq[s] != mo.seq[s - 1]) {
+            hr.push_back(Chain1Run{mo.seq[s], 0});
+            c.nruns++;
+          }
+          hr.back().count++;
+        }
+        hm.push_back(c);
+      }
+    Chain1Run* dr = dalloc<Chain1Run>(hr.size());
+    const hipError_t e = hipMemcpy(dr, hr.data(), hr.size() * sizeof(Chain1Run), hipMemcpyHostToDevice);
+    scf1_runs = dr;
+    SFX_HIP(e);
+    scf1_nruns = (int)hr.size();
+    scf1_mols = hm;
+  }
+  Scf1Args a{};
+  a.sp = sp;
+  unsigned seen = 0;
+  for (const Molecule& mo : mols) {
+    a.shared |= seen & mo.uses_mask();
+    seen |= mo.uses_mask();
+  }
+  std::copy(scf1_mols.begin(), scf1_mols.end(), a.mols);
+  a.nruns = scf1_nruns;
+  a.runs = scf1_runs;
+  a.u = d_u;
+  a.itmask = d_itmask;
+  a.fprof = d_fprof;
+  a.swf = d_swf;
+  a.swf32 = d_swf32;
+  a.store = (double*)d_store;
+  a.phi_m = d_phi_m;
+  a.phi = d_phi;
+  a.rho = d_rho;
+  a.phitot = d_phitot;
+  a.molscal = d_molscal;
+  a.phib_state = d_phib_state;
+  a.cbulk = d_cbulk;
+  return a;
+}
+
 void System::compute_phi(int prec) {
+  if (one_launch(prec, false)) {
+    launch_scf1d(lat.d, scf1_args(), false, stream);
+    gmax_valid = false;
+    phi_valid = true;
+    last_precision = prec;
+    return;
+  }
   start_phi(prec);
   // non-solvent molecules first, the solvent closes phi_b (SF_MolList1stO.cpp:280-292)
   for (int pass = 0; pass < 2; pass++)
@@ -946,6 +1009,15 @@ void System::finish_range(int m) {
 }
 
 void System::residual_internal(int prec) {
+  if (one_launch(prec, false)) {
+    Scf1Args a = scf1_args();
+    a.f = d_f;
+    launch_scf1d(lat.d, a, false, stream);
+    gmax_valid = false;
+    phi_valid = true;
+    last_precision = prec;
+    return;
+  }
   compute_phi(prec);
   launch_residual(lat.d, sp, d_itmask, d_swf, d_rho, d_phitot, d_cbulk, d_f, stream);
   SFX_HIP(hipGetLastError());
