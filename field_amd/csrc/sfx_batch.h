@@ -14,7 +14,7 @@ struct BatchProb {
   double chi_as, chi_s;
   double phib;         // homopolymer bulk volume fraction
   long long xoff;      // offset of its iteration vector (2n values)
-  long long soff;      // offset of its propagator store (N/2 ranks x (n+2))
+  long long soff;      // offset of its propagator store (every second of N/2 ranks x (n+2))
   long long hoff;      // offset of its DIIS history
   long long poff;      // offset of its phi output (2 x (n+2))
 };

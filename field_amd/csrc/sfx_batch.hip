@@ -15,8 +15,10 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 #include "sfx_batch.h"
+#include "sfx_chain1w.h"
 
 namespace sfx {
 
@@ -36,131 +38,172 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
 }
 
 // The residual of problem b at x, by the workgroup that owns it; every
-// thread of the workgroup calls it. LDS holds two ping-pong rank buffers of
-// ldsw doubles; index 0 of both stays 0 (the frozen surface layer), so the
-// lower neighbour needs no branch; the mirror1 neighbour of layer n is n.
-template <int BT>
+// thread of the workgroup calls it. The running rank is in the registers of
+// the workgroup (Chain1, K layers per lane). Of the first half's ranks the odd
+// ones go to HBM; they come back well ahead of their use, and an even one is a
+// step from the one below it, beside the running rank's own step. LDS: the two
+// exchange buffers of ldsw doubles.
+//
+// What bounds it, at 512 problems of up to 400 layers and 1000 segments: the
+// stored ranks' bytes (120 MB out, 150 MB back) and the vector units, which
+// about 2400 waves share. A residual takes 111 us (at 256 or 512 threads a
+// problem); with every rank stored 150 us; with the running rank in LDS, two
+// buffers and a barrier per rank, and every rank stored, 309 us. One layer per
+// lane for the problems that fit it, beside two for the larger ones of the same
+// batch, measured no faster.
+template <int BT, int K>
 __device__ void batch_residual(const BatchProb& p, int b, const double* __restrict__ x, double* __restrict__ f,
                                double* __restrict__ store, double* __restrict__ phi_out,
                                double* __restrict__ lngn, double* lds, int ldsw) {
-  constexpr int K = kMaxLayers / BT;  // layers per thread
+  constexpr int kBlock = K <= 2 ? 8 : K <= 5 ? 4 : 2, kRing = kBlock;  // ranks; stored rows of twice as many ranks
   __shared__ double red[BT / 64];
   const int n = p.n, N = p.N;
   const long long M = n + 2;
   const double l = p.lambda;
   const double* xb = x + p.xoff;
   double* st = store + p.soff;
-  double* cur = lds;
-  double* nxt = lds + ldsw;
   const int t = threadIdx.x;
 
-  double gA[K], gS[K], acc[K], pr[K];
+  DevLattice L{};  // surface below (the frozen wall), mirror1 above
+  L.nx = n;
+  L.l1 = l;
+  L.surf1[0] = 1;
+  Chain1<K, false, false, true> c;
+  c.init(L, ldsw, lds);
+  if (t == 0) lds[0] = lds[ldsw] = 0.0;  // read by slots without a layer; the first exchange comes after a barrier
+  double gS[K], acc[K];
 #pragma unroll
-  for (int k = 0; k < K; k++) {
-    const int z = 1 + t + k * BT;
-    gA[k] = gS[k] = acc[k] = pr[k] = 0.0;
-    if (z <= n) {
-      gA[k] = exp(-xb[2 * (z - 1)]);      // SWF of A (SF_Solve.cpp:794-852)
-      gS[k] = exp(-xb[2 * (z - 1) + 1]);  // SWF of S
-      cur[z] = gA[k];                     // rank 1
-      st[z] = gA[k];
-    }
-  }
-  if (t == 0) {
-    cur[0] = 0.0;
-    nxt[0] = 0.0;
+  for (int j = 0; j < K; j++) {
+    gS[j] = acc[j] = 0.0;
+    c.g[j] = c.x[j] >= 1 ? exp(-xb[2 * (c.x[j] - 1)]) : 0.0;             // SWF of A (SF_Solve.cpp:794-852)
+    if (c.to[j] <= n) gS[j] = exp(-xb[2 * (c.to[j] - 1) + 1]);           // SWF of S
   }
   __syncthreads();
-
-  // G_s(z) = g(z) [G(z) + l (G(z-1) - 2 G(z) + G(z+1))] on the previous rank
-#define SFX_STEP(k, z) (gA[k] * (cur[z] + l * (cur[(z) - 1] - 2.0 * cur[z] + ((z) == n ? cur[z] : cur[(z) + 1]))))
-
+  c.rank1();
   const int h = N / 2;
-  for (int s = 2; s <= h; s++) {  // stored ranks 2..N/2
-    double* row = st + (long long)(s - 1) * M;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-      const int z = 1 + t + k * BT;
-      if (z <= n) {
-        const double v = SFX_STEP(k, z);
-        nxt[z] = v;
-        row[z] = v;
-      }
+  double* row = st;
+  if (c.active) c.put(row, nullptr);
+  // ranks 2..N/2, the odd ones stored
+  auto forward = [&](bool odd) __attribute__((always_inline)) {
+    c.step();
+    if (odd) {
+      row += M;
+      c.put(row, nullptr);
     }
-    __syncthreads();
-    double* tmp = cur;
-    cur = nxt;
-    nxt = tmp;
+  };
+  for (int s = 2; s <= h; s += kBlock) {
+    const int cnt = min(kBlock, h - s + 1);
+    c.room(cnt);
+    if (!c.active) continue;
+    if (cnt == kBlock) {
+#pragma unroll
+      for (int d = 0; d < kBlock; d++) forward(d & 1);
+    } else {
+#pragma unroll 1
+      for (int d = 0; d < cnt; d++) forward(d & 1);
+    }
   }
   if (N & 1) {  // middle rank of an odd chain meets itself
+    c.room(1);
+    c.step();
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-      const int z = 1 + t + k * BT;
-      if (z <= n) {
-        const double v = SFX_STEP(k, z);
-        nxt[z] = v;
-        acc[k] += 0.5 * v * v;
+    for (int j = 0; j < K; j++) acc[j] = 0.5 * c.G[j] * c.G[j];
+  }
+  // a wave reads its neighbours' layers of the stored ranks, too: every store
+  // of the workgroup is done before the first load
+  __threadfence_block();
+  __syncthreads();
+  // ranks h+1.. (h+2.. if N is odd) to N pair with rank N-s+1: rank h down to
+  // rank 1, an even one a step from the stored odd one below it
+  double pr[kRing][K];
+  auto fetch = [&](int d) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < K; j++) pr[d][j] = c.at(row, c.x[j]);
+    row -= row != st ? M : 0;
+  };
+  auto compose = [&](const double (&q)[K]) __attribute__((always_inline)) {
+    c.step();
+#pragma unroll
+    for (int j = 0; j < K; j++) acc[j] = fma(c.G[j], q[j], acc[j]);
+  };
+  auto two = [&](const double (&q)[K]) __attribute__((always_inline)) {
+    double e[K];
+    c.average(q, e);
+#pragma unroll
+    for (int j = 0; j < K; j++) e[j] *= c.g[j];
+    compose(e);
+    compose(q);
+  };
+  if (h & 1) {
+    c.room(1);
+    if (c.active) {
+      fetch(0);
+      compose(pr[0]);
+    }
+  }
+  if (c.active) {
+#pragma unroll
+    for (int d = 0; d < kRing; d++) fetch(d);
+  }
+  for (int k = 0, pairs = h / 2; k < pairs;) {
+#pragma unroll
+    for (int o = 0; o < kRing; o += kBlock / 2) {
+      const int cnt = min(kBlock / 2, pairs - k);
+      if (cnt > 0) {
+        c.room(2 * cnt);
+        if (c.active) {
+          if (cnt == kBlock / 2) {
+#pragma unroll
+            for (int d = o; d < o + kBlock / 2; d++) two(pr[d]);
+          } else {
+#pragma unroll 1
+            for (int d = 0; d < cnt; d++) {
+              double q[K];
+#pragma unroll
+              for (int j = 0; j < K; j++) {
+                q[j] = pr[o][j];
+#pragma unroll
+                for (int e = 1; e < kBlock / 2; e++) {
+                  q[j] = d == e ? pr[o + e][j] : q[j];
+                  asm volatile("" : "+v"(q[j]));  // keeps the ring in registers
+                }
+              }
+              two(q);
+            }
+          }
+          if (k + kRing < pairs) {
+#pragma unroll
+            for (int d = 0; d < kBlock / 2; d++) fetch(o + d);
+          }
+        }
+        k += cnt;
       }
     }
-    __syncthreads();
-    double* tmp = cur;
-    cur = nxt;
-    nxt = tmp;
   }
-  // ranks N/2+1..N pair with the stored rank N-s+1; each thread reads back
-  // only the layers it wrote itself, one rank ahead
-  const int s0 = (N + 3) / 2;
-  {
-    const double* row = st + (long long)(N - s0) * M;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-      const int z = 1 + t + k * BT;
-      if (z <= n) pr[k] = row[z];
-    }
-  }
-  for (int s = s0; s <= N; s++) {
-    const double* next_row = st + (long long)(N - s - 1) * M;  // read only while s < N
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-      const int z = 1 + t + k * BT;
-      if (z <= n) {
-        const double v = SFX_STEP(k, z);
-        nxt[z] = v;
-        acc[k] += v * pr[k];
-        if (s < N) pr[k] = next_row[z];
-      }
-    }
-    __syncthreads();
-    double* tmp = cur;
-    cur = nxt;
-    nxt = tmp;
-  }
-#undef SFX_STEP
 
   // ln G_N over the interior (Lat1DFlat1stO.cpp:301-316, layer weight 1)
-  double w = 0;
+  __syncthreads();  // the exchange buffers are free
 #pragma unroll
-  for (int k = 0; k < K; k++) {
-    const int z = 1 + t + k * BT;
-    if (z <= n) w += cur[z];
-  }
+  for (int j = 0; j < K; j++) lds[c.to[j]] = c.G[j];
+  __syncthreads();
+  double w = 0;
+  for (int z = 1 + t; z <= n; z += BT) w += lds[z];
   const double GN = block_sum<BT>(w, red);
   if (t == 0 && lngn) lngn[b] = log(GN);
 
   // phi_A = 2 (phi_b / N) acc / g (free homopolymer, half store), phi_S = (1 - phi_b) g_S
   const double CA = 2.0 * p.phib / N, phibS = 1.0 - p.phib;
-  double* phA = cur;  // block_sum synchronised: every thread is done with the rank buffers
-  double* phS = nxt;
+  double* phA = lds;  // block_sum synchronised: every thread is done with the exchange buffers
+  double* phS = lds + ldsw;
   double vA[K], vS[K];
 #pragma unroll
-  for (int k = 0; k < K; k++) {
-    const int z = 1 + t + k * BT;
-    vA[k] = vS[k] = 0.0;
-    if (z <= n) {
-      vA[k] = gA[k] > 0 ? CA * acc[k] / gA[k] : 0.0;
-      vS[k] = phibS * gS[k];
-      phA[z] = vA[k];
-      phS[z] = vS[k];
+  for (int j = 0; j < K; j++) {
+    vA[j] = vS[j] = 0.0;
+    if (c.to[j] <= n) {
+      vA[j] = c.g[j] > 0 ? CA * acc[j] / c.g[j] : 0.0;
+      vS[j] = phibS * gS[j];
+      phA[c.to[j]] = vA[j];
+      phS[c.to[j]] = vS[j];
     }
   }
   __syncthreads();
@@ -176,17 +219,17 @@ __device__ void batch_residual(const BatchProb& p, int b, const double* __restri
   const double cbA = p.chi_as * phibS, cbS = p.chi_as * p.phib;
   double* fb = f + p.xoff;
 #pragma unroll
-  for (int k = 0; k < K; k++) {
-    const int z = 1 + t + k * BT;
+  for (int j = 0; j < K; j++) {
+    const int z = c.to[j];
     if (z <= n) {
       const double upA = z == n ? phA[n] : phA[z + 1];
       const double upS = z == n ? phS[n] : phS[z + 1];
-      const double sA = vA[k] + l * (phA[z - 1] - 2.0 * vA[k] + upA);
-      const double sS = vS[k] + l * (phS[z - 1] - 2.0 * vS[k] + upS);
+      const double sA = vA[j] + l * (phA[z - 1] - 2.0 * vA[j] + upA);
+      const double sS = vS[j] + l * (phS[z - 1] - 2.0 * vS[j] + upS);
       const double sW = z == 1 ? l : 0.0;  // the wall (phi 1 in layer 0) seen from layer 1
-      const double pt = vA[k] + vS[k];
-      const double uA = -log(gA[k]) - (p.chi_as * sS + p.chi_s * sW) / pt + cbA;
-      const double uS = -log(gS[k]) - (p.chi_as * sA) / pt + cbS;
+      const double pt = vA[j] + vS[j];
+      const double uA = -log(c.g[j]) - (p.chi_as * sS + p.chi_s * sW) / pt + cbA;
+      const double uS = -log(gS[j]) - (p.chi_as * sA) / pt + cbS;
       const double av = 0.5 * (uA + uS);
       fb[2 * (z - 1)] = -1.0 + 1.0 / pt + uA - av;
       fb[2 * (z - 1) + 1] = -1.0 + 1.0 / pt + uS - av;
@@ -194,7 +237,7 @@ __device__ void batch_residual(const BatchProb& p, int b, const double* __restri
   }
 }
 
-template <int BT>
+template <int BT, int K>
 __global__ void __launch_bounds__(BT) k_batch_residual(const BatchProb* __restrict__ P, const double* __restrict__ x,
                                                        double* __restrict__ f, double* __restrict__ store,
                                                        double* __restrict__ phi_out, double* __restrict__ lngn,
@@ -203,7 +246,7 @@ __global__ void __launch_bounds__(BT) k_batch_residual(const BatchProb* __restri
   const int b = blockIdx.x;
   if (active && !active[b]) return;
   const BatchProb p = P[b];
-  batch_residual<BT>(p, b, x, f, store, phi_out, lngn, lds, ldsw);
+  batch_residual<BT, K>(p, b, x, f, store, phi_out, lngn, lds, ldsw);
 }
 
 // Sums four values over the workgroup in a fixed order; every thread gets
@@ -421,7 +464,7 @@ __device__ bool batch_diis(const BatchProb& p, int b, double* __restrict__ x, co
 // iteration limit, non-finite or given up). Problems are independent, so no
 // workgroup ever waits on another and the launch ends when the slowest
 // problem does; the host neither synchronises nor relaunches per iteration.
-template <int BT>
+template <int BT, int K>
 __global__ void __launch_bounds__(BT) k_batch_solve(const BatchProb* __restrict__ P, double* __restrict__ x,
                                                     double* __restrict__ f, double* __restrict__ store,
                                                     double* __restrict__ phi_out, double* __restrict__ lngn,
@@ -431,7 +474,7 @@ __global__ void __launch_bounds__(BT) k_batch_solve(const BatchProb* __restrict_
   const int b = blockIdx.x;
   const BatchProb p = P[b];
   while (true) {
-    batch_residual<BT>(p, b, x, f, store, phi_out, lngn, lds, ldsw);
+    batch_residual<BT, K>(p, b, x, f, store, phi_out, lngn, lds, ldsw);
     __syncthreads();  // f and the rank buffers are read by other threads below
     if (batch_diis<BT>(p, b, x, f, hist, S, m, eta, tol, max_iter, backtrack)) break;
   }
@@ -478,7 +521,7 @@ void Batch::create(const sfx_adsorption_desc* d, int count, const sfx_options* o
     p.poff = po;
     p.hoff = 0;
     xo += 2LL * p.n;
-    so += (long long)(p.N / 2) * (p.n + 2);
+    so += (long long)((p.N / 2 + 1) / 2) * (p.n + 2);
     po += 2LL * (p.n + 2);
     n_max = std::max(n_max, p.n);
   }
@@ -495,42 +538,47 @@ void Batch::create(const sfx_adsorption_desc* d, int count, const sfx_options* o
   SFX_HIP(hipMalloc(&d_state, B * sizeof(BatchState)));
   SFX_HIP(hipMemcpy(d_prob, probs.data(), B * sizeof(BatchProb), hipMemcpyHostToDevice));
   SFX_HIP(hipMemset(d_x, 0, nvar * sizeof(double)));
+  SFX_HIP(hipMemset(d_store, 0, store_words * sizeof(double)));  // entry 0 of a row is the surface layer, never written
   tune();
 }
+
+// go(BT, K) with the fewest layers per lane that hold n layers in bt threads
+// (a wave owns 64 K - 16): one layer per lane is the shortest chain of
+// dependent operations per rank
+template <class F>
+static void by_threads(int bt, int n, F&& go) {
+  using std::integral_constant;
+#define TRY(BT, K)                                                       \
+  if (bt == BT && n <= BT / 64 * chain1_owned(K)) {                      \
+    go(integral_constant<int, BT>{}, integral_constant<int, K>{});       \
+    return;                                                              \
+  }
+  TRY(64, 2) TRY(64, 4) TRY(64, 8) TRY(64, 17)
+  TRY(128, 1) TRY(128, 2) TRY(128, 4) TRY(128, 9)
+  TRY(256, 1) TRY(256, 2) TRY(256, 5)
+  TRY(512, 1) TRY(512, 2) TRY(512, 3)
+#undef TRY
+  throw Error{SFX_E_INVALID, "no kernel for this many threads and layers"};
+}
+static_assert(kMaxLayers <= chain1_owned(17) && kMaxLayers <= 2 * chain1_owned(9) &&
+                  kMaxLayers <= 4 * chain1_owned(5) && kMaxLayers <= 8 * chain1_owned(3),
+              "every number of threads holds the largest lattice");
 
 void Batch::launch_residual(int bt, const int* active) {
   const int ldsw = n_max + 2;
   const size_t shm = 2 * (size_t)ldsw * sizeof(double);
-  switch (bt) {
-    case 64:
-      k_batch_residual<64><<<B, 64, shm, stream>>>(d_prob, d_x, d_f, d_store, d_phi, d_lngn, active, ldsw);
-      break;
-    case 128:
-      k_batch_residual<128><<<B, 128, shm, stream>>>(d_prob, d_x, d_f, d_store, d_phi, d_lngn, active, ldsw);
-      break;
-    case 256:
-      k_batch_residual<256><<<B, 256, shm, stream>>>(d_prob, d_x, d_f, d_store, d_phi, d_lngn, active, ldsw);
-      break;
-    default:
-      k_batch_residual<512><<<B, 512, shm, stream>>>(d_prob, d_x, d_f, d_store, d_phi, d_lngn, active, ldsw);
-      break;
-  }
+  by_threads(bt, n_max, [&](auto BT, auto K) {
+    k_batch_residual<BT(), K()><<<B, BT(), shm, stream>>>(d_prob, d_x, d_f, d_store, d_phi, d_lngn, active, ldsw);
+  });
   SFX_HIP(hipGetLastError());
 }
-
 void Batch::launch_solve(int bt, int m, double eta, double tol, int max_iter, int backtrack) {
   const int ldsw = n_max + 2;
   const size_t shm = 2 * (size_t)ldsw * sizeof(double);
-#define SOLVE(BT)                                                                                              \
-  k_batch_solve<BT><<<B, BT, shm, stream>>>(d_prob, d_x, d_f, d_store, d_phi, d_lngn, d_hist, d_state, m, eta, \
-                                            tol, max_iter, backtrack, ldsw)
-  switch (bt) {
-    case 64: SOLVE(64); break;
-    case 128: SOLVE(128); break;
-    case 256: SOLVE(256); break;
-    default: SOLVE(512); break;
-  }
-#undef SOLVE
+  by_threads(bt, n_max, [&](auto BT, auto K) {
+    k_batch_solve<BT(), K()><<<B, BT(), shm, stream>>>(d_prob, d_x, d_f, d_store, d_phi, d_lngn, d_hist, d_state, m,
+                                                       eta, tol, max_iter, backtrack, ldsw);
+  });
   SFX_HIP(hipGetLastError());
 }
 
