@@ -450,7 +450,7 @@ static void base_phi(System& S, int m, int nb, const double* lnfinal) {
   const Molecule& mo = S.mols[m];
   const size_t off = (size_t)m * S.ns * S.lat.d.M;
   double* scal = S.d_molscal + (size_t)m * MS_COUNT;
-  const bool two = sizeof(T) == 4 && S.middle_out(mo);
+  const bool two = S.middle_out(mo);
   launch_mol_finalize(mo.params(m), S.d_partial, nb, scal, lnfinal, S.d_molscal, S.nm, S.stream);
   launch_mol_phi_states<T>(S.lat.d, mo.uses_mask(), S.ns, (const T*)S.d_acc + off,
                            two ? (const T*)S.d_acc2 + off : nullptr, S.d_swf, scal, S.d_phi_m + off, S.stream);
@@ -463,9 +463,12 @@ static void base_phi(System& S, int m, int nb, const double* lnfinal) {
 // writes one word more per site-rank beside the ten of the tangent's, where
 // the base sweep moves nine); otherwise the base phi_m comes from the last
 // compute_phi at the same x.
-// FP32 tangent sweep of a first-order chain on the 3-D simple-cubic lattice,
-// several ranks per launch (sfx_block3.hip); the structure of tsweep below.
-static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const float* g32, bool base) {
+// Tangent sweep of a first-order chain on a blocked lattice, several ranks per
+// launch (sfx_block3.hip, sfx_block2.hip); the structure of tsweep below.
+template <typename T>
+static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* vt, const T* g32, bool base) {
+  const int grid = block_ranks(S.lat.d, true, sizeof(T) == 8);
+  constexpr int P = sizeof(T) == 4 ? SFX_FP32 : SFX_FP64;
   const DevLattice& L = S.lat.d;
   const long long Mn = L.M;
   Molecule& mo = S.mols[m];
@@ -475,13 +478,13 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
   double* lnb = S.d_lnb + (size_t)m * (S.maxN + 2);
   unsigned* maxf = S.d_maxf + (size_t)m * (S.maxN + 2) * kStepWords;
   unsigned* maxb = S.d_maxb + (size_t)m * (S.maxN + 2) * kStepWords;
-  float* store = (float*)S.d_store;
-  float* dstore = (float*)W.dstore.p;
-  float* pp[2] = {(float*)S.d_pp, (float*)S.d_pp + Mn};
-  float* dpp[2] = {(float*)W.dpp.p, (float*)W.dpp.p + Mn};
-  float* dacc = (float*)W.dacc.p;
+  T* store = (T*)S.d_store;
+  T* dstore = (T*)W.dstore.p;
+  T* pp[2] = {(T*)S.d_pp, (T*)S.d_pp + Mn};
+  T* dpp[2] = {(T*)W.dpp.p, (T*)W.dpp.p + Mn};
+  T* dacc = (T*)W.dacc.p;
   auto daccp = [&](int t) { return dacc + ((size_t)m * S.ns + t) * Mn; };
-  auto accp = [&](int t) { return base ? (float*)S.d_acc + ((size_t)m * S.ns + t) * Mn : nullptr; };
+  auto accp = [&](int t) { return base ? (T*)S.d_acc + ((size_t)m * S.ns + t) * Mn : nullptr; };
   auto gp = [&](int t) { return g32 + (size_t)t * Mn; };
   auto vp = [&](int t) { return vt + (size_t)t * Mn; };
   auto slot = [&](int i) { return store + (size_t)i * Mn; };
@@ -490,31 +493,35 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
   const ChainPlan& plan = mo.plan;
   {
     ZeroList zl;
+    const long long words = Mn * (long long)(sizeof(T) / 4);
     for (int t = 0; t < S.ns; t++)
       if (mo.uses[t]) {
         const size_t off = ((size_t)m * S.ns + t) * Mn;
-        zero_list_add(zl, daccp(t), Mn, st);
-        if (base) zero_list_add(zl, accp(t), Mn, st);
+        zero_list_add(zl, daccp(t), words, st);
+        if (base) zero_list_add(zl, accp(t), words, st);
         if (S.middle_out(mo)) {
-          zero_list_add(zl, (float*)W.dacc2.p + off, Mn, st);
-          if (base) zero_list_add(zl, (float*)S.d_acc2 + off, Mn, st);
+          zero_list_add(zl, (T*)W.dacc2.p + off, words, st);
+          if (base) zero_list_add(zl, (T*)S.d_acc2 + off, words, st);
         }
       }
-    zero_list_add(zl, maxf, (long long)(S.maxN + 2) * kStepWords, st);
-    zero_list_add(zl, maxb, (long long)(S.maxN + 2) * kStepWords, st);
+    if (scaled) {
+      zero_list_add(zl, maxf, (long long)(N + 2) * kStepWords, st);
+      zero_list_add(zl, maxb, (long long)(N + 2) * kStepWords, st);
+    }
     launch_zero_list(zl, st);
   }
-  auto fsc = [&](int step, int pair) { return RankScale{maxf, lnf, lnf, scal + MS_REF, step, pair}; };
-  auto bsc = [&](int step, int pair) { return RankScale{maxb, lnb, lnf, scal + MS_REF, step, pair}; };
+  RankScale none{nullptr, nullptr, nullptr, nullptr, 0, 0};
+  auto fsc = [&](int step, int pair) { return scaled ? RankScale{maxf, lnf, lnf, scal + MS_REF, step, pair} : none; };
+  auto bsc = [&](int step, int pair) { return scaled ? RankScale{maxb, lnb, lnf, scal + MS_REF, step, pair} : none; };
   auto state_of_rank = [&](int s) { return mo.seq[s - 1]; };
   auto nosplit = [](int) { return false; };
   // the arguments of ranks sa..sb of a chain from (in, din); with an
   // accumulator each rank is composed with the ranks in slots pslots[k],
   // whose log scale is lnpair[pidx[k]]
-  auto args = [&](int sa, int sb, const float* in, const float* din, int t, unsigned* maxv, double* lnv,
-                  const double* lnpair, float* const* outs, float* const* douts, const int* pslots, const int* pidx,
-                  float* acc_t, float* bacc_t) {
-    B3Args<float> a{};
+  auto args = [&](int sa, int sb, const T* in, const T* din, int t, unsigned* maxv, double* lnv,
+                  const double* lnpair, T* const* outs, T* const* douts, const int* pslots, const int* pidx,
+                  T* acc_t, T* bacc_t) {
+    B3Args<T> a{};
     a.in = in;
     a.din = din;
     a.g = gp(t);
@@ -531,23 +538,25 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
     }
     a.acc = acc_t;
     a.bacc = bacc_t;
-    a.maxv = maxv;
-    a.lnv = lnv;
-    a.lnpair = lnpair;
-    a.ref = scal + MS_REF;
-    a.gmax = S.d_gmax + (size_t)t * kStepWords;
+    if (scaled) {
+      a.maxv = maxv;
+      a.lnv = lnv;
+      a.lnpair = lnpair;
+      a.ref = scal + MS_REF;
+      a.gmax = S.d_gmax + (size_t)t * kStepWords;
+    }
     a.s0 = sa - 1;
     return a;
   };
-  auto go = [&](const B3Launch<float>& la, bool connect) {
+  auto go = [&](const B3Launch<T>& la, bool connect) {
     int nr = 0;
     for (int c = 0; c < la.nchains; c++) nr += la.a[c].nr;
-    const auto ev = S.prof.events(connect ? 3 : 2, SFX_FP32, nr);
-    launch_block3<float>(L, la, true, true, connect, st, ev.first, ev.second);
+    const auto ev = S.prof.events(connect ? 3 : 2, P, nr);
+    launch_block3<T>(L, la, true, scaled, connect, st, ev.first, ev.second);
   };
   auto launch = [&](int sa, int sb, int in_slot_or_pp, bool in_is_pp, int t, unsigned* maxv, double* lnv,
-                    float* const* outs, float* const* douts, const int* pslots, const int* pidx, bool connect) {
-    B3Launch<float> la{};
+                    T* const* outs, T* const* douts, const int* pslots, const int* pidx, bool connect) {
+    B3Launch<T> la{};
     la.a[0] = args(sa, sb, in_is_pp ? pp[in_slot_or_pp] : slot(in_slot_or_pp),
                    in_is_pp ? dpp[in_slot_or_pp] : dslot(in_slot_or_pp), t, maxv, lnv, lnf, outs, douts, pslots,
                    pidx, connect ? daccp(t) : nullptr, connect ? accp(t) : nullptr);
@@ -557,25 +566,25 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
   if (S.middle_out(mo)) {
     // the schedule of System::sweep_blocked's middle-out branch, with tangents
     const int h = N / 2;
-    float* dacc2 = (float*)W.dacc2.p;
+    T* dacc2 = (T*)W.dacc2.p;
     auto dacc2p = [&](int t) { return dacc2 + ((size_t)m * S.ns + t) * Mn; };
-    auto acc2p = [&](int t) { return base ? (float*)S.d_acc2 + ((size_t)m * S.ns + t) * Mn : nullptr; };
-    float* qq[2] = {(float*)W.dpp2.p, (float*)W.dpp2.p + Mn};  // backward running rank
-    float* dqq[2] = {(float*)W.dpp2.p + 2 * Mn, (float*)W.dpp2.p + 3 * Mn};
+    auto acc2p = [&](int t) { return base ? (T*)S.d_acc2 + ((size_t)m * S.ns + t) * Mn : nullptr; };
+    T* qq[2] = {(T*)S.d_pp2, (T*)S.d_pp2 + Mn};  // backward running rank
+    T* dqq[2] = {(T*)W.dpp2.p, (T*)W.dpp2.p + Mn};
     // (the second accumulators were cleared with the first above)
     auto rank_of = [&](int k) { return N - k + 1; };
     auto bstate = [&](int k) { return mo.seq[rank_of(k) - 1]; };
     const int tN = mo.seq[N - 1];
-    tinit2<float>(L, TInit<float>{gp(mo.seq[0]), vp(mo.seq[0]), slot(0), dslot(0), fsc(1, 0)},
-                  TInit<float>{gp(tN), vp(tN), slot(N - 1), dslot(N - 1), bsc(1, N)}, st);
-    const auto F1 = chain_launches(2, h, 2, state_of_rank);
-    const auto B1 = chain_launches(2, N - h, 2, bstate);
+    tinit2<T>(L, TInit<T>{gp(mo.seq[0]), vp(mo.seq[0]), slot(0), dslot(0), fsc(1, 0)},
+                  TInit<T>{gp(tN), vp(tN), slot(N - 1), dslot(N - 1), bsc(1, N)}, st);
+    const auto F1 = chain_launches(2, h, 2, state_of_rank, grid);
+    const auto B1 = chain_launches(2, N - h, 2, bstate, grid);
     for (size_t i = 0; i < std::max(F1.size(), B1.size()); i++) {
-      B3Launch<float> la{};
+      B3Launch<T> la{};
       if (i < F1.size()) {
         const int sa = F1[i].first, sb = F1[i].second;
-        float* outs[kB3Ranks] = {};
-        float* douts[kB3Ranks] = {};
+        T* outs[kBRanks] = {};
+        T* douts[kBRanks] = {};
         for (int s = sa; s <= sb; s++) {
           outs[s - sa] = slot(s - 1);
           douts[s - sa] = dslot(s - 1);
@@ -585,8 +594,8 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
       }
       if (i < B1.size()) {
         const int ka = B1[i].first, kb = B1[i].second;
-        float* outs[kB3Ranks] = {};
-        float* douts[kB3Ranks] = {};
+        T* outs[kBRanks] = {};
+        T* douts[kBRanks] = {};
         for (int k = ka; k <= kb; k++) {
           outs[k - ka] = slot(rank_of(k) - 1);
           douts[k - ka] = dslot(rank_of(k) - 1);
@@ -597,17 +606,17 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
       }
       go(la, false);
     }
-    launch_set_ref_pair(scal, lnf, h, lnb, N - h, st);
-    const auto F2 = chain_launches(h + 1, N, h + 1, state_of_rank);
-    const auto B2 = chain_launches(N - h + 1, N, N - h + 1, bstate);
+    launch_set_ref_pair(scal, scaled ? lnf : nullptr, h, lnb, N - h, st);
+    const auto F2 = chain_launches(h + 1, N, h + 1, state_of_rank, grid);
+    const auto B2 = chain_launches(N - h + 1, N, N - h + 1, bstate, grid);
     int fc = 0, bc = 0;
     for (size_t i = 0; i < std::max(F2.size(), B2.size()); i++) {
-      B3Launch<float> la{};
+      B3Launch<T> la{};
       if (i < F2.size()) {
         const int sa = F2[i].first, sb = F2[i].second;
-        float* outs[kB3Ranks] = {};
-        float* douts[kB3Ranks] = {};
-        int pslots[kB3Ranks] = {}, pidx[kB3Ranks] = {};
+        T* outs[kBRanks] = {};
+        T* douts[kBRanks] = {};
+        int pslots[kBRanks] = {}, pidx[kBRanks] = {};
         for (int s = sa; s <= sb; s++) {
           pslots[s - sa] = s - 1;  // backward rank s
           pidx[s - sa] = N - s + 1;
@@ -621,9 +630,9 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
       }
       if (i < B2.size()) {
         const int ka = B2[i].first, kb = B2[i].second;
-        float* outs[kB3Ranks] = {};
-        float* douts[kB3Ranks] = {};
-        int pslots[kB3Ranks] = {}, pidx[kB3Ranks] = {};
+        T* outs[kBRanks] = {};
+        T* douts[kBRanks] = {};
+        int pslots[kBRanks] = {}, pidx[kBRanks] = {};
         for (int k = ka; k <= kb; k++) {
           pslots[k - ka] = rank_of(k) - 1;  // forward rank
           pidx[k - ka] = rank_of(k);
@@ -638,17 +647,17 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
       go(la, true);
     }
     unsigned nb = grid1(L.V, kTB);
-    k_wsum2<float><<<nb, kTB, 0, st>>>(L, pp[fc], dpp[fc], S.d_partial, W.partial2.p);  // forward rank N
-    if (base) base_phi<float>(S, m, (int)nb, lnf + N);
+    k_wsum2<T><<<nb, kTB, 0, st>>>(L, pp[fc], dpp[fc], S.d_partial, W.partial2.p);  // forward rank N
+    if (base) base_phi<T>(S, m, (int)nb, scaled ? lnf + N : nullptr);
     k_tmol_finalize<<<1, 256, 0, st>>>(mo.params(m), S.d_partial, W.partial2.p, (int)nb, S.d_molscal, W.dmol.p, S.nm);
     return;
   }
-  tinit<float>(L, gp(mo.seq[0]), vp(mo.seq[0]), slot(0), dslot(0), fsc(1, 0), st);
+  tinit<T>(L, gp(mo.seq[0]), vp(mo.seq[0]), slot(0), dslot(0), fsc(1, 0), st);
   {
     int prev = 0, parity = 0;
     chain_blocks(2, plan.n, 2, state_of_rank, nosplit, [&](int sa, int sb) {
-      float* outs[kB3Ranks] = {};
-      float* douts[kB3Ranks] = {};
+      T* outs[kBRanks] = {};
+      T* douts[kBRanks] = {};
       int last = -1;
       for (int s = sa; s <= sb; s++) {
         int d = -1;
@@ -665,7 +674,7 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
       launch(sa, sb, prev, false, mo.seq[sa - 1], maxf, lnf, outs, douts, nullptr, nullptr, false);
       if (plan.c && last == plan.seg(parity)) parity ^= 1;
       prev = last;
-    });
+    }, grid);
   }
   int resident[2] = {-1, -1};
   auto get = [&](int s) -> int {
@@ -676,37 +685,37 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
       const int end = std::min(start + plan.c - 1, plan.n);
       int prev = j;
       chain_blocks(start + 1, end, 2, state_of_rank, nosplit, [&](int sa, int sb) {
-        float* outs[kB3Ranks] = {};
-        float* douts[kB3Ranks] = {};
+        T* outs[kBRanks] = {};
+        T* douts[kBRanks] = {};
         for (int s2 = sa; s2 <= sb; s2++) {
           outs[s2 - sa] = slot(plan.seg_in(set, s2 - start - 1));
           douts[s2 - sa] = dslot(plan.seg_in(set, s2 - start - 1));
         }
         launch(sa, sb, prev, false, mo.seq[sa - 1], maxf, lnf, outs, douts, nullptr, nullptr, false);
         prev = plan.seg_in(set, sb - start - 1);
-      });
+      }, grid);
       resident[set] = j;
     }
     return plan.seg_in(set, s - start - 1);
   };
   int cur = 0;
-  const float* fin = nullptr;
-  const float* dfin = nullptr;
+  const T* fin = nullptr;
+  const T* dfin = nullptr;
   if (mo.kind == 1) {
-    k_set_ref2<<<1, 1, 0, st>>>(scal, lnf, N, 1.0);
+    k_set_ref2<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, N, 1.0);
     const int tN = mo.seq[N - 1];
-    tinit<float>(L, gp(tN), vp(tN), pp[0], dpp[0], bsc(1, N), st);
+    tinit<T>(L, gp(tN), vp(tN), pp[0], dpp[0], bsc(1, N), st);
     const int iN = get(N);
-    k_tconnect<float, true><<<grid1(L.V, kTB), kTB, 0, st>>>(L, pp[0], dpp[0], slot(iN), dslot(iN), daccp(tN),
+    k_tconnect<T, sizeof(T) == 4><<<grid1(L.V, kTB), kTB, 0, st>>>(L, pp[0], dpp[0], slot(iN), dslot(iN), daccp(tN),
                                                              accp(tN), bsc(1, N), 1.0);
     auto rank_of = [&](int k) { return N - k + 1; };
     chain_blocks(
         2, N, 2, [&](int k) { return mo.seq[rank_of(k) - 1]; },
         nosplit,
         [&](int ka, int kb) {
-          float* outs[kB3Ranks] = {};
-          float* douts[kB3Ranks] = {};
-          int pslots[kB3Ranks] = {}, pidx[kB3Ranks] = {};
+          T* outs[kBRanks] = {};
+          T* douts[kBRanks] = {};
+          int pslots[kBRanks] = {}, pidx[kBRanks] = {};
           for (int k = ka; k <= kb; k++) {
             pslots[k - ka] = get(rank_of(k));
             pidx[k - ka] = rank_of(k);
@@ -715,28 +724,28 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
           douts[kb - ka] = dpp[cur ^ 1];
           launch(ka, kb, cur, true, mo.seq[rank_of(ka) - 1], maxb, lnb, outs, douts, pslots, pidx, true);
           cur ^= 1;
-        });
+        }, grid);
   } else {
     const int h = N / 2;
-    k_set_ref2<<<1, 1, 0, st>>>(scal, lnf, h, 2.0);
+    k_set_ref2<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, h, 2.0);
     const int ih = get(h);
-    launch_copy_interior<float>(L, slot(ih), pp[0], st);
-    launch_copy_interior<float>(L, dslot(ih), dpp[0], st);
+    launch_copy_interior<T>(L, slot(ih), pp[0], st);
+    launch_copy_interior<T>(L, dslot(ih), dpp[0], st);
     if (N % 2 == 1) {
       const int s = h + 1, t = mo.seq[s - 1];
-      tprop<float>(L, pp[0], dpp[0], gp(t), vp(t), pp[1], dpp[1], nullptr, nullptr, nullptr, nullptr, fsc(s, 0),
+      tprop<T>(L, pp[0], dpp[0], gp(t), vp(t), pp[1], dpp[1], nullptr, nullptr, nullptr, nullptr, fsc(s, 0),
                    st);
       cur = 1;
-      k_tconnect<float, true><<<grid1(L.V, kTB), kTB, 0, st>>>(L, pp[cur], dpp[cur], pp[cur], dpp[cur], daccp(t),
+      k_tconnect<T, sizeof(T) == 4><<<grid1(L.V, kTB), kTB, 0, st>>>(L, pp[cur], dpp[cur], pp[cur], dpp[cur], daccp(t),
                                                                accp(t), fsc(s, s), 0.5);
     }
     auto pair_of = [&](int s) { return N - s + 1; };
     chain_blocks(
         (N + 3) / 2, N, 2, state_of_rank, nosplit,
         [&](int sa, int sb) {
-          float* outs[kB3Ranks] = {};
-          float* douts[kB3Ranks] = {};
-          int pslots[kB3Ranks] = {}, pidx[kB3Ranks] = {};
+          T* outs[kBRanks] = {};
+          T* douts[kBRanks] = {};
+          int pslots[kBRanks] = {}, pidx[kBRanks] = {};
           for (int s = sa; s <= sb; s++) {
             pslots[s - sa] = get(pair_of(s));
             pidx[s - sa] = pair_of(s);
@@ -745,25 +754,22 @@ static void tsweep_blocked(System& S, Tangent& W, int m, const float* vt, const 
           douts[sb - sa] = dpp[cur ^ 1];
           launch(sa, sb, cur, true, mo.seq[sa - 1], maxf, lnf, outs, douts, pslots, pidx, true);
           cur ^= 1;
-        });
+        }, grid);
   }
   fin = pp[cur];
   dfin = dpp[cur];
   unsigned nb = grid1(L.V, kTB);
-  k_wsum2<float><<<nb, kTB, 0, st>>>(L, fin, dfin, S.d_partial, W.partial2.p);
-  if (base) base_phi<float>(S, m, (int)nb, (mo.kind == 1 ? lnb : lnf) + N);
+  k_wsum2<T><<<nb, kTB, 0, st>>>(L, fin, dfin, S.d_partial, W.partial2.p);
+  if (base) base_phi<T>(S, m, (int)nb, scaled ? (mo.kind == 1 ? lnb : lnf) + N : nullptr);
   k_tmol_finalize<<<1, 256, 0, st>>>(mo.params(m), S.d_partial, W.partial2.p, (int)nb, S.d_molscal, W.dmol.p, S.nm);
 }
 
 template <typename T>
 static void tsweep(System& S, Tangent& W, int m, bool scaled, const T* vt, const T* g32or64, const double* v64,
                    bool base) {
-  if constexpr (std::is_same<T, float>::value) {
-    const int kind = S.mols[m].kind;
-    if (scaled && S.use_block3 && (kind == 1 || kind == 2)) {
-      tsweep_blocked(S, W, m, vt, g32or64, base);
-      return;
-    }
+  if (S.use_block3 && (S.mols[m].kind == 1 || S.mols[m].kind == 2)) {
+    tsweep_blocked<T>(S, W, m, scaled, vt, g32or64, base);
+    return;
   }
   const DevLattice& L = S.lat.d;
   const long long Mn = L.M;
@@ -940,9 +946,9 @@ static void tmol_phi(System& S, Tangent& W, int m, const double* v64state) {
   const DevLattice& L = S.lat.d;
   const long long Mn = L.M;
   Molecule& mo = S.mols[m];
-  // the FP32 blocked tangent sweep of a middle-out chain leaves half of the
-  // composition in the second accumulator
-  const bool two = sizeof(T) == 4 && S.middle_out(mo);
+  // the tangent sweep of a middle-out chain leaves half of the composition in
+  // the second accumulator
+  const bool two = S.middle_out(mo);
   const size_t off = (size_t)m * S.ns * Mn;
   k_tmol_phi<T><<<grid1(L.V, kTB), kTB, 0, S.stream>>>(
       L, mo.uses_mask(), S.ns, S.d_phi_m + off, (const T*)W.dacc.p + off, two ? (const T*)W.dacc2.p + off : nullptr,
@@ -1335,16 +1341,17 @@ void vjp_at_base(System& S, const double* w, double* jtw, int precision) {
       // the transposed sweep: the tangent sweep with direction phibar / D
       k_vjp_dir<<<nbM, kTB, 0, st>>>(L, uses, S.ns, W.phibar.p, W.xdir64.p, (float*)W.xdir32.p);
       const size_t off = (size_t)m * S.ns * Mn;
+      const bool two = S.middle_out(mo);
       if (fp32) {
         tsweep<float>(S, W, m, true, (const float*)W.xdir32.p, S.d_swf32, W.xdir64.p, false);
-        const bool two = S.middle_out(mo);
         k_vjp_sweep_term<float><<<nbV, kTB, 0, st>>>(L, uses, S.ns, (const float*)W.dacc.p + off,
                                                      two ? (const float*)W.dacc2.p + off : nullptr, S.d_swf,
                                                      W.dmol.p + m * 4, W.vbar.p);
       } else {
         tsweep<double>(S, W, m, false, W.xdir64.p, S.d_swf, W.xdir64.p, false);
-        k_vjp_sweep_term<double><<<nbV, kTB, 0, st>>>(L, uses, S.ns, (const double*)W.dacc.p + off, nullptr,
-                                                      S.d_swf, W.dmol.p + m * 4, W.vbar.p);
+        k_vjp_sweep_term<double><<<nbV, kTB, 0, st>>>(L, uses, S.ns, (const double*)W.dacc.p + off,
+                                                      two ? (const double*)W.dacc2.p + off : nullptr, S.d_swf,
+                                                      W.dmol.p + m * 4, W.vbar.p);
       }
     }
   k_vjp_final<<<nbM, kTB, 0, st>>>(Mn, S.n_itvar, S.ns, S.d_st_itvar, S.d_itmask, W.vbar.p, jtw);

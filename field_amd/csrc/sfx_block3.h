@@ -15,6 +15,14 @@ namespace sfx {
 // (forward / composing) for four ranks, 8.7 / 11.0 us for two; FP64 at 128^3:
 // 65 / 113 us against 32 / 64 us, the region read half as often.
 constexpr int kB3Ranks = 4;
+constexpr int kB2Ranks = 8;        // on a 2-D lattice (sfx_block2.hip)
+constexpr int kBRanks = kB2Ranks;  // the most of any
+// ranks per launch at most of a variant (FP64 tangents in 3-D: four would need
+// 87 KB of LDS, one workgroup per CU; by twos a product at 52 x 52 x 53, N = 60,
+// takes 469 us, rank by rank and with the base swept first 974)
+inline int block_ranks(const DevLattice& L, bool tangent, bool fp64) {
+  return L.grad == 2 ? kB2Ranks : tangent && fp64 ? 2 : kB3Ranks;
+}
 
 // Ranks s0+1 .. s0+nr of one chain, all of one segment state.
 template <typename T>
@@ -23,15 +31,16 @@ struct B3Args {
   const T* din;                // its tangent (tangent sweeps)
   const T* g;                  // SWF of the state
   const T* v;                  // tangent direction of the state
-  T* out[kB3Ranks];            // where rank s0+k goes (nullptr: not kept)
-  T* dout[kB3Ranks];
-  const T* pair[kB3Ranks];     // composition partner of rank s0+k
-  const T* dpair[kB3Ranks];
+  T* out[kBRanks];            // where rank s0+k goes (nullptr: not kept)
+  T* dout[kBRanks];
+  const T* pair[kBRanks];     // composition partner of rank s0+k
+  const T* dpair[kBRanks];
   T* acc;                      // accumulator of the state (phi, or dphi for tangents)
   T* bacc;                     // tangent sweeps: phi's accumulator too, unless the base has been swept (nullptr)
   int nr;
   // FP32 log-scaling: the input is divided by max(rank s0) (maxv[s0]) and
-  // every rank by the lattice maximum of g (gmax); lnv[s] is the log of the
+  // every rank by the lattice maximum of g (gmax), in two dimensions by the
+  // power of two above each; lnv[s] is the log of the
   // divisor accumulated up to rank s, lnpair[pidx[k]] that of the partner
   unsigned* maxv;
   double* lnv;
@@ -39,7 +48,7 @@ struct B3Args {
   const double* ref;
   const unsigned* gmax;        // step-max slots of the state's lattice maximum of g
   int s0;
-  int pidx[kB3Ranks];
+  int pidx[kBRanks];
 };
 
 // One launch advancing up to two independent chains (the forward and the
@@ -56,7 +65,7 @@ struct B3Launch {
 // grid makes the partition of any stretch that starts on a grid line equal
 // to that of the whole chain, so a recomputed stretch reproduces it bit for bit.
 template <class State, class Split, class F>
-void chain_blocks(int a, int b, int g0, State state, Split split, F f, int grid = kB3Ranks) {
+void chain_blocks(int a, int b, int g0, State state, Split split, F f, int grid) {
   int s = a;
   while (s <= b) {
     int e = s;
@@ -68,7 +77,7 @@ void chain_blocks(int a, int b, int g0, State state, Split split, F f, int grid 
 
 // the launches of chain_blocks(a, b, g0, state, no extra splits) as a list
 template <class State>
-std::vector<std::pair<int, int>> chain_launches(int a, int b, int g0, State state, int grid = kB3Ranks) {
+std::vector<std::pair<int, int>> chain_launches(int a, int b, int g0, State state, int grid) {
   std::vector<std::pair<int, int>> out;
   chain_blocks(
       a, b, g0, state, [](int) { return false; }, [&](int s, int e) { out.emplace_back(s, e); }, grid);
@@ -78,6 +87,8 @@ std::vector<std::pair<int, int>> chain_launches(int a, int b, int g0, State stat
 // true when the blocked sweep applies: 3-D simple cubic, first order, every
 // side at least kB3Ranks + 1 layers (one reflection reaches the interior)
 bool block3_ok(const DevLattice& L);
+// true when the blocked sweep of 2-D lattices applies: first order, its own adjoint, images inside
+bool block2_ok(const DevLattice& L);
 
 // ev0/ev1 (optional): timing events the dispatch records at kernel start and end
 template <typename T>
@@ -85,6 +96,10 @@ void launch_block3(const DevLattice& L, const B3Args<T>& a, bool tangent, bool s
                    hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 template <typename T>
 void launch_block3(const DevLattice& L, const B3Launch<T>& la, bool tangent, bool scaled, bool connect,
+                   hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+
+template <typename T>
+void launch_block2(const DevLattice& L, const B3Launch<T>& la, bool tangent, bool scaled, bool connect,
                    hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 
 // max over the interior of each state's FP32 SWF, into step-max slots

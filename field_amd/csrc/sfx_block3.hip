@@ -331,7 +331,7 @@ static void b3_launch_h(int nr, const DevLattice& L, const B3Launch<T>& a, unsig
     b3_launch<T, TG, SC, CN, 2>(L, a, nb, st, ev0, ev1);
     return;
   }
-  b3_launch<T, TG, SC, CN, kB3Ranks>(L, a, nb, st, ev0, ev1);
+  if constexpr (!(TG && sizeof(T) == 8)) b3_launch<T, TG, SC, CN, kB3Ranks>(L, a, nb, st, ev0, ev1);
 }
 
 template <typename T>
@@ -347,28 +347,26 @@ template <typename T>
 void launch_block3(const DevLattice& L, const B3Launch<T>& a, bool tangent, bool scaled, bool connect,
                    hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
   SFX_REQUIRE(a.nchains == 1 || a.nchains == 2, SFX_E_INVALID, "a blocked launch advances one or two chains");
+  if (L.grad == 2) {
+    launch_block2<T>(L, a, tangent, scaled, connect, st, ev0, ev1);
+    return;
+  }
   int nr = 0;
   for (int c = 0; c < a.nchains; c++) {
-    SFX_REQUIRE(a.a[c].nr >= 1 && a.a[c].nr <= kB3Ranks, SFX_E_INVALID, "blocked launch of 1..4 ranks");
+    SFX_REQUIRE(a.a[c].nr >= 1 && a.a[c].nr <= block_ranks(L, tangent, sizeof(T) == 8), SFX_E_INVALID,
+                "blocked launch of 1..4 ranks");
     nr = std::max(nr, a.a[c].nr);
   }
-  SFX_REQUIRE(!(tangent && sizeof(T) == 8), SFX_E_UNSUPPORTED, "FP64 tangent sweeps run rank by rank");
   const unsigned nb = (unsigned)(((L.nx + kTX - 1) / kTX) * ((L.ny + kTY - 1) / kTY) * ((L.nz + kTZ - 1) / kTZ));
 #define B3(TG, SC, CN) b3_launch_h<T, TG, SC, CN>(nr, L, a, nb, st, ev0, ev1)
-  if (tangent) {
-    if constexpr (sizeof(T) == 4) {
-      if (scaled) {
-        if (connect) B3(true, true, true); else B3(true, true, false);
-      } else {
-        if (connect) B3(true, false, true); else B3(true, false, false);
-      }
-    }
+  if constexpr (sizeof(T) == 4) {  // FP32 sweeps are scaled, FP64 ones are not
+    SFX_REQUIRE(scaled, SFX_E_INVALID, "FP32 blocked sweeps are scaled");
+    if (tangent) { if (connect) B3(true, true, true); else B3(true, true, false); }
+    else { if (connect) B3(false, true, true); else B3(false, true, false); }
   } else {
-    if (scaled) {
-      if (connect) B3(false, true, true); else B3(false, true, false);
-    } else {
-      if (connect) B3(false, false, true); else B3(false, false, false);
-    }
+    SFX_REQUIRE(!scaled, SFX_E_INVALID, "FP64 blocked sweeps are not scaled");
+    if (tangent) { if (connect) B3(true, false, true); else B3(true, false, false); }
+    else { if (connect) B3(false, false, true); else B3(false, false, false); }
   }
 #undef B3
   SFX_HIP(hipGetLastError());

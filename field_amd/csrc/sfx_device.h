@@ -82,6 +82,17 @@ __device__ __forceinline__ T step1_curved(T lm, T lp, T a, T b, T c) {
   return b + (below + above);
 }
 
+// The 2-D steps from a site's value b, its neighbours xm, xp along x and a, c along y
+// (Lat2DFlat1stO.cpp:44, Lat2DCyl1stO.cpp:27-30)
+template <typename T>
+__device__ __forceinline__ T step2_flat(T l0, T l1x, T l1y, T xm, T xp, T a, T c, T b) {
+  return l0 * b + l1y * (a + c) + l1x * (xm + xp);
+}
+template <typename T>
+__device__ __forceinline__ T step2_curved(T lm, T lp, T l1, T xm, T xp, T a, T c, T b) {
+  return b + lm * (xm - b) + lp * (xp - b) + l1 * (a + c - b - b);
+}
+
 // Propagator stencil sum without the segment weight: sum_k lambda_k G(r+e_k).
 // Surface neighbours contribute zero. 1-D: Lat1DFlat1stO.cpp:44-46 and
 // Lat1DCyl1stO.cpp:22-23; 2-D: Lat2DFlat1stO.cpp:44, Lat2DCyl1stO.cpp:27-30;
@@ -102,8 +113,8 @@ __device__ __forceinline__ T stencil(const DevLattice& L, const T* __restrict__ 
     T c = (y == L.ny) ? (L.surf2[1] ? T(0) : G[(long long)x * jx + L.b2[1]]) : G[r + 1];
     T xm = (x == 1) ? (L.surf1[0] ? T(0) : G[(long long)L.b1[0] * jx + y]) : G[r - jx];
     T xp = (x == L.nx) ? (L.surf2[0] ? T(0) : G[(long long)L.b2[0] * jx + y]) : G[r + jx];
-    if (L.curved) return b + T(L.lm[x]) * (xm - b) + T(L.lp[x]) * (xp - b) + T(L.l1) * (a + c - b - b);
-    return T(L.l0_2d) * b + T(L.l1y) * (a + c) + T(L.l1x) * (xm + xp);
+    if (L.curved) return step2_curved(T(L.lm[x]), T(L.lp[x]), T(L.l1), xm, xp, a, c, b);
+    return step2_flat(T(L.l0_2d), T(L.l1x), T(L.l1y), xm, xp, a, c, b);
   } else {
     const int nx = L.nx, ny = L.ny, nz = L.nz;
     auto at = [&](int dx, int dy, int dz) -> T {

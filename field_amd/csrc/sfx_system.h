@@ -146,7 +146,7 @@ struct System {
   int maxN = 1, maxstore = 1;
   int store_slots = 1;     // rank slots of the propagator store (all molecules share it)
   bool checkpointed = false;
-  bool use_block3 = false;  // blocked 3-D simple-cubic sweeps (sfx_options.sweep_kernel)
+  bool use_block3 = false;  // blocked sweeps of 3-D simple-cubic and 2-D lattices (sfx_options.sweep_kernel)
   bool use_chain1 = false;  // 1-D FP64 chains in one launch per stretch (sfx_options.sweep_kernel)
   // per molecule and stretch (0 forward, 1 backward, 2 half-store second half):
   // the step list on the device, built on the first sweep (its pointers never change)
@@ -258,6 +258,7 @@ struct System {
     return use_block3 && schedule == SFX_SCHEDULE_AUTO && mo.kind == 1 && !mo.plan.c && mo.N >= 2;
   }
   int schedule = SFX_SCHEDULE_AUTO;  // sfx_options.chain_schedule
+  int sweep_kernel = SFX_SWEEP_AUTO;  // sfx_options.sweep_kernel
   bool gmax_valid = false;           // d_gmax holds the maxima of the current FP32 SWF
 };
 

@@ -138,7 +138,7 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   precision = opt ? opt->precision : SFX_FP64;
   budget = opt ? opt->memory_budget : 0;
   {
-    const int sk = opt ? opt->sweep_kernel : SFX_SWEEP_AUTO;
+    const int sk = sweep_kernel = opt ? opt->sweep_kernel : SFX_SWEEP_AUTO;
     SFX_REQUIRE(sk >= SFX_SWEEP_AUTO && sk <= SFX_SWEEP_BLOCKED, SFX_E_INVALID, "unknown sweep_kernel");
     use_block3 = sk != SFX_SWEEP_PER_RANK && block3_ok(lat.d);
     use_chain1 = sk != SFX_SWEEP_PER_RANK && chain1d_ok(lat.d);
@@ -296,6 +296,11 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   const size_t slot_bytes = comps * M * sizeof(double);
   checkpointed = budget != 0 && (size_t)maxstore * slot_bytes > budget;
   store_slots = 1;
+  // 2-D: a checkpointed store and the sequential schedule keep one launch per
+  // rank, so that they repeat each other bit for bit within the memory they
+  // took before (blocked segments need two sets of slots)
+  if (sweep_kernel != SFX_SWEEP_PER_RANK && block2_ok(lat.d) && schedule == SFX_SCHEDULE_AUTO && !checkpointed)
+    use_block3 = true;
   for (Molecule& mo : mols) {
     mo.plan.init(mo.nstore, checkpointed, use_block3 ? kB3Ranks : 1);
     store_slots = std::max(store_slots, mo.plan.slots());
@@ -623,6 +628,7 @@ void System::sweep(int m, bool scaled) {
 template <typename T>
 void System::sweep_blocked(int m, bool scaled) {
   const DevLattice& L = lat.d;
+  const int grid = block_ranks(L, false, sizeof(T) == 8);
   const long long Mn = L.M;
   Molecule& mo = mols[m];
   hipStream_t st = stream;
@@ -705,20 +711,20 @@ void System::sweep_blocked(int m, bool scaled) {
     auto bstate = [&](int k) { return mo.seq[rank_of(k) - 1]; };
     launch_init_rank2<T>(L, InitRank<T>{gp(mo.seq[0]), slot(0), fsc(1, 0)},
                          InitRank<T>{gp(mo.seq[N - 1]), slot(N - 1), bsc(1, N)}, st);
-    const auto F1 = chain_launches(2, h, 2, state_of_rank);
-    const auto B1 = chain_launches(2, N - h, 2, bstate);
+    const auto F1 = chain_launches(2, h, 2, state_of_rank, grid);
+    const auto B1 = chain_launches(2, N - h, 2, bstate, grid);
     for (size_t i = 0; i < std::max(F1.size(), B1.size()); i++) {
       B3Launch<T> la{};
       if (i < F1.size()) {
         const int sa = F1[i].first, sb = F1[i].second;
-        const T* outs[kB3Ranks] = {};
+        const T* outs[kBRanks] = {};
         for (int s = sa; s <= sb; s++) outs[s - sa] = slot(s - 1);
         la.a[la.nchains++] = args(sa, sb, slot(sa - 2), mo.seq[sa - 1], maxf, lnf, nullptr, outs, nullptr, nullptr,
                                   nullptr);
       }
       if (i < B1.size()) {
         const int ka = B1[i].first, kb = B1[i].second;
-        const T* outs[kB3Ranks] = {};
+        const T* outs[kBRanks] = {};
         for (int k = ka; k <= kb; k++) outs[k - ka] = slot(rank_of(k) - 1);
         la.a[la.nchains++] = args(ka, kb, slot(rank_of(ka - 1) - 1), bstate(ka), maxb, lnb, nullptr, outs, nullptr,
                                   nullptr, nullptr);
@@ -726,16 +732,16 @@ void System::sweep_blocked(int m, bool scaled) {
       go(la, false);
     }
     launch_set_ref_pair(scal, scaled ? lnf : nullptr, h, lnb, N - h, st);
-    const auto F2 = chain_launches(h + 1, N, h + 1, state_of_rank);
-    const auto B2 = chain_launches(N - h + 1, N, N - h + 1, bstate);
+    const auto F2 = chain_launches(h + 1, N, h + 1, state_of_rank, grid);
+    const auto B2 = chain_launches(N - h + 1, N, N - h + 1, bstate, grid);
     int fc = 0, bc = 0;
     for (size_t i = 0; i < std::max(F2.size(), B2.size()); i++) {
       B3Launch<T> la{};
       if (i < F2.size()) {
         const int sa = F2[i].first, sb = F2[i].second;
-        const T* outs[kB3Ranks] = {};
-        const T* pairs[kB3Ranks] = {};
-        int pidx[kB3Ranks] = {};
+        const T* outs[kBRanks] = {};
+        const T* pairs[kBRanks] = {};
+        int pidx[kBRanks] = {};
         for (int s = sa; s <= sb; s++) {
           pairs[s - sa] = slot(s - 1);  // backward rank s
           pidx[s - sa] = N - s + 1;     // its backward step
@@ -747,9 +753,9 @@ void System::sweep_blocked(int m, bool scaled) {
       }
       if (i < B2.size()) {
         const int ka = B2[i].first, kb = B2[i].second;
-        const T* outs[kB3Ranks] = {};
-        const T* pairs[kB3Ranks] = {};
-        int pidx[kB3Ranks] = {};
+        const T* outs[kBRanks] = {};
+        const T* pairs[kBRanks] = {};
+        int pidx[kBRanks] = {};
         for (int k = ka; k <= kb; k++) {
           pairs[k - ka] = slot(rank_of(k) - 1);  // forward rank
           pidx[k - ka] = rank_of(k);
@@ -774,7 +780,7 @@ void System::sweep_blocked(int m, bool scaled) {
   {
     int prev = 0, parity = 0;
     chain_blocks(2, plan.n, 2, state_of_rank, nosplit, [&](int sa, int sb) {
-      const T* outs[kB3Ranks] = {};
+      const T* outs[kBRanks] = {};
       int last = -1;
       for (int s = sa; s <= sb; s++) {
         int d = -1;
@@ -790,7 +796,7 @@ void System::sweep_blocked(int m, bool scaled) {
       launch(sa, sb, slot(prev), mo.seq[sa - 1], maxf, lnf, outs, nullptr, nullptr, false);
       if (plan.c && last == plan.seg(parity)) parity ^= 1;
       prev = last;
-    });
+    }, grid);
   }
   // slot of forward rank s for requests in non-increasing s; recomputes a
   // checkpoint segment with the forward pass's own launch partition
@@ -803,11 +809,11 @@ void System::sweep_blocked(int m, bool scaled) {
       const int end = std::min(start + plan.c - 1, plan.n);
       int prev = j;
       chain_blocks(start + 1, end, 2, state_of_rank, nosplit, [&](int sa, int sb) {
-        const T* outs[kB3Ranks] = {};
+        const T* outs[kBRanks] = {};
         for (int s2 = sa; s2 <= sb; s2++) outs[s2 - sa] = slot(plan.seg_in(set, s2 - start - 1));
         launch(sa, sb, slot(prev), mo.seq[sa - 1], maxf, lnf, outs, nullptr, nullptr, false);
         prev = plan.seg_in(set, sb - start - 1);
-      });
+      }, grid);
       resident[set] = j;
     }
     return plan.seg_in(set, s - start - 1);
@@ -825,9 +831,9 @@ void System::sweep_blocked(int m, bool scaled) {
         2, N, 2, [&](int k) { return mo.seq[rank_of(k) - 1]; },
         nosplit,
         [&](int ka, int kb) {
-          const T* outs[kB3Ranks] = {};
-          const T* pairs[kB3Ranks] = {};
-          int pidx[kB3Ranks] = {};
+          const T* outs[kBRanks] = {};
+          const T* pairs[kBRanks] = {};
+          int pidx[kBRanks] = {};
           for (int k = ka; k <= kb; k++) {
             pairs[k - ka] = slot(get(rank_of(k)));
             pidx[k - ka] = rank_of(k);
@@ -835,7 +841,7 @@ void System::sweep_blocked(int m, bool scaled) {
           outs[kb - ka] = pp[cur ^ 1];
           launch(ka, kb, pp[cur], mo.seq[rank_of(ka) - 1], maxb, lnb, outs, pairs, pidx, true);
           cur ^= 1;
-        });
+        }, grid);
     final_G = pp[cur];
     lnfinal = scaled ? lnb + N : nullptr;
   } else {
@@ -853,9 +859,9 @@ void System::sweep_blocked(int m, bool scaled) {
         (N + 3) / 2, N, 2, state_of_rank,
         nosplit,
         [&](int sa, int sb) {
-          const T* outs[kB3Ranks] = {};
-          const T* pairs[kB3Ranks] = {};
-          int pidx[kB3Ranks] = {};
+          const T* outs[kBRanks] = {};
+          const T* pairs[kBRanks] = {};
+          int pidx[kBRanks] = {};
           for (int s = sa; s <= sb; s++) {
             pairs[s - sa] = slot(get(pair_of(s)));
             pidx[s - sa] = pair_of(s);
@@ -863,7 +869,7 @@ void System::sweep_blocked(int m, bool scaled) {
           outs[sb - sa] = pp[cur ^ 1];
           launch(sa, sb, pp[cur], mo.seq[sa - 1], maxf, lnf, outs, pairs, pidx, true);
           cur ^= 1;
-        });
+        }, grid);
     final_G = pp[cur];
     lnfinal = scaled ? lnf + N : nullptr;
   }
