@@ -38,7 +38,7 @@ static void zero(T* p, long long n, hipStream_t st) {
 struct Tangent {
   long long M = 0;
   int maxstore = 0;
-  DevBuf<double> dstore, dpp, dacc, dphi_m, dphi, drho, dphitot, dmol, v64, v32, partial2;
+  DevBuf<double> dstore, dpp, dacc, dphi_m, dphi, drho, dmol, v64, v32;
   // transposed products (allocated by the first VJP): per-state adjoints of
   // the contact averages, of phi and of the per-state direction, the total's
   // adjoint, and the per-state sweep direction (FP64 and FP32)
@@ -66,7 +66,6 @@ struct Tangent {
     dphi_m.alloc((size_t)S.nm * S.ns * M);
     dphi.alloc((size_t)S.ns * M);
     drho.alloc((size_t)S.ns * M);
-    dphitot.alloc((size_t)M);
     dmol.alloc((size_t)S.nm * 4);
     v64.alloc((size_t)S.ns * M);
     v32.alloc((size_t)S.ns * M);  // per-state FP32 directions (half used)
@@ -75,7 +74,6 @@ struct Tangent {
       dpp2.alloc(2 * (size_t)M);
       zero<double>(dpp2.p, 2 * (long long)M, S.stream);  // halo slots are never written
     }
-    partial2.alloc((size_t)S.npart);
   }
 };
 
@@ -228,175 +226,6 @@ __global__ void k_tconnect(DevLattice L, const T* __restrict__ A, const T* __res
   if (acc) acc[r] += A[r] * B[r] * c;
 }
 
-// two weighted sums at once: sum w G and sum w dG (per block)
-template <typename T>
-__global__ void k_wsum2(DevLattice L, const T* __restrict__ G, const T* __restrict__ dG, double* __restrict__ p1,
-                        double* __restrict__ p2) {
-  long long q = site_ordinal();
-  double a = 0, b = 0;
-  if (q < L.V) {
-    int x, y, z;
-    interior_coords(L, q, x, y, z);
-    long long r = sidx(L, x, y, z);
-    double w = lngn_weight(L, x, y, z);
-    a = (double)G[r] * w;
-    b = (double)dG[r] * w;
-  }
-  __shared__ double sa[kTB / 64], sb[kTB / 64];
-  for (int o = 32; o > 0; o >>= 1) {
-    a += __shfl_xor(a, o, 64);
-    b += __shfl_xor(b, o, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    sa[threadIdx.x >> 6] = a;
-    sb[threadIdx.x >> 6] = b;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double A = 0, B = 0;
-    for (int i = 0; i < (int)(blockDim.x >> 6); i++) {
-      A += sa[i];
-      B += sb[i];
-    }
-    p1[blockIdx.x] = A;
-    p2[blockIdx.x] = B;
-  }
-}
-
-// monomer: sum w g and sum w (-v g)
-__global__ void k_wsum_mono(DevLattice L, const double* __restrict__ g, const double* __restrict__ v,
-                            double* __restrict__ p1, double* __restrict__ p2) {
-  long long q = site_ordinal();
-  double a = 0, b = 0;
-  if (q < L.V) {
-    int x, y, z;
-    interior_coords(L, q, x, y, z);
-    long long r = sidx(L, x, y, z);
-    double w = lngn_weight(L, x, y, z);
-    a = g[r] * w;
-    b = -v[r] * g[r] * w;
-  }
-  __shared__ double sa[kTB / 64], sb[kTB / 64];
-  for (int o = 32; o > 0; o >>= 1) {
-    a += __shfl_xor(a, o, 64);
-    b += __shfl_xor(b, o, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    sa[threadIdx.x >> 6] = a;
-    sb[threadIdx.x >> 6] = b;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double A = 0, B = 0;
-    for (int i = 0; i < (int)(blockDim.x >> 6); i++) {
-      A += sa[i];
-      B += sb[i];
-    }
-    p1[blockIdx.x] = A;
-    p2[blockIdx.x] = B;
-  }
-}
-
-// tangent molecule scalars: dmol[0] = dlnGN, [1] = dpref/pref, [2] = dphib
-__global__ void k_tmol_finalize(MolParams mp, const double* p1, const double* p2, int n, const double* molscal,
-                                double* dmol, int nmol) {
-  __shared__ double r1[256 / 64], r2[256 / 64];
-  double s1 = 0, s2 = 0;
-  if (p1 && p2)
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      s1 += p1[i];
-      s2 += p2[i];
-    }
-  for (int o = 32; o > 0; o >>= 1) {
-    s1 += __shfl_xor(s1, o, 64);
-    s2 += __shfl_xor(s2, o, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    r1[threadIdx.x >> 6] = s1;
-    r2[threadIdx.x >> 6] = s2;
-  }
-  __syncthreads();
-  if (threadIdx.x || blockIdx.x) return;
-  s1 = s2 = 0;
-  for (int i = 0; i < (int)(blockDim.x >> 6); i++) {
-    s1 += r1[i];
-    s2 += r2[i];
-  }
-  tmol_scalars(mp, p1 && n > 0, s1, s2, molscal + mp.index * MS_COUNT, nmol, [&](int m) { return dmol[m * 4 + 2]; },
-               dmol + mp.index * 4);
-}
-
-// dphi_{m,t} at interior sites
-template <typename T>
-__global__ void k_tmol_phi(DevLattice L, unsigned uses, int ns, const double* __restrict__ phi_m,
-                           const T* __restrict__ dacc, const T* __restrict__ dacc2, const double* __restrict__ g,
-                           const double* __restrict__ v, const double* __restrict__ dm, int monomer,
-                           double* __restrict__ dphi_m) {
-  long long q = site_ordinal();
-  if (q >= L.V) return;
-  int x, y, z;
-  interior_coords(L, q, x, y, z);
-  const long long r0 = sidx(L, x, y, z);
-  for (int t = 0; t < ns; t++) {  // every state of the molecule (bit t of uses), arrays [state][M]
-    if (!((uses >> t) & 1u)) continue;
-    const long long r = (long long)t * L.M + r0;
-    const double da = monomer ? 0.0 : (double)dacc[r] + (dacc2 ? (double)dacc2[r] : 0.0);
-    dphi_m[r] = tphi_site(monomer != 0, phi_m[r], g[r], v[r], da, dm);
-  }
-}
-
-// tangent totals (frozen states have no tangent); halos from their sources
-__global__ void k_tphi_total(DevLattice L, int nstates, int nmol, const double* __restrict__ dphi_m,
-                             const int* __restrict__ mol_uses, const int* __restrict__ frozen,
-                             double* __restrict__ dphi, double* __restrict__ dphitot) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= L.M) return;
-  int x, y, z;
-  site_coords(L, i, x, y, z);
-  int sx = remap(x, L.nx, L.b1[0], L.b2[0]);
-  int sy = L.grad >= 2 ? remap(y, L.ny, L.b1[1], L.b2[1]) : y;
-  int sz = L.grad >= 3 ? remap(z, L.nz, L.b1[2], L.b2[2]) : z;
-  long long s = sidx(L, sx, sy, sz);
-  bool surf_halo = !is_interior(L, sx, sy, sz);
-  double tot = 0;
-  for (int t = 0; t < nstates; t++) {
-    double v = 0;
-    if (!frozen[t] && !surf_halo)
-      for (int m = 0; m < nmol; m++)
-        if (mol_uses[m * nstates + t]) v += dphi_m[((long long)m * nstates + t) * L.M + s];
-    dphi[(long long)t * L.M + i] = v;
-    tot += v;
-  }
-  dphitot[i] = tot;
-}
-
-__global__ void k_tsides(DevLattice L, int nstates, const double* __restrict__ dphi, double* __restrict__ drho) {
-  long long q = site_ordinal();
-  if (q >= L.V) return;
-  int x, y, z;
-  interior_coords(L, q, x, y, z);
-  long long r = sidx(L, x, y, z);
-  for (int t = 0; t < nstates; t++) drho[(long long)t * L.M + r] = side_at(L, dphi + (long long)t * L.M, x, y, z);
-}
-
-// linearised residual (SF_Solve.cpp:554-590)
-__global__ void k_jres(DevLattice L, SysParams sp, const unsigned char* __restrict__ itmask,
-                       const double* __restrict__ v, const double* __restrict__ rho,
-                       const double* __restrict__ drho, const double* __restrict__ phitot,
-                       const double* __restrict__ dphitot, const double* __restrict__ molscal,
-                       const double* __restrict__ dmol, double* __restrict__ jv) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= L.M) return;
-  const int nv = sp.n_itvar;
-  if (!itmask[i]) {
-    for (int k = 0; k < nv; k++) jv[(long long)k * L.M + i] = 0.0;
-    return;
-  }
-  jres_site(sp, phitot[i], dphitot[i], dmol, [&](int k) { return v[(long long)k * L.M + i]; },
-            [&](int t) { return rho[(long long)t * L.M + i]; }, [&](int t) { return drho[(long long)t * L.M + i]; },
-            [&](int k, double d) { jv[(long long)k * L.M + i] = d; });
-}
-
 // per-state direction v_t = v_{itvar(t)} (zero for frozen states), in T
 // (out32 optional: the same directions rounded to FP32)
 __global__ void k_state_dir(long long M, int ns, const int* st_itvar, const double* v, double* out,
@@ -440,20 +269,7 @@ static void tprop(const DevLattice& L, const T* Gin, const T* dGin, const T* g, 
 }
 
 static __global__ void k_set_ref2(double* scal, const double* lnv, int idx, double factor) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) scal[MS_REF] = lnv ? factor * lnv[idx] : 0.0;
-}
-
-// The base part of a sweep that carries base and tangent together: the
-// molecule's constants from the partial sums of its end rank, and its phi
-template <typename T>
-static void base_phi(System& S, int m, int nb, const double* lnfinal) {
-  const Molecule& mo = S.mols[m];
-  const size_t off = (size_t)m * S.ns * S.lat.d.M;
-  double* scal = S.d_molscal + (size_t)m * MS_COUNT;
-  const bool two = S.middle_out(mo);
-  launch_mol_finalize(mo.params(m), S.d_partial, nb, scal, lnfinal, S.d_molscal, S.nm, S.stream);
-  launch_mol_phi_states<T>(S.lat.d, mo.uses_mask(), S.ns, (const T*)S.d_acc + off,
-                           two ? (const T*)S.d_acc2 + off : nullptr, S.d_swf, scal, S.d_phi_m + off, S.stream);
+  if (threadIdx.x == 0 && blockIdx.x == 0) scal[MS_REF] = factor * lnv[idx];
 }
 
 // Tangent sweep of molecule m with per-state directions vt (type T, ns*M).
@@ -606,7 +422,7 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
       }
       go(la, false);
     }
-    launch_set_ref_pair(scal, scaled ? lnf : nullptr, h, lnb, N - h, st);
+    if (scaled) launch_set_ref_pair(scal, lnf, h, lnb, N - h, st);
     const auto F2 = chain_launches(h + 1, N, h + 1, state_of_rank, grid);
     const auto B2 = chain_launches(N - h + 1, N, N - h + 1, bstate, grid);
     int fc = 0, bc = 0;
@@ -646,10 +462,7 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
       }
       go(la, true);
     }
-    unsigned nb = grid1(L.V, kTB);
-    k_wsum2<T><<<nb, kTB, 0, st>>>(L, pp[fc], dpp[fc], S.d_partial, W.partial2.p);  // forward rank N
-    if (base) base_phi<T>(S, m, (int)nb, scaled ? lnf + N : nullptr);
-    k_tmol_finalize<<<1, 256, 0, st>>>(mo.params(m), S.d_partial, W.partial2.p, (int)nb, S.d_molscal, W.dmol.p, S.nm);
+    S.add_end(m, pp[fc], dpp[fc], sizeof(T) == 4, scaled ? lnf + N : nullptr);  // forward rank N
     return;
   }
   tinit<T>(L, gp(mo.seq[0]), vp(mo.seq[0]), slot(0), dslot(0), fsc(1, 0), st);
@@ -702,7 +515,7 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
   const T* fin = nullptr;
   const T* dfin = nullptr;
   if (mo.kind == 1) {
-    k_set_ref2<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, N, 1.0);
+    if (scaled) k_set_ref2<<<1, 1, 0, st>>>(scal, lnf, N, 1.0);
     const int tN = mo.seq[N - 1];
     tinit<T>(L, gp(tN), vp(tN), pp[0], dpp[0], bsc(1, N), st);
     const int iN = get(N);
@@ -727,17 +540,23 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
         }, grid);
   } else {
     const int h = N / 2;
-    k_set_ref2<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, h, 2.0);
-    const int ih = get(h);
-    launch_copy_interior<T>(L, slot(ih), pp[0], st);
-    launch_copy_interior<T>(L, dslot(ih), dpp[0], st);
+    if (scaled) k_set_ref2<<<1, 1, 0, st>>>(scal, lnf, h, 2.0);
+    int from = get(h);  // a stored rank; in a checkpoint segment, which is overwritten, copied
+    bool in_pp = plan.c;
+    if (in_pp) {
+      launch_copy_interior<T>(L, slot(from), pp[0], st);
+      launch_copy_interior<T>(L, dslot(from), dpp[0], st);
+      from = 0;
+    }
     if (N % 2 == 1) {
       const int s = h + 1, t = mo.seq[s - 1];
-      tprop<T>(L, pp[0], dpp[0], gp(t), vp(t), pp[1], dpp[1], nullptr, nullptr, nullptr, nullptr, fsc(s, 0),
+      tprop<T>(L, in_pp ? pp[0] : slot(from), in_pp ? dpp[0] : dslot(from), gp(t), vp(t), pp[1], dpp[1], nullptr, nullptr, nullptr, nullptr, fsc(s, 0),
                    st);
       cur = 1;
       k_tconnect<T, sizeof(T) == 4><<<grid1(L.V, kTB), kTB, 0, st>>>(L, pp[cur], dpp[cur], pp[cur], dpp[cur], daccp(t),
                                                                accp(t), fsc(s, s), 0.5);
+      from = cur;
+      in_pp = true;
     }
     auto pair_of = [&](int s) { return N - s + 1; };
     chain_blocks(
@@ -752,16 +571,14 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
           }
           outs[sb - sa] = pp[cur ^ 1];
           douts[sb - sa] = dpp[cur ^ 1];
-          launch(sa, sb, cur, true, mo.seq[sa - 1], maxf, lnf, outs, douts, pslots, pidx, true);
-          cur ^= 1;
+          launch(sa, sb, from, in_pp, mo.seq[sa - 1], maxf, lnf, outs, douts, pslots, pidx, true);
+          from = cur ^= 1;
+          in_pp = true;
         }, grid);
   }
   fin = pp[cur];
   dfin = dpp[cur];
-  unsigned nb = grid1(L.V, kTB);
-  k_wsum2<T><<<nb, kTB, 0, st>>>(L, fin, dfin, S.d_partial, W.partial2.p);
-  if (base) base_phi<T>(S, m, (int)nb, scaled ? (mo.kind == 1 ? lnb : lnf) + N : nullptr);
-  k_tmol_finalize<<<1, 256, 0, st>>>(mo.params(m), S.d_partial, W.partial2.p, (int)nb, S.d_molscal, W.dmol.p, S.nm);
+  S.add_end(m, fin, dfin, sizeof(T) == 4, scaled ? (mo.kind == 1 ? lnb : lnf) + N : nullptr);
 }
 
 template <typename T>
@@ -830,7 +647,7 @@ static void tsweep(System& S, Tangent& W, int m, bool scaled, const T* vt, const
     };
     chain_forward(plan, step);
     ChainReader<decltype(step)> rd{plan, step};
-    k_set_ref2<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, N, 1.0);
+    if (scaled) k_set_ref2<<<1, 1, 0, st>>>(scal, lnf, N, 1.0);
     auto bsc2 = [&](int step, int pair) {
       RankScale r = bsc(step, pair);
       if (scaled) r.pmaxv = maxf;
@@ -854,20 +671,10 @@ static void tsweep(System& S, Tangent& W, int m, bool scaled, const T* vt, const
                        dpp6[(k - 1) & 1], wp, dwp, daccp(t), Sst, bsc2(k, s), st, accp(t));
       S.prof.end(st);
     }
-    int nb = launch_wsum6<T>(L, pp6[(N - 1) & 1], dpp6[(N - 1) & 1], S.d_partial, W.partial2.p, st);
-    if (base) base_phi<T>(S, m, nb, scaled ? lnb + N : nullptr);
-    k_tmol_finalize<<<1, 256, 0, st>>>(mo.params(m), S.d_partial, W.partial2.p, nb, S.d_molscal, dm, S.nm);
+    S.add_end(m, pp6[(N - 1) & 1], dpp6[(N - 1) & 1], sizeof(T) == 4, scaled ? lnb + N : nullptr);
   } else if (mo.kind == 0) {
-    int t = mo.seq[0];
-    unsigned nb = grid1(L.V, kTB);
-    k_wsum_mono<<<nb, kTB, 0, st>>>(L, S.d_swf + (size_t)t * Mn, v64 + (size_t)t * Mn, S.d_partial, W.partial2.p);
-    if (base) {
-      k_set_ref2<<<1, 1, 0, st>>>(scal, nullptr, 0, 0.0);
-      launch_mol_finalize(mo.params(m), S.d_partial, (int)nb, scal, nullptr, S.d_molscal, S.nm, st);
-      launch_mol_phi<double>(L, nullptr, S.d_swf + (size_t)t * Mn, scal, 1, S.d_phi_m + ((size_t)m * S.ns + t) * Mn,
-                             st);
-    }
-    k_tmol_finalize<<<1, 256, 0, st>>>(mo.params(m), S.d_partial, W.partial2.p, (int)nb, S.d_molscal, dm, S.nm);
+    const size_t off = (size_t)mo.seq[0] * Mn;
+    S.add_end(m, S.d_swf + off, v64 + off, false, nullptr);
   } else {
     auto slot = [&](int i) { return store + (size_t)i * Mn; };
     auto dslot = [&](int i) { return dstore + (size_t)i * Mn; };
@@ -881,7 +688,7 @@ static void tsweep(System& S, Tangent& W, int m, bool scaled, const T* vt, const
     chain_forward(plan, step);  // ranks 2..N (full sweep) or 2..N/2 (half store)
     ChainReader<decltype(step)> rd{plan, step};
     if (mo.kind == 1) {
-      k_set_ref2<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, N, 1.0);
+      if (scaled) k_set_ref2<<<1, 1, 0, st>>>(scal, lnf, N, 1.0);
       int tN = mo.seq[N - 1];
       tinit<T>(L, gp(tN), vp(tN), pp[0], dpp[0], bsc(1, N), st);
       const int iN = rd.get(N);
@@ -904,16 +711,24 @@ static void tsweep(System& S, Tangent& W, int m, bool scaled, const T* vt, const
       dfin = dpp[(N - 1) & 1];
     } else {
       const int h = N / 2;
-      k_set_ref2<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, h, 2.0);
+      if (scaled) k_set_ref2<<<1, 1, 0, st>>>(scal, lnf, h, 2.0);
       const int ih = rd.get(h);
-      launch_copy_interior<T>(L, slot(ih), pp[0], st);
-      launch_copy_interior<T>(L, dslot(ih), dpp[0], st);
+      const T* from = slot(ih);
+      const T* dfrom = dslot(ih);
+      if (plan.c) {  // a checkpoint segment is overwritten
+        launch_copy_interior<T>(L, from, pp[0], st);
+        launch_copy_interior<T>(L, dfrom, dpp[0], st);
+        from = pp[0];
+        dfrom = dpp[0];
+      }
       int cur = 0;
       if (N % 2 == 1) {
         int s = h + 1, t = mo.seq[s - 1];
-        tprop<T>(L, pp[cur], dpp[cur], gp(t), vp(t), pp[cur ^ 1], dpp[cur ^ 1], nullptr, nullptr, nullptr, nullptr,
+        tprop<T>(L, from, dfrom, gp(t), vp(t), pp[cur ^ 1], dpp[cur ^ 1], nullptr, nullptr, nullptr, nullptr,
                  fsc(s, 0), st);
         cur ^= 1;
+        from = pp[cur];
+        dfrom = dpp[cur];
         RankScale c = fsc(s, s);
         if (scaled)
           k_tconnect<T, true><<<grid1(L.V, kTB), kTB, 0, st>>>(L, pp[cur], dpp[cur], pp[cur], dpp[cur], daccp(t), accp(t), c,
@@ -926,33 +741,18 @@ static void tsweep(System& S, Tangent& W, int m, bool scaled, const T* vt, const
         int sinv = N - s + 1, t = mo.seq[s - 1];
         const int is = rd.get(sinv);
         S.prof.begin(3, P, st);
-        tprop<T>(L, pp[cur], dpp[cur], gp(t), vp(t), pp[cur ^ 1], dpp[cur ^ 1], slot(is), dslot(is), daccp(t),
+        tprop<T>(L, from, dfrom, gp(t), vp(t), pp[cur ^ 1], dpp[cur ^ 1], slot(is), dslot(is), daccp(t),
                  accp(t), fsc(s, sinv), st);
         S.prof.end(st);
         cur ^= 1;
+        from = pp[cur];
+        dfrom = dpp[cur];
       }
       fin = pp[cur];
       dfin = dpp[cur];
     }
-    unsigned nb = grid1(L.V, kTB);
-    k_wsum2<T><<<nb, kTB, 0, st>>>(L, fin, dfin, S.d_partial, W.partial2.p);
-    if (base) base_phi<T>(S, m, (int)nb, scaled ? (mo.kind == 1 ? lnb : lnf) + N : nullptr);
-    k_tmol_finalize<<<1, 256, 0, st>>>(mo.params(m), S.d_partial, W.partial2.p, (int)nb, S.d_molscal, dm, S.nm);
+    S.add_end(m, fin, dfin, sizeof(T) == 4, scaled ? (mo.kind == 1 ? lnb : lnf) + N : nullptr);
   }
-}
-
-template <typename T>
-static void tmol_phi(System& S, Tangent& W, int m, const double* v64state) {
-  const DevLattice& L = S.lat.d;
-  const long long Mn = L.M;
-  Molecule& mo = S.mols[m];
-  // the tangent sweep of a middle-out chain leaves half of the composition in
-  // the second accumulator
-  const bool two = S.middle_out(mo);
-  const size_t off = (size_t)m * S.ns * Mn;
-  k_tmol_phi<T><<<grid1(L.V, kTB), kTB, 0, S.stream>>>(
-      L, mo.uses_mask(), S.ns, S.d_phi_m + off, (const T*)W.dacc.p + off, two ? (const T*)W.dacc2.p + off : nullptr,
-      S.d_swf, v64state, W.dmol.p + m * 4, mo.kind == 0, W.dphi_m.p + off);
 }
 
 void tangent_free(Tangent* t) { delete t; }
@@ -965,8 +765,8 @@ static Tangent& tangent(System& S) {
   return *S.tan;
 }
 
-// dphi of every molecule for the direction v; with `base` their phi as well
-// (tsweep)
+// the tangent sweeps of every molecule for the direction v and their closing;
+// with `base` the molecules' phi as well (tsweep)
 static void tangent_sweeps(System& S, Tangent& W, const double* v, int precision, bool base) {
   hipStream_t st = S.stream;
   const long long Mn = S.lat.d.M;
@@ -978,31 +778,46 @@ static void tangent_sweeps(System& S, Tangent& W, const double* v, int precision
     launch_gmax(S.lat.d, S.d_swf32, S.ns, S.d_gmax, st);
     S.gmax_valid = true;
   }
+  S.ends.n = 0;
   for (int pass = 0; pass < 2; pass++)
     for (int m = 0; m < S.nm; m++) {
       bool solv = S.mols[m].freedom == SFX_SOLVENT;
       if ((pass == 0) == solv) continue;
-      if (fp32) {
+      if (S.mols[m].kind != 0) S.close_ends(base, W.dmol.p);
+      if (fp32)
         tsweep<float>(S, W, m, true, v32, S.d_swf32, v64, base);
-        tmol_phi<float>(S, W, m, v64);
-      } else {
+      else
         tsweep<double>(S, W, m, false, v64, S.d_swf, v64, base);
-        tmol_phi<double>(S, W, m, v64);
-      }
     }
+  S.close_ends(base, W.dmol.p);
 }
 
-// the linearised residual from dphi
-static void tangent_residual(System& S, Tangent& W, const double* v, double* jv) {
-  const DevLattice& L = S.lat.d;
-  const long long Mn = L.M;
-  hipStream_t st = S.stream;
-  k_tphi_total<<<grid1(Mn, kTB), kTB, 0, st>>>(L, S.ns, S.nm, W.dphi_m.p, S.d_mol_uses, S.d_frozen, W.dphi.p,
-                                               W.dphitot.p);
-  k_tsides<<<grid1(L.V, kTB), kTB, 0, st>>>(L, S.ns, W.dphi.p, W.drho.p);
-  k_jres<<<grid1(Mn, kTB), kTB, 0, st>>>(L, S.sp, S.d_itmask, v, S.d_rho, W.drho.p, S.d_phitot, W.dphitot.p,
-                                         S.d_molscal, W.dmol.p, jv);
-  SFX_HIP(hipGetLastError());
+// phi (base), dphi, contact averages and the linearised residual
+static void tangent_close(System& S, Tangent& W, const double* v, double* jv, int precision, bool base) {
+  PhiArgs a = S.phi_args();
+  a.base = base;
+  a.tangent = true;
+  a.dacc = W.dacc.p;
+  a.dacc2 = W.dacc2.p;
+  a.vdir = W.v64.p;
+  a.dmol = W.dmol.p;
+  a.dphi = W.dphi.p;
+  if (precision == SFX_FP32)
+    launch_phi_close<float>(S.lat.d, S.sp, a, S.stream);
+  else
+    launch_phi_close<double>(S.lat.d, S.sp, a, S.stream);
+  FieldArgs f = S.field_args();
+  f.base = base;
+  f.v = v;
+  f.dphi = W.dphi.p;
+  f.dmol = W.dmol.p;
+  f.drho = W.drho.p;
+  f.jv = jv;
+  launch_field_close(S.lat.d, S.sp, f, S.stream);
+  if (base) {
+    S.phi_valid = true;
+    S.last_precision = precision;
+  }
 }
 
 static void require_products(const System& S) {
@@ -1034,7 +849,7 @@ void jvp_at_base(System& S, const double* v, double* jv, int precision) {
   Tangent& W = tangent(S);
   if (one_launch_product(S, W, v, jv, precision, false)) return;
   tangent_sweeps(S, W, v, precision, false);
-  tangent_residual(S, W, v, jv);
+  tangent_close(S, W, v, jv, precision, false);
 }
 
 // J v at S.d_u, base and tangent in one sweep per molecule: the base sweep of
@@ -1048,8 +863,7 @@ void jvp_internal(System& S, const double* v, double* jv, int precision) {
   if (one_launch_product(S, W, v, jv, precision, true)) return;
   S.start_phi(precision);
   tangent_sweeps(S, W, v, precision, true);
-  S.finish_phi(precision);
-  tangent_residual(S, W, v, jv);
+  tangent_close(S, W, v, jv, precision, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -1342,13 +1156,16 @@ void vjp_at_base(System& S, const double* w, double* jtw, int precision) {
       k_vjp_dir<<<nbM, kTB, 0, st>>>(L, uses, S.ns, W.phibar.p, W.xdir64.p, (float*)W.xdir32.p);
       const size_t off = (size_t)m * S.ns * Mn;
       const bool two = S.middle_out(mo);
+      S.ends.n = 0;
       if (fp32) {
         tsweep<float>(S, W, m, true, (const float*)W.xdir32.p, S.d_swf32, W.xdir64.p, false);
+        S.close_ends(false, W.dmol.p);
         k_vjp_sweep_term<float><<<nbV, kTB, 0, st>>>(L, uses, S.ns, (const float*)W.dacc.p + off,
                                                      two ? (const float*)W.dacc2.p + off : nullptr, S.d_swf,
                                                      W.dmol.p + m * 4, W.vbar.p);
       } else {
         tsweep<double>(S, W, m, false, W.xdir64.p, S.d_swf, W.xdir64.p, false);
+        S.close_ends(false, W.dmol.p);
         k_vjp_sweep_term<double><<<nbV, kTB, 0, st>>>(L, uses, S.ns, (const double*)W.dacc.p + off,
                                                       two ? (const double*)W.dacc2.p + off : nullptr, S.d_swf,
                                                       W.dmol.p + m * 4, W.vbar.p);

@@ -25,8 +25,6 @@
 // launch's fixed 4 us are paid an eighth as often.
 #include <hip/hip_ext.h>
 
-#include <algorithm>
-
 #include "sfx_block3.h"
 #include "sfx_device.h"
 
@@ -44,8 +42,6 @@ bool block2_ok(const DevLattice& L) {
   // the two chains of a middle-out sweep would not agree
   bool mirror2 = false;
   for (int k = 0; k < 2; k++) mirror2 |= L.mirror2_1[k] || L.mirror2_2[k];
-  // one layer between two mirror2 bounds has no image inside
-  if (mirror2 && std::min(L.nx, L.ny) < 2) return false;
   return L.grad == 2 && L.order == 1 && !(L.curved && mirror2);
 }
 
@@ -64,7 +60,8 @@ __device__ __forceinline__ float pow2_scale(float m, double& ln) {
   return __uint_as_float((unsigned)(127 - e) << 23);
 }
 
-// interior coordinate of which c is the image; 0 behind a surface. flip: an odd
+// interior coordinate of which c is the image (every side has at least two
+// layers, so the reflections end); 0 behind a surface. flip: an odd
 // number of reflections
 __device__ __forceinline__ int image(int c, int n, int lo, int hi, bool& flip) {  // 0 surface 1 mirror1 2 mirror2 3 periodic
   flip = false;

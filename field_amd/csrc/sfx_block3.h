@@ -87,7 +87,7 @@ std::vector<std::pair<int, int>> chain_launches(int a, int b, int g0, State stat
 // true when the blocked sweep applies: 3-D simple cubic, first order, every
 // side at least kB3Ranks + 1 layers (one reflection reaches the interior)
 bool block3_ok(const DevLattice& L);
-// true when the blocked sweep of 2-D lattices applies: first order, its own adjoint, images inside
+// true when the blocked sweep of 2-D lattices applies: first order, its own adjoint
 bool block2_ok(const DevLattice& L);
 
 // ev0/ev1 (optional): timing events the dispatch records at kernel start and end

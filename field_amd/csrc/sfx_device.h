@@ -47,10 +47,12 @@ __device__ __forceinline__ long long site_ordinal() {
 }
 
 __device__ __forceinline__ void site_coords(const DevLattice& L, long long i, int& x, int& y, int& z) {
-  z = (int)(i % L.MZ);
-  long long r = i / L.MZ;
-  y = (int)(r % L.MY);
-  x = (int)(r / L.MY);
+  const unsigned q = (unsigned)i;  // lattices are below 2^31 sites
+  const unsigned r = q / (unsigned)L.MZ;
+  z = (int)(q - r * (unsigned)L.MZ);
+  const unsigned p = r / (unsigned)L.MY;
+  y = (int)(r - p * (unsigned)L.MY);
+  x = (int)p;
 }
 
 __device__ __forceinline__ bool is_interior(const DevLattice& L, int x, int y, int z) {
@@ -219,66 +221,115 @@ __device__ __forceinline__ double side_at1(const DevLattice& L, const double* __
   return b + L.l1chi * (a - b - b + c);
 }
 
-// contact averages <phi_t> (SideFraction / Sides) on every site
-__device__ inline double side_at(const DevLattice& L, const double* __restrict__ P, int x, int y, int z) {
-  // remap halo coordinates that are not surfaces
+// the layer a 1-D contact average is taken at: a halo that is no surface, at its source
+__device__ __forceinline__ int side_x1(const DevLattice& L, int x) {
+  if (x == 0 && !L.surf1[0]) return L.b1[0];
+  if (x == L.nx + 1 && !L.surf2[0]) return L.b2[0];
+  return x;
+}
+
+// contact average at an interior site of a 2-D lattice, Lat2DFlat.cpp:996-1053,
+// Lat2DCylinder.cpp:205-320 (standard lattice, l2 = 0), the neighbours'
+// offsets and the radial weights worked out once for all states
+struct Near2 {
+  unsigned b, xm, xp, ym, yp;
+  double lm, lp;
+};
+__device__ __forceinline__ Near2 near_sites2(const DevLattice& L, int x, int y) {
+  auto X = [&](int c) { return (unsigned)remap(c, L.nx, L.surf1[0] ? 0 : L.b1[0], L.surf2[0] ? L.nx + 1 : L.b2[0]); };
+  auto Y = [&](int c) { return (unsigned)remap(c, L.ny, L.surf1[1] ? 0 : L.b1[1], L.surf2[1] ? L.ny + 1 : L.b2[1]); };
+  const unsigned jx = (unsigned)L.jx, ux = (unsigned)x, uy = (unsigned)y;
+  Near2 n{ux * jx + uy, X(x - 1) * jx + uy, X(x + 1) * jx + uy, ux * jx + Y(y - 1), ux * jx + Y(y + 1), 0.0, 0.0};
+  if (L.curved) {
+    n.lm = L.lm[x];
+    n.lp = L.lp[x];
+  }
+  return n;
+}
+__device__ __forceinline__ double side_near2(const DevLattice& L, const Near2& n, const double* __restrict__ P) {
+  const double b = P[n.b], xm = P[n.xm], xp = P[n.xp], a = P[n.ym], c = P[n.yp];
+  if (L.curved) return b + n.lp * (xp - b) + n.lm * (xm - b) + L.l1 * (a + c - b - b);
+  return L.l0_2d * b + L.l1x * (xm + xp) + L.l1y * (a + c);
+}
+
+// contact average of a 2-D lattice
+__device__ __forceinline__ double side_at2(const DevLattice& L, const double* __restrict__ P, int x, int y) {
   if (x == 0 && !L.surf1[0]) x = L.b1[0];
   else if (x == L.nx + 1 && !L.surf2[0]) x = L.b2[0];
-  if (L.grad >= 2) {
-    if (y == 0 && !L.surf1[1]) y = L.b1[1];
-    else if (y == L.ny + 1 && !L.surf2[1]) y = L.b2[1];
-  }
-  if (L.grad >= 3) {
-    if (z == 0) z = L.b1[2];
-    else if (z == L.nz + 1) z = L.b2[2];
-  }
-  auto at = [&](int X, int Y, int Z) -> double {
+  if (y == 0 && !L.surf1[1]) y = L.b1[1];
+  else if (y == L.ny + 1 && !L.surf2[1]) y = L.b2[1];
+  auto at = [&](int X, int Y) -> double {
     X = remap(X, L.nx, L.surf1[0] ? 0 : L.b1[0], L.surf2[0] ? L.nx + 1 : L.b2[0]);
-    if (L.grad >= 2) Y = remap(Y, L.ny, L.surf1[1] ? 0 : L.b1[1], L.surf2[1] ? L.ny + 1 : L.b2[1]);
-    if (L.grad >= 3) Z = remap(Z, L.nz, L.b1[2], L.b2[2]);
-    return P[sidx(L, X, Y, Z)];
+    Y = remap(Y, L.ny, L.surf1[1] ? 0 : L.b1[1], L.surf2[1] ? L.ny + 1 : L.b2[1]);
+    return P[sidx(L, X, Y, 0)];
   };
-  if (L.grad == 1) return side_at1(L, P, x);
-  if (L.grad == 2) {
-    // Lat2DFlat.cpp:996-1053, Lat2DCylinder.cpp:205-320 (standard lattice, l2 = 0)
-    double b = P[sidx(L, x, y, 0)];
-    double l1 = L.l1;
-    auto lam0 = [&](int X) { return 1 - 2 * l1 - L.lp[X] - L.lm[X]; };
-    if (x == 0 || x == L.nx + 1) {
-      double a = at(x, y - 1, 0), c = at(x, y + 1, 0);
-      double in = x == 0 ? P[sidx(L, 1, y, 0)] : P[sidx(L, L.nx, y, 0)];
-      if (L.curved) return lam0(x) * b + l1 * (a + c) + (x == 0 ? L.lp[0] : L.lm[x]) * in;
-      return L.l0_2d * b + L.l1y * (a + c) + L.l1x * in;
-    }
-    if (y == 0 || y == L.ny + 1) {
-      double xm = at(x - 1, y, 0), xp = at(x + 1, y, 0);
-      double in = y == 0 ? P[sidx(L, x, 1, 0)] : P[sidx(L, x, L.ny, 0)];
-      if (L.curved) return lam0(x) * b + L.lp[x] * xp + L.lm[x] * xm + l1 * in;
-      return L.l0_2d * b + L.l1x * (xm + xp) + L.l1y * in;
-    }
-    double xm = at(x - 1, y, 0), xp = at(x + 1, y, 0), a = at(x, y - 1, 0), c = at(x, y + 1, 0);
-    if (L.curved) return b + L.lp[x] * (xp - b) + L.lm[x] * (xm - b) + l1 * (a + c - b - b);
-    return L.l0_2d * b + L.l1x * (xm + xp) + L.l1y * (a + c);
+  if (is_interior(L, x, y, 0)) return side_near2(L, near_sites2(L, x, y), P);
+  const double b = P[sidx(L, x, y, 0)], l1 = L.l1;
+  auto lam0 = [&](int X) { return 1 - 2 * l1 - L.lp[X] - L.lm[X]; };
+  if (x == 0 || x == L.nx + 1) {
+    double a = at(x, y - 1), c = at(x, y + 1);
+    double in = x == 0 ? P[sidx(L, 1, y, 0)] : P[sidx(L, L.nx, y, 0)];
+    if (L.curved) return lam0(x) * b + l1 * (a + c) + (x == 0 ? L.lp[0] : L.lm[x]) * in;
+    return L.l0_2d * b + L.l1y * (a + c) + L.l1x * in;
   }
-  // 3-D, Lat3D.cpp:1729-1784
-  if (L.kind == ST_3D_HEX) {
+  if (y == 0 || y == L.ny + 1) {
+    double xm = at(x - 1, y), xp = at(x + 1, y);
+    double in = y == 0 ? P[sidx(L, x, 1, 0)] : P[sidx(L, x, L.ny, 0)];
+    if (L.curved) return lam0(x) * b + L.lp[x] * xp + L.lm[x] * xm + l1 * in;
+    return L.l0_2d * b + L.l1x * (xm + xp) + L.l1y * in;
+  }
+  return 0.0;
+}
+
+// Contact average at an interior site of a 3-D lattice, Lat3D.cpp:1729-1784,
+// with the neighbours' offsets worked out once for all states
+struct Near {
+  unsigned x[3], y[3], z[3];  // offsets of the layers -1, 0, +1
+};
+__device__ __forceinline__ Near near_sites(const DevLattice& L, int x, int y, int z) {
+  Near n;
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    n.x[d] = (unsigned)remap(x + d - 1, L.nx, L.b1[0], L.b2[0]) * (unsigned)L.jx;
+    n.y[d] = (unsigned)remap(y + d - 1, L.ny, L.b1[1], L.b2[1]) * (unsigned)L.MZ;
+    n.z[d] = (unsigned)remap(z + d - 1, L.nz, L.b1[2], L.b2[2]);
+  }
+  return n;
+}
+template <int KIND>
+__device__ __forceinline__ double side_near(const Near& n, const double* __restrict__ P) {
+  auto at = [&](int dx, int dy, int dz) { return P[n.x[dx + 1] + n.y[dy + 1] + n.z[dz + 1]]; };
+  if constexpr (KIND == ST_3D_HEX) {
     const double lam = 1.0 / 12.0;
-    return at(x + 1, y, z) * lam + at(x - 1, y, z) * lam + at(x + 1, y - 1, z) * lam + at(x, y - 1, z) * lam +
-           at(x, y + 1, z) * lam + at(x - 1, y + 1, z) * lam + at(x, y - 1, z + 1) * lam +
-           at(x, y, z + 1) * lam + at(x - 1, y, z + 1) * lam + at(x + 1, y, z - 1) * lam +
-           at(x, y, z - 1) * lam + at(x, y + 1, z - 1) * lam;
+    return at(1, 0, 0) * lam + at(-1, 0, 0) * lam + at(1, -1, 0) * lam + at(0, -1, 0) * lam + at(0, 1, 0) * lam +
+           at(-1, 1, 0) * lam + at(0, -1, 1) * lam + at(0, 0, 1) * lam + at(-1, 0, 1) * lam + at(1, 0, -1) * lam +
+           at(0, 0, -1) * lam + at(0, 1, -1) * lam;
   }
-  if (L.kind == ST_3D_FCC) {
+  if constexpr (KIND == ST_3D_FCC) {
     const double l = 1.0 / 27.0;
     double s = 0;
+#pragma unroll
     for (int dx = -1; dx <= 1; dx++)
+#pragma unroll
       for (int dy = -1; dy <= 1; dy++)
-        for (int dz = -1; dz <= 1; dz++) s += l * at(x + dx, y + dy, z + dz);
+#pragma unroll
+        for (int dz = -1; dz <= 1; dz++) s += l * at(dx, dy, dz);
     return s;
   }
   const double l1 = 1.0 / 6.0;
-  return l1 * at(x + 1, y, z) + l1 * at(x - 1, y, z) + l1 * at(x, y + 1, z) + l1 * at(x, y - 1, z) +
-         l1 * at(x, y, z + 1) + l1 * at(x, y, z - 1);
+  return l1 * at(1, 0, 0) + l1 * at(-1, 0, 0) + l1 * at(0, 1, 0) + l1 * at(0, -1, 0) + l1 * at(0, 0, 1) +
+         l1 * at(0, 0, -1);
+}
+
+// contact averages <phi_t> (SideFraction / Sides) on every site
+__device__ inline double side_at(const DevLattice& L, const double* __restrict__ P, int x, int y, int z) {
+  if (L.grad == 1) return side_at1(L, P, side_x1(L, x));
+  if (L.grad == 2) return side_at2(L, P, x, y);
+  const Near n = near_sites(L, remap(x, L.nx, L.b1[0], L.b2[0]), remap(y, L.ny, L.b1[1], L.b2[1]),
+                            remap(z, L.nz, L.b1[2], L.b2[2]));
+  if (L.kind == ST_3D_HEX) return side_near<ST_3D_HEX>(n, P);
+  if (L.kind == ST_3D_FCC) return side_near<ST_3D_FCC>(n, P);
+  return side_near<ST_3D_SC>(n, P);
 }
 
 }  // namespace sfx

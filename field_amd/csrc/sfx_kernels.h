@@ -119,8 +119,6 @@ template <typename T>
 void launch_copy_interior(const DevLattice& L, const T* a, T* b, hipStream_t st);
 template <typename T>
 int launch_wsum(const DevLattice& L, const T* G, double* partial, hipStream_t st);
-void launch_mol_finalize(const MolParams& mp, const double* partial, int nparts, double* scal,
-                         const double* lnfN, const double* allscal, int nmol, hipStream_t st);
 // phi_m = pref (acc + acc2) / g; acc2 (the backward chain's accumulator of a
 // middle-out sweep) may be null
 template <typename A>
@@ -138,14 +136,6 @@ void launch_swf(const DevLattice& L, const double* u, const unsigned char* itmas
                 const int* st_itvar, double* swf, float* swf32, hipStream_t st, unsigned* zero = nullptr,
                 int nzero = 0);
 // sp != null: the same launch also writes the bulk fractions and ChemIntBulk
-void launch_phi_total(const DevLattice& L, int nstates, int nmol, const double* phi_m, const int* mol_uses,
-                      const double* fprof, const int* frozen, double* phi, double* phitot, hipStream_t st,
-                      const SysParams* sp = nullptr, const double* molscal = nullptr, double* phib_state = nullptr,
-                      double* cbulk = nullptr);
-void launch_sides(const DevLattice& L, int nstates, const double* phi, double* rho, hipStream_t st);
-
-void launch_residual(const DevLattice& L, const SysParams& sp, const unsigned char* itmask, const double* swf,
-                     const double* rho, const double* phitot, const double* cbulk, double* f, hipStream_t st);
 int launch_free_energy(const DevLattice& L, const SysParams& sp, const double* phi, const double* phi_m,
                        const double* rho, const double* swf, const double* u, const double* molscal,
                        double* partial, hipStream_t st);

@@ -199,26 +199,6 @@ __global__ void k_wsum(DevLattice L, const T* __restrict__ G, double* __restrict
   if (threadIdx.x == 0) partial[blockIdx.x] = v;
 }
 
-// ---------------------------------------------------------------------------
-// Molecule scalars after a sweep (mol_scalars), one workgroup
-__global__ void k_mol_finalize(MolParams mp, const double* __restrict__ partial, int nparts,
-                               double* __restrict__ scal, const double* __restrict__ lnfN,
-                               const double* __restrict__ allscal, int nmol) {
-  // the partial sums, reduced by the whole block in a fixed order
-  __shared__ double red[256 / 64];
-  double s = 0;
-  for (int i = threadIdx.x; i < nparts; i += blockDim.x) s += partial[i];
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  s = 0;
-  for (int i = 0; i < (int)(blockDim.x >> 6); i++) s += red[i];
-  // FP32: log-scale of the final rank
-  mol_scalars(mp, s, lnfN ? *lnfN : 0.0, scal[MS_REF], nmol, [&](int m) { return allscal[m * MS_COUNT + MS_PHIB]; },
-              scal);
-}
-
 // phi_{m,t} = pref_m * acc_{m,t} / g_t (g>0, else 0); monomers phi = pref * g.
 template <typename A>
 __global__ void k_mol_phi(DevLattice L, const A* __restrict__ acc, const A* __restrict__ acc2,
@@ -245,71 +225,6 @@ __global__ void k_set_ref_pair(double* scal, const double* lna, int ia, const do
 
 void launch_set_ref_pair(double* scal, const double* lna, int ia, const double* lnb, int ib, hipStream_t st) {
   k_set_ref_pair<<<1, 1, 0, st>>>(scal, lna, ia, lnb, ib);
-}
-
-// state totals over molecules + frozen profiles, halos from their sources;
-// phitot on interior sites.
-// state totals; the first thread also derives the bulk fractions and ChemIntBulk
-// from the molecules' phi_b (no dependence on the sites)
-__global__ void k_phi_total(DevLattice L, int nstates, int nmol, const double* __restrict__ phi_m,
-                            const int* __restrict__ mol_uses, const double* __restrict__ fprof,
-                            const int* __restrict__ frozen, double* __restrict__ phi,
-                            double* __restrict__ phitot, SysParams sp, const double* __restrict__ molscal,
-                            double* __restrict__ phib_state, double* __restrict__ cbulk) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0 && phib_state) bulk_fractions(sp, molscal, phib_state, cbulk);
-  if (i >= L.M) return;
-  int x, y, z;
-  site_coords(L, i, x, y, z);
-  int sx = remap(x, L.nx, L.b1[0], L.b2[0]);
-  int sy = L.grad >= 2 ? remap(y, L.ny, L.b1[1], L.b2[1]) : y;
-  int sz = L.grad >= 3 ? remap(z, L.nz, L.b1[2], L.b2[2]) : z;
-  long long s = sidx(L, sx, sy, sz);
-  bool surf_halo = !is_interior(L, sx, sy, sz);
-  double tot = 0;
-  for (int t = 0; t < nstates; t++) {
-    double v = 0;
-    if (frozen[t]) {
-      v = fprof[(long long)t * L.M + s];  // PutSides applies SetBoundaries to it as well
-    } else if (!surf_halo) {
-      for (int m = 0; m < nmol; m++)
-        if (mol_uses[m * nstates + t]) v += phi_m[((long long)m * nstates + t) * L.M + s];
-    }
-    phi[(long long)t * L.M + i] = v;
-    tot += v;
-  }
-  phitot[i] = tot;
-}
-
-// ---------------------------------------------------------------------------
-__global__ void k_sides(DevLattice L, int nstates, const double* __restrict__ phi, double* __restrict__ rho) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= L.M) return;
-  int x, y, z;
-  site_coords(L, i, x, y, z);
-  const bool side = has_side(L, x, y, z);
-  for (int t = 0; t < nstates; t++) {
-    const double* P = phi + (long long)t * L.M;
-    rho[(long long)t * L.M + i] = side ? side_at(L, P, x, y, z) : 0.0;
-  }
-}
-
-// f = -1 + 1/phitot + u'_i - <u'> per iteration site (SF_Solve.cpp:554-590),
-// written in the internal [itvar][M] layout (zero off iteration sites).
-__global__ void k_residual(DevLattice L, SysParams sp, const unsigned char* __restrict__ itmask,
-                           const double* __restrict__ swf, const double* __restrict__ rho,
-                           const double* __restrict__ phitot, const double* __restrict__ cbulk,
-                           double* __restrict__ f) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= L.M) return;
-  const int nv = sp.n_itvar;
-  if (!itmask[i]) {
-    for (int k = 0; k < nv; k++) f[(long long)k * L.M + i] = 0.0;
-    return;
-  }
-  residual_site(sp, phitot[i], cbulk, [&](int t) { return swf[(long long)t * L.M + i]; },
-                [&](int t) { return rho[(long long)t * L.M + i]; },
-                [&](int k, double v) { f[(long long)k * L.M + i] = v; });
 }
 
 // per-site free-energy density, block partials (SF_MolList1stO.cpp:815-940)
@@ -506,11 +421,6 @@ int launch_wsum(const DevLattice& L, const T* G, double* partial, hipStream_t st
   return (int)nb;
 }
 
-void launch_mol_finalize(const MolParams& mp, const double* partial, int nparts, double* scal,
-                         const double* lnfN, const double* allscal, int nmol, hipStream_t st) {
-  k_mol_finalize<<<1, 256, 0, st>>>(mp, partial, nparts, scal, lnfN, allscal, nmol);
-}
-
 template <typename A>
 void launch_mol_phi(const DevLattice& L, const A* acc, const double* g, const double* scal, int monomer,
                     double* phi_m, hipStream_t st, const A* acc2) {
@@ -548,25 +458,6 @@ void launch_swf(const DevLattice& L, const double* u, const unsigned char* itmas
   if (!zero) nzero = 0;
   k_swf<<<grid1(std::max<long long>(L.M, nzero), kBlock), kBlock, 0, st>>>(L, u, itmask, nstates, st_itvar, swf,
                                                                            swf32, zero, nzero);
-}
-
-void launch_phi_total(const DevLattice& L, int nstates, int nmol, const double* phi_m, const int* mol_uses,
-                      const double* fprof, const int* frozen, double* phi, double* phitot, hipStream_t st,
-                      const SysParams* sp, const double* molscal, double* phib_state, double* cbulk) {
-  SysParams none{};
-  k_phi_total<<<grid1(L.M, kBlock), kBlock, 0, st>>>(L, nstates, nmol, phi_m, mol_uses, fprof, frozen, phi,
-                                                     phitot, sp ? *sp : none, molscal, sp ? phib_state : nullptr,
-                                                     cbulk);
-}
-
-void launch_sides(const DevLattice& L, int nstates, const double* phi, double* rho, hipStream_t st) {
-  k_sides<<<grid1(L.M, kBlock), kBlock, 0, st>>>(L, nstates, phi, rho);
-}
-
-
-void launch_residual(const DevLattice& L, const SysParams& sp, const unsigned char* itmask, const double* swf,
-                     const double* rho, const double* phitot, const double* cbulk, double* f, hipStream_t st) {
-  k_residual<<<grid1(L.M, kBlock), kBlock, 0, st>>>(L, sp, itmask, swf, rho, phitot, cbulk, f);
 }
 
 int launch_free_energy(const DevLattice& L, const SysParams& sp, const double* phi, const double* phi_m,
@@ -698,11 +589,8 @@ void launch_range_scale(const DevLattice& L, unsigned uses, int ns, const double
 }
 
 template int launch_wsum<double>(const DevLattice&, const double*, double*, hipStream_t);
-template int launch_wsum<float>(const DevLattice&, const float*, double*, hipStream_t);
 template void launch_mol_phi<double>(const DevLattice&, const double*, const double*, const double*, int, double*,
                                      hipStream_t, const double*);
-template void launch_mol_phi<float>(const DevLattice&, const float*, const double*, const double*, int, double*,
-                                    hipStream_t, const float*);
 template void launch_mol_phi_states<double>(const DevLattice&, unsigned, int, const double*, const double*,
                                             const double*, const double*, double*, hipStream_t);
 template void launch_mol_phi_states<float>(const DevLattice&, unsigned, int, const float*, const float*,

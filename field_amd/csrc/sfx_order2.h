@@ -27,7 +27,5 @@ template <typename T>
 void launch_init2b(const DevLattice& L, bool tangent, const T* g, const T* v, T* G, T* dG, const T* Wp,
                    const T* dWp, T* acc, const RankScale& sc, hipStream_t st, T* bacc = nullptr);
 // per-block weighted sums over the six components of G (and dG)
-template <typename T>
-int launch_wsum6(const DevLattice& L, const T* G, const T* dG, double* p1, double* p2, hipStream_t st);
 
 }  // namespace sfx

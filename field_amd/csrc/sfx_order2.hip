@@ -483,47 +483,6 @@ __global__ void k_init2b(DevLattice L, const T* __restrict__ g, const T* __restr
   }
 }
 
-// weighted sums over the six components (ln G_N before /6 and the log)
-template <typename T>
-__global__ void k_wsum6(DevLattice L, const T* __restrict__ G, const T* __restrict__ dG, double* __restrict__ p1,
-                        double* __restrict__ p2) {
-  long long q = site_ordinal();
-  double a = 0, b = 0;
-  if (q < L.V) {
-    int x, y, z;
-    interior_coords(L, q, x, y, z);
-    long long r = sidx(L, x, y, z);
-    // flat 1-D sums every layer plainly (Lat1D2ndO.cpp ComputeLnGN); 2-D and 3-D
-    // halve mirror2 edges (Lat2D2ndO.cpp:387-439, Lat3D2ndO.cpp:996-1025);
-    // curved lattices weight by the layer volume (Lat1DCyl2ndO.cpp:319-330,
-    // Lat2DCyl2ndO.cpp:410-462)
-    double w = L.grad == 1 && !L.curved ? 1.0 : lngn_weight(L, x, y, z);
-    for (int k = 0; k < 6; k++) {
-      a += (double)G[(long long)k * L.M + r] * w;
-      if (dG) b += (double)dG[(long long)k * L.M + r] * w;
-    }
-  }
-  __shared__ double sa[kB2 / 64], sb[kB2 / 64];
-  for (int o = 32; o > 0; o >>= 1) {
-    a += __shfl_xor(a, o, 64);
-    b += __shfl_xor(b, o, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    sa[threadIdx.x >> 6] = a;
-    sb[threadIdx.x >> 6] = b;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double A = 0, B = 0;
-    for (int i = 0; i < (int)(blockDim.x >> 6); i++) {
-      A += sa[i];
-      B += sb[i];
-    }
-    p1[blockIdx.x] = A;
-    if (p2) p2[blockIdx.x] = B;
-  }
-}
-
 // ---------------------------------------------------------------------------
 #define SFX_O2_DISPATCH(K, ...)                 \
   do {                                          \
@@ -611,13 +570,6 @@ void launch_init2b(const DevLattice& L, bool tangent, const T* g, const T* v, T*
 }
 #undef SFX_O2_DISPATCH
 
-template <typename T>
-int launch_wsum6(const DevLattice& L, const T* G, const T* dG, double* p1, double* p2, hipStream_t st) {
-  unsigned nb = grid1(L.V, kB2);
-  k_wsum6<T><<<nb, kB2, 0, st>>>(L, G, dG, p1, p2);
-  return (int)nb;
-}
-
 template void launch_prop2f<double>(const DevLattice&, bool, const double*, const double*, const double*,
                                     const double*, double*, double*, double, const RankScale&, hipStream_t);
 template void launch_prop2f<float>(const DevLattice&, bool, const float*, const float*, const float*, const float*,
@@ -636,7 +588,5 @@ template void launch_init2b<double>(const DevLattice&, bool, const double*, cons
                                     const double*, const double*, double*, const RankScale&, hipStream_t, double*);
 template void launch_init2b<float>(const DevLattice&, bool, const float*, const float*, float*, float*, const float*,
                                    const float*, float*, const RankScale&, hipStream_t, float*);
-template int launch_wsum6<double>(const DevLattice&, const double*, const double*, double*, double*, hipStream_t);
-template int launch_wsum6<float>(const DevLattice&, const float*, const float*, double*, double*, hipStream_t);
 
 }  // namespace sfx

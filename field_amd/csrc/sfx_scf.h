@@ -111,17 +111,24 @@ __device__ __forceinline__ void bulk_fractions_wave(const SysParams& sp, const d
 }
 
 // f = -1 + 1/phitot + u'_i - <u'> of one iteration site (SF_Solve.cpp:554-590):
-// swf(t), rho(t): the site's SWF and contact average of state t; put(k, f)
-template <class Swf, class Rho, class Put>
+// swf(t), rho(t): the site's SWF and contact average of state t; put(k, f).
+// NS: a bound on the states and iteration variables; below SFX_MAXS the loops
+// unroll, for averages in registers
+template <int NS = SFX_MAXS, class Swf, class Rho, class Put>
 __device__ __forceinline__ void residual_site(const SysParams& sp, double pt, const double* cbulk, Swf&& swf,
                                               Rho&& rho, Put&& put) {
   const int nv = sp.n_itvar;
-  double up[SFX_MAXS];
+  constexpr int unroll = NS < SFX_MAXS ? NS : 1;
+  double up[NS];
   double av = 0;
-  for (int k = 0; k < nv; k++) {
+#pragma unroll unroll
+  for (int k = 0; k < NS; k++) {
+    if (k >= nv) break;
     int t = sp.itvar_rep[k];
     double ci = 0;
-    for (int j = 0; j < sp.ns; j++) {
+#pragma unroll unroll
+    for (int j = 0; j < NS; j++) {
+      if (j >= sp.ns) break;
       double x = sp.chi[t * SFX_MAXS + j];
       if (x != 0) ci += x * rho(j);
     }
@@ -132,7 +139,11 @@ __device__ __forceinline__ void residual_site(const SysParams& sp, double pt, co
     av += v;
   }
   av /= nv;
-  for (int k = 0; k < nv; k++) put(k, -1.0 + 1.0 / pt + up[k] - av);
+#pragma unroll unroll
+  for (int k = 0; k < NS; k++) {
+    if (k >= nv) break;
+    put(k, -1.0 + 1.0 / pt + up[k] - av);
+  }
 }
 
 // tangent molecule scalars from the weighted sums s1 of the end rank and s2 of
@@ -175,16 +186,21 @@ __device__ __forceinline__ double tphi_site(bool monomer, double phi, double g, 
 // linearised residual of one iteration site (SF_Solve.cpp:554-590): v(k) the
 // direction, rho/drho(t) contact averages, pt/dpt the totals, dmol the tangent
 // molecule scalars; put(k, jv)
-template <class V, class Rho, class Drho, class Put>
+template <int NS = SFX_MAXS, class V, class Rho, class Drho, class Put>
 __device__ __forceinline__ void jres_site(const SysParams& sp, double pt, double dpt, const double* dmol, V&& v,
                                           Rho&& rho, Drho&& drho, Put&& put) {
   const int nv = sp.n_itvar;
-  double du[SFX_MAXS];
+  constexpr int unroll = NS < SFX_MAXS ? NS : 1;
+  double du[NS];
   double av = 0;
-  for (int k = 0; k < nv; k++) {
+#pragma unroll unroll
+  for (int k = 0; k < NS; k++) {
+    if (k >= nv) break;
     int t = sp.itvar_rep[k];
     double ci = 0, dci = 0, dcb = 0;
-    for (int j = 0; j < sp.ns; j++) {
+#pragma unroll unroll
+    for (int j = 0; j < NS; j++) {
+      if (j >= sp.ns) break;
       double c = sp.chi[t * SFX_MAXS + j];
       if (c == 0) continue;
       ci += c * rho(j);
@@ -200,7 +216,11 @@ __device__ __forceinline__ void jres_site(const SysParams& sp, double pt, double
     av += d;
   }
   av /= nv;
-  for (int k = 0; k < nv; k++) put(k, -dpt / (pt * pt) + du[k] - av);
+#pragma unroll unroll
+  for (int k = 0; k < NS; k++) {
+    if (k >= nv) break;
+    put(k, -dpt / (pt * pt) + du[k] - av);
+  }
 }
 
 // one rank of a tangent chain and one term of its composition; the products are

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "sfx_chain1d.h"
+#include "sfx_close.h"
 #include "sfx_kernels.h"
 
 namespace sfx {
@@ -192,6 +193,7 @@ struct System {
   unsigned* d_maxf = nullptr;
   unsigned* d_maxb = nullptr;
   double* d_partial = nullptr;  // reduction partials
+  unsigned* d_ticket = nullptr;  // arrivals of an end sum's workgroups
   unsigned* d_gmax = nullptr;   // ns x kStepWords: lattice maximum of each FP32 SWF (blocked sweeps)
   double* d_phib_state = nullptr;
   double* d_cbulk = nullptr;
@@ -220,13 +222,20 @@ struct System {
   // the two internal-layout vectors of the product entry points (kept, so a
   // call allocates nothing after the first)
   void abi_vectors(double*& in, double*& out);
-  void compute_phi(int precision);  // from d_u
-  // compute_phi before and after the molecules' sweeps: a caller that sweeps
-  // base and tangent propagators together puts its own sweeps in between
+  void compute_phi(int precision, double* f = nullptr);  // from d_u; with f the residual as well
+  // compute_phi before the molecules' sweeps: a caller that sweeps base and
+  // tangent propagators together puts its own sweeps and closing behind it
   void start_phi(int precision);
-  void finish_phi(int precision);
+  // the closing launches (sfx_close.hip): a sweep leaves its molecule's end
+  // rank in `ends`; close_ends derives the scalars (of the base, and of the
+  // tangent into dmol) before the next chain overwrites the running ranks
+  EndArgs ends{};
+  void add_end(int m, const void* G, const void* dG, bool f32, const double* lnf);
+  void close_ends(bool base, double* dmol);
+  PhiArgs phi_args();
+  FieldArgs field_args();
   void residual_internal(int precision);  // d_u -> d_f
-  void finish_range(int m);  // range_restricted: the range condition fixes molecule m's constant
+  void finish_range(int m, int precision);  // range_restricted: the range condition fixes molecule m's constant
   bool has_range() const;
   // residual_internal replayed from a HIP graph captured on the first call
   // (per precision): one submission instead of a launch per rank. Plain

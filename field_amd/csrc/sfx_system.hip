@@ -23,9 +23,9 @@ static __global__ void k_fill_bytes8(unsigned long long* p, long long n) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0ull;
 }
-// scal[MS_REF] = factor * lnv[idx] (lnv == nullptr: 0)
+// scal[MS_REF] = factor * lnv[idx]
 static __global__ void k_set_ref(double* scal, const double* lnv, int idx, double factor) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) scal[MS_REF] = lnv ? factor * lnv[idx] : 0.0;
+  if (threadIdx.x == 0 && blockIdx.x == 0) scal[MS_REF] = factor * lnv[idx];
 }
 // x (SF_Solve layout) -> u[itvar][M]; u zero off the iteration sites
 static __global__ void k_unpack_sfbox(const double* x, const long long* sites, long long nsites, int nv,
@@ -68,7 +68,7 @@ System::~System() {
       if (p) (void)hipFree(p);
   void* ptrs[] = {d_u, d_f, d_swf, d_swf32, d_phi_m, d_acc, d_acc2, d_phi, d_rho, d_phitot, d_fprof, d_frozen,
                   d_st_itvar, d_mol_uses, d_itmask, d_sites, d_store, d_pp, d_pp2, d_molscal, d_lnf, d_lnb,
-                  d_maxf, d_maxb, d_partial, d_phib_state, d_cbulk, d_scalar, d_xabi, d_gmax,
+                  d_maxf, d_maxb, d_partial, d_ticket, d_phib_state, d_cbulk, d_scalar, d_xabi, d_gmax,
                   d_abi_in, d_abi_out, scf1_runs};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -320,7 +320,9 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   d_maxf = dalloc<unsigned>((size_t)nm * (maxN + 2) * kStepWords);
   d_maxb = dalloc<unsigned>((size_t)nm * (maxN + 2) * kStepWords);
   npart = (int)grid1(std::max<long long>(lat.d.M, lat.d.V), 256);
+  npart = std::max(npart, 2 * SFX_MAXM * kEndBlocks);
   d_partial = dalloc<double>(npart);
+  d_ticket = dalloc<unsigned>(2);
   d_gmax = dalloc<unsigned>((size_t)SFX_MAXS * kStepWords);
   d_phib_state = dalloc<double>(SFX_MAXS);
   d_cbulk = dalloc<double>(SFX_MAXS);
@@ -341,6 +343,7 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   zero_bytes(d_pp, 2 * comps * M * 8, stream);
   if (d_pp2) zero_bytes(d_pp2, 2 * M * 8, stream);
   zero_bytes(d_u, n_itvar * M * 8, stream);
+  zero_bytes(d_ticket, 8, stream);
   zero_bytes(d_f, n_itvar * M * 8, stream);
   zero_bytes(d_acc, (size_t)nm * ns * M * 8, stream);
   zero_bytes(d_phi_m, (size_t)nm * ns * M * 8, stream);
@@ -495,7 +498,7 @@ void System::sweep(int m, bool scaled) {
     };
     chain_forward(plan, step);
     ChainReader<decltype(step)> rd{plan, step};
-    k_set_ref<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, N, 1.0);
+    if (scaled) k_set_ref<<<1, 1, 0, st>>>(scal, lnf, N, 1.0);
     auto bsc2 = [&](int step, int pair) {
       RankScale r = bsc(step, pair);
       if (scaled) r.pmaxv = maxf;
@@ -511,18 +514,11 @@ void System::sweep(int m, bool scaled) {
                        wp, nullptr, accp(mo.seq[s - 1]), stiffness, bsc2(k, s), st);
       prof.end(st);
     }
-    int nb = launch_wsum6<T>(L, pp6[(N - 1) & 1], nullptr, d_partial, nullptr, st);
-    launch_mol_finalize(mo.params(m), d_partial, nb, scal, scaled ? lnb + N : nullptr, d_molscal, nm, st);
-    launch_mol_phi_states<A>(L, mo.uses_mask(), ns, accp(0), (const A*)nullptr, d_swf, scal,
-                             d_phi_m + (size_t)m * ns * Mn, st);
+    add_end(m, pp6[(N - 1) & 1], nullptr, sizeof(T) == 4, scaled ? lnb + N : nullptr);
     return;
   }
   if (mo.kind == 0) {
-    int t = mo.seq[0];
-    int nb = launch_wsum<double>(L, d_swf + (size_t)t * Mn, d_partial, st);
-    k_set_ref<<<1, 1, 0, st>>>(scal, nullptr, 0, 0.0);
-    launch_mol_finalize(mo.params(m), d_partial, nb, scal, nullptr, d_molscal, nm, st);
-    launch_mol_phi<double>(L, nullptr, d_swf + (size_t)t * Mn, scal, 1, d_phi_m + ((size_t)m * ns + t) * Mn, st);
+    add_end(m, d_swf + (size_t)mo.seq[0] * Mn, nullptr, false, nullptr);
     return;
   }
   if constexpr (std::is_same<T, A>::value) {
@@ -558,7 +554,7 @@ void System::sweep(int m, bool scaled) {
   }
   ChainReader<decltype(step)> rd{plan, step};
   if (mo.kind == 1) {
-    k_set_ref<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, N, 1.0);
+    if (scaled) k_set_ref<<<1, 1, 0, st>>>(scal, lnf, N, 1.0);
     // backward: step k = N-s+1 holds G_inv(s)
     launch_init_rank<T>(L, gp(mo.seq[N - 1]), pp[0], bsc(1, N), st);
     launch_connect<T, A>(L, pp[0], slot(rd.get(N)), accp(mo.seq[N - 1]), bsc(1, N), 1.0, st);
@@ -583,16 +579,22 @@ void System::sweep(int m, bool scaled) {
     lnfinal = scaled ? lnb + N : nullptr;
   } else {
     const int h = N / 2;
-    k_set_ref<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, h, 2.0);
-    // the running sweep continues the forward chain (ranks h+1..N)
-    launch_copy_interior<T>(L, slot(rd.get(h)), pp[0], st);
+    if (scaled) k_set_ref<<<1, 1, 0, st>>>(scal, lnf, h, 2.0);
+    // the running sweep continues the forward chain (ranks h+1..N) from its
+    // stored rank h; a checkpoint segment is overwritten, so that is copied
+    const T* from = slot(rd.get(h));
+    if (plan.c) {
+      launch_copy_interior<T>(L, from, pp[0], st);
+      from = pp[0];
+    }
     int cur = 0;
     if (N % 2 == 1) {
       int s = h + 1;
-      launch_prop<T, A>(L, pp[cur], gp(mo.seq[s - 1]), pp[cur ^ 1], nullptr, nullptr, fsc(s, 0), st);
+      launch_prop<T, A>(L, from, gp(mo.seq[s - 1]), pp[cur ^ 1], nullptr, nullptr, fsc(s, 0), st);
       cur ^= 1;
       RankScale c = fsc(s, s);
       launch_connect<T, A>(L, pp[cur], pp[cur], accp(mo.seq[s - 1]), c, 0.5, st);
+      from = pp[cur];
     }
     if (chain1) {
       if constexpr (std::is_same<T, double>::value && std::is_same<A, double>::value) {
@@ -600,7 +602,7 @@ void System::sweep(int m, bool scaled) {
         for (int s = (N + 3) / 2; s <= N; s++)
           hs.push_back(Chain1Step{gp(mo.seq[s - 1]), nullptr, slot(rd.get(N - s + 1)), accp(mo.seq[s - 1])});
         const int fin = cur ^ (int)(hs.size() & 1);
-        chain1_run(m, 2, hs, pp[cur], pp[fin]);
+        chain1_run(m, 2, hs, from, pp[fin]);
         cur = fin;
       }
     } else {
@@ -608,18 +610,16 @@ void System::sweep(int m, bool scaled) {
         int sinv = N - s + 1;
         const T* pair = slot(rd.get(sinv));
         prof.begin(1, P, st);
-        launch_prop<T, A>(L, pp[cur], gp(mo.seq[s - 1]), pp[cur ^ 1], pair, accp(mo.seq[s - 1]), fsc(s, sinv), st);
+        launch_prop<T, A>(L, from, gp(mo.seq[s - 1]), pp[cur ^ 1], pair, accp(mo.seq[s - 1]), fsc(s, sinv), st);
         prof.end(st);
         cur ^= 1;
+        from = pp[cur];
       }
     }
     final_G = pp[cur];
     lnfinal = scaled ? lnf + N : nullptr;
   }
-  int nb = launch_wsum<T>(L, final_G, d_partial, st);
-  launch_mol_finalize(mo.params(m), d_partial, nb, scal, lnfinal, d_molscal, nm, st);
-  launch_mol_phi_states<A>(L, mo.uses_mask(), ns, accp(0), (const A*)nullptr, d_swf, scal, d_phi_m + (size_t)m * ns * Mn,
-                           st);
+  add_end(m, final_G, nullptr, sizeof(T) == 4, lnfinal);
 }
 
 // The sweep of sweep() for a first-order chain (full or half store) on the
@@ -731,7 +731,7 @@ void System::sweep_blocked(int m, bool scaled) {
       }
       go(la, false);
     }
-    launch_set_ref_pair(scal, scaled ? lnf : nullptr, h, lnb, N - h, st);
+    if (scaled) launch_set_ref_pair(scal, lnf, h, lnb, N - h, st);
     const auto F2 = chain_launches(h + 1, N, h + 1, state_of_rank, grid);
     const auto B2 = chain_launches(N - h + 1, N, N - h + 1, bstate, grid);
     int fc = 0, bc = 0;
@@ -767,10 +767,7 @@ void System::sweep_blocked(int m, bool scaled) {
       }
       go(la, true);
     }
-    int nb = launch_wsum<T>(L, pp[fc], d_partial, st);  // forward rank N
-    launch_mol_finalize(mo.params(m), d_partial, nb, scal, scaled ? lnf + N : nullptr, d_molscal, nm, st);
-    launch_mol_phi_states<T>(L, mo.uses_mask(), ns, accp(0), acc2p(0), d_swf, scal, d_phi_m + (size_t)m * ns * Mn,
-                             st);
+    add_end(m, pp[fc], nullptr, sizeof(T) == 4, scaled ? lnf + N : nullptr);  // forward rank N
     return;
   }
   // forward chain, ranks 2..plan.n; every rank kept (full store) or the
@@ -822,7 +819,7 @@ void System::sweep_blocked(int m, bool scaled) {
   const double* lnfinal = nullptr;
   int cur = 0;
   if (mo.kind == 1) {
-    k_set_ref<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, N, 1.0);
+    if (scaled) k_set_ref<<<1, 1, 0, st>>>(scal, lnf, N, 1.0);
     // backward chain: step k holds G_inv of rank N-k+1
     launch_init_rank<T>(L, gp(mo.seq[N - 1]), pp[0], bsc(1, N), st);
     launch_connect<T, T>(L, pp[0], slot(get(N)), accp(mo.seq[N - 1]), bsc(1, N), 1.0, st);
@@ -846,13 +843,18 @@ void System::sweep_blocked(int m, bool scaled) {
     lnfinal = scaled ? lnb + N : nullptr;
   } else {
     const int h = N / 2;
-    k_set_ref<<<1, 1, 0, st>>>(scal, scaled ? lnf : nullptr, h, 2.0);
-    launch_copy_interior<T>(L, slot(get(h)), pp[0], st);
+    if (scaled) k_set_ref<<<1, 1, 0, st>>>(scal, lnf, h, 2.0);
+    const T* from = slot(get(h));
+    if (plan.c) {
+      launch_copy_interior<T>(L, from, pp[0], st);
+      from = pp[0];
+    }
     if (N % 2 == 1) {  // the middle rank meets itself
       const int s = h + 1;
-      launch_prop<T, T>(L, pp[0], gp(mo.seq[s - 1]), pp[1], nullptr, nullptr, fsc(s, 0), st);
+      launch_prop<T, T>(L, from, gp(mo.seq[s - 1]), pp[1], nullptr, nullptr, fsc(s, 0), st);
       cur = 1;
       launch_connect<T, T>(L, pp[cur], pp[cur], accp(mo.seq[s - 1]), fsc(s, s), 0.5, st);
+      from = pp[cur];
     }
     auto pair_of = [&](int s) { return N - s + 1; };
     chain_blocks(
@@ -867,20 +869,69 @@ void System::sweep_blocked(int m, bool scaled) {
             pidx[s - sa] = pair_of(s);
           }
           outs[sb - sa] = pp[cur ^ 1];
-          launch(sa, sb, pp[cur], mo.seq[sa - 1], maxf, lnf, outs, pairs, pidx, true);
+          launch(sa, sb, from, mo.seq[sa - 1], maxf, lnf, outs, pairs, pidx, true);
           cur ^= 1;
+          from = pp[cur];
         }, grid);
-    final_G = pp[cur];
+    final_G = from;
     lnfinal = scaled ? lnf + N : nullptr;
   }
-  int nb = launch_wsum<T>(L, final_G, d_partial, st);
-  launch_mol_finalize(mo.params(m), d_partial, nb, scal, lnfinal, d_molscal, nm, st);
-  launch_mol_phi_states<T>(L, mo.uses_mask(), ns, accp(0), (const T*)nullptr, d_swf, scal, d_phi_m + (size_t)m * ns * Mn,
-                           st);
+  add_end(m, final_G, nullptr, sizeof(T) == 4, lnfinal);
+}
+
+void System::add_end(int m, const void* G, const void* dG, bool f32, const double* lnf) {
+  ends.n++;
+  ends.e[ends.n - 1] = EndMol{mols[m].params(m), G, dG, lnf, f32, lnf == nullptr};
+}
+
+void System::close_ends(bool base, double* dmol) {
+  ends.nm = nm;
+  ends.molscal = d_molscal;
+  ends.dmol = dmol;
+  ends.partial = d_partial;
+  ends.ticket = d_ticket;
+  ends.base = base;
+  ends.tangent = dmol != nullptr;
+  launch_end_sums(lat.d, ends, stream);
+  ends.n = 0;
+}
+
+PhiArgs System::phi_args() {
+  PhiArgs a{};
+  a.nm = nm;
+  a.ns = ns;
+  for (int m = 0; m < nm; m++) {
+    a.uses[m] = mols[m].uses_mask();
+    a.mode[m] = mols[m].kind == 0 ? CLOSE_MONOMER : CLOSE_CHAIN;
+    a.two[m] = middle_out(mols[m]);
+  }
+  for (int t = 0; t < ns; t++) a.frozen[t] = frozen[t];
+  a.acc = d_acc;
+  a.acc2 = d_acc2;
+  a.swf = d_swf;
+  a.fprof = d_fprof;
+  a.molscal = d_molscal;
+  a.phi_m = d_phi_m;
+  a.phi = d_phi;
+  a.phib_state = d_phib_state;
+  a.cbulk = d_cbulk;
+  return a;
+}
+
+FieldArgs System::field_args() {
+  FieldArgs a{};
+  a.itmask = d_itmask;
+  a.swf = d_swf;
+  a.phi = d_phi;
+  a.phitot = d_phitot;
+  a.cbulk = d_cbulk;
+  a.rho = d_rho;
+  return a;
 }
 
 void System::start_phi(int prec) {
   const DevLattice& L = lat.d;
+  ends.n = 0;  // whatever a call that threw left
   const bool gmax = prec == SFX_FP32 && use_block3;
   launch_swf(L, d_u, d_itmask, ns, d_st_itvar, d_swf, d_swf32, stream, gmax ? d_gmax : nullptr, ns * kStepWords);
   gmax_valid = false;
@@ -946,9 +997,11 @@ Scf1Args System::scf1_args() {
   return a;
 }
 
-void System::compute_phi(int prec) {
+void System::compute_phi(int prec, double* f) {
   if (one_launch(prec, false)) {
-    launch_scf1d(lat.d, scf1_args(), false, stream);
+    Scf1Args a = scf1_args();
+    a.f = f;
+    launch_scf1d(lat.d, a, false, stream);
     gmax_valid = false;
     phi_valid = true;
     last_precision = prec;
@@ -960,21 +1013,30 @@ void System::compute_phi(int prec) {
     for (int m = 0; m < nm; m++) {
       bool solv = mols[m].freedom == SFX_SOLVENT;
       if ((pass == 0) == solv) continue;
+      // the sweeps of chains share their running ranks: the last one's end sum first
+      if (mols[m].kind != 0) close_ends(true, nullptr);
       if (prec == SFX_FP32)
         sweep<float, float>(m, true);
       else
         sweep<double, double>(m, false);
-      if (mols[m].freedom == SFX_RANGE_RESTRICTED) finish_range(m);
+      if (mols[m].freedom == SFX_RANGE_RESTRICTED) {
+        close_ends(true, nullptr);
+        finish_range(m, prec);
+      }
     }
-  finish_phi(prec);
-}
-
-void System::finish_phi(int prec) {
-  const DevLattice& L = lat.d;
-  launch_phi_total(L, ns, nm, d_phi_m, d_mol_uses, d_fprof, d_frozen, d_phi, d_phitot, stream, &sp, d_molscal,
-                   d_phib_state, d_cbulk);
-  launch_sides(L, ns, d_phi, d_rho, stream);
-  SFX_HIP(hipGetLastError());
+  close_ends(true, nullptr);
+  PhiArgs a = phi_args();
+  a.base = true;
+  for (int m = 0; m < nm; m++)
+    if (mols[m].freedom == SFX_RANGE_RESTRICTED) a.mode[m] = CLOSE_DONE;
+  if (prec == SFX_FP32)
+    launch_phi_close<float>(lat.d, sp, a, stream);
+  else
+    launch_phi_close<double>(lat.d, sp, a, stream);
+  FieldArgs fa = field_args();
+  fa.base = true;
+  fa.f = f;
+  launch_field_close(lat.d, sp, fa, stream);
   phi_valid = true;
   last_precision = prec;
 }
@@ -1006,28 +1068,26 @@ bool System::has_range() const {
 
 // SF_Copol1stO.cpp:1246-1280: phiPreNorm over the range, NormPhiFree with
 // phiRange / phiPreNorm, then theta and phi_b
-void System::finish_range(int m) {
+void System::finish_range(int m, int prec) {
   const Molecule& mo = mols[m];
-  double* phim = d_phi_m + (size_t)m * ns * lat.d.M;
+  const size_t off = (size_t)m * ns * lat.d.M;
+  double* phim = d_phi_m + off;
+  const double* scal = d_molscal + (size_t)m * MS_COUNT;
+  if (mo.kind == 0)
+    launch_mol_phi<double>(lat.d, nullptr, d_swf + (size_t)mo.seq[0] * lat.d.M, scal, 1,
+                           phim + (size_t)mo.seq[0] * lat.d.M, stream);
+  else if (prec == SFX_FP32)
+    launch_mol_phi_states<float>(lat.d, mo.uses_mask(), ns, (const float*)d_acc + off,
+                                 middle_out(mo) ? (const float*)d_acc2 + off : nullptr, d_swf, scal, phim, stream);
+  else
+    launch_mol_phi_states<double>(lat.d, mo.uses_mask(), ns, (const double*)d_acc + off,
+                                  middle_out(mo) ? (const double*)d_acc2 + off : nullptr, d_swf, scal, phim, stream);
   const int nb = launch_range_sum(lat.d, mo.range, mo.uses_mask(), ns, phim, d_partial, stream);
   launch_range_scale(lat.d, mo.uses_mask(), ns, d_partial, nb, mo.phi_range, mo.N, d_molscal + (size_t)m * MS_COUNT,
                      phim, stream);
 }
 
-void System::residual_internal(int prec) {
-  if (one_launch(prec, false)) {
-    Scf1Args a = scf1_args();
-    a.f = d_f;
-    launch_scf1d(lat.d, a, false, stream);
-    gmax_valid = false;
-    phi_valid = true;
-    last_precision = prec;
-    return;
-  }
-  compute_phi(prec);
-  launch_residual(lat.d, sp, d_itmask, d_swf, d_rho, d_phitot, d_cbulk, d_f, stream);
-  SFX_HIP(hipGetLastError());
-}
+void System::residual_internal(int prec) { compute_phi(prec, d_f); }
 
 void System::drop_graphs() {
   for (auto& g : res_graph)
