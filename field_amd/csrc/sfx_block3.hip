@@ -40,32 +40,35 @@
 namespace sfx {
 
 constexpr int kTX = 8, kTY = 8, kTZ = 16;
+static_assert(kTY % 2 == 0, "rows are numbered in pairs outside the tile");
 constexpr int kH = kB3Ranks;  // largest widening: the lattice-side bound of block3_ok
 // the tile widened by H layers; one (y, z) column of it is two threads, each
 // with px of its x planes in registers
-template <int H>
+template <int H, int KIND>
 struct B3Region {
   static constexpr int rx = kTX + 2 * H, ry = kTY + 2 * H, rz = kTZ + 2 * H;
   static constexpr int px = rx / 2;
   static constexpr int half = (ry * rz + 63) / 64 * 64;  // threads of one half
   static constexpr int threads = 2 * half;
-  // LDS words of one rank: planes 1..px-1 of each half (the outermost plane is
-  // nobody's y or z neighbour), a row of padding below and above
-  static constexpr int words = 2 * (px - 1) * half + 2 * rz;
+  // LDS words of one rank: the planes from p0 to px - 1 of each half (on the
+  // simple cubic lattice the outermost one is nobody's y or z neighbour), a row
+  // and a word of padding below and above
+  static constexpr int p0 = KIND == ST_3D_SC ? 1 : 0, planes = px - p0, pad = rz + 1;
+  static constexpr int words = 2 * planes * half + 2 * pad;
 };
 // two LDS buffers (one barrier per rank) where they leave room for three
 // workgroups per CU, else one buffer and two barriers
-template <typename T, bool TANGENT, int H>
+template <typename T, bool TANGENT, int H, int KIND>
 constexpr bool b3_double() {
-  return 2 * (TANGENT ? 2 : 1) * B3Region<H>::words * (int)sizeof(T) <= 53 * 1024;
+  return 2 * (TANGENT ? 2 : 1) * B3Region<H, KIND>::words * (int)sizeof(T) <= 53 * 1024;
 }
-template <typename T, bool TANGENT, int H>
+template <typename T, bool TANGENT, int H, int KIND>
 constexpr int b3_lds() {
-  return (b3_double<T, TANGENT, H>() ? 2 : 1) * (TANGENT ? 2 : 1) * B3Region<H>::words * (int)sizeof(T);
+  return (b3_double<T, TANGENT, H, KIND>() ? 2 : 1) * (TANGENT ? 2 : 1) * B3Region<H, KIND>::words * (int)sizeof(T);
 }
 
 bool block3_ok(const DevLattice& L) {
-  return L.grad == 3 && L.kind == ST_3D_SC && L.order == 1 && L.nx > kH && L.ny > kH && L.nz > kH;
+  return L.grad == 3 && (L.kind == ST_3D_SC || L.kind == ST_3D_FCC) && L.order == 1 && L.nx > kH && L.ny > kH && L.nz > kH;
 }
 
 // lattice coordinate c -> interior coordinate. Within kH of the lattice one
@@ -89,17 +92,17 @@ __device__ __forceinline__ float block_max_f(float v, float* red) {
   return r;
 }
 
-template <typename T, bool TANGENT, bool SCALED, bool CONNECT, int H>
-__global__ void __launch_bounds__(B3Region<H>::threads) k_block3(DevLattice L, B3Launch<T> la, int nb) {
-  using R = B3Region<H>;
+template <typename T, bool TANGENT, bool SCALED, bool CONNECT, int H, int KIND>
+__global__ void __launch_bounds__((B3Region<H, KIND>::threads)) k_block3(DevLattice L, B3Launch<T> la, int nb) {
+  using R = B3Region<H, KIND>;
   constexpr int PX = R::px, RX = R::rx, RZ = R::rz, NT = R::half;
   constexpr int OX = PX - H;  // owned planes of a half: its planes H..PX-1
-  constexpr bool DB = b3_double<T, TANGENT, H>();
+  constexpr bool DB = b3_double<T, TANGENT, H, KIND>();
   // chain of this workgroup and its tile number within that chain's grid
   const int chain = (int)blockIdx.x >= nb ? 1 : 0;
   const int bl = (int)blockIdx.x - chain * nb;
   const B3Args<T>& a = la.a[chain];
-  __shared__ __align__(16) T lds[b3_lds<T, TANGENT, H>() / sizeof(T)];
+  __shared__ __align__(16) T lds[b3_lds<T, TANGENT, H, KIND>() / sizeof(T)];
   __shared__ float red[R::threads / 64], scl[2];
   __shared__ T cfac[kB3Ranks];
 
@@ -143,7 +146,12 @@ __global__ void __launch_bounds__(B3Region<H>::threads) k_block3(DevLattice L, B
   // the planes H.. are owned where (y, z) lies in the tile and in the lattice
   const int half = __builtin_amdgcn_readfirstlane(t >= NT ? 1 : 0);
   const int c = t - half * NT;
-  const int Y = c / RZ, Z = c - Y * RZ;
+  // rows of the region from the tile's outwards, so that whole waves have no
+  // row left that a later rank needs: `row` is the wave's innermost
+  const int ring = c / RZ, Z = c - ring * RZ;
+  const int off = (ring - kTY) / 2;  // (threads past the last row keep a word of their own behind it)
+  const int Y = ring < kTY ? H + ring : ring >= R::ry ? ring : ring & 1 ? H + kTY + off : H - 1 - off;
+  const int row = __builtin_amdgcn_readfirstlane(ring);
   const bool owner = Y >= H && Y < H + kTY && Z >= H && Z < H + kTZ && y0 + Y - H <= L.ny && z0 + Z - H <= L.nz;
   const int yy = extend(y0 + Y - H, L.ny, L.periodic[1], L.mirror2_1[1], L.mirror2_2[1]);
   const int zz = extend(z0 + Z - H, L.nz, L.periodic[2], L.mirror2_1[2], L.mirror2_2[2]);
@@ -216,8 +224,34 @@ __global__ void __launch_bounds__(B3Region<H>::threads) k_block3(DevLattice L, B
       if constexpr (TANGENT) bacc[i] = T(0);
     }
   }
-  const T sixth = T(1.0 / 6.0);
-  const unsigned own = (unsigned)(RZ + c + half * (PX - 1) * NT), other = (unsigned)(RZ + c + (1 - half) * (PX - 1) * NT);
+  // LDS word of this column's plane p0, and of the other half's
+  const unsigned pos = (unsigned)(R::pad + Y * RZ + Z);
+  const unsigned own = pos + (unsigned)(half * R::planes * NT), other = pos + (unsigned)((1 - half) * R::planes * NT);
+  // the sum over the stencil at plane j, from the rank in E (registers) and buf:
+  // simple cubic six faces; FCC the in-plane diagonals and the faces of the
+  // planes before and behind, whose sums the caller rolls on
+  auto faces = [&](const T* buf, unsigned o) __attribute__((always_inline)) {
+    return buf[o - RZ] + buf[o + RZ] + buf[o - 1] + buf[o + 1];
+  };
+  auto diagonals = [&](const T* buf, unsigned o) __attribute__((always_inline)) {
+    return buf[o - RZ - 1] + buf[o - RZ + 1] + buf[o + RZ - 1] + buf[o + RZ + 1];
+  };
+  // `out`: what plane j takes from the next plane outwards, rolled on
+  auto stencil_sum = [&](const T (&E)[PX], const T* buf, int j, T& out, T& here) __attribute__((always_inline)) {
+    const unsigned o = own + (j - R::p0) * NT;
+    if constexpr (KIND == ST_3D_SC) {
+      const T in = j + 1 < PX ? E[j + 1 < PX ? j + 1 : j] : buf[other + (R::planes - 1) * NT];
+      const T s = (out + in + buf[o - RZ] + buf[o + RZ] + buf[o - 1] + buf[o + 1]) * T(1.0 / 6.0);
+      out = E[j];
+      return s;
+    } else {
+      const T in = faces(buf, j + 1 < PX ? o + NT : other + (R::planes - 1) * NT);
+      const T s = (out + in + diagonals(buf, o)) * T(1.0 / 12.0);
+      out = here;
+      here = in;
+      return s;
+    }
+  };
 #pragma unroll
   for (int k = 1; k <= H; k++) {
     if (k <= nr) {
@@ -235,27 +269,34 @@ __global__ void __launch_bounds__(B3Region<H>::threads) k_block3(DevLattice L, B
       T* const buf = lds + (DB && (k & 1) ? (TANGENT ? 2 : 1) * R::words : 0);
       T* const dbuf = buf + R::words;
       if (!DB && k > 1) __syncthreads();  // the previous rank's reads are done
+      const int rows = kTY + 2 * (nr - k);  // rows that rank k is needed on
+      if (row < rows + 2) {
 #pragma unroll
-      for (int j = k; j < PX; j++) {
-        buf[own + (j - 1) * NT] = G[j];
-        if constexpr (TANGENT) dbuf[own + (j - 1) * NT] = D[j];
+        for (int j = k - 1 + R::p0; j < PX; j++) {
+          buf[own + (j - R::p0) * NT] = G[j];
+          if constexpr (TANGENT) dbuf[own + (j - R::p0) * NT] = D[j];
+        }
       }
       __syncthreads();
-      T co = G[k - 1], dco = TANGENT ? D[k - 1] : T(0);  // the next plane outwards, old rank
+      if (row < rows) {
+        // what plane k takes from plane k - 1, and on FCC what plane k + 1 takes from k
+        T out = G[k - 1], dout = TANGENT ? D[k - 1] : T(0), here = T(0), dhere = T(0);
+        if constexpr (KIND != ST_3D_SC) {
+          out = faces(buf, own + (k - 1) * NT);
+          here = faces(buf, own + k * NT);
+          if constexpr (TANGENT) {
+            dout = faces(dbuf, own + (k - 1) * NT);
+            dhere = faces(dbuf, own + k * NT);
+          }
+        }
 #pragma unroll
-      for (int j = k; j < PX; j++) {
-        const unsigned o = own + (j - 1) * NT;
-        const T cc = G[j];
-        const T ci = j + 1 < PX ? G[j + 1 < PX ? j + 1 : j] : buf[other + (PX - 2) * NT];
-        const T s = (co + ci + buf[o - RZ] + buf[o + RZ] + buf[o - 1] + buf[o + 1]) * sixth;
-        G[j] = g[j] * s;
-        co = cc;
-        if constexpr (TANGENT) {
-          const T dc = D[j];
-          const T dci = j + 1 < PX ? D[j + 1 < PX ? j + 1 : j] : dbuf[other + (PX - 2) * NT];
-          const T ds = (dco + dci + dbuf[o - RZ] + dbuf[o + RZ] + dbuf[o - 1] + dbuf[o + 1]) * sixth;
-          D[j] = g[j] * (ds - v[j] * s);
-          dco = dc;
+        for (int j = k; j < PX; j++) {
+          const T s = stencil_sum(G, buf, j, out, here);
+          G[j] = g[j] * s;
+          if constexpr (TANGENT) {
+            const T ds = stencil_sum(D, dbuf, j, dout, dhere);
+            D[j] = g[j] * (ds - v[j] * s);
+          }
         }
       }
       // the owned tile sites of rank k: store and compose
@@ -313,25 +354,25 @@ __global__ void __launch_bounds__(B3Region<H>::threads) k_block3(DevLattice L, B
   }
 }
 
-template <typename T, bool TG, bool SC, bool CN, int H>
+template <typename T, bool TG, bool SC, bool CN, int H, int KIND>
 static void b3_launch(const DevLattice& L, const B3Launch<T>& a, unsigned nb, hipStream_t st, hipEvent_t ev0,
                       hipEvent_t ev1) {
-  static_assert(b3_lds<T, TG, H>() <= 64 * 1024, "static LDS");
+  static_assert(b3_lds<T, TG, H, KIND>() <= 64 * 1024, "static LDS");
   // with events: recorded by the dispatch itself at kernel start and end
-  hipExtLaunchKernelGGL((k_block3<T, TG, SC, CN, H>), dim3(nb * (unsigned)a.nchains), dim3(B3Region<H>::threads), 0,
-                        st, ev0, ev1, 0u, L, a, (int)nb);
+  hipExtLaunchKernelGGL((k_block3<T, TG, SC, CN, H, KIND>), dim3(nb * (unsigned)a.nchains),
+                        dim3(B3Region<H, KIND>::threads), 0, st, ev0, ev1, 0u, L, a, (int)nb);
 }
-template <typename T, bool TG, bool SC, bool CN>
+template <typename T, bool TG, bool SC, bool CN, int KIND>
 static void b3_launch_h(int nr, const DevLattice& L, const B3Launch<T>& a, unsigned nb, hipStream_t st,
                         hipEvent_t ev0, hipEvent_t ev1) {
   // launches of one or two ranks (a chain's ends, a change of the segment
   // state) load and compute a smaller region: 7.2 / 9.1 us instead of 14 / 16
   // at 75 x 61 x 90 in FP32
   if (nr <= 2) {
-    b3_launch<T, TG, SC, CN, 2>(L, a, nb, st, ev0, ev1);
+    b3_launch<T, TG, SC, CN, 2, KIND>(L, a, nb, st, ev0, ev1);
     return;
   }
-  if constexpr (!(TG && sizeof(T) == 8)) b3_launch<T, TG, SC, CN, kB3Ranks>(L, a, nb, st, ev0, ev1);
+  if constexpr (!(TG && sizeof(T) == 8)) b3_launch<T, TG, SC, CN, kB3Ranks, KIND>(L, a, nb, st, ev0, ev1);
 }
 
 template <typename T>
@@ -358,7 +399,9 @@ void launch_block3(const DevLattice& L, const B3Launch<T>& a, bool tangent, bool
     nr = std::max(nr, a.a[c].nr);
   }
   const unsigned nb = (unsigned)(((L.nx + kTX - 1) / kTX) * ((L.ny + kTY - 1) / kTY) * ((L.nz + kTZ - 1) / kTZ));
-#define B3(TG, SC, CN) b3_launch_h<T, TG, SC, CN>(nr, L, a, nb, st, ev0, ev1)
+#define B3(TG, SC, CN)                                                         \
+  (L.kind == ST_3D_FCC ? b3_launch_h<T, TG, SC, CN, ST_3D_FCC>(nr, L, a, nb, st, ev0, ev1) \
+                       : b3_launch_h<T, TG, SC, CN, ST_3D_SC>(nr, L, a, nb, st, ev0, ev1))
   if constexpr (sizeof(T) == 4) {  // FP32 sweeps are scaled, FP64 ones are not
     SFX_REQUIRE(scaled, SFX_E_INVALID, "FP32 blocked sweeps are scaled");
     if (tangent) { if (connect) B3(true, true, true); else B3(true, true, false); }

@@ -140,7 +140,7 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   {
     const int sk = sweep_kernel = opt ? opt->sweep_kernel : SFX_SWEEP_AUTO;
     SFX_REQUIRE(sk >= SFX_SWEEP_AUTO && sk <= SFX_SWEEP_BLOCKED, SFX_E_INVALID, "unknown sweep_kernel");
-    use_block3 = sk != SFX_SWEEP_PER_RANK && block3_ok(lat.d);
+    use_block3 = sk != SFX_SWEEP_PER_RANK && lat.d.kind == ST_3D_SC && block3_ok(lat.d);
     use_chain1 = sk != SFX_SWEEP_PER_RANK && chain1d_ok(lat.d);
     schedule = opt ? opt->chain_schedule : SFX_SCHEDULE_AUTO;
     SFX_REQUIRE(schedule == SFX_SCHEDULE_AUTO || schedule == SFX_SCHEDULE_SEQUENTIAL, SFX_E_INVALID,
@@ -296,10 +296,11 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   const size_t slot_bytes = comps * M * sizeof(double);
   checkpointed = budget != 0 && (size_t)maxstore * slot_bytes > budget;
   store_slots = 1;
-  // 2-D: a checkpointed store and the sequential schedule keep one launch per
+  // 2-D and FCC: a checkpointed store and the sequential schedule keep one launch per
   // rank, so that they repeat each other bit for bit within the memory they
   // took before (blocked segments need two sets of slots)
-  if (sweep_kernel != SFX_SWEEP_PER_RANK && block2_ok(lat.d) && schedule == SFX_SCHEDULE_AUTO && !checkpointed)
+  if (sweep_kernel != SFX_SWEEP_PER_RANK && (block2_ok(lat.d) || block3_ok(lat.d)) &&
+      schedule == SFX_SCHEDULE_AUTO && !checkpointed)
     use_block3 = true;
   for (Molecule& mo : mols) {
     mo.plan.init(mo.nstore, checkpointed, use_block3 ? kB3Ranks : 1);
