@@ -228,13 +228,12 @@ __global__ void k_tconnect(DevLattice L, const T* __restrict__ A, const T* __res
 
 // per-state direction v_t = v_{itvar(t)} (zero for frozen states), in T
 // (out32 optional: the same directions rounded to FP32)
-__global__ void k_state_dir(long long M, int ns, const int* st_itvar, const double* v, double* out,
-                            float* out32) {
+__global__ void k_state_dir(long long M, int ns, const int* st_itvar, SiteVec v, double* out, float* out32) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= M) return;
   for (int t = 0; t < ns; t++) {
     int iv = st_itvar[t];
-    const double d = iv >= 0 ? v[(long long)iv * M + i] : 0.0;
+    const double d = iv >= 0 ? site_get(v, M, iv, i) : 0.0;
     out[(long long)t * M + i] = d;
     if (out32) out32[(long long)t * M + i] = (float)d;
   }
@@ -767,7 +766,7 @@ static Tangent& tangent(System& S) {
 
 // the tangent sweeps of every molecule for the direction v and their closing;
 // with `base` the molecules' phi as well (tsweep)
-static void tangent_sweeps(System& S, Tangent& W, const double* v, int precision, bool base) {
+static void tangent_sweeps(System& S, Tangent& W, const SiteVec& v, int precision, bool base) {
   hipStream_t st = S.stream;
   const long long Mn = S.lat.d.M;
   double* v64 = W.v64.p;
@@ -793,7 +792,7 @@ static void tangent_sweeps(System& S, Tangent& W, const double* v, int precision
 }
 
 // phi (base), dphi, contact averages and the linearised residual
-static void tangent_close(System& S, Tangent& W, const double* v, double* jv, int precision, bool base) {
+static void tangent_close(System& S, Tangent& W, const SiteVec& v, const SiteOut& jv, int precision, bool base) {
   PhiArgs a = S.phi_args();
   a.base = base;
   a.tangent = true;
@@ -826,9 +825,10 @@ static void require_products(const System& S) {
 }
 
 // the product of a 1-D system in one launch, where that applies
-static bool one_launch_product(System& S, Tangent& W, const double* v, double* jv, int precision, bool base) {
+static bool one_launch_product(System& S, Tangent& W, const SiteVec& v, const SiteOut& jv, int precision, bool base,
+                               const double* x) {
   if (!S.one_launch(precision, true)) return false;
-  Scf1Args a = S.scf1_args();
+  Scf1Args a = S.scf1_args(x);
   a.base = base;
   a.v = v;
   a.dstore = W.dstore.p;
@@ -847,23 +847,27 @@ static bool one_launch_product(System& S, Tangent& W, const double* v, double* j
 void jvp_at_base(System& S, const double* v, double* jv, int precision) {
   require_products(S);
   Tangent& W = tangent(S);
-  if (one_launch_product(S, W, v, jv, precision, false)) return;
-  tangent_sweeps(S, W, v, precision, false);
-  tangent_close(S, W, v, jv, precision, false);
+  const SiteVec vi = S.vec_internal(v);
+  const SiteOut out = S.out_internal(jv);
+  if (one_launch_product(S, W, vi, out, precision, false, nullptr)) return;
+  tangent_sweeps(S, W, vi, precision, false);
+  tangent_close(S, W, vi, out, precision, false);
 }
 
-// J v at S.d_u, base and tangent in one sweep per molecule: the base sweep of
+// J v at x (device, the ABI's layout, as v and jv), base and tangent in one sweep per molecule: the base sweep of
 // a compute_phi before it was 33% of the product's kernel time on the 64^3 melt
 // (FP32, 443 -> 328 us without it), 39% on second-order 128^3 (52.4 -> 33.1 ms)
 // and 42% on the 64 x 128 pore (971 -> 579 us)
-void jvp_internal(System& S, const double* v, double* jv, int precision) {
-  if (S.has_range()) S.compute_phi(precision);  // phi stays defined after the refusal
+void jvp_abi(System& S, const double* x, const double* v, double* jv, int precision) {
+  if (S.has_range()) S.compute_phi(precision, x);  // phi stays defined after the refusal
   require_products(S);
   Tangent& W = tangent(S);
-  if (one_launch_product(S, W, v, jv, precision, true)) return;
-  S.start_phi(precision);
-  tangent_sweeps(S, W, v, precision, true);
-  tangent_close(S, W, v, jv, precision, true);
+  const SiteVec vi = S.vec_abi(v);
+  const SiteOut out = S.out_abi(jv);
+  if (one_launch_product(S, W, vi, out, precision, true, x)) return;
+  S.start_phi(precision, x);
+  tangent_sweeps(S, W, vi, precision, true);
+  tangent_close(S, W, vi, out, precision, true);
 }
 
 // ---------------------------------------------------------------------------

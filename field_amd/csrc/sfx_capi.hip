@@ -29,7 +29,7 @@ int last_code() { return g_code; }
 
 
 // implemented in sfx_adjoint.hip
-void jvp_internal(System& S, const double* v_internal, double* jv_internal, int precision);
+void jvp_abi(System& S, const double* x, const double* v, double* jv, int precision);
 void vjp_internal(System& S, const double* w_internal, double* jtw_internal, int precision);
 void load_vec(System& S, const double* x, int where, double* dst_internal);
 
@@ -94,8 +94,7 @@ int sfx_system_sizes(const sfx_system* s, long* nvar, long* M) {
 int sfx_compute_phi(sfx_system* s, const double* x, int where, int precision) {
   return guarded([&] {
     SFX_REQUIRE(s && x, SFX_E_INVALID, "NULL argument");
-    s->s.load_x(x, where);
-    s->s.compute_phi(precision);
+    s->s.compute_phi(precision, s->s.abi_in(x, where));
     s->s.sync();
   });
 }
@@ -103,9 +102,10 @@ int sfx_compute_phi(sfx_system* s, const double* x, int where, int precision) {
 int sfx_residual(sfx_system* s, const double* x, double* f, int where, int precision) {
   return guarded([&] {
     SFX_REQUIRE(s && x && f, SFX_E_INVALID, "NULL argument");
-    s->s.load_x(x, where);
-    s->s.residual_internal(precision);
-    s->s.store_f(s->s.d_f, f, where);
+    System& S = s->s;
+    // from host memory both go through one staging vector: x has been read when f is written
+    S.compute_phi(precision, S.abi_in(x, where), S.out_abi(where == SFX_HOST ? S.d_xabi : f));
+    S.abi_out(S.d_xabi, f, where);
   });
 }
 
@@ -113,12 +113,14 @@ int sfx_jvp(sfx_system* s, const double* x, const double* v, double* jv, int whe
   return guarded([&] {
     SFX_REQUIRE(s && x && v && jv, SFX_E_INVALID, "NULL argument");
     System& S = s->s;
-    S.load_x(x, where);
-    double *vin, *out;
-    S.abi_vectors(vin, out);
-    load_vec(S, v, where, vin);
-    jvp_internal(S, vin, out, precision);
-    S.store_f(out, jv, where);
+    const double* xd = S.abi_in(x, where);
+    double *vin = const_cast<double*>(v), *out = jv;
+    if (where == SFX_HOST) {
+      S.abi_vectors(vin, out);
+      SFX_HIP(hipMemcpyAsync(vin, v, S.nvar * sizeof(double), hipMemcpyHostToDevice, S.stream));
+    }
+    jvp_abi(S, xd, vin, out, precision);
+    S.abi_out(out, jv, where);
   });
 }
 

@@ -42,17 +42,19 @@ struct Scf1Args {
   Chain1Mol mols[SFX_MAXM];  // in the order of evaluation
   const Chain1Run* runs;
   int nruns;
-  const double* u;
+  SiteVec x;
+  double* u;              // may be null: x's copy in the internal layout
   const unsigned char* itmask;
   const double* fprof;
   double* swf;
   float* swf32;
   double *store, *phi_m, *phi, *rho, *phitot, *molscal, *phib_state, *cbulk;
-  double* f;              // may be null: phi only
+  SiteOut f;              // may be null: phi only
   // tangent
   int base;               // with the base evaluation
-  const double* v;
-  double *dstore, *dphi_m, *jv;
+  SiteVec v;
+  double *dstore, *dphi_m;
+  SiteOut jv;
 };
 
 // one workgroup evaluates the whole system (up to 1024 layers whose arrays fit LDS)

@@ -325,15 +325,17 @@ __global__ void __launch_bounds__(kScf1Threads) k_scf1d(DevLattice L, Scf1Args A
   walk.init(A.runs, A.nruns);
   if (!base && tid < sp.nm * MS_COUNT) ms[tid] = tid % MS_COUNT == MS_REF ? 0.0 : A.molscal[tid];
   __syncthreads();
+  if (A.u)
+    for (int q = tid; q < sp.n_itvar * M; q += kScf1Threads) A.u[q] = site_get(A.x, M, q / M, q % M);
   // SWF (k_swf), a thread per state and layer
   for (int q = tid; q < ns * M; q += kScf1Threads) {
     const int t = q / M, i = q - t * M;
     const int s = remap(i, n, L.b1[0], L.b2[0]);
     const int iv = sp.st_itvar[t];
-    const double g = (iv >= 0 && A.itmask[s]) ? exp(-A.u[(long long)iv * M + s]) : 0.0;
+    const double g = (iv >= 0 && A.itmask[s]) ? exp(-site_get(A.x, M, iv, s)) : 0.0;
     if (i >= 1 && i <= n) {
       lg[t * W + i] = g;
-      if constexpr (TAN) lv[t * W + i] = iv >= 0 ? A.v[(long long)iv * M + i] : 0.0;
+      if constexpr (TAN) lv[t * W + i] = iv >= 0 ? site_get(A.v, M, iv, i) : 0.0;
     }
     if (base) {
       A.swf[(long long)t * M + i] = g;
@@ -466,7 +468,7 @@ __global__ void __launch_bounds__(kScf1Threads) k_scf1d(DevLattice L, Scf1Args A
       tot += lacc[t * W + i];
       if constexpr (TAN) dtot += ldacc[t * W + i];
     }
-    double* out = TAN ? A.jv : A.f;
+    const SiteOut& out = TAN ? A.jv : A.f;
     const bool side = (i > 0 || L.surf1[0]) && (i <= n || L.surf2[0]);  // k_sides: not the other halos
     if (base) {
       A.phitot[i] = tot;
@@ -475,19 +477,19 @@ __global__ void __launch_bounds__(kScf1Threads) k_scf1d(DevLattice L, Scf1Args A
         A.rho[(long long)t * M + i] = side ? side_at1(L, lacc + t * W, i) : 0.0;
       }
     }
-    if (!out) continue;
+    if (!out.p) continue;
     if (!A.itmask[i]) {
-      for (int k = 0; k < sp.n_itvar; k++) out[(long long)k * M + i] = 0.0;
+      site_none(out, M, i);
       continue;
     }
     auto rho = [&](int t) { return base ? side_at1(L, lacc + t * W, i) : A.rho[(long long)t * M + i]; };
     if constexpr (TAN) {
-      jres_site(sp, tot, dtot, dm, [&](int k) { return A.v[(long long)k * M + i]; }, rho,
+      jres_site(sp, tot, dtot, dm, [&](int k) { return site_get(A.v, M, k, i); }, rho,
                 [&](int t) { return side_at1(L, ldacc + t * W, i); },
-                [&](int k, double d) { out[(long long)k * M + i] = d; });
+                [&](int k, double d) { site_put(out, M, k, i, d); });
     } else {
       residual_site(sp, tot, cb, [&](int t) { return lg[t * W + i]; }, rho,
-                    [&](int k, double v) { out[(long long)k * M + i] = v; });
+                    [&](int k, double v) { site_put(out, M, k, i, v); });
     }
   }
 }

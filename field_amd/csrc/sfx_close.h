@@ -53,9 +53,11 @@ struct FieldArgs {
   const unsigned char* itmask;
   const double *swf, *phi, *cbulk;
   double *rho, *phitot;
-  double* f;                                 // nullptr: contact averages alone
-  const double *v, *dphi, *dmol;             // jv: direction and tangents
-  double *drho, *jv;                         // jv nullptr: no product
+  SiteOut f;                   // p null: contact averages alone
+  SiteVec v;                   // jv: direction and tangents
+  const double *dphi, *dmol;
+  double* drho;
+  SiteOut jv;                  // p null: no product
   bool base;
 };
 void launch_field_close(const DevLattice& L, const SysParams& sp, const FieldArgs& a, hipStream_t st);

@@ -342,9 +342,9 @@ __global__ void __launch_bounds__(kCB) k_field_close(DevLattice L, SysParams sp,
   if constexpr (RES) {
     if (site)
       residual_site<NS>(sp, pt, a.cbulk, [&](int t) { return a.swf[(long long)t * L.M + i]; }, rho,
-                        [&](int k, double v) { a.f[(long long)k * L.M + i] = v; });
+                        [&](int k, double v) { site_put(a.f, L.M, k, i, v); });
     else
-      for (int k = 0; k < sp.n_itvar; k++) a.f[(long long)k * L.M + i] = 0.0;
+      site_none(a.f, L.M, i);
   }
   if constexpr (TAN) {
     auto drho = [&](int t) {
@@ -354,21 +354,21 @@ __global__ void __launch_bounds__(kCB) k_field_close(DevLattice L, SysParams sp,
         return a.drho[(long long)t * L.M + i];
     };
     if (site)
-      jres_site<NS>(sp, pt, dpt, a.dmol, [&](int k) { return a.v[(long long)k * L.M + i]; }, rho, drho,
-                    [&](int k, double d) { a.jv[(long long)k * L.M + i] = d; });
+      jres_site<NS>(sp, pt, dpt, a.dmol, [&](int k) { return site_get(a.v, L.M, k, i); }, rho, drho,
+                    [&](int k, double d) { site_put(a.jv, L.M, k, i, d); });
     else
-      for (int k = 0; k < sp.n_itvar; k++) a.jv[(long long)k * L.M + i] = 0.0;
+      site_none(a.jv, L.M, i);
   }
 }
 
 template <int NS, int KIND>
 static void field_close_k(const DevLattice& L, const SysParams& sp, const FieldArgs& a, hipStream_t st) {
   const unsigned nb = grid1(L.M, kCB);
-  if (a.jv && a.base)
+  if (a.jv.p && a.base)
     k_field_close<NS, KIND, true, false, true><<<nb, kCB, 0, st>>>(L, sp, a);
-  else if (a.jv)
+  else if (a.jv.p)
     k_field_close<NS, KIND, false, false, true><<<nb, kCB, 0, st>>>(L, sp, a);
-  else if (a.f)
+  else if (a.f.p)
     k_field_close<NS, KIND, true, true, false><<<nb, kCB, 0, st>>>(L, sp, a);
   else
     k_field_close<NS, KIND, true, false, false><<<nb, kCB, 0, st>>>(L, sp, a);

@@ -88,6 +88,39 @@ struct SysParams {
   double mol_ref[SFX_MAXM];
 };
 
+// A vector over the iteration variables, read or written by the kernels in the
+// layout it has: p[k * M + i] for variable k of site i, or, where order is
+// given, the variables of a site together in the order of the iteration sites
+// (sfx_residual's layout of the SF form). Sites off the iteration read 0.
+struct SiteVec {
+  const double* p;
+  const int* order;            // site -> its ordinal, -1 off the iteration
+  const unsigned char* mask;
+  int nv;
+};
+struct SiteOut {
+  double* p;  // may be null
+  const int* order;
+  int nv;
+};
+#ifdef __HIPCC__
+__device__ __forceinline__ double site_get(const SiteVec& v, long long M, int k, long long i) {
+  if (v.order) {
+    const int o = v.order[i];
+    return o >= 0 ? v.p[(long long)o * v.nv + k] : 0.0;
+  }
+  return v.mask[i] ? v.p[(long long)k * M + i] : 0.0;
+}
+__device__ __forceinline__ void site_put(const SiteOut& f, long long M, int k, long long i, double value) {
+  f.p[f.order ? (long long)f.order[i] * f.nv + k : (long long)k * M + i] = value;
+}
+// a site off the iteration: 0, where the layout has a place for it
+__device__ __forceinline__ void site_none(const SiteOut& f, long long M, long long i) {
+  if (!f.order)
+    for (int k = 0; k < f.nv; k++) f.p[(long long)k * M + i] = 0.0;
+}
+#endif
+
 // up to eight device arrays of 4-byte words cleared by one launch
 struct ZeroList {
   void* p[8];
@@ -131,11 +164,11 @@ void launch_mol_phi_states(const DevLattice& L, unsigned uses, int ns, const A* 
 // scal[MS_REF] = lna[ia] + lnb[ib] (0 when lna is null): the reference log of
 // a middle-out sweep's compositions
 void launch_set_ref_pair(double* scal, const double* lna, int ia, const double* lnb, int ib, hipStream_t st);
-// zero != null: the same launch also clears zero[0..nzero)
-void launch_swf(const DevLattice& L, const double* u, const unsigned char* itmask, int nstates,
+// u != null: x is copied there, in the internal layout; zero != null: the same
+// launch also clears zero[0..nzero)
+void launch_swf(const DevLattice& L, const SiteVec& x, double* u, const unsigned char* itmask, int nstates,
                 const int* st_itvar, double* swf, float* swf32, hipStream_t st, unsigned* zero = nullptr,
                 int nzero = 0);
-// sp != null: the same launch also writes the bulk fractions and ChemIntBulk
 int launch_free_energy(const DevLattice& L, const SysParams& sp, const double* phi, const double* phi_m,
                        const double* rho, const double* swf, const double* u, const double* molscal,
                        double* partial, hipStream_t st);

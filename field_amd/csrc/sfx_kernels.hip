@@ -51,7 +51,7 @@ __device__ double block_sum(double v) {
 // ---------------------------------------------------------------------------
 // SWF: g_t(r) = exp(-u_{itvar(t)}(src(r))) at iteration sites, 0 elsewhere,
 // halos from their source site (SF_Solve.cpp:794-852 + SetBoundaries).
-__global__ void k_swf(DevLattice L, const double* __restrict__ u, const unsigned char* __restrict__ itmask,
+__global__ void k_swf(DevLattice L, SiteVec x0, double* __restrict__ u, const unsigned char* __restrict__ itmask,
                       int nstates, const int* __restrict__ st_itvar, double* __restrict__ swf,
                       float* __restrict__ swf32, unsigned* __restrict__ zero, int nzero) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -64,9 +64,11 @@ __global__ void k_swf(DevLattice L, const double* __restrict__ u, const unsigned
   int sz = L.grad >= 3 ? remap(z, L.nz, L.b1[2], L.b2[2]) : z;
   long long s = sidx(L, sx, sy, sz);
   bool it = itmask[s];
+  if (u)
+    for (int k = 0; k < x0.nv; k++) u[(long long)k * L.M + i] = site_get(x0, L.M, k, i);
   for (int t = 0; t < nstates; t++) {
     int iv = st_itvar[t];
-    double g = (iv >= 0 && it) ? exp(-u[(long long)iv * L.M + s]) : 0.0;
+    double g = (iv >= 0 && it) ? exp(-site_get(x0, L.M, iv, s)) : 0.0;
     swf[(long long)t * L.M + i] = g;
     if (swf32) swf32[(long long)t * L.M + i] = (float)g;
   }
@@ -453,10 +455,10 @@ void launch_mol_phi_states(const DevLattice& L, unsigned uses, int ns, const A* 
   k_mol_phi_states<A><<<grid1(L.V, kBlock), kBlock, 0, st>>>(L, uses, ns, acc, acc2, g, scal, phi_m);
 }
 
-void launch_swf(const DevLattice& L, const double* u, const unsigned char* itmask, int nstates,
+void launch_swf(const DevLattice& L, const SiteVec& x, double* u, const unsigned char* itmask, int nstates,
                 const int* st_itvar, double* swf, float* swf32, hipStream_t st, unsigned* zero, int nzero) {
   if (!zero) nzero = 0;
-  k_swf<<<grid1(std::max<long long>(L.M, nzero), kBlock), kBlock, 0, st>>>(L, u, itmask, nstates, st_itvar, swf,
+  k_swf<<<grid1(std::max<long long>(L.M, nzero), kBlock), kBlock, 0, st>>>(L, x, u, itmask, nstates, st_itvar, swf,
                                                                            swf32, zero, nzero);
 }
 

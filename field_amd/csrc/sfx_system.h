@@ -159,7 +159,7 @@ struct System {
   // a 1-D system evaluated by one workgroup in one launch (sfx_chain1d.hip):
   // FP64, full store, no kernel timing (which reports per-rank launches)
   bool one_launch(int precision, bool tangent) const;
-  Scf1Args scf1_args();  // the system's arrays; builds the list of runs on first use
+  Scf1Args scf1_args(const double* x);  // the system's arrays; builds the list of runs on first use
   std::vector<Chain1Mol> scf1_mols;
   int scf1_nruns = 0;
   Chain1Run* scf1_runs = nullptr;
@@ -184,6 +184,7 @@ struct System {
   int* d_mol_uses = nullptr;  // nm * ns
   unsigned char* d_itmask = nullptr;
   long long* d_sites = nullptr;
+  int* d_order = nullptr;       // site -> its ordinal among the iteration sites or -1 (null: melt form)
   void* d_store = nullptr;    // maxstore * M propagator words
   void* d_pp = nullptr;       // 2 * M running propagator
   void* d_pp2 = nullptr;      // 2 * M, the backward chain's in a middle-out sweep
@@ -222,10 +223,20 @@ struct System {
   // the two internal-layout vectors of the product entry points (kept, so a
   // call allocates nothing after the first)
   void abi_vectors(double*& in, double*& out);
-  void compute_phi(int precision, double* f = nullptr);  // from d_u; with f the residual as well
+  // a vector of an entry point on the device, in its own layout: x itself, or
+  // its copy in d_xabi; and back, waiting for the stream
+  const double* abi_in(const double* x, int where);
+  void abi_out(const double* src, double* f, int where);
+  SiteVec vec_abi(const double* p) const { return SiteVec{p, d_order, d_itmask, n_itvar}; }
+  SiteVec vec_internal(const double* p) const { return SiteVec{p, nullptr, d_itmask, n_itvar}; }
+  SiteOut out_abi(double* p) const { return SiteOut{p, d_order, n_itvar}; }
+  SiteOut out_internal(double* p) const { return SiteOut{p, nullptr, n_itvar}; }
+  // from d_u, or from x (the entry points' layout, on the device), which is
+  // copied to d_u; with f the residual as well
+  void compute_phi(int precision, const double* x = nullptr, const SiteOut& f = SiteOut{});
   // compute_phi before the molecules' sweeps: a caller that sweeps base and
   // tangent propagators together puts its own sweeps and closing behind it
-  void start_phi(int precision);
+  void start_phi(int precision, const double* x);
   // the closing launches (sfx_close.hip): a sweep leaves its molecule's end
   // rank in `ends`; close_ends derives the scalars (of the base, and of the
   // tangent into dmol) before the next chain overwrites the running ranks

@@ -27,12 +27,11 @@ static __global__ void k_fill_bytes8(unsigned long long* p, long long n) {
 static __global__ void k_set_ref(double* scal, const double* lnv, int idx, double factor) {
   if (threadIdx.x == 0 && blockIdx.x == 0) scal[MS_REF] = factor * lnv[idx];
 }
-// x (SF_Solve layout) -> u[itvar][M]; u zero off the iteration sites
-static __global__ void k_unpack_sfbox(const double* x, const long long* sites, long long nsites, int nv,
-                                      long long M, double* u) {
-  long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nsites) return;
-  for (int i = 0; i < nv; i++) u[(long long)i * M + sites[k]] = x[k * nv + i];
+// x -> u[itvar][M]; u zero off the iteration sites
+static __global__ void k_load(SiteVec x, long long M, double* u) {
+  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= M) return;
+  for (int k = 0; k < x.nv; k++) u[(long long)k * M + i] = site_get(x, M, k, i);
 }
 static __global__ void k_pack_sfbox(const double* u, const long long* sites, long long nsites, int nv,
                                     long long M, double* x) {
@@ -40,13 +39,6 @@ static __global__ void k_pack_sfbox(const double* u, const long long* sites, lon
   if (k >= nsites) return;
   for (int i = 0; i < nv; i++) x[k * nv + i] = u[(long long)i * M + sites[k]];
 }
-static __global__ void k_mask_copy(const double* x, const unsigned char* mask, int nv, long long M, double* u) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M) return;
-  bool m = mask[i];
-  for (int k = 0; k < nv; k++) u[(long long)k * M + i] = m ? x[(long long)k * M + i] : 0.0;
-}
-
 static void zero_bytes(void* p, size_t bytes, hipStream_t st) {
   long long n = (long long)((bytes + 7) / 8);
   if (n) k_fill_bytes8<<<grid1(n, 256), 256, 0, st>>>((unsigned long long*)p, n);
@@ -67,7 +59,7 @@ System::~System() {
     for (Chain1Step* p : a)
       if (p) (void)hipFree(p);
   void* ptrs[] = {d_u, d_f, d_swf, d_swf32, d_phi_m, d_acc, d_acc2, d_phi, d_rho, d_phitot, d_fprof, d_frozen,
-                  d_st_itvar, d_mol_uses, d_itmask, d_sites, d_store, d_pp, d_pp2, d_molscal, d_lnf, d_lnb,
+                  d_st_itvar, d_mol_uses, d_itmask, d_sites, d_order, d_store, d_pp, d_pp2, d_molscal, d_lnf, d_lnb,
                   d_maxf, d_maxb, d_partial, d_ticket, d_phib_state, d_cbulk, d_scalar, d_xabi, d_gmax,
                   d_abi_in, d_abi_out, scf1_runs};
   for (void* p : ptrs)
@@ -290,6 +282,7 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   d_mol_uses = dalloc<int>((size_t)nm * ns);
   d_itmask = dalloc<unsigned char>(M);
   d_sites = dalloc<long long>(sites.size());
+  if (form != SFX_FORM_MELT) d_order = dalloc<int>((size_t)M);
   // propagator store: every forward rank, or sqrt(N) checkpoints when the
   // memory budget (bytes of one FP64 store) cannot hold them all
   const size_t comps = lat.d.order == 2 ? 6 : 1;
@@ -337,6 +330,11 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   SFX_HIP(hipMemcpy(d_st_itvar, st_itvar.data(), ns * sizeof(int), hipMemcpyHostToDevice));
   SFX_HIP(hipMemcpy(d_mol_uses, uses.data(), uses.size() * sizeof(int), hipMemcpyHostToDevice));
   SFX_HIP(hipMemcpy(d_itmask, itmask.data(), M, hipMemcpyHostToDevice));
+  if (d_order) {
+    std::vector<int> order((size_t)M, -1);
+    for (size_t k = 0; k < sites.size(); k++) order[(size_t)sites[k]] = (int)k;
+    SFX_HIP(hipMemcpy(d_order, order.data(), (size_t)M * sizeof(int), hipMemcpyHostToDevice));
+  }
   if (!sites.empty())
     SFX_HIP(hipMemcpy(d_sites, sites.data(), sites.size() * sizeof(long long), hipMemcpyHostToDevice));
   // zero everything once: halo slots of propagator arrays are never written
@@ -392,20 +390,20 @@ Profiler::~Profiler() {
   for (hipEvent_t e : pool) (void)hipEventDestroy(e);
 }
 
+const double* System::abi_in(const double* x, int where) {
+  if (where != SFX_HOST) return x;
+  SFX_HIP(hipMemcpyAsync(d_xabi, x, nvar * sizeof(double), hipMemcpyHostToDevice, stream));
+  return d_xabi;
+}
+
+void System::abi_out(const double* src, double* f, int where) {
+  if (where == SFX_HOST) SFX_HIP(hipMemcpyAsync(f, src, nvar * sizeof(double), hipMemcpyDeviceToHost, stream));
+  SFX_HIP(hipStreamSynchronize(stream));
+}
+
 void System::load_x(const double* x, int where) {
-  const long long Mn = lat.d.M;
-  const double* src = x;
-  if (where == SFX_HOST) {
-    SFX_HIP(hipMemcpyAsync(d_xabi, x, nvar * sizeof(double), hipMemcpyHostToDevice, stream));
-    src = d_xabi;
-  }
-  if (form == SFX_FORM_MELT) {
-    k_mask_copy<<<grid1(Mn, 256), 256, 0, stream>>>(src, d_itmask, n_itvar, Mn, d_u);
-  } else {
-    zero_bytes(d_u, (size_t)n_itvar * Mn * 8, stream);
-    k_unpack_sfbox<<<grid1((long long)sites.size(), 256), 256, 0, stream>>>(src, d_sites, (long long)sites.size(),
-                                                                            n_itvar, Mn, d_u);
-  }
+  const double* src = abi_in(x, where);
+  k_load<<<grid1(lat.d.M, 256), 256, 0, stream>>>(vec_abi(src), lat.d.M, d_u);
   SFX_HIP(hipGetLastError());
 }
 
@@ -930,11 +928,11 @@ FieldArgs System::field_args() {
   return a;
 }
 
-void System::start_phi(int prec) {
+void System::start_phi(int prec, const double* x) {
   const DevLattice& L = lat.d;
   ends.n = 0;  // whatever a call that threw left
   const bool gmax = prec == SFX_FP32 && use_block3;
-  launch_swf(L, d_u, d_itmask, ns, d_st_itvar, d_swf, d_swf32, stream, gmax ? d_gmax : nullptr, ns * kStepWords);
+  launch_swf(L, x ? vec_abi(x) : vec_internal(d_u), x ? d_u : nullptr, d_itmask, ns, d_st_itvar, d_swf, d_swf32, stream, gmax ? d_gmax : nullptr, ns * kStepWords);
   gmax_valid = false;
   if (gmax) {
     launch_gmax(L, d_swf32, ns, d_gmax, stream, true);
@@ -946,7 +944,7 @@ bool System::one_launch(int prec, bool tangent) const {
   return prec == SFX_FP64 && use_chain1 && !checkpointed && !prof.on && scf1d_ok(lat.d, ns, tangent);
 }
 
-Scf1Args System::scf1_args() {
+Scf1Args System::scf1_args(const double* x) {
   if (!scf1_runs) {
     std::vector<Chain1Mol> hm;
     std::vector<Chain1Run> hr;
@@ -982,7 +980,8 @@ Scf1Args System::scf1_args() {
   std::copy(scf1_mols.begin(), scf1_mols.end(), a.mols);
   a.nruns = scf1_nruns;
   a.runs = scf1_runs;
-  a.u = d_u;
+  a.x = x ? vec_abi(x) : vec_internal(d_u);
+  a.u = x ? d_u : nullptr;
   a.itmask = d_itmask;
   a.fprof = d_fprof;
   a.swf = d_swf;
@@ -998,9 +997,9 @@ Scf1Args System::scf1_args() {
   return a;
 }
 
-void System::compute_phi(int prec, double* f) {
+void System::compute_phi(int prec, const double* x, const SiteOut& f) {
   if (one_launch(prec, false)) {
-    Scf1Args a = scf1_args();
+    Scf1Args a = scf1_args(x);
     a.f = f;
     launch_scf1d(lat.d, a, false, stream);
     gmax_valid = false;
@@ -1008,7 +1007,7 @@ void System::compute_phi(int prec, double* f) {
     last_precision = prec;
     return;
   }
-  start_phi(prec);
+  start_phi(prec, x);
   // non-solvent molecules first, the solvent closes phi_b (SF_MolList1stO.cpp:280-292)
   for (int pass = 0; pass < 2; pass++)
     for (int m = 0; m < nm; m++) {
@@ -1088,7 +1087,7 @@ void System::finish_range(int m, int prec) {
                      phim, stream);
 }
 
-void System::residual_internal(int prec) { compute_phi(prec, d_f); }
+void System::residual_internal(int prec) { compute_phi(prec, nullptr, out_internal(d_f)); }
 
 void System::drop_graphs() {
   for (auto& g : res_graph)
