@@ -16,12 +16,14 @@ enum { MS_LNGN = 0, MS_LNC, MS_PHIB, MS_PREF, MS_REF, MS_RANGE_C, MS_COUNT = 8 }
 // multiplied by 1/maxv[k-1]. Composition multiplies by
 // exp(lnv[k] + lnpair[pair] - *ref). maxv == nullptr disables scaling.
 // The maximum of a step is spread over kMaxSlots words (workgroup b writes
-// word b mod kMaxSlots), each in a cache line of its own (kSlotStride words
-// apart): atomics on one line serialise, and a per-rank launch on a large
-// lattice has thousands of workgroups. A reader reduces the words with one
-// wave load. A step occupies kStepWords words.
+// word b mod kMaxSlots), kSlotStride words apart: atomics on one line
+// serialise, and a per-rank launch on a large lattice has thousands of
+// workgroups. A reader reduces the words with one wave load, so every line more
+// costs it too: a second-order product at 128^3 took 32.9 ms with a line per
+// word, 32.2 ms with four words a line, 35.2 ms with all in two lines. A step
+// occupies kStepWords words.
 constexpr int kMaxSlots = 64;
-constexpr int kSlotStride = 32;  // 128-byte lines
+constexpr int kSlotStride = 8;  // 32 bytes
 constexpr int kStepWords = kMaxSlots * kSlotStride;
 
 __device__ __forceinline__ void put_step_max(unsigned* maxv, int step, float m) {
