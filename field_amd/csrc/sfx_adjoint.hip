@@ -226,7 +226,8 @@ __global__ void k_tconnect(DevLattice L, const T* __restrict__ A, const T* __res
   if (acc) acc[r] += A[r] * B[r] * c;
 }
 
-// per-state direction v_t = v_{itvar(t)} (zero for frozen states), in T
+// per-state direction v_t = v_{itvar(t)} (zero for frozen states), in T, for a
+// product at a base that is there (otherwise launch_swf makes it)
 // (out32 optional: the same directions rounded to FP32)
 __global__ void k_state_dir(long long M, int ns, const int* st_itvar, SiteVec v, double* out, float* out32) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -271,6 +272,30 @@ static __global__ void k_set_ref2(double* scal, const double* lnv, int idx, doub
   if (threadIdx.x == 0 && blockIdx.x == 0) scal[MS_REF] = factor * lnv[idx];
 }
 
+// the tangent accumulators of molecule m
+static void add_tangent(ZeroList& zl, System& S, Tangent& W, int m, bool fp32) {
+  const Molecule& mo = S.mols[m];
+  const long long words = S.lat.d.M * (fp32 ? 1 : 2);
+  for (int t = 0; t < S.ns; t++)
+    if (mo.kind != 0 && mo.uses[t]) {
+      const size_t off = ((size_t)m * S.ns + t) * words;
+      zero_list_add(zl, (unsigned*)W.dacc.p + off, words, S.stream);
+      if (S.middle_out(mo)) zero_list_add(zl, (unsigned*)W.dacc2.p + off, words, S.stream);
+    }
+}
+// they and the step maxima cleared, for a sweep that carries no base (with the
+// base System::start_phi has cleared all)
+static void clear_tangent(System& S, Tangent& W, int m, bool fp32) {
+  ZeroList zl;
+  add_tangent(zl, S, W, m, fp32);
+  if (fp32) {
+    const size_t off = (size_t)m * (S.maxN + 2) * kStepWords;
+    zero_list_add(zl, S.d_maxf + off, (long long)(S.mols[m].N + 2) * kStepWords, S.stream);
+    zero_list_add(zl, S.d_maxb + off, (long long)(S.mols[m].N + 2) * kStepWords, S.stream);
+  }
+  launch_zero_list(zl, S.stream);
+}
+
 // Tangent sweep of molecule m with per-state directions vt (type T, ns*M).
 // The base propagators are computed alongside in the same precision. With
 // `base` their composition gives the molecule's phi too, and a product at a
@@ -306,25 +331,7 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
   auto dslot = [&](int i) { return dstore + (size_t)i * Mn; };
   const int N = mo.N;
   const ChainPlan& plan = mo.plan;
-  {
-    ZeroList zl;
-    const long long words = Mn * (long long)(sizeof(T) / 4);
-    for (int t = 0; t < S.ns; t++)
-      if (mo.uses[t]) {
-        const size_t off = ((size_t)m * S.ns + t) * Mn;
-        zero_list_add(zl, daccp(t), words, st);
-        if (base) zero_list_add(zl, accp(t), words, st);
-        if (S.middle_out(mo)) {
-          zero_list_add(zl, (T*)W.dacc2.p + off, words, st);
-          if (base) zero_list_add(zl, (T*)S.d_acc2 + off, words, st);
-        }
-      }
-    if (scaled) {
-      zero_list_add(zl, maxf, (long long)(N + 2) * kStepWords, st);
-      zero_list_add(zl, maxb, (long long)(N + 2) * kStepWords, st);
-    }
-    launch_zero_list(zl, st);
-  }
+  if (!base) clear_tangent(S, W, m, sizeof(T) == 4);
   RankScale none{nullptr, nullptr, nullptr, nullptr, 0, 0};
   auto fsc = [&](int step, int pair) { return scaled ? RankScale{maxf, lnf, lnf, scal + MS_REF, step, pair} : none; };
   auto bsc = [&](int step, int pair) { return scaled ? RankScale{maxb, lnb, lnf, scal + MS_REF, step, pair} : none; };
@@ -607,20 +614,7 @@ static void tsweep(System& S, Tangent& W, int m, bool scaled, const T* vt, const
   auto vp = [&](int t) { return vt + (size_t)t * Mn; };
   const int N = mo.N;
   const int P = sizeof(T) == 4 ? SFX_FP32 : SFX_FP64;
-  if (mo.kind != 0) {  // the accumulators and the step maxima, cleared by one launch
-    ZeroList zl;
-    const long long words = Mn * (long long)(sizeof(T) / 4);
-    for (int t = 0; t < S.ns; t++)
-      if (mo.uses[t]) {
-        zero_list_add(zl, daccp(t), words, st);
-        if (base) zero_list_add(zl, accp(t), words, st);
-      }
-    if (scaled) {
-      zero_list_add(zl, maxf, (long long)(N + 2) * kStepWords, st);
-      zero_list_add(zl, maxb, (long long)(N + 2) * kStepWords, st);
-    }
-    launch_zero_list(zl, st);
-  }
+  if (!base && mo.kind != 0) clear_tangent(S, W, m, sizeof(T) == 4);
   RankScale none{nullptr, nullptr, nullptr, nullptr, 0, 0};
   auto fsc = [&](int step, int pair) { return scaled ? RankScale{maxf, lnf, lnf, scal + MS_REF, step, pair} : none; };
   auto bsc = [&](int step, int pair) { return scaled ? RankScale{maxb, lnb, lnf, scal + MS_REF, step, pair} : none; };
@@ -772,7 +766,7 @@ static void tangent_sweeps(System& S, Tangent& W, const SiteVec& v, int precisio
   double* v64 = W.v64.p;
   const bool fp32 = precision == SFX_FP32;
   float* v32 = (float*)W.v32.p;
-  k_state_dir<<<grid1(Mn, kTB), kTB, 0, st>>>(Mn, S.ns, S.d_st_itvar, v, v64, fp32 ? v32 : nullptr);
+  if (!base) k_state_dir<<<grid1(Mn, kTB), kTB, 0, st>>>(Mn, S.ns, S.d_st_itvar, v, v64, fp32 ? v32 : nullptr);
   if (fp32 && S.use_block3 && !S.gmax_valid) {  // the base's FP32 SWF maxima, unless its compute_phi made them
     launch_gmax(S.lat.d, S.d_swf32, S.ns, S.d_gmax, st);
     S.gmax_valid = true;
@@ -865,7 +859,9 @@ void jvp_abi(System& S, const double* x, const double* v, double* jv, int precis
   const SiteVec vi = S.vec_abi(v);
   const SiteOut out = S.out_abi(jv);
   if (one_launch_product(S, W, vi, out, precision, true, x)) return;
-  S.start_phi(precision, x);
+  ZeroList zl;
+  for (int m = 0; m < S.nm; m++) add_tangent(zl, S, W, m, precision == SFX_FP32);
+  S.start_phi(precision, x, &zl, &vi, W.v64.p, precision == SFX_FP32 ? (float*)W.v32.p : nullptr);
   tangent_sweeps(S, W, vi, precision, true);
   tangent_close(S, W, vi, out, precision, true);
 }

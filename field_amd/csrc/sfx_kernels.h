@@ -123,10 +123,11 @@ __device__ __forceinline__ void site_none(const SiteOut& f, long long M, long lo
 }
 #endif
 
-// up to eight device arrays of 4-byte words cleared by one launch
+// device arrays of 4-byte words cleared by one launch
 struct ZeroList {
-  void* p[8];
-  long long words[8];
+  static constexpr int max = 24;
+  void* p[max];
+  long long words[max];
   int n = 0;
 };
 void launch_zero_list(const ZeroList& z, hipStream_t st);
@@ -166,11 +167,22 @@ void launch_mol_phi_states(const DevLattice& L, unsigned uses, int ns, const A* 
 // scal[MS_REF] = lna[ia] + lnb[ib] (0 when lna is null): the reference log of
 // a middle-out sweep's compositions
 void launch_set_ref_pair(double* scal, const double* lna, int ia, const double* lnb, int ib, hipStream_t st);
-// u != null: x is copied there, in the internal layout; zero != null: the same
-// launch also clears zero[0..nzero)
-void launch_swf(const DevLattice& L, const SiteVec& x, double* u, const unsigned char* itmask, int nstates,
-                const int* st_itvar, double* swf, float* swf32, hipStream_t st, unsigned* zero = nullptr,
-                int nzero = 0);
+// The SWF of every state, and what else a sweep needs beside it: x's copy in
+// the internal layout, arrays to be cleared, a product's direction per state
+struct SwfArgs {
+  SiteVec x;
+  double* u;  // may be null
+  const unsigned char* itmask;
+  int ns;
+  const int* st_itvar;
+  double* swf;
+  float* swf32;
+  ZeroList zero;
+  SiteVec v;     // direction (p null: none)
+  double* v64;
+  float* v32;    // may be null
+};
+void launch_swf(const DevLattice& L, const SwfArgs& a, hipStream_t st);
 int launch_free_energy(const DevLattice& L, const SysParams& sp, const double* phi, const double* phi_m,
                        const double* rho, const double* swf, const double* u, const double* molscal,
                        double* partial, hipStream_t st);

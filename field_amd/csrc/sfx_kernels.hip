@@ -48,14 +48,24 @@ __device__ double block_sum(double v) {
   return r;  // valid in thread 0
 }
 
+// this thread's share of the words of z, by eight bytes where an array allows
+__device__ __forceinline__ void zero_span(const ZeroList& z, long long i0, long long stride) {
+  for (int k = 0; k < z.n; k++) {
+    const long long n = z.words[k];
+    if (((size_t)z.p[k] & 7) == 0 && (n & 1) == 0) {
+      for (long long i = i0; i < n / 2; i += stride) ((unsigned long long*)z.p[k])[i] = 0ull;
+    } else {
+      for (long long i = i0; i < n; i += stride) ((unsigned*)z.p[k])[i] = 0u;
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // SWF: g_t(r) = exp(-u_{itvar(t)}(src(r))) at iteration sites, 0 elsewhere,
 // halos from their source site (SF_Solve.cpp:794-852 + SetBoundaries).
-__global__ void k_swf(DevLattice L, SiteVec x0, double* __restrict__ u, const unsigned char* __restrict__ itmask,
-                      int nstates, const int* __restrict__ st_itvar, double* __restrict__ swf,
-                      float* __restrict__ swf32, unsigned* __restrict__ zero, int nzero) {
+__global__ void k_swf(DevLattice L, SwfArgs a) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nzero) zero[i] = 0u;
+  zero_span(a.zero, i, (long long)gridDim.x * blockDim.x);
   if (i >= L.M) return;
   int x, y, z;
   site_coords(L, i, x, y, z);
@@ -63,14 +73,19 @@ __global__ void k_swf(DevLattice L, SiteVec x0, double* __restrict__ u, const un
   int sy = L.grad >= 2 ? remap(y, L.ny, L.b1[1], L.b2[1]) : y;
   int sz = L.grad >= 3 ? remap(z, L.nz, L.b1[2], L.b2[2]) : z;
   long long s = sidx(L, sx, sy, sz);
-  bool it = itmask[s];
-  if (u)
-    for (int k = 0; k < x0.nv; k++) u[(long long)k * L.M + i] = site_get(x0, L.M, k, i);
-  for (int t = 0; t < nstates; t++) {
-    int iv = st_itvar[t];
-    double g = (iv >= 0 && it) ? exp(-site_get(x0, L.M, iv, s)) : 0.0;
-    swf[(long long)t * L.M + i] = g;
-    if (swf32) swf32[(long long)t * L.M + i] = (float)g;
+  bool it = a.itmask[s];
+  if (a.u)
+    for (int k = 0; k < a.x.nv; k++) a.u[(long long)k * L.M + i] = site_get(a.x, L.M, k, i);
+  for (int t = 0; t < a.ns; t++) {
+    int iv = a.st_itvar[t];
+    double g = (iv >= 0 && it) ? exp(-site_get(a.x, L.M, iv, s)) : 0.0;
+    a.swf[(long long)t * L.M + i] = g;
+    if (a.swf32) a.swf32[(long long)t * L.M + i] = (float)g;
+    if (a.v.p) {
+      const double d = iv >= 0 ? site_get(a.v, L.M, iv, i) : 0.0;
+      a.v64[(long long)t * L.M + i] = d;
+      if (a.v32) a.v32[(long long)t * L.M + i] = (float)d;
+    }
   }
 }
 
@@ -455,11 +470,8 @@ void launch_mol_phi_states(const DevLattice& L, unsigned uses, int ns, const A* 
   k_mol_phi_states<A><<<grid1(L.V, kBlock), kBlock, 0, st>>>(L, uses, ns, acc, acc2, g, scal, phi_m);
 }
 
-void launch_swf(const DevLattice& L, const SiteVec& x, double* u, const unsigned char* itmask, int nstates,
-                const int* st_itvar, double* swf, float* swf32, hipStream_t st, unsigned* zero, int nzero) {
-  if (!zero) nzero = 0;
-  k_swf<<<grid1(std::max<long long>(L.M, nzero), kBlock), kBlock, 0, st>>>(L, x, u, itmask, nstates, st_itvar, swf,
-                                                                           swf32, zero, nzero);
+void launch_swf(const DevLattice& L, const SwfArgs& a, hipStream_t st) {
+  k_swf<<<grid1(L.M, kBlock), kBlock, 0, st>>>(L, a);
 }
 
 int launch_free_energy(const DevLattice& L, const SysParams& sp, const double* phi, const double* phi_m,
@@ -470,17 +482,8 @@ int launch_free_energy(const DevLattice& L, const SysParams& sp, const double* p
   return (int)nb;
 }
 
-__global__ void k_zero_list(ZeroList z, long long total) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (long long)gridDim.x * blockDim.x) {
-    long long off = i;
-    int k = 0;
-    while (k < z.n - 1 && off >= z.words[k]) {
-      off -= z.words[k];
-      k++;
-    }
-    ((unsigned*)z.p[k])[off] = 0u;
-  }
+__global__ void k_zero_list(ZeroList z) {
+  zero_span(z, (long long)blockIdx.x * blockDim.x + threadIdx.x, (long long)gridDim.x * blockDim.x);
 }
 
 void launch_zero_list(const ZeroList& z, hipStream_t st) {
@@ -488,12 +491,12 @@ void launch_zero_list(const ZeroList& z, hipStream_t st) {
   for (int k = 0; k < z.n; k++) total += z.words[k];
   if (total <= 0) return;
   const unsigned nb = (unsigned)std::min<long long>(grid1(total, kBlock), 4096);
-  k_zero_list<<<nb, kBlock, 0, st>>>(z, total);
+  k_zero_list<<<nb, kBlock, 0, st>>>(z);
 }
 
 void zero_list_add(ZeroList& z, void* p, long long words, hipStream_t st) {
   if (words <= 0) return;
-  if (z.n == 8) {
+  if (z.n == ZeroList::max) {
     launch_zero_list(z, st);
     z.n = 0;
   }

@@ -236,7 +236,9 @@ struct System {
   void compute_phi(int precision, const double* x = nullptr, const SiteOut& f = SiteOut{});
   // compute_phi before the molecules' sweeps: a caller that sweeps base and
   // tangent propagators together puts its own sweeps and closing behind it
-  void start_phi(int precision, const double* x);
+  // (zero: more to clear; v, v64, v32: a product's direction, see SwfArgs)
+  void start_phi(int precision, const double* x, const ZeroList* zero = nullptr, const SiteVec* v = nullptr,
+                 double* v64 = nullptr, float* v32 = nullptr);
   // the closing launches (sfx_close.hip): a sweep leaves its molecule's end
   // rank in `ends`; close_ends derives the scalars (of the base, and of the
   // tangent into dmol) before the next chain overwrites the running ranks

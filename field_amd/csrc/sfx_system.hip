@@ -455,23 +455,6 @@ void System::sweep(int m, bool scaled) {
   };
   const int N = mo.N;
   const int P = sizeof(T) == 4 ? SFX_FP32 : SFX_FP64;
-  {
-    // accumulators (also the backward chain's of a middle-out sweep) and the
-    // step maxima, cleared by one launch
-    ZeroList zl;
-    const long long aw = (long long)Mn * (long long)(sizeof(A) / 4);
-    for (int t = 0; t < ns; t++)
-      if (mo.uses[t]) {
-        zero_list_add(zl, accp(t), aw, st);
-        if constexpr (std::is_same<T, A>::value)
-          if (middle_out(mo)) zero_list_add(zl, (A*)d_acc2 + ((size_t)m * ns + t) * Mn, aw, st);
-      }
-    if (scaled) {
-      zero_list_add(zl, maxf, (long long)(N + 2) * kStepWords, st);
-      zero_list_add(zl, maxb, (long long)(N + 2) * kStepWords, st);
-    }
-    launch_zero_list(zl, st);
-  }
   RankScale none{nullptr, nullptr, nullptr, nullptr, 0, 0};
   auto fsc = [&](int step, int pair) {
     return scaled ? RankScale{maxf, lnf, lnf, scal + MS_REF, step, pair} : none;
@@ -623,7 +606,7 @@ void System::sweep(int m, bool scaled) {
 
 // The sweep of sweep() for a first-order chain (full or half store) on the
 // 3-D simple-cubic lattice, several ranks per launch (sfx_block3.hip). The
-// zeroing of the accumulators and of the scale maxima has been done by sweep().
+// accumulators and the scale maxima have been cleared by start_phi().
 template <typename T>
 void System::sweep_blocked(int m, bool scaled) {
   const DevLattice& L = lat.d;
@@ -928,11 +911,45 @@ FieldArgs System::field_args() {
   return a;
 }
 
-void System::start_phi(int prec, const double* x) {
+void System::start_phi(int prec, const double* x, const ZeroList* zero, const SiteVec* v, double* v64, float* v32) {
   const DevLattice& L = lat.d;
   ends.n = 0;  // whatever a call that threw left
   const bool gmax = prec == SFX_FP32 && use_block3;
-  launch_swf(L, x ? vec_abi(x) : vec_internal(d_u), x ? d_u : nullptr, d_itmask, ns, d_st_itvar, d_swf, d_swf32, stream, gmax ? d_gmax : nullptr, ns * kStepWords);
+  SwfArgs a{};
+  a.x = x ? vec_abi(x) : vec_internal(d_u);
+  a.u = x ? d_u : nullptr;
+  a.itmask = d_itmask;
+  a.ns = ns;
+  a.st_itvar = d_st_itvar;
+  a.swf = d_swf;
+  a.swf32 = d_swf32;
+  if (v) {
+    a.v = *v;
+    a.v64 = v64;
+    a.v32 = v32;
+  }
+  // the molecules' accumulators (also the backward chains' of middle-out
+  // sweeps) and step maxima
+  ZeroList& zl = a.zero;
+  if (zero) zl = *zero;
+  const long long w = prec == SFX_FP32 ? 1 : 2;
+  for (int m = 0; m < nm; m++) {
+    const Molecule& mo = mols[m];
+    if (mo.kind == 0) continue;
+    for (int t = 0; t < ns; t++)
+      if (mo.uses[t]) {
+        const size_t off = ((size_t)m * ns + t) * L.M * w;
+        zero_list_add(zl, (unsigned*)d_acc + off, L.M * w, stream);
+        if (middle_out(mo)) zero_list_add(zl, (unsigned*)d_acc2 + off, L.M * w, stream);
+      }
+    if (prec == SFX_FP32) {
+      const size_t off = (size_t)m * (maxN + 2) * kStepWords;
+      zero_list_add(zl, d_maxf + off, (long long)(mo.N + 2) * kStepWords, stream);
+      zero_list_add(zl, d_maxb + off, (long long)(mo.N + 2) * kStepWords, stream);
+    }
+  }
+  if (gmax) zero_list_add(zl, d_gmax, (long long)ns * kStepWords, stream);
+  launch_swf(L, a, stream);
   gmax_valid = false;
   if (gmax) {
     launch_gmax(L, d_swf32, ns, d_gmax, stream, true);
