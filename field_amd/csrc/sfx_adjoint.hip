@@ -42,7 +42,7 @@ struct Tangent {
   // transposed products (allocated by the first VJP): per-state adjoints of
   // the contact averages, of phi and of the per-state direction, the total's
   // adjoint, and the per-state sweep direction (FP64 and FP32)
-  DevBuf<double> rbar, phibar, vbar, ptbar, xdir64, xdir32, vpart;
+  DevBuf<double> rbar, phibar, vbar, ptbar, xdir64, xdir32, vpart, vcoef;
   bool vjp_ready = false;
   void init_vjp(System& S) {
     const size_t nsM = (size_t)S.ns * M;
@@ -52,7 +52,8 @@ struct Tangent {
     ptbar.alloc((size_t)M);
     xdir64.alloc(nsM);
     xdir32.alloc(nsM);  // half used
-    vpart.alloc((size_t)SFX_MAXM * S.npart);
+    vpart.alloc((size_t)3 * SFX_MAXM * S.npart);
+    vcoef.alloc(SFX_MAXM);
     vjp_ready = true;
   }
   DevBuf<double> dacc2, dpp2;   // the backward chain's, in a middle-out sweep
@@ -992,43 +993,110 @@ __global__ void k_vjp_phibar(DevLattice L, int ns, const int* __restrict__ froze
         (in && !frozen[t]) ? d * side_at(L, q + (long long)t * L.M, x, y, z) + ptbar[i] : 0.0;
 }
 
-// per-block sums over the interior of sum_{t in uses} a_t b_t (with D when weighted)
-__global__ void k_vjp_dot(DevLattice L, unsigned uses, int ns, const double* __restrict__ a,
-                          const double* __restrict__ b, int weighted, double* __restrict__ part) {
+// per-block sums over the interior, of molecule blockIdx.y: of
+// sum_t phi_m,t phibar_t into part, of D sum_t phi_m,t (theta) behind it
+struct VjpMols {
+  int nm, ns;
+  unsigned uses[SFX_MAXM];
+  int freedom[SFX_MAXM], N[SFX_MAXM], kind[SFX_MAXM];
+};
+__global__ void k_vjp_dots(DevLattice L, VjpMols a, const double* __restrict__ phi_m,
+                           const double* __restrict__ phibar, double* __restrict__ part) {
   const long long q = site_ordinal();
-  double v = 0.0;
+  const int m = blockIdx.y;
+  double v = 0.0, th = 0.0;
   if (q < L.V) {
     int x, y, z;
     interior_coords(L, q, x, y, z);
     const long long r = sidx(L, x, y, z);
-    for (int t = 0; t < ns; t++)
-      if ((uses >> t) & 1u) v += a[(long long)t * L.M + r] * (b ? b[(long long)t * L.M + r] : 1.0);
-    if (weighted) v *= lngn_weight(L, x, y, z);
+    for (int t = 0; t < a.ns; t++)
+      if ((a.uses[m] >> t) & 1u) {
+        const double p = phi_m[((long long)m * a.ns + t) * L.M + r];
+        v += p * phibar[(long long)t * L.M + r];
+        th += p;
+      }
+    th *= lngn_weight(L, x, y, z);
   }
-  __shared__ double red[kTB / 64];
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __shared__ double red[2][kTB / 64];
+  for (int o = 32; o > 0; o >>= 1) {
+    v += __shfl_xor(v, o, 64);
+    th += __shfl_xor(th, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = v;
+    red[1][threadIdx.x >> 6] = th;
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 2) {
     double s = 0.0;
-    for (int k = 0; k < (int)(blockDim.x >> 6); k++) s += red[k];
-    part[blockIdx.x] = s;
+    for (int k = 0; k < (int)(blockDim.x >> 6); k++) s += red[threadIdx.x][k];
+    part[((long long)threadIdx.x * a.nm + m) * gridDim.x + blockIdx.x] = s;
   }
 }
 
-// vbar_t += a phi_m,t phibar_t + c D phi_m,t on the interior (states in uses)
-__global__ void k_vjp_direct(DevLattice L, unsigned uses, int ns, const double* __restrict__ phi_m,
-                             const double* __restrict__ phibar, double a, double c, double* __restrict__ vbar) {
-  const long long q = site_ordinal();
-  if (q >= L.V) return;
+// one workgroup, a wave per sum: the adjoints of the molecules' bulk fractions
+// (pbpart, nbM sums each), relbar and theta (part, nbV sums each), and from them
+// each molecule's coefficient of D phi. The sums stay on the device: read back
+// they were two or three waits of the host per molecule, 0.2 ms of a product at
+// 75 x 61 x 90.
+__global__ void __launch_bounds__(1024) k_vjp_coef(VjpMols a, const double* __restrict__ pbpart, int nbM,
+                                                   const double* __restrict__ part, int nbV,
+                                                   const double* __restrict__ molscal, double* __restrict__ coef) {
+  __shared__ double sum[3 * SFX_MAXM];
+  const int lane = threadIdx.x & 63;
+  for (int k = threadIdx.x >> 6; k < 3 * a.nm; k += 16) {
+    const double* p = k < a.nm ? pbpart + (long long)k * nbM : part + (long long)(k - a.nm) * nbV;
+    const int n = k < a.nm ? nbM : nbV;
+    double s = 0.0;
+#pragma unroll 4
+    for (int i = lane; i < n; i += 64) s += p[i];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (lane == 0) sum[k] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x) return;
+  double* const pbbar = sum;
+  // molecules in the reverse order of the forward product: the solvent first
+  // (its bulk fraction closes on the others'), then the rest
+  for (int pass = 0; pass < 2; pass++)
+    for (int m = 0; m < a.nm; m++) {
+      const bool solv = a.freedom[m] == SFX_SOLVENT;
+      if ((pass == 0) != solv) continue;
+      const double relbar = sum[a.nm + m], theta = sum[2 * a.nm + m], phib = molscal[m * MS_COUNT + MS_PHIB];
+      double lnbar = 0.0;
+      if (solv) {
+        // rel = dphib / phib, dphib = -sum_{m' != solvent} dphib_m'
+        const double dpb = (phib != 0 ? relbar / phib : 0.0) + pbbar[m];
+        for (int o = 0; o < a.nm; o++)
+          if (o != m) pbbar[o] -= dpb;
+      } else if (a.freedom[m] == SFX_RESTRICTED) {
+        // rel = -dlnGN, dphib = -phib dlnGN
+        lnbar = -relbar - phib * pbbar[m];
+      }
+      // dlnGN = -(N / theta) sum_t,r D phi_m,t v_t, theta = sum D phi_m
+      coef[m] = lnbar != 0.0 ? -lnbar * a.N[m] / theta : 0.0;
+    }
+}
+
+// vbar_t = sum_m +-phi_m,t phibar_t + coef_m D phi_m,t on the interior, 0 elsewhere
+// (a monomer's phi falls with its own direction)
+__global__ void k_vjp_direct(DevLattice L, VjpMols a, const double* __restrict__ phi_m,
+                             const double* __restrict__ phibar, const double* __restrict__ coef,
+                             double* __restrict__ vbar) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= L.M) return;
   int x, y, z;
-  interior_coords(L, q, x, y, z);
-  const long long r0 = sidx(L, x, y, z);
-  const double d = lngn_weight(L, x, y, z);
-  for (int t = 0; t < ns; t++) {
-    if (!((uses >> t) & 1u)) continue;
-    const long long r = (long long)t * L.M + r0;
-    vbar[r] += phi_m[r] * (a * phibar[r] + c * d);
+  site_coords(L, i, x, y, z);
+  const bool in = is_interior(L, x, y, z);
+  const double d = in ? lngn_weight(L, x, y, z) : 0.0;
+  for (int t = 0; t < a.ns; t++) {
+    const long long r = (long long)t * L.M + i;
+    double v = 0.0;
+    if (in)
+      for (int m = 0; m < a.nm; m++)
+        if ((a.uses[m] >> t) & 1u)
+          v += phi_m[(long long)m * a.ns * L.M + r] * ((a.kind[m] == 0 ? -1.0 : 1.0) * phibar[r] + coef[m] * d);
+    vbar[r] = v;
   }
 }
 
@@ -1081,15 +1149,6 @@ __global__ void k_vjp_final(long long M, int nv, int ns, const int* __restrict__
   }
 }
 
-static double host_sum(const double* part, int n, hipStream_t st) {
-  std::vector<double> h(n);
-  SFX_HIP(hipMemcpyAsync(h.data(), part, n * sizeof(double), hipMemcpyDeviceToHost, st));
-  SFX_HIP(hipStreamSynchronize(st));
-  double s = 0.0;
-  for (double v : h) s += v;
-  return s;
-}
-
 // J^T w at the base state of the last compute_phi at S.d_u
 void vjp_at_base(System& S, const double* w, double* jtw, int precision) {
   require_products(S);
@@ -1104,54 +1163,35 @@ void vjp_at_base(System& S, const double* w, double* jtw, int precision) {
   hipStream_t st = S.stream;
   const bool fp32 = precision == SFX_FP32;
   const unsigned nbM = grid1(Mn, kTB), nbV = grid1(L.V, kTB);
+  VjpMols vm{};
+  vm.nm = S.nm;
+  vm.ns = S.ns;
+  for (int m = 0; m < S.nm; m++) {
+    vm.uses[m] = S.mols[m].uses_mask();
+    vm.freedom[m] = S.mols[m].freedom;
+    vm.N[m] = S.mols[m].N;
+    vm.kind[m] = S.mols[m].kind;
+  }
+  double* const pbpart = W.vpart.p;
+  double* const part = W.vpart.p + (size_t)SFX_MAXM * S.npart;
   // residual: the direct part, the contact averages' and the total's adjoints,
   // and each molecule's bulk-fraction adjoint through ChemIntBulk
-  k_vjp_res<<<nbM, kTB, 0, st>>>(L, S.sp, S.d_itmask, w, S.d_rho, S.d_phitot, jtw, W.rbar.p, W.ptbar.p, W.vpart.p);
-  std::vector<double> pbbar(S.nm, 0.0);
-  for (int m = 0; m < S.nm; m++) pbbar[m] = host_sum(W.vpart.p + (size_t)m * nbM, (int)nbM, st);
+  k_vjp_res<<<nbM, kTB, 0, st>>>(L, S.sp, S.d_itmask, w, S.d_rho, S.d_phitot, jtw, W.rbar.p, W.ptbar.p, pbpart);
   // the contact averages and phi_total, transposed
   k_vjp_q<<<nbM, kTB, 0, st>>>(L, S.ns, S.d_frozen, W.rbar.p, W.xdir64.p);
   k_vjp_phibar<<<nbM, kTB, 0, st>>>(L, S.ns, S.d_frozen, W.xdir64.p, W.ptbar.p, W.phibar.p);
-  SFX_HIP(hipMemsetAsync(W.vbar.p, 0, (size_t)S.ns * Mn * sizeof(double), st));
-  std::vector<double> molscal((size_t)S.nm * MS_COUNT);
-  SFX_HIP(hipMemcpyAsync(molscal.data(), S.d_molscal, molscal.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-  SFX_HIP(hipStreamSynchronize(st));
+  k_vjp_dots<<<dim3(nbV, S.nm), kTB, 0, st>>>(L, vm, S.d_phi_m, W.phibar.p, part);
+  k_vjp_coef<<<1, 1024, 0, st>>>(vm, pbpart, (int)nbM, part, (int)nbV, S.d_molscal, W.vcoef.p);
+  k_vjp_direct<<<nbM, kTB, 0, st>>>(L, vm, S.d_phi_m, W.phibar.p, W.vcoef.p, W.vbar.p);
   if (fp32 && S.use_block3 && !S.gmax_valid) {
     launch_gmax(L, S.d_swf32, S.ns, S.d_gmax, st);
     S.gmax_valid = true;
   }
-  // molecules in the reverse order of the forward product: the solvent first
-  // (its bulk fraction closes on the others'), then the rest
   for (int pass = 0; pass < 2; pass++)
     for (int m = 0; m < S.nm; m++) {
       const Molecule& mo = S.mols[m];
-      const bool solv = mo.freedom == SFX_SOLVENT;
-      if ((pass == 0) != solv) continue;
+      if ((pass == 0) != (mo.freedom == SFX_SOLVENT) || mo.kind == 0) continue;
       const unsigned uses = mo.uses_mask();
-      const double* phi_m = S.d_phi_m + (size_t)m * S.ns * Mn;
-      k_vjp_dot<<<nbV, kTB, 0, st>>>(L, uses, S.ns, phi_m, W.phibar.p, 0, W.vpart.p);
-      const double relbar = host_sum(W.vpart.p, (int)nbV, st);
-      const double phib = molscal[(size_t)m * MS_COUNT + MS_PHIB];
-      const bool monomer = mo.kind == 0;
-      double lnbar = 0.0;
-      if (solv) {
-        // rel = dphib / phib, dphib = -sum_{m' != solvent} dphib_m'
-        const double dpb = (phib != 0 ? relbar / phib : 0.0) + pbbar[m];
-        for (int o = 0; o < S.nm; o++)
-          if (o != m) pbbar[o] -= dpb;
-      } else if (mo.freedom == SFX_RESTRICTED) {
-        // rel = -dlnGN, dphib = -phib dlnGN
-        lnbar = -relbar - phib * pbbar[m];
-      }
-      // dlnGN = -(N / theta) sum_t,r D phi_m,t v_t, theta = sum D phi_m
-      double coef = 0.0;
-      if (lnbar != 0.0) {
-        k_vjp_dot<<<nbV, kTB, 0, st>>>(L, uses, S.ns, phi_m, nullptr, 1, W.vpart.p);
-        const double theta = host_sum(W.vpart.p, (int)nbV, st);
-        coef = -lnbar * mo.N / theta;
-      }
-      k_vjp_direct<<<nbV, kTB, 0, st>>>(L, uses, S.ns, phi_m, W.phibar.p, monomer ? -1.0 : 1.0, coef, W.vbar.p);
-      if (monomer) continue;
       // the transposed sweep: the tangent sweep with direction phibar / D
       k_vjp_dir<<<nbM, kTB, 0, st>>>(L, uses, S.ns, W.phibar.p, W.xdir64.p, (float*)W.xdir32.p);
       const size_t off = (size_t)m * S.ns * Mn;
