@@ -223,6 +223,9 @@ struct System {
   // the two internal-layout vectors of the product entry points (kept, so a
   // call allocates nothing after the first)
   void abi_vectors(double*& in, double*& out);
+  // two host vectors of nvar values that kernels can read and write, kept with the system
+  void host_vectors(double*& a, double*& b);
+  double* h_vec = nullptr;
   // a vector of an entry point on the device, in its own layout: x itself, or
   // its copy in d_xabi; and back, waiting for the stream
   const double* abi_in(const double* x, int where);
@@ -254,10 +257,11 @@ struct System {
   // (per precision): one submission instead of a launch per rank. Plain
   // launches while kernel timing is on. Kernels take their parameters by
   // value, so set_chi drops the graphs.
-  void residual_replay(int precision);
+  // host: x and f are the two vectors of host_vectors() instead
+  void residual_replay(int precision, bool host = false);
   void drop_graphs();
-  hipGraphExec_t res_graph[2] = {nullptr, nullptr};
-  bool res_graph_gmax[2] = {false, false};
+  hipGraphExec_t res_graph[3] = {nullptr, nullptr, nullptr};  // FP64, FP32, FP64 on the host vectors
+  bool res_graph_gmax[3] = {false, false, false};
   bool graph_ok = true;  // false once a capture was refused: plain launches from then on
   long long graph_replays = 0;  // residuals replayed from a graph so far
   double free_energy();

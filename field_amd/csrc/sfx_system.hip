@@ -64,6 +64,7 @@ System::~System() {
                   d_abi_in, d_abi_out, scf1_runs};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
+  if (h_vec) (void)hipHostFree(h_vec);
   tangent_free(tan);
   precond_free(precond);
   solve_work_free(work);
@@ -414,6 +415,17 @@ void System::abi_vectors(double*& in, double*& out) {
   }
   in = d_abi_in;
   out = d_abi_out;
+}
+
+void System::host_vectors(double*& a, double*& b) {
+  if (!h_vec &&
+      hipHostMalloc((void**)&h_vec, 2 * (size_t)nvar * sizeof(double), hipHostMallocCoherent) != hipSuccess) {
+    (void)hipGetLastError();
+    h_vec = nullptr;
+    throw Error{SFX_E_OOM, "hipHostMalloc failed"};
+  }
+  a = h_vec;
+  b = h_vec + nvar;
 }
 
 // internal [itvar][M] vector -> ABI layout (host or device)
@@ -1114,10 +1126,17 @@ void System::drop_graphs() {
     }
 }
 
-void System::residual_replay(int prec) {
-  const int k = prec == SFX_FP32 ? 1 : 0;
+void System::residual_replay(int prec, bool host) {
+  SFX_REQUIRE(!host || (prec == SFX_FP64 && h_vec), SFX_E_INVALID, "no host vectors");
+  const int k = host ? 2 : prec == SFX_FP32 ? 1 : 0;
+  auto run = [&] {
+    if (host)
+      compute_phi(prec, h_vec, out_abi(h_vec + nvar));
+    else
+      residual_internal(prec);
+  };
   if (prof.on || !graph_ok) {
-    residual_internal(prec);
+    run();
     return;
   }
   if (!res_graph[k]) {
@@ -1125,7 +1144,7 @@ void System::residual_replay(int prec) {
     // settings such as dynamic LDS attributes outside any capture), then
     // records them for the calls after it: a capture executes nothing. A
     // runtime that refuses the capture leaves the system on plain launches.
-    residual_internal(prec);
+    run();
     const bool gm = gmax_valid;
     hipGraph_t g = nullptr;
     if (hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
@@ -1135,7 +1154,7 @@ void System::residual_replay(int prec) {
     }
     bool captured = true;
     try {
-      residual_internal(prec);
+      run();
     } catch (...) {
       captured = false;
     }
