@@ -39,14 +39,14 @@
 
 namespace sfx {
 
-constexpr int kTX = 8, kTY = 8, kTZ = 16;
+constexpr int kTX = 8, kTY = 8, kTZ = 16;  // (x: or 2 kTX, see b3_launch_h)
 static_assert(kTY % 2 == 0, "rows are numbered in pairs outside the tile");
 constexpr int kH = kB3Ranks;  // largest widening: the lattice-side bound of block3_ok
 // the tile widened by H layers; one (y, z) column of it is two threads, each
 // with px of its x planes in registers
-template <int H, int KIND>
+template <int H, int KIND, int TX = kTX>
 struct B3Region {
-  static constexpr int rx = kTX + 2 * H, ry = kTY + 2 * H, rz = kTZ + 2 * H;
+  static constexpr int rx = TX + 2 * H, ry = kTY + 2 * H, rz = kTZ + 2 * H;
   static constexpr int px = rx / 2;
   static constexpr int half = (ry * rz + 63) / 64 * 64;  // threads of one half
   static constexpr int threads = 2 * half;
@@ -58,13 +58,13 @@ struct B3Region {
 };
 // two LDS buffers (one barrier per rank) where they leave room for three
 // workgroups per CU, else one buffer and two barriers
-template <typename T, bool TANGENT, int H, int KIND>
+template <typename T, bool TANGENT, int H, int KIND, int TX = kTX>
 constexpr bool b3_double() {
-  return 2 * (TANGENT ? 2 : 1) * B3Region<H, KIND>::words * (int)sizeof(T) <= 53 * 1024;
+  return 2 * (TANGENT ? 2 : 1) * B3Region<H, KIND, TX>::words * (int)sizeof(T) <= 53 * 1024;
 }
-template <typename T, bool TANGENT, int H, int KIND>
+template <typename T, bool TANGENT, int H, int KIND, int TX = kTX>
 constexpr int b3_lds() {
-  return (b3_double<T, TANGENT, H, KIND>() ? 2 : 1) * (TANGENT ? 2 : 1) * B3Region<H, KIND>::words * (int)sizeof(T);
+  return (b3_double<T, TANGENT, H, KIND, TX>() ? 2 : 1) * (TANGENT ? 2 : 1) * B3Region<H, KIND, TX>::words * (int)sizeof(T);
 }
 
 bool block3_ok(const DevLattice& L) {
@@ -92,17 +92,17 @@ __device__ __forceinline__ float block_max_f(float v, float* red) {
   return r;
 }
 
-template <typename T, bool TANGENT, bool SCALED, bool CONNECT, int H, int KIND>
-__global__ void __launch_bounds__((B3Region<H, KIND>::threads)) k_block3(DevLattice L, B3Launch<T> la, int nb) {
-  using R = B3Region<H, KIND>;
+template <typename T, bool TANGENT, bool SCALED, bool CONNECT, int H, int KIND, int TX = kTX>
+__global__ void __launch_bounds__((B3Region<H, KIND, TX>::threads)) k_block3(DevLattice L, B3Launch<T> la, int nb) {
+  using R = B3Region<H, KIND, TX>;
   constexpr int PX = R::px, RX = R::rx, RZ = R::rz, NT = R::half;
   constexpr int OX = PX - H;  // owned planes of a half: its planes H..PX-1
-  constexpr bool DB = b3_double<T, TANGENT, H, KIND>();
+  constexpr bool DB = b3_double<T, TANGENT, H, KIND, TX>();
   // chain of this workgroup and its tile number within that chain's grid
   const int chain = (int)blockIdx.x >= nb ? 1 : 0;
   const int bl = (int)blockIdx.x - chain * nb;
   const B3Args<T>& a = la.a[chain];
-  __shared__ __align__(16) T lds[b3_lds<T, TANGENT, H, KIND>() / sizeof(T)];
+  __shared__ __align__(16) T lds[b3_lds<T, TANGENT, H, KIND, TX>() / sizeof(T)];
   __shared__ float red[R::threads / 64], scl[2];
   __shared__ T cfac[kB3Ranks];
 
@@ -138,7 +138,7 @@ __global__ void __launch_bounds__((B3Region<H, KIND>::threads)) k_block3(DevLatt
   b /= nbz;
   const int by = b % nby;
   const int bx = b / nby;
-  const int x0 = 1 + bx * kTX, y0 = 1 + by * kTY, z0 = 1 + bz * kTZ;  // tile origin (interior coords)
+  const int x0 = 1 + bx * TX, y0 = 1 + by * kTY, z0 = 1 + bz * kTZ;  // tile origin (interior coords)
 
   // this thread's (y, z) column and its half of it: plane j of the lower half
   // is region plane j, of the upper half region plane RX-1-j, so that in both
@@ -164,7 +164,7 @@ __global__ void __launch_bounds__((B3Region<H, KIND>::threads)) k_block3(DevLatt
 #pragma unroll
   for (int j = 0; j < PX; j++) px[j] = (unsigned)__builtin_amdgcn_readlane((int)xoff, j);
   // owned plane j lies in the lattice
-  auto inside = [&](int j) { return x0 + (half ? kTX - 1 - (j - H) : j - H) <= L.nx; };
+  auto inside = [&](int j) { return x0 + (half ? TX - 1 - (j - H) : j - H) <= L.nx; };
 
   // rank s0 (and its tangent), g (and v) of the column: the plane's offset is
   // uniform, the lane's is one 32-bit word
@@ -354,25 +354,40 @@ __global__ void __launch_bounds__((B3Region<H, KIND>::threads)) k_block3(DevLatt
   }
 }
 
-template <typename T, bool TG, bool SC, bool CN, int H, int KIND>
-static void b3_launch(const DevLattice& L, const B3Launch<T>& a, unsigned nb, hipStream_t st, hipEvent_t ev0,
-                      hipEvent_t ev1) {
-  static_assert(b3_lds<T, TG, H, KIND>() <= 64 * 1024, "static LDS");
+static unsigned b3_tiles(const DevLattice& L, int tx) {
+  return (unsigned)(((L.nx + tx - 1) / tx) * ((L.ny + kTY - 1) / kTY) * ((L.nz + kTZ - 1) / kTZ));
+}
+template <typename T, bool TG, bool SC, bool CN, int H, int KIND, int TX = kTX>
+static void b3_launch(const DevLattice& L, const B3Launch<T>& a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+  static_assert(b3_lds<T, TG, H, KIND, TX>() <= 64 * 1024, "static LDS");
+  const unsigned nb = b3_tiles(L, TX);
   // with events: recorded by the dispatch itself at kernel start and end
-  hipExtLaunchKernelGGL((k_block3<T, TG, SC, CN, H, KIND>), dim3(nb * (unsigned)a.nchains),
-                        dim3(B3Region<H, KIND>::threads), 0, st, ev0, ev1, 0u, L, a, (int)nb);
+  hipExtLaunchKernelGGL((k_block3<T, TG, SC, CN, H, KIND, TX>), dim3(nb * (unsigned)a.nchains),
+                        dim3(B3Region<H, KIND, TX>::threads), 0, st, ev0, ev1, 0u, L, a, (int)nb);
 }
 template <typename T, bool TG, bool SC, bool CN, int KIND>
-static void b3_launch_h(int nr, const DevLattice& L, const B3Launch<T>& a, unsigned nb, hipStream_t st,
-                        hipEvent_t ev0, hipEvent_t ev1) {
+static void b3_launch_h(int nr, const DevLattice& L, const B3Launch<T>& a, hipStream_t st, hipEvent_t ev0,
+                        hipEvent_t ev1) {
   // launches of one or two ranks (a chain's ends, a change of the segment
   // state) load and compute a smaller region: 7.2 / 9.1 us instead of 14 / 16
   // at 75 x 61 x 90 in FP32
   if (nr <= 2) {
-    b3_launch<T, TG, SC, CN, 2, KIND>(L, a, nb, st, ev0, ev1);
+    b3_launch<T, TG, SC, CN, 2, KIND>(L, a, st, ev0, ev1);
     return;
   }
-  if constexpr (!(TG && sizeof(T) == 8)) b3_launch<T, TG, SC, CN, kB3Ranks, KIND>(L, a, nb, st, ev0, ev1);
+  // FP32 base ranks: a tile of 16 planes reads 4.5 times itself instead of 6,
+  // from 3.5 workgroups of the smaller tile per CU on. With fewer the chip runs
+  // out of waves (residuals at 40 x 42 x 45: 166 us by 8 planes, 193 by 16; at
+  // 64 x 66 x 69 240 and 235; at 100 x 102 x 105 518 and 480). FP64 and
+  // tangents, with twice the registers and LDS, are slower by it throughout
+  // (100 x 102 x 105: 618 and 656 us in FP64, products 829 and 920 in FP32).
+  if constexpr (!TG && sizeof(T) == 4 && KIND == ST_3D_SC) {
+    if (b3_tiles(L, kTX) * (unsigned)a.nchains >= 896) {
+      b3_launch<T, TG, SC, CN, kB3Ranks, KIND, 2 * kTX>(L, a, st, ev0, ev1);
+      return;
+    }
+  }
+  if constexpr (!(TG && sizeof(T) == 8)) b3_launch<T, TG, SC, CN, kB3Ranks, KIND>(L, a, st, ev0, ev1);
 }
 
 template <typename T>
@@ -398,10 +413,9 @@ void launch_block3(const DevLattice& L, const B3Launch<T>& a, bool tangent, bool
                 "blocked launch of 1..4 ranks");
     nr = std::max(nr, a.a[c].nr);
   }
-  const unsigned nb = (unsigned)(((L.nx + kTX - 1) / kTX) * ((L.ny + kTY - 1) / kTY) * ((L.nz + kTZ - 1) / kTZ));
 #define B3(TG, SC, CN)                                                         \
-  (L.kind == ST_3D_FCC ? b3_launch_h<T, TG, SC, CN, ST_3D_FCC>(nr, L, a, nb, st, ev0, ev1) \
-                       : b3_launch_h<T, TG, SC, CN, ST_3D_SC>(nr, L, a, nb, st, ev0, ev1))
+  (L.kind == ST_3D_FCC ? b3_launch_h<T, TG, SC, CN, ST_3D_FCC>(nr, L, a, st, ev0, ev1) \
+                       : b3_launch_h<T, TG, SC, CN, ST_3D_SC>(nr, L, a, st, ev0, ev1))
   if constexpr (sizeof(T) == 4) {  // FP32 sweeps are scaled, FP64 ones are not
     SFX_REQUIRE(scaled, SFX_E_INVALID, "FP32 blocked sweeps are scaled");
     if (tangent) { if (connect) B3(true, true, true); else B3(true, true, false); }
