@@ -1,5 +1,5 @@
-// sfx_block3.hip -- temporally blocked propagator ranks on the 3-D simple-cubic
-// lattice: one launch advances a chain by up to four ranks.
+// sfx_block3.hip -- temporally blocked propagator ranks on 3-D simple-cubic and
+// FCC lattices: one launch advances a chain by up to four ranks.
 //
 // A workgroup owns an 8 x 8 x 16 output tile. It loads the previous rank and
 // the state's SWF on the tile widened by the number of ranks nr in every
@@ -9,6 +9,8 @@
 // on the tile widened by nr - k:
 //   G_k(r) = g(r) (1/6) sum_6 G_{k-1}(r + e)            (Lat3D1stO.cpp:53-260)
 //   dG_k(r) = g(r) ((1/6) sum_6 dG_{k-1} - v(r) (1/6) sum_6 G_{k-1})
+// (FCC: (1/12) sum_12 over the edge neighbours, Lat3DFCC1stO.cpp:77-89; at 50 x
+// 41 x 63 four FP64 ranks take 10.3 / 11.2 us where one took 3.7 / 4.0)
 // Two threads hold one (y, z) column of the widened tile, half of its x planes
 // each, in registers, with g (and v) beside them: the x neighbours are
 // registers, the y and z neighbours come from LDS, where every rank is
@@ -17,15 +19,16 @@
 // acc += G_k G_pair c_k (ConnectG, Lat3D1stO.cpp:299-312; tangent
 // dacc += (dG_k G_pair + G_k dG_pair) c_k), and acc goes to HBM once.
 //
-// What bounds it: at 64^3 the instructions a wave issues one after the other
-// (the arrays stay in the caches), at 128^3 the LDS exchange and HBM. The form
-// before gave each thread of a 1024-thread workgroup one site at a time and
-// spent most of its instructions on the divisions that found it; its reads
-// from LDS were seven a site, now five. Four ranks of two chains at 64^3,
-// FP32: 17.5 / 21.5 us then, 9.4 / 11.2 us now (forward / composing), tangents
-// 25 / 29 us then, 14.4 / 16.2 us now; FP64 at 128^3, four ranks: 122 / 160 us
-// then, 65 / 113 us now. One thread per column (twice the planes each) took
-// 11.7 / 14.7 us in FP32: half the waves, each twice as long.
+// What bounds it: at 64^3 a launch is one chain of waits, 5-10k of 22k cycles on
+// the region's loads (rows of 96 bytes touch 1.7 lines, near the L2's rate), 3k
+// on the scale factors and the first barrier, 11k in four ranks; 12% fewer loads
+// and instructions changed nothing. At 128^3 it is the region's reads and HBM.
+// The form before gave each thread of a 1024-thread workgroup one site at a time
+// and spent most of its instructions on the divisions that found it. Four ranks
+// of two chains at 64^3, FP32: 17.5 / 21.5 us then, 9.0 / 11.1 us now (forward /
+// composing), tangents 25 / 29 us then, 14.4 / 18.0 us now, base and tangent
+// composed together; FP64 at 128^3: 122 / 160 us then, 63 / 112 us now. One
+// thread per column (twice the planes each) took 11.7 / 14.7 us in FP32.
 //
 // FP32 scaling: the input is divided by max(rank s0) and every rank by the
 // lattice maximum of g, so no rank exceeds 1 and at most nr ranks decay

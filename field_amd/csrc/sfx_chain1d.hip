@@ -301,9 +301,8 @@ __device__ double2 scf1_layer_sums(int n, Val&& val, Dval&& dval, double* wsum) 
 
 // The residual (u -> SWF -> propagators -> phi -> f), or with TAN the product
 // J v (A.base: with phi and the contact averages on the way; otherwise at those
-// of the last evaluation), of a 1-D first-order system in FP64: the sequence of
-// kernels of System::residual_internal and jvp_internal in one workgroup, same
-// bits. SWF, accumulators and profiles are in LDS, indexed by layer with W
+// of the last evaluation), of a 1-D first-order system in FP64: the launches of a
+// residual or a product in one workgroup, same bits. SWF, accumulators and profiles are in LDS, indexed by layer with W
 // words per state; the first wave sweeps the chains.
 template <int K, bool CURVED, bool TAN>
 __global__ void __launch_bounds__(kScf1Threads) k_scf1d(DevLattice L, Scf1Args A) {
@@ -432,7 +431,7 @@ __global__ void __launch_bounds__(kScf1Threads) k_scf1d(DevLattice L, Scf1Args A
     __syncthreads();
   }
 
-  // state totals (k_phi_total, k_tphi_total): a state of one molecule has its
+  // state totals (k_phi_close): a state of one molecule has its
   // phi in LDS; one of several is summed over the phi_m this thread wrote
   for (int x = 1 + tid; x <= n; x += kScf1Threads)
     for (int t = 0; t < ns; t++) {
@@ -461,7 +460,7 @@ __global__ void __launch_bounds__(kScf1Threads) k_scf1d(DevLattice L, Scf1Args A
   }
   if (base && tid < sp.nm * MS_COUNT) A.molscal[tid] = ms[tid];
   __syncthreads();
-  // contact averages (k_sides, k_tsides) and the residual or its linearisation
+  // contact averages and the residual or its linearisation
   for (int i = tid; i < M; i += kScf1Threads) {
     double tot = 0, dtot = 0;
     for (int t = 0; t < ns; t++) {
@@ -469,7 +468,7 @@ __global__ void __launch_bounds__(kScf1Threads) k_scf1d(DevLattice L, Scf1Args A
       if constexpr (TAN) dtot += ldacc[t * W + i];
     }
     const SiteOut& out = TAN ? A.jv : A.f;
-    const bool side = (i > 0 || L.surf1[0]) && (i <= n || L.surf2[0]);  // k_sides: not the other halos
+    const bool side = (i > 0 || L.surf1[0]) && (i <= n || L.surf2[0]);  // not the other halos
     if (base) {
       A.phitot[i] = tot;
       for (int t = 0; t < ns; t++) {

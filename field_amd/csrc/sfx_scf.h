@@ -235,7 +235,7 @@ __device__ __forceinline__ T tan_compose(T dG, T Gp, T G, T dGp) {  // dG Gp + G
 }
 
 // contact averages of one site, halo sites that are not surfaces excluded
-// (SetBoundaries fills those; k_sides)
+// (SetBoundaries fills those)
 __device__ __forceinline__ bool has_side(const DevLattice& L, int x, int y, int z) {
   if (is_interior(L, x, y, z)) return true;
   const int c[3] = {x, y, z}, n[3] = {L.nx, L.ny, L.nz};

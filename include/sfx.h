@@ -131,9 +131,10 @@ typedef struct sfx_options {
                              SFX_SWEEP_PER_RANK (one launch per rank) or
                              SFX_SWEEP_BLOCKED (up to four ranks per launch through
                              LDS, where every side exceeds four layers). AUTO and
-                             BLOCKED also advance first-order 2-D sweeps by up to
-                             eight ranks per launch (fully stored, chain_schedule
-                             AUTO, a curved lattice without mirror2 sides), and run
+                             BLOCKED also advance first-order FCC sweeps by four and
+                             2-D sweeps by eight ranks per launch (fully stored,
+                             chain_schedule AUTO, a curved lattice without mirror2
+                             sides), and run
                              a 1-D first-order FP64 evaluation in one workgroup
                              launch, or above 1024 layers each stretch of a chain's
                              ranks in one (up to 4000 layers) */
