@@ -281,7 +281,7 @@ static void add_tangent(ZeroList& zl, System& S, Tangent& W, int m, bool fp32) {
     if (mo.kind != 0 && mo.uses[t]) {
       const size_t off = ((size_t)m * S.ns + t) * words;
       zero_list_add(zl, (unsigned*)W.dacc.p + off, words, S.stream);
-      if (S.middle_out(mo)) zero_list_add(zl, (unsigned*)W.dacc2.p + off, words, S.stream);
+      if (S.middle_out(mo, fp32 ? SFX_FP32 : SFX_FP64)) zero_list_add(zl, (unsigned*)W.dacc2.p + off, words, S.stream);
     }
 }
 // they and the step maxima cleared, for a sweep that carries no base (with the
@@ -367,6 +367,7 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
       a.lnpair = lnpair;
       a.ref = scal + MS_REF;
       a.gmax = S.d_gmax + (size_t)t * kStepWords;
+      a.low = mo.blocked_rank(sa - 1) ? S.low_word() : nullptr;
     }
     a.s0 = sa - 1;
     return a;
@@ -386,7 +387,7 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
     la.nchains = 1;
     go(la, connect);
   };
-  if (S.middle_out(mo)) {
+  if (S.middle_out(mo, P)) {
     // the schedule of System::sweep_blocked's middle-out branch, with tangents
     const int h = N / 2;
     T* dacc2 = (T*)W.dacc2.p;
@@ -470,6 +471,7 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
       go(la, true);
     }
     S.add_end(m, pp[fc], dpp[fc], sizeof(T) == 4, scaled ? lnf + N : nullptr);  // forward rank N
+    if (scaled) S.check_end(m, N, N);
     return;
   }
   tinit<T>(L, gp(mo.seq[0]), vp(mo.seq[0]), slot(0), dslot(0), fsc(1, 0), st);
@@ -586,12 +588,13 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
   fin = pp[cur];
   dfin = dpp[cur];
   S.add_end(m, fin, dfin, sizeof(T) == 4, scaled ? (mo.kind == 1 ? lnb : lnf) + N : nullptr);
+  if (scaled) S.check_end(m, N, mo.kind == 1 ? N : 0);
 }
 
 template <typename T>
 static void tsweep(System& S, Tangent& W, int m, bool scaled, const T* vt, const T* g32or64, const double* v64,
                    bool base) {
-  if (S.use_block3 && (S.mols[m].kind == 1 || S.mols[m].kind == 2)) {
+  if (S.blocked(sizeof(T) == 4 ? SFX_FP32 : SFX_FP64) && (S.mols[m].kind == 1 || S.mols[m].kind == 2)) {
     tsweep_blocked<T>(S, W, m, scaled, vt, g32or64, base);
     return;
   }
@@ -768,7 +771,7 @@ static void tangent_sweeps(System& S, Tangent& W, const SiteVec& v, int precisio
   const bool fp32 = precision == SFX_FP32;
   float* v32 = (float*)W.v32.p;
   if (!base) k_state_dir<<<grid1(Mn, kTB), kTB, 0, st>>>(Mn, S.ns, S.d_st_itvar, v, v64, fp32 ? v32 : nullptr);
-  if (fp32 && S.use_block3 && !S.gmax_valid) {  // the base's FP32 SWF maxima, unless its compute_phi made them
+  if (fp32 && S.blocked(precision) && !S.gmax_valid) {  // the base's FP32 SWF maxima, unless its compute_phi made them
     launch_gmax(S.lat.d, S.d_swf32, S.ns, S.d_gmax, st);
     S.gmax_valid = true;
   }
@@ -788,7 +791,7 @@ static void tangent_sweeps(System& S, Tangent& W, const SiteVec& v, int precisio
 
 // phi (base), dphi, contact averages and the linearised residual
 static void tangent_close(System& S, Tangent& W, const SiteVec& v, const SiteOut& jv, int precision, bool base) {
-  PhiArgs a = S.phi_args();
+  PhiArgs a = S.phi_args(precision);
   a.base = base;
   a.tangent = true;
   a.dacc = W.dacc.p;
@@ -849,7 +852,7 @@ void jvp_at_base(System& S, const double* v, double* jv, int precision) {
   tangent_close(S, W, vi, out, precision, false);
 }
 
-// J v at x (device, the ABI's layout, as v and jv), base and tangent in one sweep per molecule: the base sweep of
+// J v at x (device, the ABI's layout, as v and jv; null: at S.d_u), base and tangent in one sweep per molecule: the base sweep of
 // a compute_phi before it was 33% of the product's kernel time on the 64^3 melt
 // (FP32, 443 -> 328 us without it), 39% on second-order 128^3 (52.4 -> 33.1 ms)
 // and 42% on the 64 x 128 pore (971 -> 579 us)
@@ -1183,7 +1186,7 @@ void vjp_at_base(System& S, const double* w, double* jtw, int precision) {
   k_vjp_dots<<<dim3(nbV, S.nm), kTB, 0, st>>>(L, vm, S.d_phi_m, W.phibar.p, part);
   k_vjp_coef<<<1, 1024, 0, st>>>(vm, pbpart, (int)nbM, part, (int)nbV, S.d_molscal, W.vcoef.p);
   k_vjp_direct<<<nbM, kTB, 0, st>>>(L, vm, S.d_phi_m, W.phibar.p, W.vcoef.p, W.vbar.p);
-  if (fp32 && S.use_block3 && !S.gmax_valid) {
+  if (fp32 && S.blocked(precision) && !S.gmax_valid) {
     launch_gmax(L, S.d_swf32, S.ns, S.d_gmax, st);
     S.gmax_valid = true;
   }
@@ -1195,7 +1198,7 @@ void vjp_at_base(System& S, const double* w, double* jtw, int precision) {
       // the transposed sweep: the tangent sweep with direction phibar / D
       k_vjp_dir<<<nbM, kTB, 0, st>>>(L, uses, S.ns, W.phibar.p, W.xdir64.p, (float*)W.xdir32.p);
       const size_t off = (size_t)m * S.ns * Mn;
-      const bool two = S.middle_out(mo);
+      const bool two = S.middle_out(mo, precision);
       S.ends.n = 0;
       if (fp32) {
         tsweep<float>(S, W, m, true, (const float*)W.xdir32.p, S.d_swf32, W.xdir64.p, false);

@@ -165,6 +165,7 @@ __global__ void __launch_bounds__(kB2Threads) k_block2(DevLattice L, B3Launch<T>
         ma = fmaxf(ma, __shfl_xor(ma, o, 64));
         mb = fmaxf(mb, __shfl_xor(mb, o, 64));
       }
+      if (lane == 0 && bl == 0 && a.low && !(ma >= kLowMax)) *a.low = 1u;
       double lna;
       const float sa = pow2_scale(ma, lna), sb = pow2_scale(mb, lng);
       if (lane == 0) {

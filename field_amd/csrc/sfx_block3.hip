@@ -193,6 +193,7 @@ __global__ void __launch_bounds__((B3Region<H, KIND, TX>::threads)) k_block3(Dev
         ma = fmaxf(ma, __shfl_xor(ma, o, 64));
         mb = fmaxf(mb, __shfl_xor(mb, o, 64));
       }
+      if (lane == 0 && bl == 0 && a.low && !(ma >= kLowMax)) *a.low = 1u;
       if (!(ma > 0.f)) ma = 1.f;
       if (!(mb > 0.f)) mb = 1.f;
       if (lane == 0) {

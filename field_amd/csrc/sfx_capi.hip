@@ -94,8 +94,13 @@ int sfx_system_sizes(const sfx_system* s, long* nvar, long* M) {
 int sfx_compute_phi(sfx_system* s, const double* x, int where, int precision) {
   return guarded([&] {
     SFX_REQUIRE(s && x, SFX_E_INVALID, "NULL argument");
-    s->s.compute_phi(precision, s->s.abi_in(x, where));
-    s->s.sync();
+    System& S = s->s;
+    const double* xd = S.abi_in(x, where);
+    S.checked(precision, [&] {
+      S.compute_phi(precision, xd);
+      S.sync();
+      xd = nullptr;  // a second pass takes the copy in d_u
+    });
   });
 }
 
@@ -104,8 +109,12 @@ int sfx_residual(sfx_system* s, const double* x, double* f, int where, int preci
     SFX_REQUIRE(s && x && f, SFX_E_INVALID, "NULL argument");
     System& S = s->s;
     // from host memory both go through one staging vector: x has been read when f is written
-    S.compute_phi(precision, S.abi_in(x, where), S.out_abi(where == SFX_HOST ? S.d_xabi : f));
-    S.abi_out(S.d_xabi, f, where);
+    const double* xd = S.abi_in(x, where);
+    S.checked(precision, [&] {
+      S.compute_phi(precision, xd, S.out_abi(where == SFX_HOST ? S.d_xabi : f));
+      S.abi_out(S.d_xabi, f, where);
+      xd = nullptr;  // f may have been written over x: a second pass takes the copy in d_u
+    });
   });
 }
 
@@ -119,8 +128,21 @@ int sfx_jvp(sfx_system* s, const double* x, const double* v, double* jv, int whe
       S.abi_vectors(vin, out);
       SFX_HIP(hipMemcpyAsync(vin, v, S.nvar * sizeof(double), hipMemcpyHostToDevice, S.stream));
     }
-    jvp_abi(S, xd, vin, out, precision);
-    S.abi_out(out, jv, where);
+    // a second pass reads v again: a product written over it goes through a vector of its own
+    const bool over = where != SFX_HOST && jv == v && precision == SFX_FP32 && S.blocked(precision);
+    if (over) {
+      double* in;
+      S.abi_vectors(in, out);
+    }
+    S.checked(precision, [&] {
+      jvp_abi(S, xd, vin, out, precision);
+      S.abi_out(out, jv, where);
+      xd = nullptr;
+    });
+    if (over) {
+      SFX_HIP(hipMemcpyAsync(jv, out, S.nvar * sizeof(double), hipMemcpyDeviceToDevice, S.stream));
+      S.sync();
+    }
   });
 }
 
@@ -132,8 +154,10 @@ int sfx_vjp(sfx_system* s, const double* x, const double* w, double* jtw, int wh
     double *win, *out;
     S.abi_vectors(win, out);
     load_vec(S, w, where, win);
-    vjp_internal(S, win, out, precision);
-    S.store_f(out, jtw, where);
+    S.checked(precision, [&] {
+      vjp_internal(S, win, out, precision);
+      S.store_f(out, jtw, where);
+    });
   });
 }
 

@@ -16,6 +16,10 @@ struct EndMol {
   const void* dG;     // tangent, of the same type; for a monomer the direction v (dG = -v g)
   const double* lnf;  // FP32: log scale of the end rank; nullptr: unscaled, MS_REF becomes 0
   bool f32, unscaled;
+  // FP32 by blocked launches: step maxima of the chains' last ranks that no
+  // launch reads, and the word set when one is below kLowMax (null: no check)
+  const unsigned* endmax[2];
+  unsigned* low;
 };
 struct EndArgs {
   int n;  // entries; a solvent may only close on entries before it or finished molecules

@@ -89,6 +89,11 @@ __global__ void __launch_bounds__(NT) k_end_sums(DevLattice L, EndArgs a) {
     ph[t] = a.molscal[t * MS_COUNT + MS_PHIB];
     if constexpr (TAN) dph[t] = a.dmol[t * 4 + 2];
   }
+  float em[2] = {1.f, 1.f};
+  const bool check = e.low && blockIdx.x == 0 && wave == 0;
+  if (check)
+    for (int k = 0; k < 2; k++)
+      if (e.endmax[k]) em[k] = __uint_as_float(e.endmax[k][lane * kSlotStride]);
   double s = 0, ds = 0;
   if (e.f32)
     end_sum<float, TAN, NT>(L, e, s, ds);
@@ -97,6 +102,13 @@ __global__ void __launch_bounds__(NT) k_end_sums(DevLattice L, EndArgs a) {
   for (int o = 32; o > 0; o >>= 1) {
     s += __shfl_xor(s, o, 64);
     if constexpr (TAN) ds += __shfl_xor(ds, o, 64);
+  }
+  if (check) {
+    for (int o = 32; o > 0; o >>= 1) {
+      em[0] = fmaxf(em[0], __shfl_xor(em[0], o, 64));
+      em[1] = fmaxf(em[1], __shfl_xor(em[1], o, 64));
+    }
+    if (lane == 0 && !(fminf(em[0], em[1]) >= kLowMax)) *e.low = 1u;
   }
   if (lane == 0) {
     r1[wave] = s;

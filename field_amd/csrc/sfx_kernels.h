@@ -63,6 +63,16 @@ __device__ __forceinline__ float get_step_max(const unsigned* maxv, int step) {
   return v;
 }
 
+// A launch of several ranks divides by the lattice maximum of g alone, so its
+// ranks decay wherever the chain's weight is far from that maximum (an isolated
+// deep site, a block entering another's region), and the composition multiplies
+// a rank of either chain before their logs make up for it. Below this maximum of
+// a launch's last rank (22 kT lost within it) the evaluation is repeated rank by
+// rank. A composed product of two such ranks is still 2^62 above FP32's smallest
+// normal number; unchecked, transposed products lost digits from a decay of
+// 2^-60 on and sums of 2^-127 became log(0).
+constexpr float kLowMax = 0x1p-32f;
+
 struct RankScale {
   unsigned* maxv;
   double* lnv;

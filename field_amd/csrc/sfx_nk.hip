@@ -70,13 +70,28 @@ void solve_nk(System& S, const sfx_solver_opts& o, sfx_solve_stats& st) {
   SFX_HIP(hipEventRecord(e0, S.stream));
 
   int prec = o.fp64_switch > 0 ? SFX_FP32 : SFX_FP64;
+  // a sweep that decayed too far within a launch, seen after a wait for the
+  // stream: the solve goes on rank by rank in FP32, and the caller repeats it
+  struct PerRank {
+    System& S;
+    bool take() {
+      if (!S.took_low()) return false;
+      S.set_fp32_per_rank(true);
+      return true;
+    }
+    ~PerRank() { S.set_fp32_per_rank(false); }
+  } per_rank{S};
   auto eval = [&](int p) {
-    S.residual_replay(p);
-    if (p == SFX_FP32)
-      st.residual_evals_fp32++;
-    else
-      st.residual_evals++;
-    return std::sqrt(V.dot(r, r));
+    double norm;
+    do {
+      S.residual_replay(p);
+      if (p == SFX_FP32)
+        st.residual_evals_fp32++;
+      else
+        st.residual_evals++;
+      norm = std::sqrt(V.dot(r, r));
+    } while (per_rank.take());
+    return norm;
   };
   double rn = eval(prec);
   int it = 0;
@@ -109,9 +124,11 @@ void solve_nk(System& S, const sfx_solver_opts& o, sfx_solve_stats& st) {
         V.scale(-1.0 / rn, r, Vk(0));
         beta = rn;
       } else {
-        op(dx, wv, pz);
-        V.axpby(-1.0, r, -1.0, wv);  // w = -r - J P z
-        beta = std::sqrt(V.dot(wv, wv));
+        do {
+          op(dx, wv, pz);
+          V.axpby(-1.0, r, -1.0, wv);  // w = -r - J P z
+          beta = std::sqrt(V.dot(wv, wv));
+        } while (per_rank.take());
         lin = beta;
         if (beta <= eta * beta0) break;
         V.scale(1.0 / beta, wv, Vk(0));
@@ -121,34 +138,36 @@ void solve_nk(System& S, const sfx_solver_opts& o, sfx_solve_stats& st) {
       int j = 0;
       double res = beta;
       for (; j < m && total < o.gmres_max_iter; j++) {
-        op(Vk(j), wv, pc ? Zk(j) : pz);
         total++;
         // classical Gram-Schmidt, twice, with the projections kept on the
         // device; one read-back per Arnoldi step brings both passes and ||w||^2
         std::vector<double> h(j + 1, 0.0), hb(2 * kGsPass + 1);
-        for (int pass = 0; pass < 2; pass++) {
-          for (int base = 0; base <= j; base += 16) {
-            DotList dl{};
-            dl.count = std::min(16, j + 1 - base);
-            for (int i = 0; i < dl.count; i++) {
-              dl.a[i] = Vk(base + i);
-              dl.b[i] = wv;
+        do {
+          op(Vk(j), wv, pc ? Zk(j) : pz);
+          for (int pass = 0; pass < 2; pass++) {
+            for (int base = 0; base <= j; base += 16) {
+              DotList dl{};
+              dl.count = std::min(16, j + 1 - base);
+              for (int i = 0; i < dl.count; i++) {
+                dl.a[i] = Vk(base + i);
+                dl.b[i] = wv;
+              }
+              V.dots_dev(dl, gs + pass * kGsPass + base, pass * kGsPass + base);
             }
-            V.dots_dev(dl, gs + pass * kGsPass + base, pass * kGsPass + base);
+            VecList vl{};
+            vl.count = j + 2;
+            for (int i = 0; i <= j; i++) vl.v[i] = Vk(i);
+            vl.v[j + 1] = wv;
+            V.subtract_projections(vl, gs + pass * kGsPass, wv);
           }
-          VecList vl{};
-          vl.count = j + 2;
-          for (int i = 0; i <= j; i++) vl.v[i] = Vk(i);
-          vl.v[j + 1] = wv;
-          V.subtract_projections(vl, gs + pass * kGsPass, wv);
-        }
-        {
-          DotList dl{};
-          dl.count = 1;
-          dl.a[0] = dl.b[0] = wv;
-          V.dots_dev(dl, gs + 2 * kGsPass, 2 * kGsPass);
-        }
-        V.wait_host(2 * kGsPass + 1, hb.data());
+          {
+            DotList dl{};
+            dl.count = 1;
+            dl.a[0] = dl.b[0] = wv;
+            V.dots_dev(dl, gs + 2 * kGsPass, 2 * kGsPass);
+          }
+          V.wait_host(2 * kGsPass + 1, hb.data());
+        } while (per_rank.take());
         for (int i = 0; i <= j; i++) h[i] = (0.0 + hb[i]) + hb[kGsPass + i];
         double hn = std::sqrt(hb[2 * kGsPass]);
         for (int i = 0; i <= j; i++) H[(size_t)i * m + j] = h[i];

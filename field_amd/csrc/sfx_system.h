@@ -95,6 +95,9 @@ struct Molecule {
   double phi_range = 0;
   int nstore = 0;         // forward ranks the backward pass needs
   ChainPlan plan;         // how they are kept
+  // rank s of either chain comes out of a launch of several ranks: not the first
+  // one, nor the middle rank of an odd palindrome
+  bool blocked_rank(int s) const { return s >= 2 && !(kind == 2 && N % 2 == 1 && s == N / 2 + 1); }
   MolParams params(int index) const {
     return MolParams{index, N, freedom, kind, phib, theta};
   }
@@ -247,8 +250,10 @@ struct System {
   // tangent into dmol) before the next chain overwrites the running ranks
   EndArgs ends{};
   void add_end(int m, const void* G, const void* dG, bool f32, const double* lnf);
+  // the last entry's maxima to be checked (steps of d_maxf and d_maxb, 0: none)
+  void check_end(int m, int fstep, int bstep);
   void close_ends(bool base, double* dmol);
-  PhiArgs phi_args();
+  PhiArgs phi_args(int precision);
   FieldArgs field_args();
   void residual_internal(int precision);  // d_u -> d_f
   void finish_range(int m, int precision);  // range_restricted: the range condition fixes molecule m's constant
@@ -280,11 +285,35 @@ struct System {
   // middle-out: its forward and backward chains advance in the same launches.
   // The base and the tangent sweeps must agree on this (their compositions
   // share the reference log).
-  bool middle_out(const Molecule& mo) const {
-    return use_block3 && schedule == SFX_SCHEDULE_AUTO && mo.kind == 1 && !mo.plan.c && mo.N >= 2;
+  bool middle_out(const Molecule& mo, int precision) const {
+    return blocked(precision) && schedule == SFX_SCHEDULE_AUTO && mo.kind == 1 && !mo.plan.c && mo.N >= 2;
   }
   int schedule = SFX_SCHEDULE_AUTO;  // sfx_options.chain_schedule
   int sweep_kernel = SFX_SWEEP_AUTO;  // sfx_options.sweep_kernel
+  // FP32 sweeps of several ranks per launch set the word low_word() where a rank
+  // decayed too far within a launch (kLowMax). took_low(), after a wait for the
+  // stream, says so and clears it; the caller then repeats the evaluation with
+  // fp32_per_rank set, which renormalises every rank. checked() does both
+  bool fp32_per_rank = false;
+  bool blocked(int precision) const { return use_block3 && !(precision == SFX_FP32 && fp32_per_rank); }
+  void set_fp32_per_rank(bool on);
+  unsigned* low_word();
+  bool took_low();
+  unsigned* h_low = nullptr;
+  // run(): an evaluation in `precision` and a wait for the stream
+  template <class Run>
+  void checked(int precision, Run&& run) {
+    run();
+    if (precision != SFX_FP32 || !took_low()) return;
+    set_fp32_per_rank(true);
+    try {
+      run();
+    } catch (...) {
+      set_fp32_per_rank(false);
+      throw;
+    }
+    set_fp32_per_rank(false);
+  }
   bool gmax_valid = false;           // d_gmax holds the maxima of the current FP32 SWF
 };
 

@@ -65,6 +65,7 @@ System::~System() {
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (h_vec) (void)hipHostFree(h_vec);
+  if (h_low) (void)hipHostFree(h_low);
   tangent_free(tan);
   precond_free(precond);
   solve_work_free(work);
@@ -516,7 +517,7 @@ void System::sweep(int m, bool scaled) {
     return;
   }
   if constexpr (std::is_same<T, A>::value) {
-    if (use_block3) {
+    if (blocked(P)) {
       sweep_blocked<T>(m, scaled);
       return;
     }
@@ -671,6 +672,7 @@ void System::sweep_blocked(int m, bool scaled) {
       a.lnpair = lnpair;
       a.ref = scal + MS_REF;
       a.gmax = d_gmax + (size_t)t * kStepWords;
+      a.low = mo.blocked_rank(sa - 1) ? low_word() : nullptr;
     }
     a.s0 = sa - 1;
     return a;
@@ -689,7 +691,7 @@ void System::sweep_blocked(int m, bool scaled) {
     la.nchains = 1;
     go(la, connect);
   };
-  if (middle_out(mo)) {
+  if (middle_out(mo, P)) {
     // Launch i advances the forward chain through ranks 2..h (stored) and the
     // backward chain through ranks N-1..h+1 (stored) together. Then the
     // forward chain continues through ranks h+1..N composed with the stored
@@ -762,6 +764,7 @@ void System::sweep_blocked(int m, bool scaled) {
       go(la, true);
     }
     add_end(m, pp[fc], nullptr, sizeof(T) == 4, scaled ? lnf + N : nullptr);  // forward rank N
+    if (scaled) check_end(m, N, N);
     return;
   }
   // forward chain, ranks 2..plan.n; every rank kept (full store) or the
@@ -871,11 +874,52 @@ void System::sweep_blocked(int m, bool scaled) {
     lnfinal = scaled ? lnf + N : nullptr;
   }
   add_end(m, final_G, nullptr, sizeof(T) == 4, lnfinal);
+  if (scaled) check_end(m, N, mo.kind == 1 ? N : 0);
+}
+
+void System::check_end(int m, int fstep, int bstep) {
+  const Molecule& mo = mols[m];
+  const size_t off = (size_t)m * (maxN + 2) * kStepWords;
+  EndMol& e = ends.e[ends.n - 1];
+  e.endmax[0] = d_maxf + off + (size_t)fstep * kStepWords;
+  // an odd palindrome's middle rank is made from rank N/2 by a launch of its own
+  if (mo.kind == 2 && mo.N % 2 == 1 && mo.blocked_rank(mo.N / 2))
+    e.endmax[1] = d_maxf + off + (size_t)(mo.N / 2) * kStepWords;
+  else
+    e.endmax[1] = bstep ? d_maxb + off + (size_t)bstep * kStepWords : nullptr;
+  e.low = low_word();
+}
+
+unsigned* System::low_word() {
+  if (!h_low) {
+    if (hipHostMalloc((void**)&h_low, sizeof(unsigned), hipHostMallocCoherent) != hipSuccess) {
+      (void)hipGetLastError();
+      h_low = nullptr;
+      throw Error{SFX_E_OOM, "hipHostMalloc failed"};
+    }
+    *h_low = 0u;
+  }
+  return h_low;
+}
+
+bool System::took_low() {
+  if (!h_low || !*(volatile unsigned*)h_low) return false;
+  *(volatile unsigned*)h_low = 0u;
+  return true;
+}
+
+void System::set_fp32_per_rank(bool on) {
+  if (fp32_per_rank == on) return;
+  fp32_per_rank = on;
+  if (res_graph[1]) {
+    (void)hipGraphExecDestroy(res_graph[1]);
+    res_graph[1] = nullptr;
+  }
 }
 
 void System::add_end(int m, const void* G, const void* dG, bool f32, const double* lnf) {
   ends.n++;
-  ends.e[ends.n - 1] = EndMol{mols[m].params(m), G, dG, lnf, f32, lnf == nullptr};
+  ends.e[ends.n - 1] = EndMol{mols[m].params(m), G, dG, lnf, f32, lnf == nullptr, {nullptr, nullptr}, nullptr};
 }
 
 void System::close_ends(bool base, double* dmol) {
@@ -890,14 +934,14 @@ void System::close_ends(bool base, double* dmol) {
   ends.n = 0;
 }
 
-PhiArgs System::phi_args() {
+PhiArgs System::phi_args(int prec) {
   PhiArgs a{};
   a.nm = nm;
   a.ns = ns;
   for (int m = 0; m < nm; m++) {
     a.uses[m] = mols[m].uses_mask();
     a.mode[m] = mols[m].kind == 0 ? CLOSE_MONOMER : CLOSE_CHAIN;
-    a.two[m] = middle_out(mols[m]);
+    a.two[m] = middle_out(mols[m], prec);
   }
   for (int t = 0; t < ns; t++) a.frozen[t] = frozen[t];
   a.acc = d_acc;
@@ -926,7 +970,7 @@ FieldArgs System::field_args() {
 void System::start_phi(int prec, const double* x, const ZeroList* zero, const SiteVec* v, double* v64, float* v32) {
   const DevLattice& L = lat.d;
   ends.n = 0;  // whatever a call that threw left
-  const bool gmax = prec == SFX_FP32 && use_block3;
+  const bool gmax = prec == SFX_FP32 && blocked(prec);
   SwfArgs a{};
   a.x = x ? vec_abi(x) : vec_internal(d_u);
   a.u = x ? d_u : nullptr;
@@ -952,7 +996,7 @@ void System::start_phi(int prec, const double* x, const ZeroList* zero, const Si
       if (mo.uses[t]) {
         const size_t off = ((size_t)m * ns + t) * L.M * w;
         zero_list_add(zl, (unsigned*)d_acc + off, L.M * w, stream);
-        if (middle_out(mo)) zero_list_add(zl, (unsigned*)d_acc2 + off, L.M * w, stream);
+        if (middle_out(mo, prec)) zero_list_add(zl, (unsigned*)d_acc2 + off, L.M * w, stream);
       }
     if (prec == SFX_FP32) {
       const size_t off = (size_t)m * (maxN + 2) * kStepWords;
@@ -1054,7 +1098,7 @@ void System::compute_phi(int prec, const double* x, const SiteOut& f) {
       }
     }
   close_ends(true, nullptr);
-  PhiArgs a = phi_args();
+  PhiArgs a = phi_args(prec);
   a.base = true;
   for (int m = 0; m < nm; m++)
     if (mols[m].freedom == SFX_RANGE_RESTRICTED) a.mode[m] = CLOSE_DONE;
@@ -1107,10 +1151,10 @@ void System::finish_range(int m, int prec) {
                            phim + (size_t)mo.seq[0] * lat.d.M, stream);
   else if (prec == SFX_FP32)
     launch_mol_phi_states<float>(lat.d, mo.uses_mask(), ns, (const float*)d_acc + off,
-                                 middle_out(mo) ? (const float*)d_acc2 + off : nullptr, d_swf, scal, phim, stream);
+                                 middle_out(mo, prec) ? (const float*)d_acc2 + off : nullptr, d_swf, scal, phim, stream);
   else
     launch_mol_phi_states<double>(lat.d, mo.uses_mask(), ns, (const double*)d_acc + off,
-                                  middle_out(mo) ? (const double*)d_acc2 + off : nullptr, d_swf, scal, phim, stream);
+                                  middle_out(mo, prec) ? (const double*)d_acc2 + off : nullptr, d_swf, scal, phim, stream);
   const int nb = launch_range_sum(lat.d, mo.range, mo.uses_mask(), ns, phim, d_partial, stream);
   launch_range_scale(lat.d, mo.uses_mask(), ns, d_partial, nb, mo.phi_range, mo.N, d_molscal + (size_t)m * MS_COUNT,
                      phim, stream);
