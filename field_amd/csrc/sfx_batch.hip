@@ -25,16 +25,39 @@ namespace sfx {
 constexpr int kMaxLayers = 1024;
 constexpr int kMaxDiis = 15;
 
+// Sums over a problem are taken as a workgroup of kSumThreads takes them,
+// whatever number of threads runs it: a thread adds the terms of kSumThreads /
+// BT such threads separately (terms t + r BT, t + r BT + kSumThreads, ...), the
+// waves are reduced one by one and added in order. With the rounding of every
+// other operation written out, residuals and DIIS iterates do not depend on what
+// tune() chooses; DIIS amplifies a last bit into another path and, where the
+// bulk is unstable, into another number of converged problems.
+constexpr int kSumThreads = 512;
 template <int BT>
-__device__ __forceinline__ double block_sum(double v, double* red) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double r = 0;
+constexpr int kSumParts = kSumThreads / BT;
+
+// red holds NV * kSumThreads / 64 doubles; every thread gets the totals
+template <int BT, int NV>
+__device__ __forceinline__ void block_sum(double (&v)[kSumParts<BT>][NV], double (&out)[NV], double* red) {
+  constexpr int R = kSumParts<BT>, W = BT / 64;
 #pragma unroll
-  for (int i = 0; i < BT / 64; i++) r += red[i];
-  return r;
+  for (int r = 0; r < R; r++)
+#pragma unroll
+    for (int j = 0; j < NV; j++)
+      for (int o = 32; o > 0; o >>= 1) v[r][j] += __shfl_xor(v[r][j], o, 64);
+  __syncthreads();  // red may still be read from the previous call
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+      for (int j = 0; j < NV; j++) red[j * (R * W) + r * W + (threadIdx.x >> 6)] = v[r][j];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    double s = 0;
+    for (int w = 0; w < R * W; w++) s += red[j * (R * W) + w];
+    out[j] = s;
+  }
 }
 
 // The residual of problem b at x, by the workgroup that owns it; every
@@ -56,7 +79,7 @@ __device__ void batch_residual(const BatchProb& p, int b, const double* __restri
                                double* __restrict__ store, double* __restrict__ phi_out,
                                double* __restrict__ lngn, double* lds, int ldsw) {
   constexpr int kBlock = K <= 2 ? 8 : K <= 5 ? 4 : 2, kRing = kBlock;  // ranks; stored rows of twice as many ranks
-  __shared__ double red[BT / 64];
+  __shared__ double red[kSumThreads / 64];
   const int n = p.n, N = p.N;
   const long long M = n + 2;
   const double l = p.lambda;
@@ -186,10 +209,14 @@ __device__ void batch_residual(const BatchProb& p, int b, const double* __restri
 #pragma unroll
   for (int j = 0; j < K; j++) lds[c.to[j]] = c.G[j];
   __syncthreads();
-  double w = 0;
-  for (int z = 1 + t; z <= n; z += BT) w += lds[z];
-  const double GN = block_sum<BT>(w, red);
-  if (t == 0 && lngn) lngn[b] = log(GN);
+  double w[kSumParts<BT>][1], GN[1];
+#pragma unroll
+  for (int q = 0; q < kSumParts<BT>; q++) {
+    w[q][0] = 0;
+    for (int z = 1 + t + q * BT; z <= n; z += kSumThreads) w[q][0] += lds[z];
+  }
+  block_sum<BT, 1>(w, GN, red);
+  if (t == 0 && lngn) lngn[b] = log(GN[0]);
 
   // phi_A = 2 (phi_b / N) acc / g (free homopolymer, half store), phi_S = (1 - phi_b) g_S
   const double CA = 2.0 * p.phib / N, phibS = 1.0 - p.phib;
@@ -215,24 +242,28 @@ __device__ void batch_residual(const BatchProb& p, int b, const double* __restri
       po[M + z] = in ? phS[z] : 0.0;
     }
   }
-  // contact averages and the residual (two iteration variables, A and S)
-  const double cbA = p.chi_as * phibS, cbS = p.chi_as * p.phib;
-  double* fb = f + p.xoff;
+  // contact averages and the residual (two iteration variables, A and S), each
+  // operation rounded as written
+  {
+#pragma clang fp contract(off)
+    const double cbA = p.chi_as * phibS, cbS = p.chi_as * p.phib;
+    double* fb = f + p.xoff;
 #pragma unroll
-  for (int j = 0; j < K; j++) {
-    const int z = c.to[j];
-    if (z <= n) {
-      const double upA = z == n ? phA[n] : phA[z + 1];
-      const double upS = z == n ? phS[n] : phS[z + 1];
-      const double sA = vA[j] + l * (phA[z - 1] - 2.0 * vA[j] + upA);
-      const double sS = vS[j] + l * (phS[z - 1] - 2.0 * vS[j] + upS);
-      const double sW = z == 1 ? l : 0.0;  // the wall (phi 1 in layer 0) seen from layer 1
-      const double pt = vA[j] + vS[j];
-      const double uA = -log(c.g[j]) - (p.chi_as * sS + p.chi_s * sW) / pt + cbA;
-      const double uS = -log(gS[j]) - (p.chi_as * sA) / pt + cbS;
-      const double av = 0.5 * (uA + uS);
-      fb[2 * (z - 1)] = -1.0 + 1.0 / pt + uA - av;
-      fb[2 * (z - 1) + 1] = -1.0 + 1.0 / pt + uS - av;
+    for (int j = 0; j < K; j++) {
+      const int z = c.to[j];
+      if (z <= n) {
+        const double upA = z == n ? phA[n] : phA[z + 1];
+        const double upS = z == n ? phS[n] : phS[z + 1];
+        const double sA = fma(l, (phA[z - 1] - 2.0 * vA[j]) + upA, vA[j]);
+        const double sS = fma(l, (phS[z - 1] - 2.0 * vS[j]) + upS, vS[j]);
+        const double sW = z == 1 ? l : 0.0;  // the wall (phi 1 in layer 0) seen from layer 1
+        const double pt = vA[j] + vS[j];
+        const double uA = -log(c.g[j]) - fma(p.chi_as, sS, p.chi_s * sW) / pt + cbA;
+        const double uS = -log(gS[j]) - (p.chi_as * sA) / pt + cbS;
+        const double av = 0.5 * (uA + uS);
+        fb[2 * (z - 1)] = -1.0 + 1.0 / pt + uA - av;
+        fb[2 * (z - 1) + 1] = -1.0 + 1.0 / pt + uS - av;
+      }
     }
   }
 }
@@ -247,26 +278,6 @@ __global__ void __launch_bounds__(BT) k_batch_residual(const BatchProb* __restri
   if (active && !active[b]) return;
   const BatchProb p = P[b];
   batch_residual<BT, K>(p, b, x, f, store, phi_out, lngn, lds, ldsw);
-}
-
-// Sums four values over the workgroup in a fixed order; every thread gets
-// the totals. red holds 4 * (BT / 64) doubles.
-template <int BT>
-__device__ __forceinline__ void block_reduce4(double (&v)[4], double* red) {
-#pragma unroll
-  for (int j = 0; j < 4; j++)
-    for (int o = 32; o > 0; o >>= 1) v[j] += __shfl_xor(v[j], o, 64);
-  __syncthreads();  // red may still be read from the previous call
-  if ((threadIdx.x & 63) == 0)
-#pragma unroll
-    for (int j = 0; j < 4; j++) red[j * (BT / 64) + (threadIdx.x >> 6)] = v[j];
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    double r = 0;
-    for (int w = 0; w < BT / 64; w++) r += red[j * (BT / 64) + w];
-    v[j] = r;
-  }
 }
 
 // X = A^{-1} 1 by Gaussian elimination with partial pivoting; A (k x k, row
@@ -290,13 +301,13 @@ __device__ void diis_solve(double* A, double* rhs, int k, double* X) {
     const double d = A[c * k + c];
     for (int r = c + 1; r < k; r++) {
       const double fct = A[r * k + c] / d;
-      for (int j = c; j < k; j++) A[r * k + j] -= fct * A[c * k + j];
-      rhs[r] -= fct * rhs[c];
+      for (int j = c; j < k; j++) A[r * k + j] = fma(-fct, A[c * k + j], A[r * k + j]);
+      rhs[r] = fma(-fct, rhs[c], rhs[r]);
     }
   }
   for (int i = k - 1; i >= 0; i--) {
     double s = rhs[i];
-    for (int j = i + 1; j < k; j++) s -= A[i * k + j] * X[j];
+    for (int j = i + 1; j < k; j++) s = fma(-A[i * k + j], X[j], s);
     X[i] = s / A[i * k + i];
   }
 }
@@ -316,7 +327,8 @@ template <int BT>
 __device__ bool batch_diis(const BatchProb& p, int b, double* __restrict__ x, const double* __restrict__ g,
                            double* __restrict__ hist, BatchState* __restrict__ S, int m, double eta, double tol,
                            int max_iter, int backtrack) {
-  __shared__ double red[4 * (BT / 64)];
+  constexpr int R = kSumParts<BT>;
+  __shared__ double red[4 * kSumThreads / 64];
   __shared__ double dts[kMaxDiis + 1];
   __shared__ double Ap[kMaxDiis * kMaxDiis], rhs[kMaxDiis], coef[kMaxDiis];
   __shared__ int decision, save_best, finished;
@@ -337,20 +349,25 @@ __device__ bool batch_diis(const BatchProb& p, int b, double* __restrict__ x, co
   const double eta_p = backtrack ? st.eta : eta;
 
   // new point x - eta g and its step; |g|^2 and the step's own product
-  double gg = 0.0, dd = 0.0;
-  for (long long q = t; q < nv; q += BT) {
-    const double xi = xb[q], gi = gb[q];
-    const double xn = xi - eta_p * gi;
-    const double d = xn - xi;
-    x0[q] = xi;
-    xR[(long long)k * nv + q] = xn;
-    xx0[(long long)k * nv + q] = d;
-    gg += gi * gi;
-    dd += d * d;
-  }
   {
-    double two[4] = {gg, dd, 0.0, 0.0};
-    block_reduce4<BT>(two, red);
+    double part[R][2], two[2];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      double gg = 0.0, dd = 0.0;
+      for (long long q = t + r * BT; q < nv; q += kSumThreads) {
+        const double xi = xb[q], gi = gb[q];
+        const double xn = fma(-eta_p, gi, xi);
+        const double d = xn - xi;
+        x0[q] = xi;
+        xR[(long long)k * nv + q] = xn;
+        xx0[(long long)k * nv + q] = d;
+        gg = fma(gi, gi, gg);
+        dd = fma(d, d, dd);
+      }
+      part[r][0] = gg;
+      part[r][1] = dd;
+    }
+    block_sum<BT, 2>(part, two, red);
     if (t == 0) {
       dts[kMaxDiis] = two[0];
       dts[kd - 1] = two[1];
@@ -359,19 +376,24 @@ __device__ bool batch_diis(const BatchProb& p, int b, double* __restrict__ x, co
   // the products of the step with the kept steps, four per pass (a thread
   // reads back only the step entries it wrote itself)
   for (int i0 = 0; i0 < kd - 1; i0 += 4) {
-    double a4[4] = {0.0, 0.0, 0.0, 0.0};
-    for (long long q = t; q < nv; q += BT) {
-      const double d = xx0[(long long)k * nv + q];
+    double part[R][4], a4[4];
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        if (i0 + j < kd - 1) {
-          int posi = k - kd + 1 + i0 + j;
-          if (posi < 0) posi += m;
-          a4[j] += xx0[(long long)posi * nv + q] * d;
+    for (int r = 0; r < R; r++) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) part[r][j] = 0.0;
+      for (long long q = t + r * BT; q < nv; q += kSumThreads) {
+        const double d = xx0[(long long)k * nv + q];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          if (i0 + j < kd - 1) {
+            int posi = k - kd + 1 + i0 + j;
+            if (posi < 0) posi += m;
+            part[r][j] = fma(xx0[(long long)posi * nv + q], d, part[r][j]);
+          }
         }
       }
     }
-    block_reduce4<BT>(a4, red);
+    block_sum<BT, 4>(part, a4, red);
     if (t == 0)
       for (int j = 0; j < 4 && i0 + j < kd - 1; j++) dts[i0 + j] = a4[j];
   }
@@ -448,7 +470,7 @@ __device__ bool batch_diis(const BatchProb& p, int b, double* __restrict__ x, co
       for (int i = 0; i < kd; i++) {
         int posi = k - kd + 1 + i;
         if (posi < 0) posi += m;
-        s += coef[i] * xR[(long long)posi * nv + q];
+        s = fma(coef[i], xR[(long long)posi * nv + q], s);
       }
       xb[q] = s;
     }
@@ -722,6 +744,15 @@ int sfx_batch_tuning(const sfx_batch* b, int* threads, float* ms) {
     *threads = b->b.block;
     if (ms)
       for (int i = 0; i < 4; i++) ms[i] = b->b.tuned_ms[i];
+  });
+}
+
+int sfx_batch_set_threads(sfx_batch* b, int threads) {
+  return guarded([&] {
+    SFX_REQUIRE(b, SFX_E_INVALID, "NULL argument");
+    SFX_REQUIRE(threads == 64 || threads == 128 || threads == 256 || threads == 512, SFX_E_INVALID,
+                "64, 128, 256 or 512 threads per problem");
+    b->b.block = threads;
   });
 }
 

@@ -51,6 +51,7 @@ _SIGS = {
     "sfx_batch_destroy": (C.c_int, [C.c_void_p]),
     "sfx_batch_sizes": (C.c_int, [C.c_void_p, C.POINTER(C.c_longlong), C.c_void_p]),
     "sfx_batch_tuning": (C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.c_void_p]),
+    "sfx_batch_set_threads": (C.c_int, [C.c_void_p, C.c_int]),
     "sfx_batch_residual": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int]),
     "sfx_batch_solve": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p,
                                   C.c_void_p]),
@@ -414,6 +415,10 @@ class Batch:
         ms = (C.c_float * 4)()
         check(lib().sfx_batch_tuning(self.h, C.byref(th), ms))
         return th.value, list(ms)
+
+    def set_threads(self, threads: int):
+        """Threads per problem instead of the tuner's choice; results are the same bits."""
+        check(lib().sfx_batch_set_threads(self.h, threads))
 
     def split(self, v):
         return [v[self.offsets[i]:self.offsets[i + 1]] for i in range(len(self.problems))]

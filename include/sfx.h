@@ -344,6 +344,9 @@ int sfx_batch_sizes(const sfx_batch* b, long long* nvar, long long* offsets);
 /* Threads per problem the tuner chose at creation and the residual time (ms)
  * it measured at 64, 128, 256 and 512 threads (ms: 4 floats, may be NULL). */
 int sfx_batch_tuning(const sfx_batch* b, int* threads, float* ms);
+/* This many threads per problem (64, 128, 256 or 512) instead of the tuner's
+ * choice. Results are the same bits at each. */
+int sfx_batch_set_threads(sfx_batch* b, int threads);
 /* Residuals of every problem at x (host or device per `where`). */
 int sfx_batch_residual(sfx_batch* b, const double* x, double* f, int where);
 /* DIIS (MPS.cpp:228-284) on every problem at once from x (in/out), in one
