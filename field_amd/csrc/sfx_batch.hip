@@ -559,8 +559,10 @@ void Batch::create(const sfx_adsorption_desc* d, int count, const sfx_options* o
   SFX_HIP(hipMalloc(&d_lngn, B * sizeof(double)));
   SFX_HIP(hipMalloc(&d_state, B * sizeof(BatchState)));
   SFX_HIP(hipMemcpy(d_prob, probs.data(), B * sizeof(BatchProb), hipMemcpyHostToDevice));
-  SFX_HIP(hipMemset(d_x, 0, nvar * sizeof(double)));
-  SFX_HIP(hipMemset(d_store, 0, store_words * sizeof(double)));  // entry 0 of a row is the surface layer, never written
+  // on the stream of the launches that read them: it does not wait for the default stream
+  SFX_HIP(hipMemsetAsync(d_x, 0, nvar * sizeof(double), stream));
+  // (entry 0 of a store row is the surface layer, never written)
+  SFX_HIP(hipMemsetAsync(d_store, 0, store_words * sizeof(double), stream));
   tune();
 }
 

@@ -37,3 +37,21 @@ def test_other_numbers_of_threads_are_refused(sfx):
     for threads in (0, 32, 96, 1024):
         with pytest.raises(sfx.SFError):
             B.set_threads(threads)
+
+
+def test_first_residual_of_a_batch_in_used_memory(sfx):
+    """The store's surface entries are cleared before any launch reads them, also
+    in memory that held something else: the first residual is the second's bits."""
+    import torch
+
+    x = None
+    for _ in range(3):
+        junk = torch.full((1 << 25,), float("nan"), dtype=torch.float64, device="cuda")
+        del junk
+        torch.cuda.empty_cache()
+        B = sfx.Batch(configs.batch_1d(256))
+        if x is None:
+            x = np.random.default_rng(3).normal(0, 0.1, B.nvar)
+            ref = B.residual(x)
+        assert np.isfinite(ref).all() and np.array_equal(B.residual(x), ref)
+        B.close()
