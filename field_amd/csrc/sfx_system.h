@@ -184,10 +184,9 @@ struct System {
   double* d_fprof = nullptr;  // ns * M
   int* d_frozen = nullptr;
   int* d_st_itvar = nullptr;
-  int* d_mol_uses = nullptr;  // nm * ns
   unsigned char* d_itmask = nullptr;
   long long* d_sites = nullptr;
-  int* d_order = nullptr;       // site -> its ordinal among the iteration sites or -1 (null: melt form)
+  int* d_order = nullptr;       // site -> its ordinal among the iteration sites or -1, behind d_sites (null: melt form)
   void* d_store = nullptr;    // maxstore * M propagator words
   void* d_pp = nullptr;       // 2 * M running propagator
   void* d_pp2 = nullptr;      // 2 * M, the backward chain's in a middle-out sweep
@@ -197,7 +196,7 @@ struct System {
   unsigned* d_maxf = nullptr;
   unsigned* d_maxb = nullptr;
   double* d_partial = nullptr;  // reduction partials
-  unsigned* d_ticket = nullptr;  // arrivals of an end sum's workgroups
+  unsigned* d_ticket = nullptr;  // arrivals of an end sum's workgroups (behind d_scalar's 16)
   unsigned* d_gmax = nullptr;   // ns x kStepWords: lattice maximum of each FP32 SWF (blocked sweeps)
   double* d_phib_state = nullptr;
   double* d_cbulk = nullptr;

@@ -27,6 +27,19 @@ static __global__ void k_fill_bytes8(unsigned long long* p, long long n) {
 static __global__ void k_set_ref(double* scal, const double* lnv, int idx, double factor) {
   if (threadIdx.x == 0 && blockIdx.x == 0) scal[MS_REF] = factor * lnv[idx];
 }
+// order[i] = ordinal of site i among the (ascending) iteration sites, -1 off them
+static __global__ void k_order(const unsigned char* itmask, const long long* sites, long long nsites, long long M,
+                               int* order) {
+  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= M) return;
+  long long lo = 0, hi = itmask[i] ? nsites : 0;
+  while (hi - lo > 1) {
+    const long long mid = (lo + hi) / 2;
+    if (sites[mid] <= i) lo = mid;
+    else hi = mid;
+  }
+  order[i] = itmask[i] ? (int)lo : -1;
+}
 // x -> u[itvar][M]; u zero off the iteration sites
 static __global__ void k_load(SiteVec x, long long M, double* u) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -58,9 +71,9 @@ System::~System() {
   for (auto& a : chain1_dev)
     for (Chain1Step* p : a)
       if (p) (void)hipFree(p);
-  void* ptrs[] = {d_u, d_f, d_swf, d_swf32, d_phi_m, d_acc, d_acc2, d_phi, d_rho, d_phitot, d_fprof, d_frozen,
-                  d_st_itvar, d_mol_uses, d_itmask, d_sites, d_order, d_store, d_pp, d_pp2, d_molscal, d_lnf, d_lnb,
-                  d_maxf, d_maxb, d_partial, d_ticket, d_phib_state, d_cbulk, d_scalar, d_xabi, d_gmax,
+  void* ptrs[] = {d_u, d_f, d_swf, d_swf32, d_phi_m, d_acc, d_phi, d_rho, d_phitot, d_fprof, d_frozen,
+                  d_st_itvar, d_itmask, d_sites, d_store, d_pp, d_molscal, d_lnf, d_lnb,
+                  d_maxf, d_maxb, d_partial, d_phib_state, d_cbulk, d_scalar, d_xabi, d_gmax,
                   d_abi_in, d_abi_out, scf1_runs};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -274,17 +287,15 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   d_swf = dalloc<double>(ns * M);
   d_swf32 = dalloc<float>(ns * M);
   d_phi_m = dalloc<double>((size_t)nm * ns * M);
-  d_acc = dalloc<double>((size_t)nm * ns * M);
   d_phi = dalloc<double>(ns * M);
   d_rho = dalloc<double>(ns * M);
   d_phitot = dalloc<double>(M);
   d_fprof = dalloc<double>(ns * M);
   d_frozen = dalloc<int>(ns);
   d_st_itvar = dalloc<int>(ns);
-  d_mol_uses = dalloc<int>((size_t)nm * ns);
   d_itmask = dalloc<unsigned char>(M);
-  d_sites = dalloc<long long>(sites.size());
-  if (form != SFX_FORM_MELT) d_order = dalloc<int>((size_t)M);
+  d_sites = dalloc<long long>(sites.size() + (form != SFX_FORM_MELT ? (M + 1) / 2 : 0));
+  if (form != SFX_FORM_MELT) d_order = (int*)(d_sites + sites.size());
   // propagator store: every forward rank, or sqrt(N) checkpoints when the
   // memory budget (bytes of one FP64 store) cannot hold them all
   const size_t comps = lat.d.order == 2 ? 6 : 1;
@@ -305,10 +316,13 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
     SFX_REQUIRE((size_t)store_slots * slot_bytes <= budget, SFX_E_OOM,
                 "memory budget below the checkpointed propagator store (2 sqrt(N) ranks)");
   d_store = dalloc<double>((size_t)store_slots * comps * M);  // sized for FP64 so both precisions fit
-  d_pp = dalloc<double>(2 * comps * M);
+  // with the backward chains' of middle-out sweeps behind them
+  const size_t n_acc = (size_t)nm * ns * M, n_pp = 2 * comps * M;
+  d_acc = dalloc<double>(use_block3 ? 2 * n_acc : n_acc);
+  d_pp = dalloc<double>(use_block3 ? n_pp + 2 * M : n_pp);
   if (use_block3) {
-    d_acc2 = dalloc<double>((size_t)nm * ns * M);
-    d_pp2 = dalloc<double>(2 * M);
+    d_acc2 = (double*)d_acc + n_acc;
+    d_pp2 = (double*)d_pp + n_pp;
   }
   d_molscal = dalloc<double>((size_t)nm * MS_COUNT);
   d_lnf = dalloc<double>((size_t)nm * (maxN + 2));
@@ -318,35 +332,27 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   npart = (int)grid1(std::max<long long>(lat.d.M, lat.d.V), 256);
   npart = std::max(npart, 2 * SFX_MAXM * kEndBlocks);
   d_partial = dalloc<double>(npart);
-  d_ticket = dalloc<unsigned>(2);
   d_gmax = dalloc<unsigned>((size_t)SFX_MAXS * kStepWords);
   d_phib_state = dalloc<double>(SFX_MAXS);
   d_cbulk = dalloc<double>(SFX_MAXS);
-  d_scalar = dalloc<double>(16);
+  d_scalar = dalloc<double>(17);
+  d_ticket = (unsigned*)(d_scalar + 16);
   d_xabi = dalloc<double>((size_t)nvar);
-  std::vector<int> uses((size_t)nm * ns);
-  for (int m = 0; m < nm; m++)
-    for (int t = 0; t < ns; t++) uses[(size_t)m * ns + t] = mols[m].uses[t];
   SFX_HIP(hipMemcpy(d_fprof, fprof.data(), ns * M * sizeof(double), hipMemcpyHostToDevice));
   SFX_HIP(hipMemcpy(d_frozen, frozen.data(), ns * sizeof(int), hipMemcpyHostToDevice));
   SFX_HIP(hipMemcpy(d_st_itvar, st_itvar.data(), ns * sizeof(int), hipMemcpyHostToDevice));
-  SFX_HIP(hipMemcpy(d_mol_uses, uses.data(), uses.size() * sizeof(int), hipMemcpyHostToDevice));
   SFX_HIP(hipMemcpy(d_itmask, itmask.data(), M, hipMemcpyHostToDevice));
-  if (d_order) {
-    std::vector<int> order((size_t)M, -1);
-    for (size_t k = 0; k < sites.size(); k++) order[(size_t)sites[k]] = (int)k;
-    SFX_HIP(hipMemcpy(d_order, order.data(), (size_t)M * sizeof(int), hipMemcpyHostToDevice));
-  }
   if (!sites.empty())
     SFX_HIP(hipMemcpy(d_sites, sites.data(), sites.size() * sizeof(long long), hipMemcpyHostToDevice));
+  if (d_order)
+    k_order<<<grid1(Mn, 256), 256, 0, stream>>>(d_itmask, d_sites, (long long)sites.size(), Mn, d_order);
   // zero everything once: halo slots of propagator arrays are never written
   zero_bytes(d_store, (size_t)store_slots * comps * M * 8, stream);
-  zero_bytes(d_pp, 2 * comps * M * 8, stream);
-  if (d_pp2) zero_bytes(d_pp2, 2 * M * 8, stream);
+  zero_bytes(d_pp, (use_block3 ? n_pp + 2 * M : n_pp) * 8, stream);
   zero_bytes(d_u, n_itvar * M * 8, stream);
   zero_bytes(d_ticket, 8, stream);
   zero_bytes(d_f, n_itvar * M * 8, stream);
-  zero_bytes(d_acc, (size_t)nm * ns * M * 8, stream);
+  zero_bytes(d_acc, n_acc * 8, stream);
   zero_bytes(d_phi_m, (size_t)nm * ns * M * 8, stream);
   zero_bytes(d_molscal, (size_t)nm * MS_COUNT * 8, stream);
   SFX_HIP(hipStreamSynchronize(stream));
