@@ -14,6 +14,7 @@
 // The transpose product J^T w runs the same recursions backwards (adjoint
 // propagators with the transposed stencil, applied as a scatter).
 #include <cmath>
+#include <memory>
 #include <type_traits>
 
 #include "sfx_scf.h"
@@ -756,8 +757,9 @@ void tangent_free(Tangent* t) { delete t; }
 
 static Tangent& tangent(System& S) {
   if (!S.tan) {
-    S.tan = new Tangent();
-    S.tan->init(S);
+    std::unique_ptr<Tangent> t(new Tangent());  // the system's only once it has all its buffers
+    t->init(S);
+    S.tan = t.release();
   }
   return *S.tan;
 }

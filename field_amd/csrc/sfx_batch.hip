@@ -638,6 +638,7 @@ void Batch::ensure_history(int m) {
   if (hist_m == m) return;
   if (d_hist) SFX_HIP(hipFree(d_hist));
   d_hist = nullptr;
+  hist_m = 0;
   long long ho = 0;
   for (int i = 0; i < B; i++) {
     probs[i].hoff = ho;

@@ -22,17 +22,21 @@ struct DevBuf {
   size_t n = 0;
   DevBuf() = default;
   explicit DevBuf(size_t n_) { alloc(n_); }
+  // whatever was held before is given back first, also when this throws
   void alloc(size_t n_) {
+    release();
+    if (hipMalloc(&p, (n_ ? n_ : 1) * sizeof(T)) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+      throw Error{SFX_E_OOM, "hipMalloc failed"};
+    }
     n = n_;
-    if (hipMalloc(&p, (n ? n : 1) * sizeof(T)) != hipSuccess) throw Error{SFX_E_OOM, "hipMalloc failed"};
   }
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
-  }
-  void reset(size_t n_) {
+  ~DevBuf() { release(); }
+  void release() {
     if (p) (void)hipFree(p);
     p = nullptr;
-    alloc(n_);
+    n = 0;
   }
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;

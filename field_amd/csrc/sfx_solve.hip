@@ -112,11 +112,12 @@ void VecOps::init(long long n_, hipStream_t st) {
   if (partial) (void)hipFree(partial);
   if (dres) (void)hipFree(dres);
   partial = dres = nullptr;
-  n = n_;
-  nblk = (int)std::min<long long>(grid1(n, kDotBlock), 1024);
+  n = 0;  // until all of it is there
+  nblk = (int)std::min<long long>(grid1(n_, kDotBlock), 1024);
   SFX_HIP(hipMalloc(&partial, sizeof(double) * kMaxDots * nblk));
   SFX_HIP(hipMalloc(&dres, sizeof(double) * kMaxDots));
   if (!hres) SFX_HIP(hipHostMalloc(&hres, sizeof(double) * kHostWords, hipHostMallocCoherent));
+  n = n_;
 }
 VecOps::~VecOps() {
   if (partial) (void)hipFree(partial);
@@ -168,7 +169,8 @@ SolveWork& solve_work(System& S, long long n, size_t nvec) {
   if (!S.work) S.work = new SolveWork();
   SolveWork& w = *S.work;
   if (w.n != n || w.nvec < nvec) {  // grows only: a hipFree waits for the device
-    w.vecs.reset((size_t)n * nvec);
+    w.n = 0;
+    w.vecs.alloc((size_t)n * nvec);
     w.n = n;
     w.nvec = nvec;
   }

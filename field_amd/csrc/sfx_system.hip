@@ -62,7 +62,10 @@ static T* dalloc(size_t n) {
   T* p = nullptr;
   if (n == 0) n = 1;
   hipError_t e = hipMalloc(&p, n * sizeof(T));
-  if (e != hipSuccess) throw Error{SFX_E_OOM, std::string("hipMalloc: ") + hipGetErrorString(e)};
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    throw Error{SFX_E_OOM, std::string("hipMalloc: ") + hipGetErrorString(e)};
+  }
   return p;
 }
 
@@ -416,10 +419,8 @@ void System::load_x(const double* x, int where) {
 }
 
 void System::abi_vectors(double*& in, double*& out) {
-  if (!d_abi_in) {
-    d_abi_in = dalloc<double>((size_t)n_itvar * lat.d.M);
-    d_abi_out = dalloc<double>((size_t)n_itvar * lat.d.M);
-  }
+  if (!d_abi_in) d_abi_in = dalloc<double>((size_t)n_itvar * lat.d.M);
+  if (!d_abi_out) d_abi_out = dalloc<double>((size_t)n_itvar * lat.d.M);
   in = d_abi_in;
   out = d_abi_out;
 }
@@ -1044,8 +1045,9 @@ Scf1Args System::scf1_args(const double* x) {
       }
     Chain1Run* dr = dalloc<Chain1Run>(hr.size());
     const hipError_t e = hipMemcpy(dr, hr.data(), hr.size() * sizeof(Chain1Run), hipMemcpyHostToDevice);
-    scf1_runs = dr;
+    if (e != hipSuccess) (void)hipFree(dr);
     SFX_HIP(e);
+    scf1_runs = dr;
     scf1_nruns = (int)hr.size();
     scf1_mols = hm;
   }
