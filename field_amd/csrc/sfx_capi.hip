@@ -41,6 +41,25 @@ struct sfx_system {
   System s;
 };
 
+namespace {
+// an entry point's work; where it finds no memory it starts again without the
+// blocked sweeps' second accumulators (nothing of the caller's has been written
+// when an allocation fails)
+template <class F>
+int guarded_fit(sfx_system* s, F&& f) {
+  return guarded([&] {
+    SFX_REQUIRE(s, SFX_E_INVALID, "NULL argument");
+    try {
+      f();
+      return;
+    } catch (const Error& e) {
+      if (e.code != SFX_E_OOM || !s->s.drop_blocked()) throw;
+    }
+    f();
+  });
+}
+}  // namespace
+
 extern "C" {
 
 int sfx_abi_version(void) { return SFX_ABI_VERSION; }
@@ -92,7 +111,7 @@ int sfx_system_sizes(const sfx_system* s, long* nvar, long* M) {
 }
 
 int sfx_compute_phi(sfx_system* s, const double* x, int where, int precision) {
-  return guarded([&] {
+  return guarded_fit(s, [&] {
     SFX_REQUIRE(s && x, SFX_E_INVALID, "NULL argument");
     System& S = s->s;
     const double* xd = S.abi_in(x, where);
@@ -105,7 +124,7 @@ int sfx_compute_phi(sfx_system* s, const double* x, int where, int precision) {
 }
 
 int sfx_residual(sfx_system* s, const double* x, double* f, int where, int precision) {
-  return guarded([&] {
+  return guarded_fit(s, [&] {
     SFX_REQUIRE(s && x && f, SFX_E_INVALID, "NULL argument");
     System& S = s->s;
     // from host memory both go through one staging vector: x has been read when f is written
@@ -119,7 +138,7 @@ int sfx_residual(sfx_system* s, const double* x, double* f, int where, int preci
 }
 
 int sfx_jvp(sfx_system* s, const double* x, const double* v, double* jv, int where, int precision) {
-  return guarded([&] {
+  return guarded_fit(s, [&] {
     SFX_REQUIRE(s && x && v && jv, SFX_E_INVALID, "NULL argument");
     System& S = s->s;
     const double* xd = S.abi_in(x, where);
@@ -147,7 +166,7 @@ int sfx_jvp(sfx_system* s, const double* x, const double* v, double* jv, int whe
 }
 
 int sfx_vjp(sfx_system* s, const double* x, const double* w, double* jtw, int where, int precision) {
-  return guarded([&] {
+  return guarded_fit(s, [&] {
     SFX_REQUIRE(s && x && w && jtw, SFX_E_INVALID, "NULL argument");
     System& S = s->s;
     S.load_x(x, where);
@@ -264,7 +283,7 @@ int sfx_precondition(sfx_system* s, const double* r, double* out, int where) {
 }
 
 int sfx_solve(sfx_system* s, const sfx_solver_opts* o, double* x, int where, sfx_solve_stats* stats) {
-  return guarded([&] {
+  return guarded_fit(s, [&] {
     SFX_REQUIRE(s && o && x, SFX_E_INVALID, "NULL argument");
     System& S = s->s;
     sfx_solve_stats st{};

@@ -151,6 +151,10 @@ struct System {
   int store_slots = 1;     // rank slots of the propagator store (all molecules share it)
   bool checkpointed = false;
   bool use_block3 = false;  // blocked sweeps of 3-D simple-cubic and 2-D lattices (sfx_options.sweep_kernel)
+  // 2-D and FCC lattices, swept rank by rank where their second accumulators do
+  // not fit: gives these (and the tangents') back; false if there is nothing to give
+  bool drop_blocked();
+  double* d_second = nullptr;  // d_pp2, then d_acc2
   bool use_chain1 = false;  // 1-D FP64 chains in one launch per stretch (sfx_options.sweep_kernel)
   // per molecule and stretch (0 forward, 1 backward, 2 half-store second half):
   // the step list on the device, built on the first sweep (its pointers never change)

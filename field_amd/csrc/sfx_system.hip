@@ -75,7 +75,7 @@ System::~System() {
     for (Chain1Step* p : a)
       if (p) (void)hipFree(p);
   void* ptrs[] = {d_u, d_f, d_swf, d_swf32, d_phi_m, d_acc, d_phi, d_rho, d_phitot, d_fprof, d_frozen,
-                  d_st_itvar, d_itmask, d_sites, d_store, d_pp, d_molscal, d_lnf, d_lnb,
+                  d_st_itvar, d_itmask, d_sites, d_store, d_pp, d_second, d_molscal, d_lnf, d_lnb,
                   d_maxf, d_maxb, d_partial, d_phib_state, d_cbulk, d_scalar, d_xabi, d_gmax,
                   d_abi_in, d_abi_out, scf1_runs};
   for (void* p : ptrs)
@@ -319,14 +319,9 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
     SFX_REQUIRE((size_t)store_slots * slot_bytes <= budget, SFX_E_OOM,
                 "memory budget below the checkpointed propagator store (2 sqrt(N) ranks)");
   d_store = dalloc<double>((size_t)store_slots * comps * M);  // sized for FP64 so both precisions fit
-  // with the backward chains' of middle-out sweeps behind them
-  const size_t n_acc = (size_t)nm * ns * M, n_pp = 2 * comps * M;
-  d_acc = dalloc<double>(use_block3 ? 2 * n_acc : n_acc);
-  d_pp = dalloc<double>(use_block3 ? n_pp + 2 * M : n_pp);
-  if (use_block3) {
-    d_acc2 = (double*)d_acc + n_acc;
-    d_pp2 = (double*)d_pp + n_pp;
-  }
+  const size_t n_acc = (size_t)nm * ns * M;
+  d_acc = dalloc<double>(n_acc);
+  d_pp = dalloc<double>(2 * comps * M);
   d_molscal = dalloc<double>((size_t)nm * MS_COUNT);
   d_lnf = dalloc<double>((size_t)nm * (maxN + 2));
   d_lnb = dalloc<double>((size_t)nm * (maxN + 2));
@@ -341,6 +336,17 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   d_scalar = dalloc<double>(17);
   d_ticket = (unsigned*)(d_scalar + 16);
   d_xabi = dalloc<double>((size_t)nvar);
+  // the backward chains' running ranks and accumulators of middle-out sweeps,
+  // last: 2-D and FCC lattices do without them where memory is short
+  if (use_block3) {
+    try {
+      d_second = dalloc<double>(2 * M + n_acc);
+      d_pp2 = d_second;
+      d_acc2 = d_second + 2 * M;
+    } catch (const Error&) {
+      if (!drop_blocked()) throw;
+    }
+  }
   SFX_HIP(hipMemcpy(d_fprof, fprof.data(), ns * M * sizeof(double), hipMemcpyHostToDevice));
   SFX_HIP(hipMemcpy(d_frozen, frozen.data(), ns * sizeof(int), hipMemcpyHostToDevice));
   SFX_HIP(hipMemcpy(d_st_itvar, st_itvar.data(), ns * sizeof(int), hipMemcpyHostToDevice));
@@ -351,7 +357,8 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
     k_order<<<grid1(Mn, 256), 256, 0, stream>>>(d_itmask, d_sites, (long long)sites.size(), Mn, d_order);
   // zero everything once: halo slots of propagator arrays are never written
   zero_bytes(d_store, (size_t)store_slots * comps * M * 8, stream);
-  zero_bytes(d_pp, (use_block3 ? n_pp + 2 * M : n_pp) * 8, stream);
+  zero_bytes(d_pp, 2 * comps * M * 8, stream);
+  if (d_pp2) zero_bytes(d_pp2, 2 * M * 8, stream);
   zero_bytes(d_u, n_itvar * M * 8, stream);
   zero_bytes(d_ticket, 8, stream);
   zero_bytes(d_f, n_itvar * M * 8, stream);
@@ -360,6 +367,20 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
   zero_bytes(d_molscal, (size_t)nm * MS_COUNT * 8, stream);
   SFX_HIP(hipStreamSynchronize(stream));
   SFX_HIP(hipGetLastError());
+}
+
+bool System::drop_blocked() {
+  if (!use_block3 || checkpointed || lat.d.kind == ST_3D_SC) return false;
+  if (stream) SFX_HIP(hipStreamSynchronize(stream));
+  drop_graphs();
+  if (d_second) (void)hipFree(d_second);
+  d_second = nullptr;
+  d_pp2 = d_acc2 = nullptr;
+  tangent_free(tan);
+  tan = nullptr;
+  use_block3 = false;
+  gmax_valid = false;
+  return true;
 }
 
 void System::sync() { SFX_HIP(hipStreamSynchronize(stream)); }

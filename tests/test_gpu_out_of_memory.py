@@ -47,10 +47,13 @@ class Filled:
         return self
 
     def leave(self, n):
-        self.more = None
+        self.more = []
         torch.cuda.empty_cache()
-        free, _ = torch.cuda.mem_get_info()
-        self.more = torch.empty(max(free - n, 0), dtype=torch.uint8, device="cuda")
+        for _ in range(8):  # what a large allocation really takes is known after it
+            free, _ = torch.cuda.mem_get_info()
+            if free - n < 4 << 20:
+                return
+            self.more.append(torch.empty(free - n, dtype=torch.uint8, device="cuda"))
 
     def __exit__(self, *_):
         self.hold = self.more = None
@@ -86,3 +89,45 @@ def test_refused_twice_and_served_later(sfx):
     for G in systems.values():
         for name, run in calls(G, x, v).items():
             assert np.array_equal(run(), ref[name]), name
+
+
+def used():
+    free, total = torch.cuda.mem_get_info()
+    return total - free
+
+
+def test_fcc_fits_where_it_fitted_rank_by_rank(sfx):
+    """The second accumulators of blocked FCC sweeps are left out, or given back,
+    where they do not fit; the system is then swept rank by rank."""
+    lat, sysd = system((120, 120, 120), "fcc")  # 14 MiB an array; second accumulators and ranks 111 MiB
+    x, v = inputs(sysd.nvar(lat))
+    for lattice in (lat, system((9, 9, 9), "fcc")[0]):  # the kernels of both paths have run once
+        for kernel in ("auto", "per_rank"):
+            S = sfx.System(lattice, sysd, sweep_kernel=kernel)
+            xs, vs = inputs(S.nvar)
+            S.jvp(xs, vs), S.vjp(xs, vs), S.residual(xs)
+            S.close()
+    gc.collect()
+    torch.cuda.empty_cache()
+    u0 = used()
+    P = sfx.System(lat, sysd, sweep_kernel="per_rank")
+    need = used() - u0
+    f = P.residual(x)
+    u1 = used()
+    jv = P.jvp(x, v)
+    tangents = used() - u1
+    jtw = P.vjp(x, v)
+    P.close()
+    assert tangents > 200 << 20
+    with Filled(2 << 30) as memory:
+        memory.leave(need + (40 << 20))
+        G = sfx.System(lat, sysd)
+        assert np.array_equal(G.residual(x), f)
+        G.close()
+    G = sfx.System(lat, sysd)
+    assert np.abs(G.residual(x) - f).max() <= 1e-12 * np.abs(f).max()
+    with Filled(2 << 30) as memory:
+        memory.leave(tangents - (50 << 20))
+        assert np.array_equal(G.jvp(x, v), jv)
+        assert np.array_equal(G.residual(x), f)
+    assert np.array_equal(G.vjp(x, v), jtw)
