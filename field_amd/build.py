@@ -26,9 +26,7 @@ FLAGS = [
     "-fPIC",
     "-std=c++17",
     "-Wall",
-    "-Wno-unused-function",
-    "-Wno-unused-variable",
-    # packed FP32 instructions stay disabled (the hardware pool requires it)
+    # packed FP32 instructions stay disabled: some of their forms have given wrong results
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 

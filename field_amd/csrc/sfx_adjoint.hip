@@ -80,16 +80,6 @@ struct Tangent {
 };
 
 
-static __global__ void k_to_f32(const double* a, float* b, long long n) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = (float)a[i];
-}
-
-template <typename T>
-__device__ __forceinline__ T vdir(const DevLattice& L, const T* v, int x, int y, int z) {
-  return v[sidx(L, x, y, z)];
-}
-
 // rank 1: G = g, dG = -v g
 template <typename T>
 struct TInit {
@@ -625,7 +615,6 @@ static void tsweep(System& S, Tangent& W, int m, bool scaled, const T* vt, const
   auto bsc = [&](int step, int pair) { return scaled ? RankScale{maxb, lnb, lnf, scal + MS_REF, step, pair} : none; };
   const T* fin = nullptr;
   const T* dfin = nullptr;
-  double* dm = W.dmol.p;
   const ChainPlan& plan = mo.plan;
   if (mo.kind == 3) {
     const long long M6 = 6 * Mn;

@@ -45,7 +45,6 @@ struct Batch {
   hipStream_t stream = nullptr;
   // results of the last solve
   std::vector<BatchState> last;
-  int residual_launches = 0;
 
   ~Batch();
   void create(const sfx_adsorption_desc* d, int count, const sfx_options* opt);

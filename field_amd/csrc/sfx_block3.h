@@ -93,9 +93,6 @@ bool block2_ok(const DevLattice& L);
 
 // ev0/ev1 (optional): timing events the dispatch records at kernel start and end
 template <typename T>
-void launch_block3(const DevLattice& L, const B3Args<T>& a, bool tangent, bool scaled, bool connect,
-                   hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
-template <typename T>
 void launch_block3(const DevLattice& L, const B3Launch<T>& la, bool tangent, bool scaled, bool connect,
                    hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 
@@ -104,7 +101,7 @@ void launch_block2(const DevLattice& L, const B3Launch<T>& la, bool tangent, boo
                    hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 
 // max over the interior of each state's FP32 SWF, into step-max slots
-// gmax + t * kStepWords (zeroed here; read with get_step_max(.., 0))
+// gmax + t * kStepWords (zeroed here)
 // zeroed: gmax[0, ns * kStepWords) is already 0 on st (launch_swf can clear it)
 void launch_gmax(const DevLattice& L, const float* swf32, int ns, unsigned* gmax, hipStream_t st,
                  bool zeroed = false);

@@ -395,15 +395,6 @@ static void b3_launch_h(int nr, const DevLattice& L, const B3Launch<T>& a, hipSt
 }
 
 template <typename T>
-void launch_block3(const DevLattice& L, const B3Args<T>& a, bool tangent, bool scaled, bool connect,
-                   hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
-  B3Launch<T> la{};
-  la.a[0] = a;
-  la.nchains = 1;
-  launch_block3<T>(L, la, tangent, scaled, connect, st, ev0, ev1);
-}
-
-template <typename T>
 void launch_block3(const DevLattice& L, const B3Launch<T>& a, bool tangent, bool scaled, bool connect,
                    hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
   SFX_REQUIRE(a.nchains == 1 || a.nchains == 2, SFX_E_INVALID, "a blocked launch advances one or two chains");
@@ -465,10 +456,6 @@ void launch_gmax(const DevLattice& L, const float* swf32, int ns, unsigned* gmax
   SFX_HIP(hipGetLastError());
 }
 
-template void launch_block3<float>(const DevLattice&, const B3Args<float>&, bool, bool, bool, hipStream_t,
-                                   hipEvent_t, hipEvent_t);
-template void launch_block3<double>(const DevLattice&, const B3Args<double>&, bool, bool, bool, hipStream_t,
-                                    hipEvent_t, hipEvent_t);
 template void launch_block3<float>(const DevLattice&, const B3Launch<float>&, bool, bool, bool, hipStream_t,
                                    hipEvent_t, hipEvent_t);
 template void launch_block3<double>(const DevLattice&, const B3Launch<double>&, bool, bool, bool, hipStream_t,

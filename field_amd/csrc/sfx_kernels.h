@@ -55,14 +55,6 @@ __device__ __forceinline__ void block_step_max2(const unsigned* maxa, int sa, co
   mb = sh[1];
 }
 
-// called by every lane of a wave; all lanes get the maximum
-__device__ __forceinline__ float get_step_max(const unsigned* maxv, int step) {
-  const int lane = threadIdx.x & 63;
-  float v = lane < kMaxSlots ? __uint_as_float(maxv[(long long)step * kStepWords + lane * kSlotStride]) : 0.f;
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
-
 // A launch of several ranks divides by the lattice maximum of g alone, so its
 // ranks decay wherever the chain's weight is far from that maximum (an isolated
 // deep site, a block entering another's region), and the composition multiplies

@@ -26,6 +26,5 @@ void launch_init2f(const DevLattice& L, bool tangent, const T* g, const T* v, T*
 template <typename T>
 void launch_init2b(const DevLattice& L, bool tangent, const T* g, const T* v, T* G, T* dG, const T* Wp,
                    const T* dWp, T* acc, const RankScale& sc, hipStream_t st, T* bacc = nullptr);
-// per-block weighted sums over the six components of G (and dG)
 
 }  // namespace sfx

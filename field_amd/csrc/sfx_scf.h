@@ -67,28 +67,8 @@ __device__ __forceinline__ double phi_site(double acc, double g, double pref) {
 }
 
 // segment bulk fractions and ChemIntBulk (SF_MolStructure.cpp:605-612,
-// SF_SegmentList.cpp:610-623); one thread
-__device__ inline void bulk_fractions(const SysParams& sp, const double* molscal, double* phib_state, double* cbulk) {
-  for (int t = 0; t < sp.ns; t++) {
-    double pb = 0;
-    if (sp.melt)
-      pb = sp.melt_phib[t];
-    else if (!sp.frozen[t])
-      for (int m = 0; m < sp.nm; m++) pb += molscal[m * MS_COUNT + MS_PHIB] * sp.mol_frac[m * SFX_MAXS + t];
-    phib_state[t] = pb;
-  }
-  for (int t = 0; t < sp.ns; t++) {
-    double c = 0;
-    if (!sp.frozen[t])
-      for (int j = 0; j < sp.ns; j++) {
-        double x = sp.chi[t * SFX_MAXS + j];
-        if (x != 0) c += x * phib_state[j];
-      }
-    cbulk[t] = c;
-  }
-}
-
-// bulk_fractions by one wave, a lane per state; cb: ChemIntBulk in LDS as well
+// SF_SegmentList.cpp:610-623) by one wave, a lane per state; cb: ChemIntBulk in
+// LDS as well
 __device__ __forceinline__ void bulk_fractions_wave(const SysParams& sp, const double* molscal, double* phib_state,
                                                     double* cbulk, double* cb) {
   const int t = (int)threadIdx.x & 63;

@@ -136,13 +136,6 @@ void VecOps::wait_host(int count, double* host_out) {
   SFX_HIP(hipStreamSynchronize(stream));
   std::memcpy(host_out, hres, sizeof(double) * count);
 }
-void VecOps::fetch(const double* dsrc, int count, double* host_out) {
-  SFX_REQUIRE(count >= 0 && count <= kHostWords, SFX_E_INVALID, "too many words to read back");
-  if (count == 0) return;
-  SFX_HIP(hipMemcpyAsync(hres, dsrc, sizeof(double) * count, hipMemcpyDeviceToHost, stream));
-  SFX_HIP(hipStreamSynchronize(stream));
-  std::memcpy(host_out, hres, sizeof(double) * count);
-}
 void VecOps::dots(const DotList& dl, double* host_out) {
   if (dl.count <= 0) return;
   dots_dev(dl, dres, 0);

@@ -15,10 +15,6 @@
 
 namespace sfx {
 
-static __global__ void k_fill_u32(unsigned* p, unsigned v, long long n) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
 static __global__ void k_fill_bytes8(unsigned long long* p, long long n) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0ull;
