@@ -386,7 +386,7 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
     auto acc2p = [&](int t) { return base ? (T*)S.d_acc2 + ((size_t)m * S.ns + t) * Mn : nullptr; };
     T* qq[2] = {(T*)S.d_pp2, (T*)S.d_pp2 + Mn};  // backward running rank
     T* dqq[2] = {(T*)W.dpp2.p, (T*)W.dpp2.p + Mn};
-    // (the second accumulators were cleared with the first above)
+    // (the second accumulators were cleared with the first, by start_phi or above)
     auto rank_of = [&](int k) { return N - k + 1; };
     auto bstate = [&](int k) { return mo.seq[rank_of(k) - 1]; };
     const int tN = mo.seq[N - 1];

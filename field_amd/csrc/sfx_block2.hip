@@ -14,15 +14,17 @@
 // with them), behind a surface 0.
 //   G_k(r) = g(r) A[G_{k-1}](r)  (Lat2DFlat1stO.cpp:31-52, Lat2DCyl1stO.cpp:16-39)
 // Composition and tangents are those of sfx_block3.hip, and so is FP32 scaling
-// but that its divisors are powers of two.
+// but that its divisors are powers of two: of eight ranks, up to eight decay
+// between renormalisations (kLowMax).
 //
 // What bounds it: the ranks' dependent operations and barriers, and the
 // launch's loads and dispatch before them. At 64 x 128 a launch of eight ranks
 // takes 6.3 / 9.9 us (forward / composing, both chains) in FP64 and 9.2 / 12.3
-// us for an FP32 product; the N = 40 residual went from 376 to 154 us and the
-// product from 978 to 217 us. Why eight ranks: the widened tile
-// costs four times the tile's work, which the idle chip has to spare, and a
-// launch's fixed 4 us are paid an eighth as often.
+// us for an FP32 product; with it the N = 40 residual went from 376 to 154 us and
+// the product from 978 to 217 us (100 and 143 us since the launches around it were
+// fused). Why eight ranks: the widened tile costs four times the tile's work,
+// which the idle chip has to spare, and a launch's fixed 4 us are paid an eighth
+// as often.
 #include <hip/hip_ext.h>
 
 #include "sfx_block3.h"

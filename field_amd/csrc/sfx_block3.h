@@ -1,5 +1,5 @@
-// sfx_block3.h -- several propagator ranks per launch on the 3-D simple-cubic
-// lattice (temporal blocking through LDS tiles).
+// sfx_block3.h -- several propagator ranks per launch on 3-D simple-cubic and FCC
+// lattices and on 2-D ones (temporal blocking through LDS tiles).
 #pragma once
 
 #include <utility>
@@ -62,7 +62,8 @@ struct B3Launch {
 };
 
 // Splits chain steps a..b (ascending) into launches: a launch ends at a grid
-// line ((step - g0 + 1) % grid == 0), before a step of another segment state, or before a step that split() marks. f(first, last) per launch. The
+// line ((step - g0 + 1) % grid == 0), before a step of another segment state, or
+// before a step that split() marks. f(first, last) per launch. The
 // grid makes the partition of any stretch that starts on a grid line equal
 // to that of the whole chain, so a recomputed stretch reproduces it bit for bit.
 template <class State, class Split, class F>
@@ -85,7 +86,7 @@ std::vector<std::pair<int, int>> chain_launches(int a, int b, int g0, State stat
   return out;
 }
 
-// true when the blocked sweep applies: 3-D simple cubic, first order, every
+// true when the blocked sweep applies: 3-D simple cubic or FCC, first order, every
 // side at least kB3Ranks + 1 layers (one reflection reaches the interior)
 bool block3_ok(const DevLattice& L);
 // true when the blocked sweep of 2-D lattices applies: first order, its own adjoint

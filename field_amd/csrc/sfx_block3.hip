@@ -32,7 +32,8 @@
 //
 // FP32 scaling: the input is divided by max(rank s0) and every rank by the
 // lattice maximum of g, so no rank exceeds 1 and at most nr ranks decay
-// between renormalisations; the logs of the divisors go to lnv.
+// between renormalisations; the logs of the divisors go to lnv. Where a launch's
+// ranks decay too far, it says so (kLowMax).
 #include <hip/hip_ext.h>
 
 #include <algorithm>

@@ -61,18 +61,21 @@ void launch_chain1d(const DevLattice& L, const double* in0, const Chain1Step* st
 // ---------------------------------------------------------------------------
 // A whole evaluation of a 1-D system in one workgroup. It takes the place of
 // the 22 launches of a residual (2-22 us each, most of them at the launch
-// floor) and of the 150 to 300 of a product. 100 layers, A_100: 106 us of
-// kernels before, 24 us in this one (chain 9 us, molecule constants 4 us, the
-// residual's logs 3 us, the rest latencies), 133 -> 57 us a call; a product of
-// 237 layers and 151 segments 600 us before, 42 us now, 709 -> 85 us a call.
+// floor) and of the 150 to 300 of a product. 100 layers, A_100: 20 us of
+// dependent steps (chain 9 us, molecule constants 4 us, the residual's logs 3
+// us, the rest latencies) instead of 106 us of kernels, 136 -> 38 us a call; a
+// product of 237 layers and 151 segments about 40 us instead of 600, 720 -> 58
+// us a call. Four layers a lane (897 to 1024 layers) with tangents spill 107
+// registers (flat; 164 curved), two 6 (15): a product of 1000 layers takes 160
+// us all the same, 756 by launches.
 // Larger lattices (1025 to 4000 layers), lattices of at most kChain1Halo layers
 // and systems whose arrays do not fit LDS keep the launches (k_chain1d).
 // ---------------------------------------------------------------------------
 constexpr int kScf1Waves = 8, kScf1Threads = 64 * kScf1Waves;
 constexpr int kScf1Lds = 156 * 1024;  // of 160 KB, the static words beside it
 
-// every lambda of the sweep is inlined: one that is not would put the ring of
-// partner rows into memory
+// every lambda of the sweep is inlined: one that is not would put the whole ring
+// of partner rows into memory
 #define SFX_INLINE __attribute__((always_inline))
 
 // words of LDS per layer of a system with ns states
@@ -302,8 +305,9 @@ __device__ double2 scf1_layer_sums(int n, Val&& val, Dval&& dval, double* wsum) 
 // The residual (u -> SWF -> propagators -> phi -> f), or with TAN the product
 // J v (A.base: with phi and the contact averages on the way; otherwise at those
 // of the last evaluation), of a 1-D first-order system in FP64: the launches of a
-// residual or a product in one workgroup, same bits. SWF, accumulators and profiles are in LDS, indexed by layer with W
-// words per state; the first wave sweeps the chains.
+// residual or a product in one workgroup; a residual's bits are the launches'.
+// SWF, accumulators and profiles are in LDS, indexed by layer with W words per
+// state; every wave sweeps its layers of the chains.
 template <int K, bool CURVED, bool TAN>
 __global__ void __launch_bounds__(kScf1Threads) k_scf1d(DevLattice L, Scf1Args A) {
   extern __shared__ double lds[];

@@ -147,9 +147,10 @@ struct Chain1 {
 #pragma unroll
     for (int j = 0; j < K; j++) G[j] = g[j] * A[j];
   }
-  // the owned layers to a rank's row in the store, and a partner's from it (a
-  // lane without one reads what nobody wants). No lane is masked off: that
-  // costs more than the rank's arithmetic
+  // the owned layers to a rank's row in the store, and a partner's from it. No
+  // lane is masked off (that costs more than the rank's arithmetic): lanes
+  // without a layer all use the row's last word, the upper halo, so no kernel
+  // may read that word of a 1-D store
   static __device__ __forceinline__ double& at(double* row, int i) {
     return *(double*)((char*)row + (unsigned)(i * 8));
   }

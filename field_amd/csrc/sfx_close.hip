@@ -5,9 +5,9 @@
 // As a launch per molecule and quantity this was 11 to 15 launches, 40 us or
 // more on any lattice. Every launch costs 2.5 us of dispatch and drain whatever
 // it does, and a profile written by one is read again by the next. Together
-// they take 18 us now on the 64 x 128 pore (a residual 154 -> 130 us, a product
-// 217 -> 178), 34 us for a product at 64^3 (327 -> 300 us) and 103 us at 128^3,
-// where 70 are the profiles' traffic (139 us before).
+// they take 18 us on the 64 x 128 pore (with them a residual went from 154 to 130
+// us, a product from 217 to 178), 34 us for a product at 64^3 (327 to 300 us) and
+// 103 us at 128^3, where 70 are the profiles' traffic (139 us before).
 //   k_end_sums    every molecule's end sum; the workgroup that finishes last
 //                 adds the partial sums in a fixed order and derives the
 //                 scalars, which were a launch of one workgroup each

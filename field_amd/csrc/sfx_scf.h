@@ -1,7 +1,8 @@
 // sfx_scf.h -- the arithmetic of one site, one molecule and one system, shared
 // by the kernels that run it launch by launch over a whole lattice and by the
-// one that runs a 1-D system in a single workgroup (sfx_chain1d.hip): both
-// give the same bits.
+// one that runs a 1-D system in a single workgroup (sfx_chain1d.hip): both give
+// the same bits, but for a product's last operations, which the compiler fuses
+// in each as it finds them.
 #pragma once
 
 #include "sfx_device.h"

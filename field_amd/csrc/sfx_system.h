@@ -150,7 +150,7 @@ struct System {
   int maxN = 1, maxstore = 1;
   int store_slots = 1;     // rank slots of the propagator store (all molecules share it)
   bool checkpointed = false;
-  bool use_block3 = false;  // blocked sweeps of 3-D simple-cubic and 2-D lattices (sfx_options.sweep_kernel)
+  bool use_block3 = false;  // blocked sweeps of 3-D simple-cubic, FCC and 2-D lattices (sfx_options.sweep_kernel)
   // 2-D and FCC lattices, swept rank by rank where their second accumulators do
   // not fit: gives these (and the tangents') back; false if there is nothing to give
   bool drop_blocked();

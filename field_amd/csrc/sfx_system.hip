@@ -351,7 +351,8 @@ void System::create(const sfx_lattice_desc& ld, const sfx_system_desc& sd, const
     SFX_HIP(hipMemcpy(d_sites, sites.data(), sites.size() * sizeof(long long), hipMemcpyHostToDevice));
   if (d_order)
     k_order<<<grid1(Mn, 256), 256, 0, stream>>>(d_itmask, d_sites, (long long)sites.size(), Mn, d_order);
-  // zero everything once: halo slots of propagator arrays are never written
+  // zero everything once: halo slots of propagator arrays are never written, but
+  // for the upper one of a 1-D store's rows (Chain1::put), and never read
   zero_bytes(d_store, (size_t)store_slots * comps * M * 8, stream);
   zero_bytes(d_pp, 2 * comps * M * 8, stream);
   if (d_pp2) zero_bytes(d_pp2, 2 * M * 8, stream);
@@ -641,9 +642,9 @@ void System::sweep(int m, bool scaled) {
   add_end(m, final_G, nullptr, sizeof(T) == 4, lnfinal);
 }
 
-// The sweep of sweep() for a first-order chain (full or half store) on the
-// 3-D simple-cubic lattice, several ranks per launch (sfx_block3.hip). The
-// accumulators and the scale maxima have been cleared by start_phi().
+// The sweep of sweep() for a first-order chain (full or half store) on a
+// simple-cubic, FCC or 2-D lattice, several ranks per launch (sfx_block3.hip,
+// sfx_block2.hip). The accumulators and the scale maxima have been cleared by start_phi().
 template <typename T>
 void System::sweep_blocked(int m, bool scaled) {
   const DevLattice& L = lat.d;
@@ -726,7 +727,7 @@ void System::sweep_blocked(int m, bool scaled) {
     T* acc2 = (T*)d_acc2;
     auto acc2p = [&](int t) { return acc2 + ((size_t)m * ns + t) * Mn; };
     T* qq[2] = {(T*)d_pp2, (T*)d_pp2 + Mn};
-    // (the second accumulators were cleared with the first by sweep())
+    // (start_phi cleared the second accumulators with the first)
     auto rank_of = [&](int k) { return N - k + 1; };  // backward step k holds rank N-k+1
     auto bstate = [&](int k) { return mo.seq[rank_of(k) - 1]; };
     launch_init_rank2<T>(L, InitRank<T>{gp(mo.seq[0]), slot(0), fsc(1, 0)},

@@ -65,6 +65,18 @@ def test_deep_site(sfx, lattice, chain, depth):
 
 
 @pytest.mark.parametrize("chain", CHAINS)
+@pytest.mark.parametrize("options", [dict(chain_schedule="sequential"), dict(memory_budget=20 * 8 * LATTICES["sc"].M)],
+                         ids=["sequential", "checkpointed"])
+def test_other_schedules(sfx, chain, options):
+    lat, sysd = system("sc", chain)
+    G, P = sfx.System(lat, sysd, **options), sfx.System(lat, sysd, sweep_kernel="per_rank")
+    x, w = fields(lat, sysd, 24)
+    assert np.array_equal(G.residual(x, precision="fp32"), P.residual(x, precision="fp32"))
+    assert np.array_equal(G.jvp(x, w, precision="fp32"), P.jvp(x, w, precision="fp32"))
+    assert np.array_equal(G.vjp(x, w, precision="fp32"), P.vjp(x, w, precision="fp32"))
+
+
+@pytest.mark.parametrize("chain", CHAINS)
 def test_results_over_the_inputs(sfx, chain):
     """A repeated evaluation takes its inputs from where the first pass has not written."""
     lat, sysd = system("2d", chain)
