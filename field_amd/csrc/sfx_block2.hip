@@ -40,11 +40,12 @@ constexpr int kB2Threads = 64 * kB2Waves;
 static_assert(kB2H % kB2Rows == 0 && kB2X % kB2Rows == 0, "a wave's rows are all owned or none");
 
 bool block2_ok(const DevLattice& L) {
-  // a curved lattice with a mirror2 side: its sweep is not its own adjoint, so
-  // the two chains of a middle-out sweep would not agree
-  bool mirror2 = false;
-  for (int k = 0; k < 2; k++) mirror2 |= L.mirror2_1[k] || L.mirror2_2[k];
-  return L.grad == 2 && L.order == 1 && !(L.curved && mirror2);
+  // a curved lattice with a mirror2 side or radial wrap-around (layers of
+  // different volumes exchange through one weight each): its sweep is not its own
+  // adjoint, so the two chains of a middle-out sweep would not agree
+  bool adjoint = !L.periodic[0];
+  for (int k = 0; k < 2; k++) adjoint &= !L.mirror2_1[k] && !L.mirror2_2[k];
+  return L.grad == 2 && L.order == 1 && (!L.curved || adjoint);
 }
 
 // The factor 2^-e that a step maximum m stands for, 2^(e-1) <= m < 2^e, and

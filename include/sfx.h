@@ -134,7 +134,7 @@ typedef struct sfx_options {
                              BLOCKED also advance first-order FCC sweeps by four and
                              2-D sweeps by eight ranks per launch (fully stored,
                              chain_schedule AUTO, a curved lattice without mirror2
-                             sides; rank by rank where device memory has no room
+                             or radially periodic sides; rank by rank where device memory has no room
                              for their second accumulators), and run
                              a 1-D first-order FP64 evaluation in one workgroup
                              launch, or above 1024 layers each stretch of a chain's
