@@ -877,7 +877,7 @@ void jvp_abi(System& S, const double* x, const double* v, double* jv, int precis
 
 // true where the backward sweep is the forward sweep's adjoint in D. Not so:
 // the 2-D cylinder's second-order sweep (its outward step is not split, as in
-// the reference); a curved lattice with a mirror2 side; a 1-D flat lattice
+// the reference); a curved lattice with a mirror2 or radially periodic side; a 1-D flat lattice
 // with a layer adjustment other than 1; a mirror on a HEX lattice (its
 // neighbour set is not symmetric under reflection, so the mirrored stencil is
 // not); a second-order 1-D or 2-D lattice with a mirror2 lower bound (the
@@ -885,6 +885,7 @@ void jvp_abi(System& S, const double* x, const double* v, double* jv, int precis
 bool vjp_supported(const System& S) {
   const DevLattice& L = S.lat.d;
   if (L.curved) {
+    if (L.periodic[0]) return false;
     for (int k = 0; k < L.grad; k++)
       if (L.mirror2_1[k] || L.mirror2_2[k]) return false;
     if (L.grad == 2 && L.order == 2) return false;
@@ -1148,7 +1149,7 @@ void vjp_at_base(System& S, const double* w, double* jtw, int precision) {
   require_products(S);
   SFX_REQUIRE(vjp_supported(S), SFX_E_UNSUPPORTED,
               "transposed products need a backward sweep that is the forward sweep's adjoint: not on a curved "
-              "lattice with a mirror2 side, the second-order 2-D cylinder, a layer adjustment other than 1, a "
+              "lattice with a mirror2 or radially periodic side, the second-order 2-D cylinder, a layer adjustment other than 1, a "
               "mirror on a HEX lattice or a second-order 1-D/2-D mirror2 lower bound");
   Tangent& W = tangent(S);
   if (!W.vjp_ready) W.init_vjp(S);

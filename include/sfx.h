@@ -198,7 +198,8 @@ int sfx_jvp(sfx_system* s, const double* x, const double* v, double* jv, int whe
  * of its partition function wherever the backward sweep is the forward sweep's
  * adjoint in the site-volume inner product, so the transposed sweep is the
  * tangent sweep with a rescaled direction. SFX_E_UNSUPPORTED where that does
- * not hold: a curved lattice with a mirror2 side, the second-order 2-D
+ * not hold: a curved lattice with a mirror2 or radially
+ * periodic side, the second-order 2-D
  * cylinder (the reference's backward sweep does not split its outward step,
  * Lat2DCyl2ndO.cpp:223-227), a 1-D flat layer adjustment other than 1, a
  * mirror side on a HEX lattice (its neighbour set is not reflection
