@@ -267,7 +267,10 @@ __device__ __forceinline__ double side_at2(const DevLattice& L, const double* __
   const double b = P[sidx(L, x, y, 0)], l1 = L.l1;
   auto lam0 = [&](int X) { return 1 - 2 * l1 - L.lp[X] - L.lm[X]; };
   if (x == 0 || x == L.nx + 1) {
-    double a = at(x, y - 1), c = at(x, y + 1);
+    // where two surfaces meet only the two neighbours on the lattice count
+    // (Lat2DFlat.cpp:996-1010, Lat2DCylinder.cpp:205-220); there is nothing
+    // behind the corner to read
+    double a = y > 0 ? at(x, y - 1) : 0.0, c = y <= L.ny ? at(x, y + 1) : 0.0;
     double in = x == 0 ? P[sidx(L, 1, y, 0)] : P[sidx(L, L.nx, y, 0)];
     if (L.curved) return lam0(x) * b + l1 * (a + c) + (x == 0 ? L.lp[0] : L.lm[x]) * in;
     return L.l0_2d * b + L.l1y * (a + c) + L.l1x * in;
