@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(kTB) k_tprop(DevLattice L, const T* __restrict
     float mprev, unused;
     block_step_max2(sc.maxv, sc.step - 1, nullptr, 0, mprev, unused);
     if (!(mprev > 0.f)) mprev = 1.f;
-    lncum = l0 + log((double)mprev);
+    lncum = l0 + log((double)(sc.prev_blocked ? mprev * kBlockDown : mprev));
     scale = (T)(1.f / mprev);
     if constexpr (CONNECT) cfac = (T)exp(lncum + lp - rf);
   }
@@ -210,7 +210,7 @@ __global__ void k_tconnect(DevLattice L, const T* __restrict__ A, const T* __res
   long long q = site_ordinal();
   if (q >= L.V) return;
   T c = T(half);
-  if constexpr (SCALED) c = (T)(half * exp(sc.lnv[sc.step] + sc.lnpair[sc.pair] - *sc.ref));
+  if constexpr (SCALED) c = (T)connect_factor(sc, half);
   int x, y, z;
   interior_coords(L, q, x, y, z);
   long long r = sidx(L, x, y, z);
@@ -261,7 +261,10 @@ static void tprop(const DevLattice& L, const T* Gin, const T* dGin, const T* g, 
 }
 
 static __global__ void k_set_ref2(double* scal, const double* lnv, int idx, double factor) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) scal[MS_REF] = factor * lnv[idx];
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    scal[MS_REF] = factor * lnv[idx];
+    scal[MS_POW] = 0.0;
+  }
 }
 
 // the tangent accumulators of molecule m
@@ -327,6 +330,15 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
   RankScale none{nullptr, nullptr, nullptr, nullptr, 0, 0};
   auto fsc = [&](int step, int pair) { return scaled ? RankScale{maxf, lnf, lnf, scal + MS_REF, step, pair} : none; };
   auto bsc = [&](int step, int pair) { return scaled ? RankScale{maxb, lnb, lnf, scal + MS_REF, step, pair} : none; };
+  // launches of one rank between blocked ones: what they read carries kBlockScale
+  auto carried = [&](RankScale sc, int carry) {
+    if (scaled) {
+      sc.prev_blocked = mo.blocked_rank(sc.step - 1);
+      sc.pow = scal + MS_POW;
+      sc.carry = carry;
+    }
+    return sc;
+  };
   auto state_of_rank = [&](int s) { return mo.seq[s - 1]; };
   auto nosplit = [](int) { return false; };
   // the arguments of ranks sa..sb of a chain from (in, din); with an
@@ -358,7 +370,8 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
       a.lnpair = lnpair;
       a.ref = scal + MS_REF;
       a.gmax = S.d_gmax + (size_t)t * kStepWords;
-      a.low = mo.blocked_rank(sa - 1) ? S.low_word() : nullptr;
+      a.low = S.low_word();
+      a.carried = mo.blocked_rank(sa - 1);
     }
     a.s0 = sa - 1;
     return a;
@@ -421,7 +434,7 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
       }
       go(la, false);
     }
-    if (scaled) launch_set_ref_pair(scal, lnf, h, lnb, N - h, st);
+    if (scaled) launch_set_ref_block(scal, maxf, lnf, h, maxb, lnb, N - h, st);
     const auto F2 = chain_launches(h + 1, N, h + 1, state_of_rank, grid);
     const auto B2 = chain_launches(N - h + 1, N, N - h + 1, bstate, grid);
     int fc = 0, bc = 0;
@@ -515,12 +528,12 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
   const T* fin = nullptr;
   const T* dfin = nullptr;
   if (mo.kind == 1) {
-    if (scaled) k_set_ref2<<<1, 1, 0, st>>>(scal, lnf, N, 1.0);
+    if (scaled) launch_set_ref_block(scal, maxf, lnf, N, nullptr, nullptr, 0, st);
     const int tN = mo.seq[N - 1];
     tinit<T>(L, gp(tN), vp(tN), pp[0], dpp[0], bsc(1, N), st);
     const int iN = get(N);
     k_tconnect<T, sizeof(T) == 4><<<grid1(L.V, kTB), kTB, 0, st>>>(L, pp[0], dpp[0], slot(iN), dslot(iN), daccp(tN),
-                                                             accp(tN), bsc(1, N), 1.0);
+                                                             accp(tN), carried(bsc(1, N), 1), 1.0);
     auto rank_of = [&](int k) { return N - k + 1; };
     chain_blocks(
         2, N, 2, [&](int k) { return mo.seq[rank_of(k) - 1]; },
@@ -540,7 +553,7 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
         }, grid);
   } else {
     const int h = N / 2;
-    if (scaled) k_set_ref2<<<1, 1, 0, st>>>(scal, lnf, h, 2.0);
+    if (scaled) launch_set_ref_block(scal, maxf, lnf, h, maxf, lnf, h, st);
     int from = get(h);  // a stored rank; in a checkpoint segment, which is overwritten, copied
     bool in_pp = plan.c;
     if (in_pp) {
@@ -550,11 +563,11 @@ static void tsweep_blocked(System& S, Tangent& W, int m, bool scaled, const T* v
     }
     if (N % 2 == 1) {
       const int s = h + 1, t = mo.seq[s - 1];
-      tprop<T>(L, in_pp ? pp[0] : slot(from), in_pp ? dpp[0] : dslot(from), gp(t), vp(t), pp[1], dpp[1], nullptr, nullptr, nullptr, nullptr, fsc(s, 0),
+      tprop<T>(L, in_pp ? pp[0] : slot(from), in_pp ? dpp[0] : dslot(from), gp(t), vp(t), pp[1], dpp[1], nullptr, nullptr, nullptr, nullptr, carried(fsc(s, 0), 0),
                    st);
       cur = 1;
       k_tconnect<T, sizeof(T) == 4><<<grid1(L.V, kTB), kTB, 0, st>>>(L, pp[cur], dpp[cur], pp[cur], dpp[cur], daccp(t),
-                                                               accp(t), fsc(s, s), 0.5);
+                                                               accp(t), carried(fsc(s, s), 0), 0.5);
       from = cur;
       in_pp = true;
     }

@@ -110,6 +110,7 @@ __global__ void __launch_bounds__(kB2Threads) k_block2(DevLattice L, B3Launch<T>
   // the maxima and logs of earlier launches first (sfx_block3.hip)
   float ma = 0.f, mb = 0.f;
   double lnv0 = 0.0, lnp = 0.0, lref = 0.0;
+  int power = 0;  // of this lane's composition factor
   if constexpr (SCALED) {
     if (wave == 0) {
       ma = __uint_as_float(a.maxv[(long long)a.s0 * kStepWords + lane * kSlotStride]);
@@ -122,6 +123,7 @@ __global__ void __launch_bounds__(kB2Threads) k_block2(DevLattice L, B3Launch<T>
           if (lane == k) pi = a.pidx[k];
         if (lane < nr) lnp = a.lnpair[pi];
         lref = *a.ref;
+        power = (int)a.ref[MS_POW - MS_REF] - kBlockPower * (pi >= 2 ? 2 : 1);
       }
     }
   }
@@ -168,17 +170,18 @@ __global__ void __launch_bounds__(kB2Threads) k_block2(DevLattice L, B3Launch<T>
         ma = fmaxf(ma, __shfl_xor(ma, o, 64));
         mb = fmaxf(mb, __shfl_xor(mb, o, 64));
       }
-      if (lane == 0 && bl == 0 && a.low && !(ma >= kLowMax)) *a.low = 1u;
+      if (a.carried) ma *= kBlockDown;
+      if (lane == 0 && bl == 0 && low_input(ma, a.carried)) *a.low = 1u;
       double lna;
       const float sa = pow2_scale(ma, lna), sb = pow2_scale(mb, lng);
       if (lane == 0) {
-        scl[0] = sa;
+        scl[0] = sa * (a.carried ? 1.f : kBlockScale);
         scl[1] = sb;
       }
       if (CONNECT || bl == 0) {
         ln_base = lnv0 + lna;
         if constexpr (CONNECT) {
-          const double cf = lane < nr ? exp(ln_base + (lane + 1) * lng + lnp - lref) : 1.0;
+          const double cf = lane < nr ? ldexp(exp(ln_base + (lane + 1) * lng + lnp - lref), power) : 1.0;
           if (lane < kB2Ranks) cfac[lane] = (T)cf;
         }
       }

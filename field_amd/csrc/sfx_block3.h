@@ -47,7 +47,8 @@ struct B3Args {
   const double* lnpair;
   const double* ref;
   const unsigned* gmax;        // step-max slots of the state's lattice maximum of g
-  unsigned* low;               // set when max(rank s0) is below kLowMax (null: rank s0 is not of a blocked launch)
+  unsigned* low;               // set when rank s0 has decayed too far (low_input)
+  bool carried;                // rank s0 carries kBlockScale: it comes out of a blocked launch
   int s0;
   int pidx[kBRanks];
 };

@@ -32,8 +32,9 @@
 //
 // FP32 scaling: the input is divided by max(rank s0) and every rank by the
 // lattice maximum of g, so no rank exceeds 1 and at most nr ranks decay
-// between renormalisations; the logs of the divisors go to lnv. Where a launch's
-// ranks decay too far, it says so (kLowMax).
+// between renormalisations; the logs of the divisors go to lnv. Stored ranks and
+// maxima carry a factor 2^32, and a launch whose ranks decay too far says so
+// (kLowMax).
 #include <hip/hip_ext.h>
 
 #include <algorithm>
@@ -118,6 +119,7 @@ __global__ void __launch_bounds__((B3Region<H, KIND, TX>::threads)) k_block3(Dev
   // arrive before the region and are worked on while it is in flight
   float ma = 0.f, mb = 0.f;
   double lnv0 = 0.0, lnp = 0.0, lref = 0.0;
+  int power = 0;  // of this lane's composition factor
   if constexpr (SCALED) {
     if (t < 64) {
       ma = __uint_as_float(a.maxv[(long long)a.s0 * kStepWords + lane * kSlotStride]);
@@ -130,6 +132,7 @@ __global__ void __launch_bounds__((B3Region<H, KIND, TX>::threads)) k_block3(Dev
           if (lane == k) pi = a.pidx[k];
         if (lane < nr) lnp = a.lnpair[pi];
         lref = *a.ref;
+        power = (int)a.ref[MS_POW - MS_REF] - kBlockPower * (pi >= 2 ? 2 : 1);
       }
     }
   }
@@ -194,11 +197,12 @@ __global__ void __launch_bounds__((B3Region<H, KIND, TX>::threads)) k_block3(Dev
         ma = fmaxf(ma, __shfl_xor(ma, o, 64));
         mb = fmaxf(mb, __shfl_xor(mb, o, 64));
       }
-      if (lane == 0 && bl == 0 && a.low && !(ma >= kLowMax)) *a.low = 1u;
+      if (a.carried) ma *= kBlockDown;
+      if (lane == 0 && bl == 0 && low_input(ma, a.carried)) *a.low = 1u;
       if (!(ma > 0.f)) ma = 1.f;
       if (!(mb > 0.f)) mb = 1.f;
       if (lane == 0) {
-        scl[0] = 1.f / ma;
+        scl[0] = 1.f / ma * (a.carried ? 1.f : kBlockScale);
         scl[1] = 1.f / mb;
       }
       if (CONNECT || bl == 0) {
@@ -206,7 +210,7 @@ __global__ void __launch_bounds__((B3Region<H, KIND, TX>::threads)) k_block3(Dev
         ln_base = lnv0 + __shfl(lv, 0, 64);
         lng = __shfl(lv, 1, 64);
         if constexpr (CONNECT) {
-          const double cf = lane < nr ? exp(ln_base + (lane + 1) * lng + lnp - lref) : 1.0;
+          const double cf = lane < nr ? ldexp(exp(ln_base + (lane + 1) * lng + lnp - lref), power) : 1.0;
           if (lane < kB3Ranks) cfac[lane] = (T)cf;
         }
       }

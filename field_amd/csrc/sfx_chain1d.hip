@@ -326,7 +326,7 @@ __global__ void __launch_bounds__(kScf1Threads) k_scf1d(DevLattice L, Scf1Args A
   for (int i = tid; i < scf1_words(ns, TAN) * W; i += kScf1Threads) lds[i] = 0.0;
   RunWalk walk;
   walk.init(A.runs, A.nruns);
-  if (!base && tid < sp.nm * MS_COUNT) ms[tid] = tid % MS_COUNT == MS_REF ? 0.0 : A.molscal[tid];
+  if (!base && tid < sp.nm * MS_COUNT) ms[tid] = tid % MS_COUNT == MS_REF || tid % MS_COUNT == MS_POW ? 0.0 : A.molscal[tid];
   __syncthreads();
   if (A.u)
     for (int q = tid; q < sp.n_itvar * M; q += kScf1Threads) A.u[q] = site_get(A.x, M, q / M, q % M);
@@ -379,8 +379,8 @@ __global__ void __launch_bounds__(kScf1Threads) k_scf1d(DevLattice L, Scf1Args A
         wsum);
     if (base) {
       if (tid == 0) {
-        mscal[MS_REF] = 0.0;
-        mol_scalars(mp, sums.x, 0.0, 0.0, sp.nm, [&](int m) { return ms[m * MS_COUNT + MS_PHIB]; }, mscal);
+        mscal[MS_REF] = mscal[MS_POW] = 0.0;
+        mol_scalars(mp, sums.x, 0.0, 0.0, 0, sp.nm, [&](int m) { return ms[m * MS_COUNT + MS_PHIB]; }, mscal);
       }
       __syncthreads();
       const double pref = mscal[MS_PREF];

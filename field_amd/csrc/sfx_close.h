@@ -17,7 +17,8 @@ struct EndMol {
   const double* lnf;  // FP32: log scale of the end rank; nullptr: unscaled, MS_REF becomes 0
   bool f32, unscaled;
   // FP32 by blocked launches: step maxima of the chains' last ranks that no
-  // launch reads, and the word set when one is below kLowMax (null: no check)
+  // launch reads, and the word set when one is below kLowMax (null: not by blocked
+  // launches; with it G and the maxima carry kBlockScale)
   const unsigned* endmax[2];
   unsigned* low;
 };

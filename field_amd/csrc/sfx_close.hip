@@ -79,7 +79,10 @@ __global__ void __launch_bounds__(NT) k_end_sums(DevLattice L, EndArgs a) {
     mp = m.mp;
     if (m.lnf) lnf = *m.lnf;
     const double* const old = a.molscal + mp.index * MS_COUNT;
-    if (!m.unscaled) sc[MS_REF] = old[MS_REF];
+    if (!m.unscaled) {
+      sc[MS_REF] = old[MS_REF];
+      sc[MS_POW] = old[MS_POW];
+    }
     if (!a.base) {
       sc[MS_LNGN] = old[MS_LNGN];
       sc[MS_PHIB] = old[MS_PHIB];
@@ -89,7 +92,7 @@ __global__ void __launch_bounds__(NT) k_end_sums(DevLattice L, EndArgs a) {
     ph[t] = a.molscal[t * MS_COUNT + MS_PHIB];
     if constexpr (TAN) dph[t] = a.dmol[t * 4 + 2];
   }
-  float em[2] = {1.f, 1.f};
+  float em[2] = {kBlockScale, kBlockScale};
   const bool check = e.low && blockIdx.x == 0 && wave == 0;
   if (check)
     for (int k = 0; k < 2; k++)
@@ -108,7 +111,7 @@ __global__ void __launch_bounds__(NT) k_end_sums(DevLattice L, EndArgs a) {
       em[0] = fmaxf(em[0], __shfl_xor(em[0], o, 64));
       em[1] = fmaxf(em[1], __shfl_xor(em[1], o, 64));
     }
-    if (lane == 0 && !(fminf(em[0], em[1]) >= kLowMax)) *e.low = 1u;
+    if (lane == 0 && !(fminf(em[0], em[1]) * kBlockDown >= kLowMax)) *e.low = 1u;
   }
   if (lane == 0) {
     r1[wave] = s;
@@ -155,7 +158,7 @@ __global__ void __launch_bounds__(NT) k_end_sums(DevLattice L, EndArgs a) {
   for (int pass = 0; pass < 2; pass++) {
     if (t < a.n && (mp.freedom == SFX_SOLVENT) == (pass == 1)) {
       if (a.base) {
-        mol_scalars(mp, s1[t], lnf, sc[MS_REF], a.nm, [&](int o) { return ph[o]; }, sc);
+        mol_scalars(mp, a.e[t].low ? s1[t] * kBlockDown : s1[t], lnf, sc[MS_REF], (int)sc[MS_POW], a.nm, [&](int o) { return ph[o]; }, sc);
         ph[mp.index] = sc[MS_PHIB];
         out[MS_LNGN] = sc[MS_LNGN];
         out[MS_LNC] = sc[MS_LNC];
@@ -163,6 +166,7 @@ __global__ void __launch_bounds__(NT) k_end_sums(DevLattice L, EndArgs a) {
         out[MS_PREF] = sc[MS_PREF];
       }
       out[MS_REF] = sc[MS_REF];
+      out[MS_POW] = sc[MS_POW];
       if constexpr (TAN) {
         double d[4];
         tmol_scalars(mp, true, s1[t], s2[t], sc, a.nm, [&](int o) { return dph[o]; }, d);

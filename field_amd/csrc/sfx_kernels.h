@@ -9,7 +9,7 @@
 namespace sfx {
 
 // per-molecule device scalars
-enum { MS_LNGN = 0, MS_LNC, MS_PHIB, MS_PREF, MS_REF, MS_RANGE_C, MS_COUNT = 8 };
+enum { MS_LNGN = 0, MS_LNC, MS_PHIB, MS_PREF, MS_REF, MS_RANGE_C, MS_POW, MS_COUNT = 8 };
 
 // FP32 per-rank log-scaling context of one sweep. Step k writes max|G| of its
 // output into maxv[k] and the cumulative log scale into lnv[k]; its output is
@@ -57,13 +57,24 @@ __device__ __forceinline__ void block_step_max2(const unsigned* maxa, int sa, co
 
 // A launch of several ranks divides by the lattice maximum of g alone, so its
 // ranks decay wherever the chain's weight is far from that maximum (an isolated
-// deep site, a block entering another's region), and the composition multiplies
-// a rank of either chain before their logs make up for it. Below this maximum of
-// a launch's last rank (22 kT lost within it) the evaluation is repeated rank by
-// rank. A composed product of two such ranks is still 2^62 above FP32's smallest
-// normal number; unchecked, transposed products lost digits from a decay of
-// 2^-60 on and sums of 2^-127 became log(0).
-constexpr float kLowMax = 0x1p-32f;
+// deep site, a block entering another's region, strong noise). Its ranks carry a
+// factor kBlockScale = 2^32 (their values and maxima; lnv is the log without it),
+// and where a launch's last rank has fallen below kLowMax = 2^-24 of its input (17
+// kT) the evaluation is repeated rank by rank. The accumulators carry 2^MS_POW,
+// which puts the ranks that the reference log is taken from at 2^kAccPower. So
+// every rank, composed product and accumulator has at least the range above FP32's
+// smallest numbers that the per-rank kernels leave it, whose ranks are at most g's
+// maximum (up to exp(5.5)). With a maximum of 1 and no check, transposed products
+// lost digits from a loss of 2^-60 on, sums of 2^-127 became log(0), and a profile
+// fixed by its amount in a box far from the chain's weight came out 0. Powers of
+// two round nothing: a field without such decays gives the bits it gave without.
+constexpr int kBlockPower = 32, kAccPower = 32;
+constexpr float kBlockScale = 0x1p32f, kBlockDown = 0x1p-32f;
+constexpr float kLowMax = 0x1p-24f;
+// a launch's input of maximum m (without kBlockScale) has decayed too far; or, if it
+// is a first rank, which does not carry the factor yet, kBlockScale / m may be no
+// number (a field of 62 kT everywhere)
+__host__ __device__ constexpr bool low_input(float m, bool carried) { return !(m >= (carried ? kLowMax : 0x1p-90f)); }
 
 struct RankScale {
   unsigned* maxv;
@@ -72,8 +83,20 @@ struct RankScale {
   const double* ref;
   int step;
   int pair;
-  const unsigned* pmaxv;  // step maxima of the partner chain (second order recovers its rank)
+  const unsigned* pmaxv = nullptr;  // step maxima of the partner chain (second order recovers its rank)
+  // beside blocked launches: rank step - 1 carries kBlockScale; a composition in
+  // their accumulators (MS_POW), of `carry` ranks that carry it
+  bool prev_blocked = false;
+  const double* pow = nullptr;
+  int carry = 0;
 };
+
+#ifdef __HIPCC__
+__device__ __forceinline__ double connect_factor(const RankScale& sc, double half) {
+  const double c = half * exp(sc.lnv[sc.step] + sc.lnpair[sc.pair] - *sc.ref);
+  return sc.pow ? ldexp(c, (int)*sc.pow - kBlockPower * sc.carry) : c;
+}
+#endif
 
 struct MolParams {
   int index, N, freedom, kind;  // kind: 0 monomer, 1 full sweep, 2 half-stored (palindrome), 3 second order
@@ -166,9 +189,11 @@ void launch_mol_phi(const DevLattice& L, const A* acc, const double* g, const do
 template <typename A>
 void launch_mol_phi_states(const DevLattice& L, unsigned uses, int ns, const A* acc, const A* acc2, const double* g,
                            const double* scal, double* phi_m, hipStream_t st);
-// scal[MS_REF] = lna[ia] + lnb[ib] (0 when lna is null): the reference log of
-// a middle-out sweep's compositions
-void launch_set_ref_pair(double* scal, const double* lna, int ia, const double* lnb, int ib, hipStream_t st);
+// scal[MS_REF], scal[MS_POW] = the reference log of a blocked sweep's compositions
+// and their accumulators' power of two, from the logs and maxima of the ranks that
+// the chains' first halves end with (lnb null: of one)
+void launch_set_ref_block(double* scal, const unsigned* maxa, const double* lna, int ia, const unsigned* maxb,
+                          const double* lnb, int ib, hipStream_t st);
 // The SWF of every state, and what else a sweep needs beside it: x's copy in
 // the internal layout, arrays to be cleared, a product's direction per state
 struct SwfArgs {

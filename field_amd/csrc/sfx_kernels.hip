@@ -123,7 +123,7 @@ __device__ __forceinline__ float step_scale(const RankScale& sc, double& lncum) 
   float mprev, unused;
   block_step_max2(sc.maxv, sc.step - 1, nullptr, 0, mprev, unused);
   if (!(mprev > 0.f)) mprev = 1.f;  // all-zero propagator: keep it unscaled
-  lncum = l0 + log((double)mprev);
+  lncum = l0 + log((double)(sc.prev_blocked ? mprev * kBlockDown : mprev));
   return 1.f / mprev;
 }
 
@@ -185,7 +185,7 @@ __global__ void k_connect(DevLattice L, const T* __restrict__ Ga, const T* __res
   long long q = site_ordinal();
   if (q >= L.V) return;
   T cfac = T(half);
-  if constexpr (SCALED) cfac = (T)(half * exp(sc.lnv[sc.step] + sc.lnpair[sc.pair] - *sc.ref));
+  if constexpr (SCALED) cfac = (T)connect_factor(sc, half);
   int x, y, z;
   interior_coords(L, q, x, y, z);
   long long r = sidx(L, x, y, z);
@@ -236,12 +236,29 @@ __global__ void k_mol_phi(DevLattice L, const A* __restrict__ acc, const A* __re
   phi_m[r] = v;
 }
 
-__global__ void k_set_ref_pair(double* scal, const double* lna, int ia, const double* lnb, int ib) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) scal[MS_REF] = lna ? lna[ia] + lnb[ib] : 0.0;
+// one wave: the logs of ranks ia and ib, and kAccPower less the powers of two above
+// their maxima
+__global__ void __launch_bounds__(64) k_set_ref_block(double* scal, const unsigned* maxa, const double* lna, int ia,
+                                                      const unsigned* maxb, const double* lnb, int ib) {
+  const int lane = threadIdx.x;
+  float a = __uint_as_float(maxa[(long long)ia * kStepWords + lane * kSlotStride]);
+  float b = lnb ? __uint_as_float(maxb[(long long)ib * kStepWords + lane * kSlotStride]) : 0.f;
+  for (int o = 32; o > 0; o >>= 1) {
+    a = fmaxf(a, __shfl_xor(a, o, 64));
+    b = fmaxf(b, __shfl_xor(b, o, 64));
+  }
+  if (lane) return;
+  // rank 1 does not come out of a blocked launch
+  auto power = [](float m, int rank) {
+    return m > 0.f && m < INFINITY ? ilogbf(m) + 1 - (rank >= 2 ? kBlockPower : 0) : 0;
+  };
+  scal[MS_REF] = lnb ? lna[ia] + lnb[ib] : lna[ia];
+  scal[MS_POW] = kAccPower - power(a, ia) - (lnb ? power(b, ib) : 0);
 }
 
-void launch_set_ref_pair(double* scal, const double* lna, int ia, const double* lnb, int ib, hipStream_t st) {
-  k_set_ref_pair<<<1, 1, 0, st>>>(scal, lna, ia, lnb, ib);
+void launch_set_ref_block(double* scal, const unsigned* maxa, const double* lna, int ia, const unsigned* maxb,
+                          const double* lnb, int ib, hipStream_t st) {
+  k_set_ref_block<<<1, 64, 0, st>>>(scal, maxa, lna, ia, maxb, lnb, ib);
 }
 
 // per-site free-energy density, block partials (SF_MolList1stO.cpp:815-940)

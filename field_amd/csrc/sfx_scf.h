@@ -13,10 +13,10 @@ namespace sfx {
 // Molecule scalars after a sweep from the weighted sum s of its end rank (one
 // thread). Normalisation per freedom: SF_Monomer1stO.cpp:110-130,
 // SF_Homopol1stO.cpp:599-619, SF_Copol1stO.cpp:1242-1275. phib_of(m): the bulk
-// fraction of another molecule.
+// fraction of another molecule. The accumulators carry exp(-ref) 2^power.
 template <class PhibOf>
-__device__ __forceinline__ void mol_scalars(const MolParams& mp, double s, double lnscale, double ref, int nmol,
-                                            PhibOf&& phib_of, double* scal) {
+__device__ __forceinline__ void mol_scalars(const MolParams& mp, double s, double lnscale, double ref, int power,
+                                            int nmol, PhibOf&& phib_of, double* scal) {
   const double lnsum = mp.kind == 3 ? log(s / 6.0) : log(s);  // second order: Lat3D2ndO.cpp:1024
   const double lnGN = lnsum + lnscale;                        // FP32: plus the log-scale of the final rank
   const double N = mp.N;
@@ -49,7 +49,7 @@ __device__ __forceinline__ void mol_scalars(const MolParams& mp, double s, doubl
   scal[MS_LNGN] = lnGN;
   scal[MS_LNC] = lnC;
   scal[MS_PHIB] = phib;
-  scal[MS_PREF] = pref;
+  scal[MS_PREF] = ldexp(pref, -power);
 }
 
 // range_restricted: the constant from the profile's sum s over the box, after mol_scalars
@@ -140,6 +140,7 @@ __device__ __forceinline__ void tmol_scalars(const MolParams& mp, bool any, doub
     d[3] = f * exp(log(mp.theta) - ms[MS_LNGN] - (mp.kind == 0 ? 0.0 : log((double)mp.N)) + ms[MS_REF]);
   else
     d[3] = f * (mp.kind == 0 ? phib : phib / mp.N) * exp(ms[MS_REF]);
+  d[3] = ldexp(d[3], -(int)ms[MS_POW]);
   d[0] = dln;
   if (mp.freedom == SFX_RESTRICTED) {
     d[1] = -dln;

@@ -21,7 +21,10 @@ static __global__ void k_fill_bytes8(unsigned long long* p, long long n) {
 }
 // scal[MS_REF] = factor * lnv[idx]
 static __global__ void k_set_ref(double* scal, const double* lnv, int idx, double factor) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) scal[MS_REF] = factor * lnv[idx];
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    scal[MS_REF] = factor * lnv[idx];
+    scal[MS_POW] = 0.0;
+  }
 }
 // order[i] = ordinal of site i among the (ascending) iteration sites, -1 off them
 static __global__ void k_order(const unsigned char* itmask, const long long* sites, long long nsites, long long M,
@@ -672,6 +675,15 @@ void System::sweep_blocked(int m, bool scaled) {
   RankScale none{nullptr, nullptr, nullptr, nullptr, 0, 0};
   auto fsc = [&](int step, int pair) { return scaled ? RankScale{maxf, lnf, lnf, scal + MS_REF, step, pair} : none; };
   auto bsc = [&](int step, int pair) { return scaled ? RankScale{maxb, lnb, lnf, scal + MS_REF, step, pair} : none; };
+  // launches of one rank between blocked ones: what they read carries kBlockScale
+  auto carried = [&](RankScale sc, int carry) {
+    if (scaled) {
+      sc.prev_blocked = mo.blocked_rank(sc.step - 1);
+      sc.pow = scal + MS_POW;
+      sc.carry = carry;
+    }
+    return sc;
+  };
   auto state_of_rank = [&](int s) { return mo.seq[s - 1]; };
   auto nosplit = [](int) { return false; };
   // the arguments of ranks sa..sb of a chain from the rank in `in`; with an
@@ -697,7 +709,8 @@ void System::sweep_blocked(int m, bool scaled) {
       a.lnpair = lnpair;
       a.ref = scal + MS_REF;
       a.gmax = d_gmax + (size_t)t * kStepWords;
-      a.low = mo.blocked_rank(sa - 1) ? low_word() : nullptr;
+      a.low = low_word();
+      a.carried = mo.blocked_rank(sa - 1);
     }
     a.s0 = sa - 1;
     return a;
@@ -752,7 +765,7 @@ void System::sweep_blocked(int m, bool scaled) {
       }
       go(la, false);
     }
-    if (scaled) launch_set_ref_pair(scal, lnf, h, lnb, N - h, st);
+    if (scaled) launch_set_ref_block(scal, maxf, lnf, h, maxb, lnb, N - h, st);
     const auto F2 = chain_launches(h + 1, N, h + 1, state_of_rank, grid);
     const auto B2 = chain_launches(N - h + 1, N, N - h + 1, bstate, grid);
     int fc = 0, bc = 0;
@@ -841,10 +854,10 @@ void System::sweep_blocked(int m, bool scaled) {
   const double* lnfinal = nullptr;
   int cur = 0;
   if (mo.kind == 1) {
-    if (scaled) k_set_ref<<<1, 1, 0, st>>>(scal, lnf, N, 1.0);
+    if (scaled) launch_set_ref_block(scal, maxf, lnf, N, nullptr, nullptr, 0, st);
     // backward chain: step k holds G_inv of rank N-k+1
     launch_init_rank<T>(L, gp(mo.seq[N - 1]), pp[0], bsc(1, N), st);
-    launch_connect<T, T>(L, pp[0], slot(get(N)), accp(mo.seq[N - 1]), bsc(1, N), 1.0, st);
+    launch_connect<T, T>(L, pp[0], slot(get(N)), accp(mo.seq[N - 1]), carried(bsc(1, N), 1), 1.0, st);
     auto rank_of = [&](int k) { return N - k + 1; };
     chain_blocks(
         2, N, 2, [&](int k) { return mo.seq[rank_of(k) - 1]; },
@@ -865,7 +878,7 @@ void System::sweep_blocked(int m, bool scaled) {
     lnfinal = scaled ? lnb + N : nullptr;
   } else {
     const int h = N / 2;
-    if (scaled) k_set_ref<<<1, 1, 0, st>>>(scal, lnf, h, 2.0);
+    if (scaled) launch_set_ref_block(scal, maxf, lnf, h, maxf, lnf, h, st);
     const T* from = slot(get(h));
     if (plan.c) {
       launch_copy_interior<T>(L, from, pp[0], st);
@@ -873,9 +886,9 @@ void System::sweep_blocked(int m, bool scaled) {
     }
     if (N % 2 == 1) {  // the middle rank meets itself
       const int s = h + 1;
-      launch_prop<T, T>(L, from, gp(mo.seq[s - 1]), pp[1], nullptr, nullptr, fsc(s, 0), st);
+      launch_prop<T, T>(L, from, gp(mo.seq[s - 1]), pp[1], nullptr, nullptr, carried(fsc(s, 0), 0), st);
       cur = 1;
-      launch_connect<T, T>(L, pp[cur], pp[cur], accp(mo.seq[s - 1]), fsc(s, s), 0.5, st);
+      launch_connect<T, T>(L, pp[cur], pp[cur], accp(mo.seq[s - 1]), carried(fsc(s, s), 0), 0.5, st);
       from = pp[cur];
     }
     auto pair_of = [&](int s) { return N - s + 1; };

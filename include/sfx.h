@@ -134,13 +134,13 @@ typedef struct sfx_options {
                              BLOCKED also advance first-order FCC sweeps by four and
                              2-D sweeps by eight ranks per launch (fully stored,
                              chain_schedule AUTO, a curved lattice without mirror2
-                             or radially periodic sides; rank by rank where device memory has no room
-                             for their second accumulators), and run
-                             a 1-D first-order FP64 evaluation in one workgroup
+                             or radially periodic sides; rank by rank where device
+                             memory has no room for their second accumulators), and
+                             run a 1-D first-order FP64 evaluation in one workgroup
                              launch, or above 1024 layers each stretch of a chain's
                              ranks in one (up to 4000 layers). An FP32 evaluation
-                             whose ranks lose more than 2^-32 within a launch is
-                             repeated with one launch per rank */
+                             with ranks that fall below 2^-24 of their launch's input
+                             is repeated with one launch per rank */
   int chain_schedule;     /* SFX_SCHEDULE_AUTO: a first-order chain without mirror
                              symmetry, fully stored, on a blocked lattice advances its
                              forward and backward chains in the same launches (each

@@ -1,12 +1,13 @@
 """FP32 sweeps of several ranks per launch where a chain's weight lies far from
 the lattice maximum of g: a site of u = 0 in a lattice of u = depth, on lattices
 whose step gives a site no weight of its own, so that two ranks lose the factor
-exp(-depth). A launch renormalises only its input; from some 22 kT within one
+exp(-depth). A launch renormalises only its input; from some 17 kT within one
 launch on the evaluation is repeated rank by rank, so every depth has to give
 the FP64 result: rounding of 1e-7 per rank over at most 41 ranks, 2e-5 of the
 largest entry. Depths below and above that line, and ones at which the ranks of
 a launch reach FP32's smallest numbers. A second polymer, without a field, fills
-the lattice.
+the lattice. Strong noise reaches FP32's range in every kernel: there the blocked
+sweeps may be no further off than four times the per-rank ones, or 2e-5.
 """
 import numpy as np
 import pytest
@@ -113,3 +114,25 @@ def test_newton_krylov_steps(sfx, lattice, chain):
     f = G.residual(y, precision="fp32")
     G.solve(x, **opts)
     assert np.array_equal(G.residual(y, precision="fp32"), f)
+
+
+@pytest.mark.parametrize("lattice", LATTICES)
+@pytest.mark.parametrize("sigma", [0.5, 1.0, 1.5])
+@pytest.mark.parametrize("seed", range(4))
+def test_strong_noise(sfx, lattice, sigma, seed):
+    """Also of a molecule whose amount is fixed in a box that its weight avoids."""
+    lat = LATTICES[lattice]
+    chi = np.array([[0.0, 0.8, 0.4], [0.8, 0.0, 0.6], [0.4, 0.6, 0.0]])
+    far = tuple(max(1, n // 4) for n in lat.n_layers) + (1,) * (3 - len(lat.n_layers))
+    box = MoleculeSpec("b", "(A)26", "range_restricted", range_lo=far, range_hi=far, phi_range=1.0)
+    for molecules, products in (([MoleculeSpec("p", "(A)20(B)21", "restricted", theta=9.0)], True), ([box], False)):
+        sysd = SystemSpec(("A", "B", "S"), chi, molecules + [MoleculeSpec("q", "(B)9", "free", phibulk=0.05),
+                                                             MoleculeSpec("s", "(S)1", "solvent")])
+        G, P = sfx.System(lat, sysd), sfx.System(lat, sysd, sweep_kernel="per_rank")
+        rng = np.random.default_rng(seed)
+        x, w = rng.normal(0, sigma, G.nvar), rng.normal(0, 1, G.nvar)
+        for what in ("residual", "jvp", "vjp") if products else ("residual",):
+            arg = (x,) if what == "residual" else (x, w)
+            ref = getattr(G, what)(*arg)
+            a, b = (np.abs(getattr(S, what)(*arg, precision="fp32") - ref).max() for S in (G, P))
+            assert a <= max(4 * b, 2e-5 * np.abs(ref).max()) or not np.isfinite(b), (what, a, b)
