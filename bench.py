@@ -165,7 +165,7 @@ def batch_leg(args):
             "algorithmic_bytes": nbytes,
             "achieved_GBs": round(nbytes / st["seconds"] / 1e9, 1),
             "frac_of_hbm_peak": round(nbytes / st["seconds"] / 1e9 / PEAK_HBM_GBS, 4),
-            "bound": "latency: a chain of N barriered rank steps per residual in each workgroup"}
+            "bound": "latency: a chain of N dependent rank steps per residual in each workgroup"}
 
 
 def transfer_compare(args):

@@ -1,7 +1,7 @@
 /*
  * orc.h -- ORACLE (test infrastructure only). FP64 CPU restatement of the
- * reference's Scheutjens-Fleer hot path. Loaded by tests/, smoke() (as the
- * checker) and bench.py's cpu_baseline leg only; never by the product path.
+ * reference's Scheutjens-Fleer hot path. Loaded by tests/, smoke() (to
+ * compare with) and bench.py's cpu_baseline leg only; never by the product path.
  */
 #ifndef ORC_H
 #define ORC_H

@@ -2,7 +2,7 @@
 
 ctypes access to liborc.so, the FP64 CPU restatement of the reference's SCF
 hot path. Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline
-leg import this module: as the checker, or as the timed CPU baseline.
+leg import this module: to compare with, or as the timed CPU baseline.
 """
 from __future__ import annotations
 

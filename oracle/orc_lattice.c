@@ -1,7 +1,7 @@
 /*
  * orc_lattice.c -- ORACLE (test infrastructure only): FP64 CPU restatement of
  * the reference's lattice layer. Only tests/, __graft_entry__.smoke() and
- * bench.py's cpu_baseline leg may load it, and only as the checker or the
+ * bench.py's cpu_baseline leg may load it, and only to compare with or as the
  * timed CPU baseline; the product path never does.
  *
  * Site arrays use the reference layout shifted to 0-based indices:
