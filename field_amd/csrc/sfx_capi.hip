@@ -49,13 +49,23 @@ template <class F>
 int guarded_fit(sfx_system* s, F&& f) {
   return guarded([&] {
     SFX_REQUIRE(s, SFX_E_INVALID, "NULL argument");
+    System& S = s->s;
+    auto work = [&] {
+      try {
+        f();
+      } catch (...) {  // a low rank of what it had launched is not the next call's
+        (void)hipStreamSynchronize(S.stream);
+        (void)S.took_low();
+        throw;
+      }
+    };
     try {
-      f();
+      work();
       return;
     } catch (const Error& e) {
-      if (e.code != SFX_E_OOM || !s->s.drop_blocked()) throw;
+      if (e.code != SFX_E_OOM || !S.drop_blocked()) throw;
     }
-    f();
+    work();
   });
 }
 }  // namespace

@@ -136,3 +136,20 @@ def test_strong_noise(sfx, lattice, sigma, seed):
             ref = getattr(G, what)(*arg)
             a, b = (np.abs(getattr(S, what)(*arg, precision="fp32") - ref).max() for S in (G, P))
             assert a <= max(4 * b, 2e-5 * np.abs(ref).max()) or not np.isfinite(b), (what, a, b)
+
+
+def test_a_refused_call_leaves_nothing_behind(sfx):
+    """A product that is refused after its sweep has found low ranks: the next
+    evaluation, of an ordinary field, is by blocked launches, to the same bits."""
+    lat = LATTICES["2d"]
+    box = MoleculeSpec("b", "(A)26", "range_restricted", range_lo=(6, 15, 1), range_hi=(9, 20, 1), phi_range=1.0)
+    sysd = SystemSpec(("A", "S"), np.array([[0.0, 0.4], [0.4, 0.0]]), [box, MoleculeSpec("s", "(S)1", "solvent")])
+    G = sfx.System(lat, sysd)
+    rng = np.random.default_rng(2)
+    x, steep = rng.normal(0, 0.1, G.nvar), rng.normal(0, 3.0, G.nvar)
+    f = G.residual(x, precision="fp32")
+    with pytest.raises(sfx.SFError):
+        G.jvp(steep, x, precision="fp32")
+    assert np.array_equal(G.residual(x, precision="fp32"), f)
+    P = sfx.System(lat, sysd, sweep_kernel="per_rank")  # the two paths can be told apart
+    assert not np.array_equal(P.residual(x, precision="fp32"), f)
